@@ -947,19 +947,23 @@ bool dc_small_supported(int n_units, int region, int k_eff, int group, int hd, b
     return (int64_t)n_units * p.bpu <= (int64_t)occ;
 }
 
+// Both sizes below cover every region of up to `region` rows, not this one alone: a caller sizes
+// its workspace for the longest region its store can hold, and a shorter one may have more blocks
+// per unit (32700 rows of 8 units: 64 blocks; 32828 rows: 43 blocks of three steps).
 size_t dc_small_workspace_bytes(int n_units, int region, int group, int hd) {
-    const SmallPlan p = plan_small(n_units, region);
-    if (!p.ok) return 0;
-    return carve_attn(nullptr, n_units, group, hd, p.bpu).bytes;
+    if (n_units < 1 || n_units > kSmallBlocks || region < 1) return 0;
+    const int steps = (region + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
+    const int bpu = kSmallBlocks / n_units;
+    return carve_attn(nullptr, n_units, group, hd, bpu < steps ? bpu : steps).bytes;
 }
 
 // The route's own candidate lists: one packed (key, id) word per region row.  They are not shared
 // with the lists of the other routes, so a workspace whose state is ready stays ready for this
 // route whichever route the calls in between took.
 size_t dc_small_cand_bytes(int n_units, int region) {
-    const SmallPlan p = plan_small(n_units, region);
-    if (!p.ok) return 0;
-    return dc_align_up((size_t)n_units * (size_t)region * 8, 256);
+    if (n_units < 1 || n_units > kSmallBlocks || region < 1) return 0;
+    const int64_t most = kSmallTotalRows / n_units;  // longer regions take other routes
+    return dc_align_up((size_t)n_units * (size_t)(region < most ? region : most) * 8, 256);
 }
 
 namespace {

@@ -307,3 +307,14 @@ def test_snapshot_roundtrip_many_nodes(tmp_path):
     snap = snapshot.read(path)
     assert np.array_equal(snap["keys"], keys) and np.array_equal(snap["vals"], vals)
     assert snap["num_nodes"] == n and snap["options"]["n_max"] == n
+
+
+@pytest.mark.parametrize("n_units", [1, 8, 12, 64, 512])
+def test_layer_workspace_of_a_long_region_covers_every_shorter_one(n_units):
+    """DiffCache sizes its workspace once, for the longest region its store can hold; the blocks per unit
+    of the one-kernel route fall when the region grows past a multiple of its grid (8 units: 32768 rows)."""
+    from diffcache_amd import _hip
+    lib = _hip.lib
+    regions = sorted({r + d for r in (256, 1024, 4096, 16384, 32768, 40960, 65536, 81920, 131072) for d in (-68, 0, 1, 60)})
+    need = [lib.dc_layer_workspace_bytes(n_units, r, 1024, 4, 128, 1024 + 4 + 128 + 1) for r in regions]
+    assert all(a <= b for a, b in zip(need, need[1:]))
