@@ -29,7 +29,8 @@ SYMBOLS = (
     "dc_version", "dc_last_error", "dc_group_mean_bf16", "dc_score_bf16",
     "dc_topk_workspace_bytes", "dc_topk_select", "dc_gather_rows_bf16",
     "dc_attn_workspace_bytes", "dc_gather_attn_bf16", "dc_gather_attn_static_bf16", "dc_append_kv_bf16",
-    "dc_step_advance", "dc_step_state_advance", "dc_step_state_rollover", "dc_ingest_kv_bf16", "dc_layer_workspace_bytes", "dc_decode_layer",
+    "dc_step_advance", "dc_step_state_advance", "dc_step_state_rollover", "dc_ingest_kv_bf16",
+    "dc_prefill_workspace_bytes", "dc_prefill_layer_bf16", "dc_layer_workspace_bytes", "dc_decode_layer",
     "dc_decode_layer_status", "dc_set_wait_limit", "dc_decode_layer_route", "dc_last_route",
     "dc_decode_layer_errors", "dc_one_kernel_guard",
     "dc_pq_build_lut", "dc_pq_adc_scan", "dc_score_gathered_bf16", "dc_compose_idx",
@@ -67,6 +68,21 @@ class LayerArgs(C.Structure):
     ]
 
 
+class PrefillArgs(C.Structure):
+    """struct dc_prefill_args of include/diffcache_hip.h"""
+    _fields_ = [
+        ("k_src", C.c_void_p), ("v_src", C.c_void_p), ("k_store", C.c_void_p), ("v_store", C.c_void_p),
+        ("k_buf", C.c_void_p), ("v_buf", C.c_void_p), ("codes", C.c_void_p), ("scale", C.c_void_p),
+        ("resid", C.c_void_p), ("r_sq", C.c_void_p), ("step_state", C.c_void_p), ("workspace", C.c_void_p),
+        ("workspace_bytes", C.c_size_t),
+        ("batch_stride", C.c_int64), ("head_stride", C.c_int64), ("row_stride", C.c_int64),
+        ("buf_batch_stride", C.c_int64), ("buf_head_stride", C.c_int64), ("buf_row_stride", C.c_int64),
+        ("code_batch_stride", C.c_int64), ("code_head_stride", C.c_int64), ("code_row_stride", C.c_int64),
+        ("n_b", C.c_int), ("n_h", C.c_int), ("seq", C.c_int), ("hd", C.c_int),
+        ("n_prefix", C.c_int), ("n_suffix", C.c_int),
+    ]
+
+
 def _load() -> C.CDLL:
     if not os.path.exists(LIB_PATH):
         raise ImportError(
@@ -92,6 +108,8 @@ def _load() -> C.CDLL:
         "dc_step_state_advance": (i, [p, i, i, p]),
         "dc_step_state_rollover": (i, [p, i, i, p]),
         "dc_ingest_kv_bf16": (i, [p, p, i, i, i, i, i64, i64, i64, i64, p]),
+        "dc_prefill_workspace_bytes": (sz, [i, i]),
+        "dc_prefill_layer_bf16": (i, [C.POINTER(PrefillArgs), p]),
         "dc_layer_workspace_bytes": (sz, [i, i, i, i, i, i]),
         "dc_decode_layer": (i, [C.POINTER(LayerArgs), p]),
         "dc_decode_layer_status": (i, [C.POINTER(LayerArgs), p]),
@@ -522,6 +540,59 @@ def ingest_kv(store: torch.Tensor, src: torch.Tensor, dst_pos: int = 0) -> None:
         raise DiffCacheError(f"rows [{dst_pos}, {dst_pos + seq}) outside the store of {n_max} rows")
     _check(lib.dc_ingest_kv_bf16(_dev(store, "store"), _dev(src, "src"), b, seq, h, hd, dst_pos, sb, sh,
                                  sr, _stream()))
+
+
+def prefill_layer(store_k: torch.Tensor, store_v: torch.Tensor, k_src: torch.Tensor, v_src: torch.Tensor,
+                  n_prefix: int, n_suffix: int, buf_k: Optional[torch.Tensor] = None,
+                  buf_v: Optional[torch.Tensor] = None, sketch: Optional[Sketch] = None,
+                  r_sq: Optional[torch.Tensor] = None, step_state: Optional[torch.Tensor] = None,
+                  workspace: Optional[torch.Tensor] = None) -> None:
+    """dc_prefill_layer_bf16: k_src, v_src (b, seq, h, hd) bf16 into rows [0, seq) of the stores; the prefix
+    and suffix rows also to rows [0, n_prefix + n_suffix) of ``buf_k`` / ``buf_v`` (b, h, rows, hd); the sketch
+    of the rows between them; ``r_sq`` (h) fp32 receives the largest squared key norm of every head."""
+    sb, sh, sr = _store_strides(store_k)
+    if _store_strides(store_v) != (sb, sh, sr):
+        raise DiffCacheError("K and V stores must share their strides")
+    b, h, n_max, hd = store_k.shape
+    k_src, v_src = k_src.contiguous(), v_src.contiguous()
+    for src in (k_src, v_src):
+        if src.dtype != torch.bfloat16 or src.dim() != 4 or src.shape[0] != b or src.shape[2] != h \
+                or src.shape[3] != hd or src.shape[1] != k_src.shape[1]:
+            raise DiffCacheError("k_src and v_src must be (b, seq, h, hd) bf16 tensors matching the store")
+    seq = k_src.shape[1]
+    if seq > n_max or n_prefix < 0 or n_suffix < 0 or n_prefix + n_suffix > seq:
+        raise DiffCacheError(f"{seq} rows ({n_prefix} prefix, {n_suffix} suffix) do not fit the store of {n_max} rows")
+    a = PrefillArgs()
+    a.k_src, a.v_src = _dev(k_src, "k_src"), _dev(v_src, "v_src")
+    a.k_store, a.v_store = _dev(store_k, "store_k"), _dev(store_v, "store_v")
+    a.batch_stride, a.head_stride, a.row_stride = sb, sh, sr
+    a.n_b, a.n_h, a.seq, a.hd, a.n_prefix, a.n_suffix = b, h, seq, hd, n_prefix, n_suffix
+    if buf_k is not None and n_prefix + n_suffix > 0:
+        db, dh, dr = _store_strides(buf_k)
+        if _store_strides(buf_v) != (db, dh, dr) or buf_k.shape != buf_v.shape or buf_k.shape[0] != b \
+                or buf_k.shape[1] != h or buf_k.shape[2] < n_prefix + n_suffix or buf_k.shape[3] != hd:
+            raise DiffCacheError("buf_k / buf_v must be (b, h, >= n_prefix + n_suffix, hd) tensors of equal strides")
+        a.k_buf, a.v_buf = _dev(buf_k, "buf_k"), _dev(buf_v, "buf_v")
+        a.buf_batch_stride, a.buf_head_stride, a.buf_row_stride = db, dh, dr
+    if sketch is not None:
+        c = sketch.codes
+        if c.shape != store_k.shape:
+            raise DiffCacheError("the sketch does not belong to this store")
+        need = int(lib.dc_prefill_workspace_bytes(b * h, hd))
+        if workspace is None:
+            workspace = torch.empty((need,), dtype=torch.uint8, device=store_k.device)
+        a.codes, a.scale, a.resid = _dev(c, "codes"), _dev(sketch.scale, "scale"), _dev(sketch.resid, "resid")
+        a.code_batch_stride, a.code_head_stride, a.code_row_stride = c.stride(0), c.stride(1), c.stride(2)
+        a.workspace, a.workspace_bytes = _dev(workspace, "workspace"), workspace.numel()
+    if r_sq is not None:
+        if r_sq.dtype != torch.float32 or r_sq.numel() < h or not r_sq.is_contiguous():
+            raise DiffCacheError("r_sq must be a contiguous fp32 tensor of h elements")
+        a.r_sq = _dev(r_sq, "r_sq")
+    if step_state is not None:
+        if step_state.dtype != torch.int32 or step_state.numel() < 4 or not step_state.is_contiguous():
+            raise DiffCacheError("the step state must be a contiguous int32 tensor of 4 elements in GPU memory")
+        a.step_state = _dev(step_state, "step_state")
+    _check(lib.dc_prefill_layer_bf16(C.byref(a), _stream()))
 
 
 def layer_workspace_bytes(n_units: int, n_region: int, budget: int, group: int, hd: int,

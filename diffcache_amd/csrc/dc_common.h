@@ -58,6 +58,10 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
                           int n_sink, int64_t recent_lo, int n_recent, const int32_t *n_recent_dev, int64_t ksb,
                           int64_t ksh, int64_t ksr, int64_t vsb, int64_t vsh, int64_t vsr, float scale,
                           void *workspace, size_t workspace_bytes, void *stream, const int32_t *recent_lo_dev);
+// sketch.hip: the quantising pass of dc_sketch_build_bf16
+int dc_sketch_quantise_launch(const char *who, const void *k, uint8_t *codes, const float *scale, float *resid,
+                              int n_units, int n_h, int n_rows, int hd, int64_t sb, int64_t sh, int64_t sr, int64_t cb,
+                              int64_t ch, int64_t cr, int scale_is_amax, float *scale_out, void *stream);
 // small.hip: a whole decode layer in one kernel, for short contexts
 bool dc_small_supported(int n_units, int region, int k_eff, int group, int hd, bool has_sketch);
 size_t dc_small_workspace_bytes(int n_units, int region, int group, int hd);

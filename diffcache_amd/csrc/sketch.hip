@@ -67,16 +67,17 @@ __global__ __launch_bounds__(kThreads) void sketch_absmax_kernel(
 }
 
 // quantise rows with a_d = amax_d / 127 (scale_is_amax) or a_d = scale_d, write the
-// codes, and raise resid_d to the largest |k - a c| seen
+// codes, and raise resid_d to the largest |k - a c| seen; scale_out (or null) receives a_d
 template <int HD>
 __global__ __launch_bounds__(kThreads) void sketch_quantise_kernel(
     const uint16_t *__restrict__ K, uint8_t *__restrict__ C, const float *__restrict__ scale,
     uint32_t *__restrict__ resid_bits, int n_h, int n_rows, int64_t sb, int64_t sh, int64_t sr, int64_t cb,
-    int64_t ch, int64_t cr, int blocks_per_unit, int scale_is_amax) {
+    int64_t ch, int64_t cr, int n_units, int rows_per_block, int scale_is_amax, float *__restrict__ scale_out) {
     constexpr int LPR = HD / 8;
     constexpr int GROUPS = kThreads / LPR;
+    constexpr int kInFlight = 4;  // rows of a lane group requested together
     __shared__ uint32_t smax[GROUPS][HD];
-    const int unit = blockIdx.x / blocks_per_unit, blk = blockIdx.x % blocks_per_unit;
+    const int unit = blockIdx.x % n_units, blk = blockIdx.x / n_units;
     const int b = unit / n_h, h = unit % n_h;
     const int grp = threadIdx.x / LPR, col = threadIdx.x % LPR;
     const uint16_t *Ku = K + b * sb + h * sh + col * 8;
@@ -89,28 +90,44 @@ __global__ __launch_bounds__(kThreads) void sketch_quantise_kernel(
         inv[i] = a[i] > 0.f ? 1.0f / a[i] : 0.f;
         res[i] = 0.f;
     }
-    const int64_t r0 = (int64_t)blk * kRowsPerBlock;
-    int64_t r1 = r0 + kRowsPerBlock;
-    if (r1 > n_rows) r1 = n_rows;
-    for (int64_t r = r0 + grp; r < r1; r += GROUPS) {
-        const uint4 w = dc_load_stream16(Ku + r * sr);
-        const float kv[8] = {dc_bf16_lo(w.x), dc_bf16_hi(w.x), dc_bf16_lo(w.y), dc_bf16_hi(w.y),
-                             dc_bf16_lo(w.z), dc_bf16_hi(w.z), dc_bf16_lo(w.w), dc_bf16_hi(w.w)};
-        uint32_t code[8];
+    if (scale_out && blk == 0 && grp == 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            float c = rintf(kv[i] * inv[i]);
-            c = c > 127.f ? 127.f : (c < -127.f ? -127.f : c);
-            if (!(c == c)) c = 0.f;  // NaN key or 0 * inf
-            const float e = fabsf(fmaf(-a[i], c, kv[i]));
-            // a NaN residual must poison the bound, not vanish in the max
-            if (!(e <= res[i])) res[i] = (e == e) ? e : __builtin_inff();
-            code[i] = (uint32_t)((int)c + 128);
+        for (int i = 0; i < 8; ++i) scale_out[(int64_t)unit * HD + col * 8 + i] = a[i];
+    }
+    const int64_t r0 = (int64_t)blk * rows_per_block;
+    int64_t r1 = r0 + rows_per_block;
+    if (r1 > n_rows) r1 = n_rows;
+    for (int64_t rb = r0 + grp; rb < r1; rb += GROUPS * kInFlight) {
+        uint4 wv[kInFlight];
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            int64_t r = rb + (int64_t)u * GROUPS;
+            r = r < r1 ? r : r1 - 1;
+            wv[u] = dc_load_stream16(Ku + r * sr);
         }
-        uint2 packed;
-        packed.x = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
-        packed.y = code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24);
-        dc_store_stream8(Cu + r * cr, packed);
+#pragma unroll
+        for (int u = 0; u < kInFlight; ++u) {
+            const int64_t r = rb + (int64_t)u * GROUPS;
+            if (r >= r1) break;
+            const uint4 w = wv[u];
+            const float kv[8] = {dc_bf16_lo(w.x), dc_bf16_hi(w.x), dc_bf16_lo(w.y), dc_bf16_hi(w.y),
+                                 dc_bf16_lo(w.z), dc_bf16_hi(w.z), dc_bf16_lo(w.w), dc_bf16_hi(w.w)};
+            uint32_t code[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float c = rintf(kv[i] * inv[i]);
+                c = c > 127.f ? 127.f : (c < -127.f ? -127.f : c);
+                if (!(c == c)) c = 0.f;  // NaN key or 0 * inf
+                const float e = fabsf(fmaf(-a[i], c, kv[i]));
+                // a NaN residual must poison the bound, not vanish in the max
+                if (!(e <= res[i])) res[i] = (e == e) ? e : __builtin_inff();
+                code[i] = (uint32_t)((int)c + 128);
+            }
+            uint2 packed;
+            packed.x = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
+            packed.y = code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24);
+            dc_store_stream8(Cu + r * cr, packed);
+        }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) smax[grp][col * 8 + i] = __float_as_uint(res[i]);
@@ -128,6 +145,30 @@ __global__ void sketch_finalise_kernel(float *scale, int64_t n) {
 }
 
 }  // namespace
+
+// The quantising pass on its own: scale holds amax_d (scale_is_amax) or a_d, resid is raised from
+// what it holds.  Arguments are the caller's to check.
+int dc_sketch_quantise_launch(const char *who, const void *k, uint8_t *codes, const float *scale, float *resid,
+                              int n_units, int n_h, int n_rows, int hd, int64_t sb, int64_t sh, int64_t sr, int64_t cb,
+                              int64_t ch, int64_t cr, int scale_is_amax, float *scale_out, void *stream) {
+    // rows per block: as many as leave about 2048 blocks, from 256 (a block ends with an LDS pass and
+    // HD atomics) to kRowsPerBlock
+    int64_t rpb = (int64_t)n_units * n_rows / 2048 / 256 * 256;
+    rpb = rpb < 256 ? 256 : (rpb > kRowsPerBlock ? kRowsPerBlock : rpb);
+    const int64_t blocks = ((int64_t)n_rows + rpb - 1) / rpb * n_units;
+    DC_REQUIRE(blocks < (1ll << 31), "%s: grid too large", who);
+    const dim3 grid((unsigned)blocks);
+    hipStream_t st = (hipStream_t)stream;
+#define DC_LAUNCH_SKQ(HD)                                                                                   \
+    hipLaunchKernelGGL(sketch_quantise_kernel<HD>, grid, dim3(kThreads), 0, st, (const uint16_t *)k, codes, scale, \
+                       (uint32_t *)resid, n_h, n_rows, sb, sh, sr, cb, ch, cr, n_units, (int)rpb, scale_is_amax, scale_out)
+    if (hd == 64) DC_LAUNCH_SKQ(64);
+    else if (hd == 128) DC_LAUNCH_SKQ(128);
+    else DC_LAUNCH_SKQ(256);
+#undef DC_LAUNCH_SKQ
+    DC_CHECK_LAUNCH(who);
+    return DC_OK;
+}
 
 extern "C" int dc_sketch_build_bf16(const void *k, uint8_t *codes, float *scale, float *resid, int n_b,
                                     int n_h, int n_rows, int hd, int64_t sb, int64_t sh, int64_t sr,
@@ -155,20 +196,19 @@ extern "C" int dc_sketch_build_bf16(const void *k, uint8_t *codes, float *scale,
     }
     if (bpu == 0) return DC_OK;
     const dim3 grid((unsigned)(n_units * bpu));
-#define DC_LAUNCH_SKB(HD)                                                                               \
-    do {                                                                                                \
-        if (!keep_scale)                                                                                \
-            hipLaunchKernelGGL(sketch_absmax_kernel<HD>, grid, dim3(kThreads), 0, st, (const uint16_t *)k, \
-                               (uint32_t *)scale, n_h, n_rows, sb, sh, sr, (int)bpu);                   \
-        hipLaunchKernelGGL(sketch_quantise_kernel<HD>, grid, dim3(kThreads), 0, st, (const uint16_t *)k, \
-                           codes, scale, (uint32_t *)resid, n_h, n_rows, sb, sh, sr, cb, ch, cr, (int)bpu, \
-                           keep_scale ? 0 : 1);                                                         \
-    } while (0)
-    if (hd == 64) DC_LAUNCH_SKB(64);
-    else if (hd == 128) DC_LAUNCH_SKB(128);
-    else DC_LAUNCH_SKB(256);
+#define DC_LAUNCH_SKB(HD)                                                                            \
+    hipLaunchKernelGGL(sketch_absmax_kernel<HD>, grid, dim3(kThreads), 0, st, (const uint16_t *)k,   \
+                       (uint32_t *)scale, n_h, n_rows, sb, sh, sr, (int)bpu)
+    if (!keep_scale) {
+        if (hd == 64) DC_LAUNCH_SKB(64);
+        else if (hd == 128) DC_LAUNCH_SKB(128);
+        else DC_LAUNCH_SKB(256);
+        DC_CHECK_LAUNCH(who);
+    }
 #undef DC_LAUNCH_SKB
-    DC_CHECK_LAUNCH(who);
+    const int rc = dc_sketch_quantise_launch(who, k, codes, scale, resid, (int)n_units, n_h, n_rows, hd, sb, sh, sr, cb, ch,
+                                             cr, keep_scale ? 0 : 1, nullptr, stream);
+    if (rc) return rc;
     if (!keep_scale) {
         hipLaunchKernelGGL(sketch_finalise_kernel, sgrid, dim3(256), 0, st, scale, n_sc);
         DC_CHECK_LAUNCH(who);

@@ -79,6 +79,23 @@ def _as_bf16(x: ArrayLike, device: torch.device) -> torch.Tensor:
     return t.to(device, non_blocking=True)
 
 
+class DeviceRSq:
+    """The largest squared key norm of every head, as a prefill left it on the device.  It is part of what a
+    snapshot records and nothing on the decode path asks for it, so it crosses to the host when it is first
+    read instead of holding a prefill up once per layer.  Rounded to bf16, the type the reference's
+    reduction over bf16 keys returns (src/diffcache/kvcache/diffcache.py:151-156)."""
+
+    def __init__(self, values: torch.Tensor) -> None:
+        self._values: Optional[torch.Tensor] = values
+        self._list: List[float] = []
+
+    def tolist(self) -> List[float]:
+        if self._values is not None:
+            self._list = self._values.to(torch.bfloat16).tolist()
+            self._values = None
+        return list(self._list)
+
+
 class DiffCacheHIP:
     def __init__(self, bsz: int, q_head_num: int, kv_head_num: int, head_dim: int, **kwargs) -> None:
         opt = dict(_DEFAULTS)
@@ -96,7 +113,7 @@ class DiffCacheHIP:
         self.bsz, self.q_head_num, self.kv_head_num, self.head_dim = bsz, q_head_num, kv_head_num, head_dim
         self.max_ctx_len = int(opt["max_ctx_len"])
         self.m, self.ef_cons = int(opt["m"]), int(opt["ef_cons"])
-        self.r_sq: List[float] = list(opt["r_sq"]) if opt["r_sq"] is not None else [4.0] * kv_head_num
+        self.r_sq = opt["r_sq"] if opt["r_sq"] is not None else [4.0] * kv_head_num
         self.batch_search = bool(opt["batch_search"])
         self.name = str(opt["name"])
         self.use_bruteforce = bool(opt["use_bruteforce"])   # the scan here is always exact
@@ -124,6 +141,16 @@ class DiffCacheHIP:
         # optional 8-bit sketch of the keys: queries scan it instead of the bf16 rows and
         # rescore the rows that can still matter; the ids are the same
         self.sketch: Optional[hip.Sketch] = hip.Sketch(self.keys) if opt["key_sketch"] else None
+
+    @property
+    def r_sq(self) -> List[float]:
+        if isinstance(self._r_sq, DeviceRSq):
+            self._r_sq = self._r_sq.tolist()
+        return self._r_sq
+
+    @r_sq.setter
+    def r_sq(self, value) -> None:
+        self._r_sq = value if isinstance(value, DeviceRSq) else list(value)
 
     def _resketch(self) -> None:
         if self.sketch is not None and self.ctx_len > 0:

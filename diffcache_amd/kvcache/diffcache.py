@@ -64,7 +64,7 @@ from typing import List, Optional
 import torch
 
 from .. import _hip as hip
-from ..data_layer import DiffCacheHIP, init_metrics
+from ..data_layer import DeviceRSq, DiffCacheHIP, init_metrics
 
 
 class DiffCache:
@@ -152,6 +152,8 @@ class DiffCache:
             self.sketch = [hip.Sketch(self.kstore[l], codes=self._cslab[l]) for l in range(num_layers)]
 
         n_units = batch_size * num_kv_heads
+        self._prefill_ws = torch.empty((int(hip.lib.dc_prefill_workspace_bytes(n_units, head_dim)),),
+                                       device=self.device, dtype=torch.uint8)
         self.group = num_q_heads // num_kv_heads
         # group-mean query of the current layer (the reference's pinned qbuf_cpu, diffcache.py:80)
         self.qbuf = torch.zeros((batch_size, num_kv_heads, head_dim), device=self.device, dtype=torch.bfloat16)
@@ -191,6 +193,18 @@ class DiffCache:
         init_metrics()
 
     # ------------------------------------------------------------------ helpers
+    @property
+    def r_sq(self) -> List[List[float]]:
+        """Largest squared key norm per layer and head (waits for the device after a prefill)."""
+        for layer_idx, value in enumerate(self._r_sq):
+            if isinstance(value, DeviceRSq):
+                self._r_sq[layer_idx] = value.tolist()
+        return self._r_sq
+
+    @r_sq.setter
+    def r_sq(self, value) -> None:
+        self._r_sq = list(value)
+
     def _region(self):
         lo = self.kvbuf_prefix_len
         return lo, lo + self.retrieval_region_len
@@ -282,33 +296,25 @@ class DiffCache:
         """key_states / value_states (bsz, seq_len, num_kv_heads, head_dim) bf16 on the
         GPU (diffcache.py:149-184)."""
         seq_len = key_states.size(1)
-        hip.require(seq_len <= self.max_length, "prompt longer than max_length")
-
-        # r_sq from the prefill keys, as the reference does; only the graph build needed it
-        r_sq = torch.einsum("bshd,bshd->bsh", key_states, key_states).max(dim=1).values.max(dim=0).values.tolist()
-        self.r_sq[layer_idx] = r_sq
-
-        # all rows into the store, (b, s, h, d) -> (b, h, s, d)
-        hip.ingest_kv(self.kstore[layer_idx], key_states, 0)
-        hip.ingest_kv(self.vstore[layer_idx], value_states, 0)
-
+        hip.require(0 < seq_len <= self.max_length, "the prompt is empty or longer than max_length")
         prefix_len = min(self._prefix0, seq_len)                    # diffcache.py:163
         suffix_len = min(self._suffix0, seq_len - prefix_len)       # diffcache.py:169
-        self.kvbuf_prefix_len = prefix_len
-        self.retrieval_region_len = seq_len - prefix_len - suffix_len
-        self._set_suffix_len(suffix_len)
-        self._store_suffix_rows = suffix_len
-        if self.key_sketch and self.retrieval_region_len > 0:
-            self.sketch[layer_idx].build(self.kstore[layer_idx], prefix_len, self.retrieval_region_len)
-
-        # prefix and suffix rows of the assembled buffer (diffcache.py:164-171)
+        hip.require(suffix_len <= self.kvbuf_suffix_maxlen, "kvbuf_suffix_len exceeds kvbuf_suffix_maxlen")
+        region = seq_len - prefix_len - suffix_len
+        # One call: all rows into the store, (b, s, h, d) -> (b, h, s, d); the sketch of the region; the
+        # prefix and suffix rows of the assembled buffer (diffcache.py:164-171); r_sq of the prompt's
+        # keys (which only the reference's graph build needs; here snapshots record it); the step state
+        r_sq = torch.empty((self.num_kv_heads,), device=self.device, dtype=torch.float32)
         b0 = self.retrieval_budget
-        ks, vs = self.kstore[layer_idx], self.vstore[layer_idx]
-        self.kbuf[layer_idx][:, :, b0:b0 + prefix_len].copy_(ks[:, :, :prefix_len])
-        self.vbuf[layer_idx][:, :, b0:b0 + prefix_len].copy_(vs[:, :, :prefix_len])
-        s0 = seq_len - suffix_len
-        self.kbuf[layer_idx][:, :, b0 + prefix_len:b0 + prefix_len + suffix_len].copy_(ks[:, :, s0:seq_len])
-        self.vbuf[layer_idx][:, :, b0 + prefix_len:b0 + prefix_len + suffix_len].copy_(vs[:, :, s0:seq_len])
+        hip.prefill_layer(self.kstore[layer_idx], self.vstore[layer_idx], key_states, value_states, prefix_len,
+                          suffix_len, self.kbuf[layer_idx][:, :, b0:], self.vbuf[layer_idx][:, :, b0:],
+                          sketch=self.sketch[layer_idx] if region > 0 else None, r_sq=r_sq, step_state=self._state,
+                          workspace=self._prefill_ws)
+        self._r_sq[layer_idx] = DeviceRSq(r_sq)
+        self.kvbuf_prefix_len = prefix_len
+        self.retrieval_region_len = region
+        self.kvbuf_suffix_len = suffix_len
+        self._store_suffix_rows = suffix_len
 
         self._bind_data_layer(layer_idx)
         return key_states, value_states
@@ -320,7 +326,7 @@ class DiffCache:
         self.data_layers[layer_idx] = DiffCacheHIP(
             bsz=self.batch_size, q_head_num=self.num_q_heads, kv_head_num=self.num_kv_heads,
             head_dim=self.head_dim, max_ctx_len=n, m=self.nsw_m, ef_cons=self.nsw_ef_cons,
-            r_sq=self.r_sq[layer_idx], name=f"l{layer_idx:03d}",
+            r_sq=self._r_sq[layer_idx], name=f"l{layer_idx:03d}",
             attn_mass_threshold=self.attn_mass_threshold, k_check_seq=self.k_check_seq,
             key_mode=self.key_mode, device=str(self.device),
             storage=(self.kstore[layer_idx][:, :, lo:hi], self.vstore[layer_idx][:, :, lo:hi]))

@@ -322,6 +322,40 @@ int dc_ingest_kv_bf16(void *store, const void *src, int n_b, int seq, int n_h, i
                       int64_t row_stride, void *stream);
 
 /*
+ * A whole prompt into one layer of a cache: dc_ingest_kv_bf16 of K and V to rows [0, seq) of the
+ * store, the sketch of the retrieval region [n_prefix, seq - n_suffix) as dc_sketch_build_bf16
+ * (keep_scale == 0) makes it, the prefix and suffix rows of the assembled buffer, the largest
+ * squared key norm of every head and the step state, from one pass over V and two over K.
+ *   k_src, v_src   (n_b, seq, n_h, hd) bf16, contiguous
+ *   k_buf, v_buf   NULL, or the assembled buffer at the row of its first prefix row: rows
+ *                  [0, n_prefix) and [seq - n_suffix, seq) go to rows [0, n_prefix + n_suffix) there
+ *   codes, scale, resid  NULL, or the sketch of the store (row 0 = store row 0) and its
+ *                  (n_b*n_h, hd) scales and bounds; strides of the codes in bytes
+ *   r_sq           NULL, or (n_h) fp32: max over batch and rows of sum_d k_d^2 (fp32 sums)
+ *   step_state     NULL, or a dc_step_state: n_recent, region_hi and append_pos are set
+ *   workspace      dc_prefill_workspace_bytes(n_b*n_h, hd) bytes, needed with codes only
+ * Replaces src/diffcache/kvcache/diffcache.py:149-184 (r_sq, permute, host copies, prefix and
+ * suffix) and the memcpy of Index::prefill (diffcache_cpu/src/nsw.rs:503-508).
+ */
+typedef struct dc_prefill_args {
+    const void *k_src, *v_src;
+    void *k_store, *v_store;
+    void *k_buf, *v_buf;
+    uint8_t *codes;
+    float *scale, *resid, *r_sq;
+    int32_t *step_state;
+    void *workspace;
+    size_t workspace_bytes;
+    int64_t batch_stride, head_stride, row_stride;             /* of the stores */
+    int64_t buf_batch_stride, buf_head_stride, buf_row_stride; /* of k_buf and v_buf */
+    int64_t code_batch_stride, code_head_stride, code_row_stride;
+    int n_b, n_h, seq, hd;
+    int n_prefix, n_suffix;
+} dc_prefill_args;
+size_t dc_prefill_workspace_bytes(int n_units, int hd);
+int dc_prefill_layer_bf16(const dc_prefill_args *args, void *stream);
+
+/*
  * One decode layer of the path: score -> select -> attend, enqueued back to back.
  * All pointers are device pointers; see the single-step calls for the meaning
  * of each field.  n_ctx rows are valid per unit; the retrieval region is
