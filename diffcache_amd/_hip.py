@@ -38,7 +38,7 @@ SYMBOLS = (
     "dc_sparse_select", "dc_score_select_bf16",
     "dc_sketch_build_bf16", "dc_sketch_select_workspace_bytes", "dc_sketch_select_state_init",
     "dc_score_select_sketch_bf16", "dc_kcheck_f32",
-    "dc_pq_search_workspace_bytes", "dc_pq_search_bf16",
+    "dc_pq_search_workspace_bytes", "dc_pq_search_bf16", "dc_pq_encode_bf16",
     "dc_data_layer_create", "dc_data_layer_destroy", "dc_data_layer_ctx_len", "dc_data_layer_sizes",
     "dc_data_layer_bind", "dc_data_layer_prefill", "dc_data_layer_insert", "dc_data_layer_query",
 )
@@ -119,6 +119,7 @@ def _load() -> C.CDLL:
         "dc_decode_layer_errors": (C.c_uint, []),
         "dc_one_kernel_guard": (i, [i, i, i, i, i]),
         "dc_pq_build_lut": (i, [p, p, p, i, i, i, i, p]),
+        "dc_pq_encode_bf16": (i, [p, i64, i64, p, p, i64, i, i, i, p]),
         "dc_pq_adc_scan": (i, [p, p, p, p, i, i, i, i64, p]),
         "dc_score_gathered_bf16": (i, [p, p, p, p, i, i, i, i64, i, i64, i64, i64, i64, i64, p]),
         "dc_compose_idx": (i, [p, i64, p, i64, p, i64, i, i, p]),
@@ -743,6 +744,29 @@ def pq_build_lut(q: torch.Tensor, books: torch.Tensor, n_b: int) -> torch.Tensor
     _check(lib.dc_pq_build_lut(_dev(q, "q"), _dev(books, "books"), _dev(lut, "lut"), n_b, n_h, m * ds, m,
                                _stream()))
     return lut
+
+
+def pq_encode_supported(keys: torch.Tensor, books: torch.Tensor) -> bool:
+    """Whether dc_pq_encode_bf16 takes these: bf16 keys (n, hd) and fp32 books in GPU memory, at most 256
+    centroids, 2, 4, 8 or 16 columns per subspace, rows aligned to them."""
+    m, nc, ds = books.shape
+    align = min(2 * ds, 16)
+    return (keys.is_cuda and books.is_cuda and keys.dtype == torch.bfloat16 and books.dtype == torch.float32
+            and keys.dim() == 2 and keys.stride(1) == 1 and keys.shape[1] == m * ds and ds in (2, 4, 8, 16)
+            and 1 <= nc <= 256 and keys.stride(0) >= m * ds
+            and keys.data_ptr() % align == 0 and keys.stride(0) * 2 % align == 0)
+
+
+def pq_encode(keys: torch.Tensor, books: torch.Tensor) -> torch.Tensor:
+    """keys (n, hd) bf16, books (m, nc, ds) fp32 -> codes (n, m) uint8 (dc_pq_encode_bf16)."""
+    if not pq_encode_supported(keys, books):
+        raise DiffCacheError("dc_pq_encode_bf16 does not take these keys and books")
+    m, nc, ds = books.shape
+    books = books.contiguous()
+    codes = torch.empty((keys.shape[0], m), dtype=torch.uint8, device=keys.device)
+    _check(lib.dc_pq_encode_bf16(_dev(keys, "keys"), keys.stride(0), keys.shape[0], _dev(books, "books"),
+                                 _dev(codes, "codes"), codes.stride(0), m * ds, m, nc, _stream()))
+    return codes
 
 
 def pq_adc_scan(codes: torch.Tensor, lut: torch.Tensor, hist: Optional[torch.Tensor] = None

@@ -4,8 +4,8 @@ pipeline ADC scan -> candidates -> exact bf16 rerank.
 The reference's PQ baseline directory (evaluation/impl/pqcache) is empty, so
 this follows the benchmark configuration only: M subspaces x 256 centroids,
 8-bit codes, per-query fp32 lookup tables, 4096 candidates reranked to top-k.
-Training and encoding are one-off preparation and use torch ops on the device;
-everything a query touches runs in libdiffcache_hip.so.
+Training is one-off preparation and uses torch ops on the device around the encoding kernel;
+encoding and everything a query touches run in libdiffcache_hip.so.
 """
 from __future__ import annotations
 
@@ -29,8 +29,9 @@ def train_codebooks(keys: torch.Tensor, m: int, iters: int = 8, seed: int = 0,
     for j in range(m):
         xs = x[:, j * ds:(j + 1) * ds].contiguous()
         c = xs[torch.randint(0, n, (n_centroids,), generator=g, device=x.device)].clone()
+        cols = keys[:, j * ds:(j + 1) * ds]
         for _ in range(iters):
-            a = torch.cdist(xs, c).argmin(dim=1)
+            a = encode(cols, c.unsqueeze(0)).view(-1).long()
             sums = torch.zeros_like(c).index_add_(0, a, xs)
             cnt = torch.bincount(a, minlength=n_centroids).to(xs.dtype)
             nz = cnt > 0
@@ -42,6 +43,9 @@ def train_codebooks(keys: torch.Tensor, m: int, iters: int = 8, seed: int = 0,
 def encode(keys: torch.Tensor, books: torch.Tensor, chunk: int = 1 << 18) -> torch.Tensor:
     """keys (n, hd) bf16/fp32, books (m, 256, ds) -> codes (n, m) uint8: nearest
     centroid by squared L2 per subspace."""
+    if hip.pq_encode_supported(keys, books):
+        return hip.pq_encode(keys, books)
+    # fp32 keys, other subspace widths: torch's distances
     m, nc, ds = books.shape
     n = keys.shape[0]
     codes = torch.empty((n, m), dtype=torch.uint8, device=keys.device)

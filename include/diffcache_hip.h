@@ -515,6 +515,16 @@ int dc_compose_idx(const uint32_t *outer, int64_t outer_unit_stride, const uint3
                    int n_inner, void *stream);
 
 /*
+ * PQ codes of keys: codes[i, s] = the centroid c of subspace s with the least |x - c|^2, x = columns
+ * [s*ds, (s+1)*ds) of key i, ds = hd / m (2, 4, 8 or 16); equal distances -> the lower number.
+ * Decided in fp32 by |c|^2 / 2 - x.c, every product exact.  keys bf16, key_stride elements from row to row;
+ * books (m, n_centroids <= 256, ds) fp32; codes code_stride bytes from row to row.
+ * No reference code (see above).
+ */
+int dc_pq_encode_bf16(const void *keys, int64_t key_stride, int64_t n, const float *books, uint8_t *codes,
+                      int64_t code_stride, int hd, int m, int n_centroids, void *stream);
+
+/*
  * The whole PQ search in one call, without a dense ADC score array:
  *   candidates = the min(n_cand, n_rows) keys of every unit with the largest ADC
  *                scores (ties to the lower id), scores as dc_pq_adc_scan computes them;

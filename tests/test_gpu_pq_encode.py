@@ -1,0 +1,48 @@
+"""dc_pq_encode_bf16 against float64 distances."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("n,m,ds,nc", [
+    (1, 32, 4, 256), (255, 32, 4, 256), (257, 16, 8, 256),      # below, at and past a block of 256 keys
+    (3001, 32, 2, 256), (3001, 16, 16, 256),                    # the other subspace widths
+    (700, 3, 4, 200), (513, 5, 8, 17), (300, 1, 4, 1),          # odd subspace counts, fewer centroids
+])
+def test_pq_encode_picks_a_nearest_centroid(n, m, ds, nc):
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(n * m + ds)
+    x = torch.randn((n, m * ds + 16), generator=g, device=DEV).to(torch.bfloat16)[:, :m * ds]     # strided rows
+    books = torch.randn((m, nc, ds), generator=g, device=DEV)
+    if nc > 40:
+        books[:, 33] = books[:, 7]          # equal centroids: the lower number
+    codes = hip.pq_encode(x, books).long()
+    assert codes.shape == (n, m) and int(codes.max()) < nc
+    assert nc <= 40 or not bool((codes == 33).any())
+    X, B = x.double().view(n, m, ds), books.double()
+    for j in range(m):
+        d = 0.5 * (B[j] ** 2).sum(-1)[None] - X[:, j] @ B[j].t()
+        # ds + 3 fp32 roundings of terms no larger than their sum of magnitudes, on either side
+        size = 0.5 * (B[j] ** 2).sum(-1)[None] + X[:, j].abs() @ B[j].abs().t()
+        err = (ds + 3) * 2.0 ** -24 * size.amax(dim=1)
+        got = d.gather(1, codes[:, j:j + 1])[:, 0]
+        assert bool((got <= d.amin(dim=1) + 2 * err).all())
+    if m == 32 and ds == 4 and n > 1:
+        # a single nearest centroid wherever fp32 can tell: at most a handful of keys are undecided
+        exact = torch.stack([torch.cdist(X[:, j], B[j]).argmin(1) for j in range(m)], 1)
+        assert (exact != codes).float().mean() < 1e-3
+
+
+def test_encode_takes_what_it_took_before():
+    """fp32 keys and subspace widths the kernel is not built for still go through torch's distances."""
+    from diffcache_amd.pq import encode
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn((400, 24), generator=g, device=DEV)
+    for m in (2, 6):
+        books = torch.randn((m, 16, 24 // m), generator=g, device=DEV)
+        for keys in (x, x.to(torch.bfloat16)):
+            want = torch.stack([torch.cdist(keys.float().view(400, m, -1)[:, j].contiguous(), books[j]).argmin(1)
+                                for j in range(m)], 1)
+            assert (encode(keys, books).long() != want).float().mean() < 1e-2
