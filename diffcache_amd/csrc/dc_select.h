@@ -315,4 +315,147 @@ __device__ __forceinline__ void dc_finalize_unit(const uint32_t *ck, const uint3
     });
 }
 
+// Bitonic sort of n (a power of two, >= 128) 64-bit words in LDS by all kFinalThreads threads.  Stages with a
+// stride of at most 64 stay inside 128 elements, a wave's block: the wave keeps the block in
+// registers, two elements per lane, exchanges across lanes with shuffles and touches LDS once per
+// run of those stages.  Only the stages that cross waves (stride >= 128) go through LDS with a
+// block barrier.  The caller's stores to buf must be followed by a barrier; ends with one.
+__device__ __forceinline__ void dc_bitonic_lds(unsigned long long *buf, int n) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    auto local_stages = [&](int size_lo, int size_hi) {
+        for (int blk = tid >> 6; blk * 128 < n; blk += kFinalThreads / 64) {  // wave-uniform
+            const int i0 = blk * 128 + lane, i1 = i0 + 64;
+            unsigned long long a = buf[i0], b = buf[i1];
+            for (int size = size_lo; size <= size_hi; size <<= 1) {
+                int s = size >> 1;
+                if (s >= 64) {  // the two elements of the lane meet; both sort the same way
+                    const bool asc = (i0 & size) == 0;
+                    const unsigned long long lo = a < b ? a : b, hi = a < b ? b : a;
+                    a = asc ? lo : hi;
+                    b = asc ? hi : lo;
+                    s = 32;
+                }
+                const bool asc_a = (i0 & size) == 0, asc_b = (i1 & size) == 0;
+                for (; s >= 1; s >>= 1) {
+                    const unsigned long long pa = __shfl_xor(a, s, 64), pb = __shfl_xor(b, s, 64);
+                    const bool lower = (lane & s) == 0;
+                    a = ((lower == asc_a) == (a < pa)) ? a : pa;  // keep the smaller iff lower == asc
+                    b = ((lower == asc_b) == (b < pb)) ? b : pb;
+                }
+            }
+            buf[i0] = a;
+            buf[i1] = b;
+        }
+    };
+    local_stages(2, 128);
+    __syncthreads();
+    for (int size = 256; size <= n; size <<= 1) {
+        for (int stride = size >> 1, ls = __ffs(size) - 2; stride >= 128; stride >>= 1, --ls) {
+            for (int t = tid; t < (n >> 1); t += kFinalThreads) {
+                const int i = ((t >> ls) << (ls + 1)) | (t & (stride - 1));
+                const int j = i + stride;
+                const bool asc = (i & size) == 0;
+                unsigned long long a = buf[i], b = buf[j];
+                if ((a > b) == asc) {
+                    buf[i] = b;
+                    buf[j] = a;
+                }
+            }
+            __syncthreads();
+        }
+        local_stages(size, size);
+        __syncthreads();
+    }
+}
+
+// The `need` smallest (key, id) pairs of a list in LDS by one counting pass over the highest kRadixBits bits in
+// which the keys differ: the histogram's prefix is the rank of a bin's first member, so every member
+// of a bin below the threshold's has its slot from the bin's cursor, and only the threshold's bin has to
+// be ranked.
+//   SORTED: out(rank, key, id) in ascending order: the bins up to the threshold's are scattered to their
+//           stretches of buf (need + kSortBinMost words) and ranked among bin mates.  Returns
+//           false, with nothing put out, when a bin holds more than kSortBinMost (runs of equal keys, one
+//           far outlier): ranking inside bins is quadratic.
+//   else:   out(slot, key, id) with the slots below need in no particular order; buf (kFinalThreads words)
+//           takes the threshold's bin.  Returns false when that holds more than kFinalThreads.
+// need <= n.  Called by all threads with uniform arguments, after a barrier.
+constexpr int kSortMost = 4096;      // longest sorted selection
+constexpr int kSortBinMost = 128;
+template <bool SORTED, typename Out>
+__device__ __forceinline__ bool dc_select_counted(const uint32_t *ck, const uint32_t *ci, uint32_t n, uint32_t need,
+                                                  unsigned long long *buf, uint32_t *lh, uint32_t *wtot, uint32_t *sres,
+                                                  uint32_t *smisc, Out out) {
+    const int tid = threadIdx.x;
+    if (tid == 0) smisc[0] = smisc[1] = 0u;
+    for (int i = tid; i < kRadixBins; i += kFinalThreads) lh[i] = 0u;
+    __syncthreads();
+    const uint32_t k0 = ck[0];
+    uint32_t diff = 0u;
+    for (uint32_t i = tid; i < n; i += kFinalThreads) diff |= ck[i] ^ k0;
+    // one addition per wave: a thousand lanes updating one LDS word are served one after the other
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) diff |= (uint32_t)__shfl_xor((int)diff, d, 64);
+    if ((tid & 63) == 0 && diff) atomicOr(&smisc[0], diff);
+    __syncthreads();
+    diff = smisc[0];
+    const int top = diff ? 32 - __clz(diff) : 0;
+    const int shift = top > kRadixBits ? top - kRadixBits : 0;
+    const uint32_t mask = diff ? (uint32_t)kRadixBins - 1u : 0u;  // the bits above are the same in every key
+    auto bin_of = [&](uint32_t key) { return (key >> shift) & mask; };
+    for (uint32_t i = tid; i < n; i += kFinalThreads) atomicAdd(&lh[bin_of(ck[i])], 1u);
+    __syncthreads();
+    const uint32_t h0 = lh[2 * tid], h1 = lh[2 * tid + 1];
+    uint32_t total;
+    const uint32_t excl = block_excl_scan<kFinalThreads>(h0 + h1, wtot, &total);
+    lh[2 * tid] = excl;
+    lh[2 * tid + 1] = excl + h0;
+    if (SORTED) {
+        uint32_t most = 0u;  // largest bin up to the threshold's
+        if (excl < need) most = h0;
+        if (excl + h0 < need && h1 > most) most = h1;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            const uint32_t o = (uint32_t)__shfl_xor((int)most, d, 64);
+            most = o > most ? o : most;
+        }
+        if ((tid & 63) == 0 && most) atomicMax(&smisc[1], most);
+    }
+    if (excl < need && need <= excl + h0 + h1) {
+        const bool first = excl + h0 >= need;
+        sres[0] = 2 * tid + (first ? 0 : 1);
+        sres[1] = first ? excl : excl + h0;
+        sres[2] = first ? h0 : h1;
+    }
+    __syncthreads();
+    const uint32_t t_bin = sres[0], t_lo = sres[1], t_cnt = sres[2];
+    if (SORTED ? smisc[1] > (uint32_t)kSortBinMost : t_cnt > (uint32_t)kFinalThreads) return false;
+    for (uint32_t i = tid; i < n; i += kFinalThreads) {
+        const uint32_t key = ck[i], bin = bin_of(key);
+        if (bin > t_bin) continue;
+        const uint32_t slot = atomicAdd(&lh[bin], 1u);
+        const unsigned long long pair = ((unsigned long long)key << 32) | ci[i];
+        if (SORTED) buf[slot] = pair;
+        else if (bin == t_bin) buf[slot - t_lo] = pair;
+        else out(slot, key, ci[i]);
+    }
+    __syncthreads();
+    if (SORTED) {
+        // a bin's cursor now stands at its end, which is the start of the next bin
+        for (uint32_t i = tid; i < t_lo + t_cnt; i += kFinalThreads) {
+            const unsigned long long mine = buf[i];
+            const uint32_t bin = bin_of((uint32_t)(mine >> 32));
+            const uint32_t lo = bin ? lh[bin - 1] : 0u, hi = lh[bin];
+            uint32_t rank = lo;
+            for (uint32_t j = lo; j < hi; ++j) rank += buf[j] < mine ? 1u : 0u;
+            if (rank < need) out(rank, (uint32_t)(mine >> 32), (uint32_t)mine);
+        }
+    } else if ((uint32_t)tid < t_cnt) {
+        const unsigned long long mine = buf[tid];
+        uint32_t rank = t_lo;
+        for (uint32_t j = 0; j < t_cnt; ++j) rank += buf[j] < mine ? 1u : 0u;
+        if (rank < need) out(rank, (uint32_t)(mine >> 32), (uint32_t)mine);
+    }
+    return true;
+}
+
 }  // namespace

@@ -815,8 +815,12 @@ __global__ __launch_bounds__(kThreads) void pq_rescore_kernel(
     }
 }
 
-// One block per unit: radix select among the candidates of the threshold bucket
-// fills idx_out[c_less, k).  Leaves the unit's list cursors at zero.
+// One block per unit: a selection among the candidates of the threshold bucket
+// fills idx_out[c_less, k).  Leaves the unit's list cursors at zero.  A chain of block barriers on few CUs: the
+// counting pass that hands out the slots itself (dc_select_counted) takes 5.9 us at 8 units and 7.0 us at
+// 64 (2048 of about 3600 candidates); a radix pass whose members reserve slots wave by wave took 7.5
+// and 8.8 us.  Lists that do not fit the LDS and threshold bins of more than kFinalThreads (ties by the
+// thousand) take the radix passes of dc_finalize_unit.
 __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     uint32_t *__restrict__ hist, UnitState *__restrict__ state, uint32_t *__restrict__ cand_key,
     uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride,
@@ -826,6 +830,7 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     __shared__ uint32_t sres[4];
     __shared__ uint32_t smisc[2];
     __shared__ uint32_t lck[kCandLds], lci[kCandLds];  // candidates are staged in LDS when they fit
+    __shared__ unsigned long long tie[kFinalThreads];
     const int unit = blockIdx.x;
     const int tid = threadIdx.x;
     UnitState *st = state + unit;
@@ -882,37 +887,114 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     if (c_less >= kk) return;
     uint32_t need = kk - c_less;
     if (need > n_c) need = n_c;
-    if (n_c <= 128u) {
-        // Short list: every thread ranks its own candidate among all of them by
-        // (key, id).  The packed pairs sit in lh, padded with a sentinel to a multiple
-        // of 8; the reads in the loop are wave-uniform 16-byte broadcasts.
-        unsigned long long *comp = reinterpret_cast<unsigned long long *>(lh);
-        const unsigned long long mine = ((unsigned long long)hk[0] << 32) | hi[0];
-        comp[tid] = (uint32_t)tid < n_c ? mine : ~0ull;
-        __syncthreads();
-        if ((uint32_t)tid < n_c) {
-            const ulonglong2 *c2 = reinterpret_cast<const ulonglong2 *>(comp);
-            const uint32_t n8 = (n_c + 7u) / 8u;
-            uint32_t rank = 0;
-            for (uint32_t j = 0; j < n8; ++j) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const ulonglong2 t = c2[4 * j + u];
-                    rank += (t.x < mine ? 1u : 0u) + (t.y < mine ? 1u : 0u);
-                }
-            }
-            if (rank < need) {
-                io[c_less + rank] = hi[0];
-                if (ko) ko[c_less + rank] = hk[0];
-            }
-        }
-        return;
-    }
+    auto put = [&](uint32_t slot, uint32_t key, uint32_t id) {
+        io[c_less + slot] = id;
+        if (ko) ko[c_less + slot] = key;
+    };
+    if (staged && dc_select_counted<false>(lck, lci, n_c, need, tie, lh, wtot, sres, smisc, put)) return;
+    __syncthreads();
     // Two calls, so that the staged list is read with LDS instructions: through a pointer chosen
     // at run time every access would be a flat one, and waiting for a flat load also waits for
     // the stores issued above.
     if (staged) dc_finalize_unit<true>(lck, lci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
     else dc_finalize_unit(ck, ci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
+}
+
+// The same for ids in best-first order (k <= kSortMost): the unit's certain members (which classify_kernel
+// wrote to idx_out and sel_keys) and its candidates are ordered together by one counting pass
+// (dc_select_counted), which is the selection as well.  4 units, 1024 of about 1400 candidates: 5.6 us,
+// against 6.1 us for a selection and 8.6 us for a bitonic sort of its result in a kernel of its own.
+// Lists that do not fit the LDS and keys that crowd into few bins take the selection above and the
+// bitonic sort.
+constexpr int kSortedLds = 12288;
+
+__global__ __launch_bounds__(kFinalThreads) void select_sorted_kernel(
+    uint32_t *__restrict__ hist, UnitState *__restrict__ state, const uint32_t *__restrict__ cand_key,
+    const uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride,
+    uint32_t *__restrict__ sel_keys, int n_rows, int k_eff, int reinit) {
+    __shared__ uint32_t lh[kRadixBins];
+    __shared__ uint32_t wtot[kFinalThreads / 64 + 1];
+    __shared__ uint32_t sres[4];
+    __shared__ uint32_t smisc[2];
+    __shared__ uint32_t lck[kSortedLds], lci[kSortedLds];
+    __shared__ unsigned long long buf[kSortMost + kSortBinMost];
+    const int unit = blockIdx.x;
+    const int tid = threadIdx.x;
+    UnitState *st = state + unit;
+    const uint32_t *ck = cand_key + (int64_t)unit * n_rows;
+    const uint32_t *ci = cand_idx + (int64_t)unit * n_rows;
+    uint32_t *io = idx_out + (int64_t)unit * idx_stride;
+    uint32_t *ko = sel_keys + (int64_t)unit * k_eff;
+    // the head of the candidate list is fetched before its length is known
+    constexpr int kHead = 4;
+    uint32_t hk[kHead], hi[kHead];
+#pragma unroll
+    for (int j = 0; j < kHead; ++j) {
+        const int i = tid + j * kFinalThreads;
+        hk[j] = hi[j] = 0;
+        if (i < n_rows) {
+            hk[j] = ck[i];
+            hi[j] = ci[i];
+        }
+    }
+    uint32_t n_c = st->cand_cnt;
+    const uint32_t kk = (uint32_t)k_eff;
+    uint32_t c_less = st->c_less;
+    if (n_c > (uint32_t)n_rows) n_c = n_rows;
+    if (c_less > kk) c_less = kk;
+    const uint32_t n = c_less + n_c, need = kk < n ? kk : n;
+    const bool staged = n <= (uint32_t)kSortedLds;
+    if (staged) {
+        for (uint32_t i = tid; i < c_less; i += kFinalThreads) {
+            lck[i] = ko[i];
+            lci[i] = io[i];
+        }
+#pragma unroll
+        for (int j = 0; j < kHead; ++j) {
+            const uint32_t i = (uint32_t)(tid + j * kFinalThreads);
+            if (i < n_c) {
+                lck[c_less + i] = hk[j];
+                lci[c_less + i] = hi[j];
+            }
+        }
+        for (uint32_t i = tid + kHead * kFinalThreads; i < n_c; i += kFinalThreads) {
+            lck[c_less + i] = ck[i];
+            lci[c_less + i] = ci[i];
+        }
+    }
+    __syncthreads();  // every thread has read the counters
+    if (reinit) {
+        uint4 *hz = reinterpret_cast<uint4 *>(hist + (int64_t)unit * DC_HIST_BINS);
+        if (tid < DC_HIST_BINS / 4) hz[tid] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    if (tid == 0) {
+        if (reinit) {
+            st->tb_run = DC_HIST_BINS;
+            st->surv_cnt = 0;
+        }
+        st->win_cnt = 0;
+        st->cand_cnt = 0;
+    }
+    if (need == 0u) return;
+    if (staged && dc_select_counted<true>(lck, lci, n, need, buf, lh, wtot, sres, smisc,
+                                   [&](uint32_t rank, uint32_t, uint32_t id) { io[rank] = id; }))
+        return;
+    __syncthreads();
+    if (c_less < need) {
+        if (staged)
+            dc_finalize_unit<true>(lck + c_less, lci + c_less, n_c, need - c_less, io + c_less, n_rows, lh, wtot, sres, smisc,
+                                   ko + c_less);
+        else
+            dc_finalize_unit(ck, ci, n_c, need - c_less, io + c_less, n_rows, lh, wtot, sres, smisc, ko + c_less);
+    }
+    __syncthreads();
+    int pow2 = 128;
+    while (pow2 < (int)need) pow2 <<= 1;
+    for (int i = tid; i < pow2; i += kFinalThreads)
+        buf[i] = i < (int)need ? ((unsigned long long)ko[i] << 32) | io[i] : ~0ull;
+    __syncthreads();
+    dc_bitonic_lds(buf, pow2);
+    for (int i = tid; i < (int)need; i += kFinalThreads) io[i] = (uint32_t)buf[i];
 }
 
 }  // namespace
@@ -1037,6 +1119,12 @@ namespace {
 int launch_finish(const char *who, const FusedWs &w, uint32_t *idx_out, int64_t idx_unit_stride, int n_units,
                   int n_rows, int k_eff, int mode, int order, int reinit, hipStream_t st) {
     uint32_t *sel_keys = order == DC_ORDER_BEST ? w.sel_keys : nullptr;
+    if (order == DC_ORDER_BEST && k_eff <= kSortMost) {
+        hipLaunchKernelGGL(select_sorted_kernel, dim3(n_units), dim3(kFinalThreads), 0, st, w.hist, w.state,
+                           w.cand_key, w.cand_idx, idx_out, idx_unit_stride, sel_keys, n_rows, k_eff, reinit);
+        DC_CHECK_LAUNCH(who);
+        return DC_OK;
+    }
     hipLaunchKernelGGL(select_finish_kernel, dim3(n_units), dim3(kFinalThreads), 0, st, w.hist, w.state,
                        w.cand_key, w.cand_idx, idx_out, idx_unit_stride, sel_keys, n_rows, k_eff, reinit);
     DC_CHECK_LAUNCH(who);
