@@ -152,8 +152,6 @@ class DiffCache:
             self.sketch = [hip.Sketch(self.kstore[l], codes=self._cslab[l]) for l in range(num_layers)]
 
         n_units = batch_size * num_kv_heads
-        self._prefill_ws = torch.empty((int(hip.lib.dc_prefill_workspace_bytes(n_units, head_dim)),),
-                                       device=self.device, dtype=torch.uint8)
         self.group = num_q_heads // num_kv_heads
         # group-mean query of the current layer (the reference's pinned qbuf_cpu, diffcache.py:80)
         self.qbuf = torch.zeros((batch_size, num_kv_heads, head_dim), device=self.device, dtype=torch.bfloat16)
@@ -297,6 +295,8 @@ class DiffCache:
         GPU (diffcache.py:149-184)."""
         seq_len = key_states.size(1)
         hip.require(0 < seq_len <= self.max_length, "the prompt is empty or longer than max_length")
+        # a replay would move the rows and leave the host's lengths as they are
+        hip.require(not torch.cuda.is_current_stream_capturing(), "a prefill cannot be captured in a graph")
         prefix_len = min(self._prefix0, seq_len)                    # diffcache.py:163
         suffix_len = min(self._suffix0, seq_len - prefix_len)       # diffcache.py:169
         hip.require(suffix_len <= self.kvbuf_suffix_maxlen, "kvbuf_suffix_len exceeds kvbuf_suffix_maxlen")
@@ -308,8 +308,7 @@ class DiffCache:
         b0 = self.retrieval_budget
         hip.prefill_layer(self.kstore[layer_idx], self.vstore[layer_idx], key_states, value_states, prefix_len,
                           suffix_len, self.kbuf[layer_idx][:, :, b0:], self.vbuf[layer_idx][:, :, b0:],
-                          sketch=self.sketch[layer_idx] if region > 0 else None, r_sq=r_sq, step_state=self._state,
-                          workspace=self._prefill_ws)
+                          sketch=self.sketch[layer_idx] if region > 0 else None, r_sq=r_sq, step_state=self._state)
         self._r_sq[layer_idx] = DeviceRSq(r_sq)
         self.kvbuf_prefix_len = prefix_len
         self.retrieval_region_len = region

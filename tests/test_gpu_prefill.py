@@ -75,3 +75,40 @@ def test_r_sq_of_a_prefill_reads_as_before():
         assert isinstance(got, list) and all(isinstance(x, float) for x in got)
         assert all(abs(a - b) <= 2.0 ** -7 * b for a, b in zip(got, want))     # one bf16 ulp
     assert cache.r_sq[0] == [4.0, 4.0] and mine == [[4.0, 4.0], [4.0, 4.0]]
+
+
+def test_layers_prefilled_on_two_streams_share_nothing_and_r_sq_waits_for_its_own():
+    """Layers ingested on different streams at the same time: each sketch is that of its own keys, and r_sq read
+    from a third stream is the finished value."""
+    from diffcache_amd import DiffCache, _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(11)
+    cache = DiffCache(num_layers=2, batch_size=2, max_length=20100, num_kv_heads=4, num_q_heads=8, head_dim=128,
+                      retrieval_budget=64, nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8,
+                      kvbuf_suffix_maxlen=16, attn_mass_threshold=0.9, k_check_seq=[100], r_sq=[[4.0] * 4] * 2)
+    ks = [torch.randn((2, 20011, 4, 128), generator=g, device=DEV).mul_(10.0 ** l).to(torch.bfloat16) for l in range(2)]
+    want = [k.float().pow(2).sum(-1).amax(dim=(0, 1)).to(torch.bfloat16).tolist() for k in ks]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for l, stream in enumerate((torch.cuda.Stream(), torch.cuda.Stream())):
+            with torch.cuda.stream(stream):
+                cache.prefill_update_kv_cache(ks[l], ks[l], l)
+        for l in range(2):
+            assert all(abs(a - b) <= 2.0 ** -7 * b for a, b in zip(cache.data_layers[l].r_sq, want[l]))   # one bf16 ulp
+        torch.cuda.synchronize()
+        for l in range(2):
+            ref = hip.Sketch(cache.kstore[l])
+            ref.build(cache.kstore[l], 4, 20011 - 12)
+            assert torch.equal(cache.sketch[l].scale, ref.scale) and torch.equal(cache.sketch[l].resid, ref.resid)
+            assert torch.equal(cache.sketch[l].codes[:, :, 4:20003], ref.codes[:, :, 4:20003])
+
+
+def test_a_prefill_under_capture_is_refused():
+    from diffcache_amd import DiffCache
+    cache = DiffCache(num_layers=1, batch_size=1, max_length=300, num_kv_heads=1, num_q_heads=1, head_dim=64,
+                      retrieval_budget=16, nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8,
+                      kvbuf_suffix_maxlen=16, attn_mass_threshold=0.9, k_check_seq=[100], r_sq=[[4.0]])
+    k = torch.ones((1, 200, 1, 64), device=DEV, dtype=torch.bfloat16)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+        with pytest.raises(Exception, match="captured"):
+            cache.prefill_update_kv_cache(k, k, 0)
