@@ -31,7 +31,7 @@ SYMBOLS = (
     "dc_attn_workspace_bytes", "dc_gather_attn_bf16", "dc_gather_attn_static_bf16", "dc_append_kv_bf16",
     "dc_step_advance", "dc_step_state_advance", "dc_step_state_rollover", "dc_ingest_kv_bf16",
     "dc_prefill_workspace_bytes", "dc_prefill_layer_bf16", "dc_layer_workspace_bytes", "dc_decode_layer",
-    "dc_decode_layer_status", "dc_set_wait_limit", "dc_decode_layer_route", "dc_last_route",
+    "dc_decode_layer_step", "dc_decode_layer_status", "dc_set_wait_limit", "dc_decode_layer_route", "dc_last_route",
     "dc_decode_layer_errors", "dc_one_kernel_guard",
     "dc_pq_build_lut", "dc_pq_adc_scan", "dc_score_gathered_bf16", "dc_compose_idx",
     "dc_score_select_workspace_bytes", "dc_select_state_init", "dc_score_prune_bf16",
@@ -65,6 +65,14 @@ class LayerArgs(C.Structure):
         ("n_recent_dev", C.c_void_p),
         ("one_kernel", C.c_int),
         ("region_hi_dev", C.c_void_p),
+    ]
+
+
+class StepArgs(C.Structure):
+    """struct dc_step_args of include/diffcache_hip.h"""
+    _fields_ = [
+        ("append", C.c_int), ("advance_limit", C.c_int), ("pos", C.c_int64), ("pos_end", C.c_int64),
+        ("pos_dev", C.c_void_p), ("advance_state", C.c_void_p),
     ]
 
 
@@ -112,6 +120,7 @@ def _load() -> C.CDLL:
         "dc_prefill_layer_bf16": (i, [C.POINTER(PrefillArgs), p]),
         "dc_layer_workspace_bytes": (sz, [i, i, i, i, i, i]),
         "dc_decode_layer": (i, [C.POINTER(LayerArgs), p]),
+        "dc_decode_layer_step": (i, [C.POINTER(LayerArgs), C.POINTER(StepArgs), p]),
         "dc_decode_layer_status": (i, [C.POINTER(LayerArgs), p]),
         "dc_set_wait_limit": (None, [i]),
         "dc_decode_layer_route": (i, [C.POINTER(LayerArgs)]),
@@ -664,18 +673,41 @@ def decode_layer(q: torch.Tensor, store_k: torch.Tensor, store_v: torch.Tensor, 
                  sketch: Optional["Sketch"] = None,
                  n_recent_dev: Optional[torch.Tensor] = None,
                  one_kernel: int = ONE_KERNEL_AUTO,
-                 region_hi_dev: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 region_hi_dev: Optional[torch.Tensor] = None,
+                 append: Optional[Tuple[int, Optional[torch.Tensor], int]] = None,
+                 advance: Optional[Tuple[torch.Tensor, int]] = None) -> torch.Tensor:
     """score -> select -> attend for one layer, enqueued on the current stream.
     ``n_recent_dev``: the suffix length as a device-side int32 (``n_recent`` = capacity).
     ``select_state_ready``: see dc_layer_args in the header (skips the init kernel).
     ``sketch``: scan the 8-bit sketch of the keys instead of the keys (same result).
     ``one_kernel``: ONE_KERNEL_* policy for short contexts (see the header).
     ``region_hi_dev``: the end of the retrieval region as a device-side int32 (``recent_lo`` = its
-    largest value), for captured steps that outlive a rollover of the recent window."""
+    largest value), for captured steps that outlive a rollover of the recent window.
+    ``append`` (pos, pos_dev, pos_end): new_k / new_v also go to that row of the store, as append_kv
+    puts them there; ``advance`` (state, limit): step_state_advance by one behind the layer.  Both ride
+    in the layer's own launches."""
     a = _layer_args(q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores, idx_out, out, workspace,
                     new_k, new_v, lse, mode, order, scale, select_state_ready, scan_events, sketch, n_recent_dev,
                     one_kernel, region_hi_dev)
-    _check(lib.dc_decode_layer(C.byref(a), _stream()))
+    if append is None and advance is None:
+        _check(lib.dc_decode_layer(C.byref(a), _stream()))
+        return out
+    s = StepArgs()
+    if append is not None:
+        b, h, n_max, hd = store_k.shape
+        if not 0 <= append[0] < n_max:
+            raise DiffCacheError(f"append position {append[0]} outside the store of {n_max} rows")
+        for t in (new_k, new_v):
+            if t is None or t.numel() != b * h * hd or not t.is_contiguous():
+                raise DiffCacheError("new_k/new_v must be contiguous and hold (b, h, hd) values")
+        s.append, s.pos, s.pos_end = 1, append[0], min(append[2], n_max)
+        s.pos_dev = _counter(append[1])
+    if advance is not None:
+        state, s.advance_limit = advance
+        if not state.is_cuda or state.dtype != torch.int32 or state.numel() < 4 or not state.is_contiguous():
+            raise DiffCacheError("the step state must be a contiguous int32 tensor of 4 elements in GPU memory")
+        s.advance_state = state.data_ptr()
+    _check(lib.dc_decode_layer_step(C.byref(a), C.byref(s), _stream()))
     return out
 
 

@@ -72,7 +72,9 @@ extern "C" size_t dc_layer_workspace_bytes(int n_units, int n_region_rows, int b
     return carve_layer(nullptr, n_units, n_region_rows, budget, group, hd, n_rows_attended).bytes;
 }
 
-extern "C" int dc_decode_layer(const dc_layer_args *a, void *stream) {
+extern "C" int dc_decode_layer(const dc_layer_args *a, void *stream) { return dc_decode_layer_step(a, nullptr, stream); }
+
+extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *step, void *stream) {
     DC_REQUIRE(a, "dc_decode_layer: null args");
     DC_REQUIRE(a->q && a->k && a->v && a->out && a->idx_out, "dc_decode_layer: null pointer in args");
     DC_REQUIRE(a->n_b >= 0 && a->n_h >= 1 && a->group >= 1 && a->n_sink >= 0 && a->n_recent >= 0 &&
@@ -82,8 +84,11 @@ extern "C" int dc_decode_layer(const dc_layer_args *a, void *stream) {
     DC_REQUIRE(a->recent_lo >= a->n_sink, "dc_decode_layer: recent_lo %lld < n_sink %d",
                (long long)a->recent_lo, a->n_sink);
     DC_REQUIRE(!(a->region_hi_dev && a->scores), "dc_decode_layer: region_hi_dev needs scores == NULL");
+    const int rc_step = dc_step_check("dc_decode_layer", a, step);
+    if (rc_step) return rc_step;
+    int32_t *adv = step ? step->advance_state : nullptr;
     const int n_units = a->n_b * a->n_h;
-    if (n_units == 0) return DC_OK;
+    if (n_units == 0) return adv ? dc_step_state_advance(adv, 1, step->advance_limit, stream) : DC_OK;
     const int64_t region64 = a->recent_lo - a->n_sink;
     DC_REQUIRE(region64 < (1ll << 31), "dc_decode_layer: region too long");
     const int region = (int)region64;
@@ -126,12 +131,13 @@ extern "C" int dc_decode_layer(const dc_layer_args *a, void *stream) {
             ready = 1;
         }
         if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
-        rc = dc_small_try(a, region, k_eff, w.topk, w.small_cand, w.attn, w.attn_bytes, stream);
+        rc = dc_small_try(a, region, k_eff, w.topk, w.small_cand, w.attn, w.attn_bytes, stream, step);
         if (rc < 0) return rc;
         if (rc == 1) {
             if (a->ev_scan_end) (void)hipEventRecord((hipEvent_t)a->ev_scan_end, st);
             g_last_route = DC_ROUTE_ONE_KERNEL;
-            return DC_OK;
+            // (every block of that kernel reads the state at a time of its own)
+            return adv ? dc_step_state_advance(adv, 1, step->advance_limit, stream) : DC_OK;
         }
     }
     if (k_eff > 0 && !a->scores && a->sketch_codes && region <= DC_SKETCH_MAX_ROWS) {
@@ -178,7 +184,7 @@ extern "C" int dc_decode_layer(const dc_layer_args *a, void *stream) {
                                a->n_b, a->n_h, a->group, a->hd, k_eff, a->idx_unit_stride, nullptr, a->n_sink,
                                a->n_sink, a->recent_lo, a->n_recent, a->n_recent_dev, a->kv_batch_stride,
                                a->kv_head_stride, a->kv_row_stride, a->kv_batch_stride, a->kv_head_stride,
-                               a->kv_row_stride, a->scale, w.attn, w.attn_bytes, stream, a->region_hi_dev);
+                               a->kv_row_stride, a->scale, w.attn, w.attn_bytes, stream, a->region_hi_dev, step);
     return rc;
 }
 

@@ -84,6 +84,7 @@ struct AttnArgs {
     int n_recent, n_total, n_splits;
     int64_t ksb, ksh, ksr, vsb, vsh, vsr;
     float scale;
+    DcAppend app;
 };
 
 struct AttnShared {
@@ -246,6 +247,8 @@ __device__ __forceinline__ void dc_attn_split(const AttnArgs &a, int unit, int s
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[g][i] += __shfl_xor(acc[g][i], off, 64);
         }
+    DcNewRow<HD> fresh;
+    fresh.load(a.app, a.new_k, a.new_v, unit, split == a.n_splits - 1);
     if (lane < LPR) {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -273,6 +276,7 @@ __device__ __forceinline__ void dc_attn_split(const AttnArgs &a, int unit, int s
         ml[0] = mm;
         ml[1] = l;
     }
+    fresh.store(a.app, b * a.ksb + h * a.ksh, a.ksr, b * a.vsb + h * a.vsh, a.vsr);
 }
 
 
@@ -494,6 +498,8 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int
     lloc += __shfl_xor(lloc, 16, 64);
     lloc += __shfl_xor(lloc, 32, 64);
     if (q == 0) s_l[wave * 16 + c] = lloc;
+    DcNewRow<HD> fresh;
+    fresh.load(a.app, a.new_k, a.new_v, unit, split == a.n_splits - 1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int head = 4 * q + i;
@@ -522,6 +528,7 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int
         ml[0] = mm;
         ml[1] = l;
     }
+    fresh.store(a.app, b * a.ksb + h * a.ksh, a.ksr, b * a.vsb + h * a.vsh, a.vsr);
 }
 
 }  // namespace

@@ -57,7 +57,8 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
                           int hd, int n_idx, int64_t idx_unit_stride, const uint32_t *n_idx_unit, int64_t region_lo,
                           int n_sink, int64_t recent_lo, int n_recent, const int32_t *n_recent_dev, int64_t ksb,
                           int64_t ksh, int64_t ksr, int64_t vsb, int64_t vsh, int64_t vsr, float scale,
-                          void *workspace, size_t workspace_bytes, void *stream, const int32_t *recent_lo_dev);
+                          void *workspace, size_t workspace_bytes, void *stream, const int32_t *recent_lo_dev,
+                          const dc_step_args *step = nullptr);
 // sketch.hip: the quantising pass of dc_sketch_build_bf16
 int dc_sketch_quantise_launch(const char *who, const void *k, uint8_t *codes, const float *scale, float *resid,
                               int n_units, int n_h, int n_rows, int hd, int64_t sb, int64_t sh, int64_t sr, int64_t cb,
@@ -68,14 +69,70 @@ size_t dc_small_workspace_bytes(int n_units, int region, int group, int hd);
 size_t dc_small_cand_bytes(int n_units, int region);
 int dc_small_state_init(int n_units, int region, void *cand, void *stream);
 int dc_small_try(const dc_layer_args *a, int region, int k_eff, void *sel_ws, void *cand, void *attn_ws,
-                 size_t attn_ws_bytes, void *stream);
+                 size_t attn_ws_bytes, void *stream, const dc_step_args *step);
 bool dc_ws_state_trusted(const void *workspace);
 void dc_ws_state_initialised(const void *workspace);
+
+// kv.hip: the checks of dc_append_kv_bf16 on the append part of a step (DC_OK when there is none)
+int dc_step_check(const char *who, const dc_layer_args *a, const dc_step_args *step);
 
 static inline bool dc_aligned16(const void *p) { return (((uintptr_t)p) & 15u) == 0; }
 static inline size_t dc_align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // ---- device side -----------------------------------------------------------
+// dc_step_state_advance, by one thread
+__device__ __forceinline__ void dc_state_advance(int32_t *s, int delta, int limit) {
+    int64_t n = (int64_t)s[0] + delta;
+    if (n > limit) {  // the window is full: this token has no row (the caller had to roll it over)
+        s[3] = 1;
+        n = limit;
+    }
+    if (n < 0) n = 0;
+    s[0] = (int32_t)n;
+    s[2] = s[1] + (int32_t)n;
+}
+
+// The token's row on its way into the store (dc_append_kv_bf16 inside another kernel): HD/4 threads of one
+// block per unit carry 16 bytes each, the first half of K, the second of V.  load() goes in front of the
+// block's last reduction, where registers are free, and store() behind it, so that nothing waits for it
+// (in front of the gathered rows it costs the attention a fourth wave per SIMD).
+struct DcAppend {
+    uint16_t *k, *v;  // the stores (row 0 of unit (0, 0)); k null: nothing to append
+    const int32_t *pos_dev;
+    int64_t pos, pos_end;
+};
+inline DcAppend dc_append_of(const dc_step_args *step, const void *k, const void *v) {
+    DcAppend a = {nullptr, nullptr, nullptr, 0, 0};
+    if (step && step->append)
+        a = {(uint16_t *)const_cast<void *>(k), (uint16_t *)const_cast<void *>(v), step->pos_dev, step->pos, step->pos_end};
+    return a;
+}
+template <int HD>
+struct DcNewRow {
+    uint4 w;
+    int64_t at;  // uniform
+    bool live;
+    __device__ __forceinline__ void load(const DcAppend &a, const uint16_t *new_k, const uint16_t *new_v, int unit, bool mine) {
+        const int t = threadIdx.x;
+        mine = mine && a.k;
+        live = mine && t < HD / 4;
+        at = a.pos;
+        if (mine && a.pos_dev) at += (int64_t)*a.pos_dev;
+        if (live) {
+            const uint16_t *src = t < HD / 8 ? new_k : new_v;
+            w = *reinterpret_cast<const uint4 *>(src + (int64_t)unit * HD + (t % (HD / 8)) * 8);
+        }
+    }
+    // ku, vu: element offset of the unit's row 0 in the stores
+    __device__ __forceinline__ void store(const DcAppend &a, int64_t ku, int64_t ksr, int64_t vu, int64_t vsr) const {
+        const int t = threadIdx.x;
+        if (live && at >= 0 && at < a.pos_end) {
+            uint16_t *dst = t < HD / 8 ? a.k + ku + at * ksr : a.v + vu + at * vsr;
+            *reinterpret_cast<uint4 *>(dst + (t % (HD / 8)) * 8) = w;
+        }
+    }
+};
+
 // 16-byte load of data that is read once (the scans stream gigabytes through the
 // caches): the non-temporal hint keeps the lines from displacing what is reused, and the
 // streaming kernels reach the plain read rate of the part with it (about 8 % faster).

@@ -37,16 +37,7 @@ __global__ void step_advance_kernel(int32_t *counter, int delta, int limit) {
 
 // The step state of a sequence as four device words (dc_step_state in the header): one thread.
 __global__ void step_state_advance_kernel(int32_t *s, int delta, int limit) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        int64_t n = (int64_t)s[0] + delta;
-        if (n > limit) {  // the window is full: this token has no row (the caller had to roll it over)
-            s[3] = 1;
-            n = limit;
-        }
-        if (n < 0) n = 0;
-        s[0] = (int32_t)n;
-        s[2] = s[1] + (int32_t)n;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) dc_state_advance(s, delta, limit);
 }
 __global__ void step_state_rollover_kernel(int32_t *s, int moved, int keep) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -94,6 +85,16 @@ extern "C" int dc_append_kv_bf16(void *k_store, void *v_store, const void *new_k
                        (const uint16_t *)new_k, (const uint16_t *)new_v, n_h, hd, pos, pos_dev, pos_end, sb, sh,
                        sr, total);
     DC_CHECK_LAUNCH("dc_append_kv_bf16");
+    return DC_OK;
+}
+
+int dc_step_check(const char *who, const dc_layer_args *a, const dc_step_args *step) {
+    if (!step) return DC_OK;
+    DC_REQUIRE(!step->advance_state || step->advance_limit >= 0, "%s: negative limit", who);
+    if (!step->append) return DC_OK;
+    DC_REQUIRE(a->new_k && a->new_v, "%s: append without new_k and new_v", who);
+    DC_REQUIRE(step->pos >= 0 && step->pos < step->pos_end, "%s: append position %lld outside the store's %lld rows", who,
+               (long long)step->pos, (long long)step->pos_end);
     return DC_OK;
 }
 

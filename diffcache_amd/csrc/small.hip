@@ -72,6 +72,7 @@ struct SmallArgs {
     int spin_limit;
     uint32_t *mailbox;    // one word of pinned host memory (device address), or null: receives launch_seq when a wait runs out
     uint32_t launch_seq;  // never zero
+    DcAppend app;
 };
 
 __device__ __forceinline__ void stores_done() {
@@ -224,6 +225,7 @@ __global__ __launch_bounds__(kThreads) void small_layer_kernel(SmallArgs a) {
         if (a.lse && tid < G) a.lse[unit * G + tid] = __uint_as_float(0x7fc00000u);
         for (int i = tid; i < a.k_eff; i += kThreads) io[i] = 0xffffffffu;
     };
+    DcNewRow<HD> fresh;  // the token's row goes to the store with the unit's last block
     // ---------------- 1: scores of this block's rows ----------------
     for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
     if (tid < 4) s_cnt[tid] = 0;
@@ -270,6 +272,8 @@ __global__ __launch_bounds__(kThreads) void small_layer_kernel(SmallArgs a) {
     __syncthreads();
     if (s_bad != 0u) {  // every block of the unit sees the same word: none of them goes on
         poison();
+        fresh.load(a.app, a.new_k, a.new_v, unit, blk == a.bpu - 1);
+        fresh.store(a.app, b * a.sb + h * a.sh, a.sr, b * a.sb + h * a.sh, a.sr);
         return;
     }
     // What an addition returns -- the rows of that bucket counted before this block's -- is the
@@ -566,6 +570,7 @@ __global__ __launch_bounds__(kThreads) void small_layer_kernel(SmallArgs a) {
         sm.template absorb<R>(x, vw);
     }
 
+    fresh.load(a.app, a.new_k, a.new_v, unit, blk == a.bpu - 1);
     // the block's partial: combine its lane groups (the candidate list in LDS is dead)
     __syncthreads();
     float *s_red = reinterpret_cast<float *>(smem);  // [kAttnWaves][G]
@@ -608,6 +613,7 @@ __global__ __launch_bounds__(kThreads) void small_layer_kernel(SmallArgs a) {
         }
     }
     __syncthreads();
+    fresh.store(a.app, b * a.sb + h * a.sh, a.sr, b * a.sb + h * a.sh, a.sr);
     const int n_splits = a.bpu;
     const int64_t slot = (int64_t)unit * n_splits + blk;
     for (int o = tid; o < G * HD; o += kThreads) {
@@ -992,7 +998,7 @@ int dc_small_state_init(int n_units, int region, void *cand, void *stream) {
 // left ready by the previous call; cand: dc_small_cand_bytes(...) bytes, every slot empty;
 // attn_ws: dc_small_workspace_bytes(...) bytes.
 int dc_small_try(const dc_layer_args *a, int region, int k_eff, void *sel_ws, void *cand, void *attn_ws,
-                 size_t attn_ws_bytes, void *stream) {
+                 size_t attn_ws_bytes, void *stream, const dc_step_args *step) {
     const char *who = "dc_decode_layer(one kernel)";
     const int n_units = a->n_b * a->n_h;
     const SmallPlan p = plan_small(n_units, region);
@@ -1090,6 +1096,7 @@ int dc_small_try(const dc_layer_args *a, int region, int k_eff, void *sel_ws, vo
     s.mailbox = d.mail_dev;
     if (++g_launch_seq == 0u) g_launch_seq = 1u;
     s.launch_seq = g_launch_seq;
+    s.app = dc_append_of(step, a->k, a->v);
     dim3 grid((unsigned)(n_units * p.bpu));
     int rc;
     if (a->hd == 64) rc = launch_small<64>(a->group, grid, st, s);

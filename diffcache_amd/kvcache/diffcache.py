@@ -415,19 +415,22 @@ class DiffCache:
         hi_cap = self.max_length - self.kvbuf_suffix_maxlen
         if dev_region:
             # the token's row is the device's append position; never past the end of the store
-            hip.append_kv(self.kstore[layer_idx], self.vstore[layer_idx], nk, nv, 0, pos_dev=self._state[2:3],
-                          pos_end=self.max_length)
+            append = (0, self._state[2:3], self.max_length)
         else:
             # the token's row: hi + (device-side window length); never past the window's capacity
-            hip.append_kv(self.kstore[layer_idx], self.vstore[layer_idx], nk, nv, hi, pos_dev=self.step_state,
-                          pos_end=min(hi + self.kvbuf_suffix_maxlen, self.max_length))
+            append = (hi, self.step_state, min(hi + self.kvbuf_suffix_maxlen, self.max_length))
+        last = layer_idx == self.num_layers - 1
         if out is None:
             if self._attn_out is None:
                 self._attn_out = torch.empty((b, hq, hd), device=self.device, dtype=torch.bfloat16)
             out = self._attn_out
         ws = self._ensure_workspace()
         if self.use_k_check and min(hi - lo, self.retrieval_budget) > 0:
+            hip.append_kv(self.kstore[layer_idx], self.vstore[layer_idx], nk, nv, append[0], pos_dev=append[1],
+                          pos_end=append[2])
             self._decode_attention_k_check(layer_idx, q, nk, nv, out, ws)
+            if last:
+                hip.step_state_advance(self._state, 1, self.kvbuf_suffix_maxlen)
         else:
             # attended: [selected | prefix | the window's rows before this token | this token]
             # (a call with the region's end on the device has other launch sizes than one without:
@@ -439,15 +442,14 @@ class DiffCache:
                              select_state_ready=self._ws_ready and self._ws_order == tag,
                              sketch=self.sketch[layer_idx], n_recent_dev=self.step_state,
                              one_kernel=self.one_kernel,
-                             region_hi_dev=self._state[1:2] if dev_region else None)
+                             region_hi_dev=self._state[1:2] if dev_region else None, append=append,
+                             advance=(self._state, self.kvbuf_suffix_maxlen) if last else None)
             self._ws_ready = True
             self._ws_order = tag        # the state is left ready for a call of the same kind only
             self._hook_ws_ready = False
-        if layer_idx == self.num_layers - 1:
-            hip.step_state_advance(self._state, 1, self.kvbuf_suffix_maxlen)
-            if not capturing:       # a captured step is counted when it is replayed (advance_host_step)
-                self.kvbuf_suffix_len += 1
-                self._store_suffix_rows += 1
+        if last and not capturing:  # a captured step is counted when it is replayed (advance_host_step)
+            self.kvbuf_suffix_len += 1
+            self._store_suffix_rows += 1
         return out
 
     def _note_failures(self) -> None:

@@ -416,6 +416,24 @@ typedef struct dc_layer_args {
 size_t dc_layer_workspace_bytes(int n_units, int n_region_rows, int budget, int group, int hd,
                                 int n_rows_attended);
 int dc_decode_layer(const dc_layer_args *args, void *stream);
+
+/*
+ * dc_decode_layer together with what a decode step does around it, in the same launches: the
+ * token's row into the store (dc_append_kv_bf16 of new_k / new_v; the row must lie outside the
+ * rows this call scans and attends to, as the next free row of the recent window does) and, in the call of the last layer,
+ * the step state (dc_step_state_advance by one), which may be the words n_recent_dev,
+ * region_hi_dev and pos_dev point into: the call reads them as they were before.  step == NULL: dc_decode_layer.
+ * Replaces the insert and the kvbuf_suffix_len bookkeeping around the attention call
+ * (diffcache_cpu/src/lib.rs:352-369, src/diffcache/kvcache/diffcache.py:221-223).
+ */
+typedef struct dc_step_args {
+    int append;              /* 0: the store is left alone */
+    int advance_limit;       /* window capacity, the limit of dc_step_state_advance */
+    int64_t pos, pos_end;    /* as in dc_append_kv_bf16 */
+    const int32_t *pos_dev;
+    int32_t *advance_state;  /* NULL, or the dc_step_state to advance */
+} dc_step_args;
+int dc_decode_layer_step(const dc_layer_args *args, const dc_step_args *step, void *stream);
 /*
  * Short contexts.  With scores == NULL, order == DC_ORDER_ANY and at most 640 Ki region rows
  * over all units (and, when a sketch is passed, whose chain of kernels is the faster one, at most
