@@ -222,28 +222,12 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
                        surv + (int64_t)unit * n_cap, refresh, (uint32_t)k_eff);
 }
 
-// sum over aligned groups of LPR lanes (4, 8 or 16)
+// largest value of aligned groups of LPR lanes (8, 16 or 32), in every lane of the group
 template <int LPR>
-__device__ __forceinline__ float sketch_group_sum(float v) {
-    if (LPR == 4) {
-        v += __builtin_amdgcn_update_dpp(0.0f, v, 0xB1, 0xF, 0xF, true);  // quad_perm [1,0,3,2]
-        v += __builtin_amdgcn_update_dpp(0.0f, v, 0x4E, 0xF, 0xF, true);  // quad_perm [2,3,0,1]
-        return v;
-    }
-    return dc_group_sum<(LPR == 8 ? 8 : 16)>(v);
-}
-
-// 16 code bytes (value + 128) times 16 weights, added to acc
-__device__ __forceinline__ float sketch_dot16(const uint4 &c, const float (&w)[16], float acc) {
-    const uint32_t x[4] = {c.x, c.y, c.z, c.w};
+__device__ __forceinline__ float group_max(float v) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        acc = fmaf((float)(x[i] & 0xffu), w[4 * i + 0], acc);
-        acc = fmaf((float)((x[i] >> 8) & 0xffu), w[4 * i + 1], acc);
-        acc = fmaf((float)((x[i] >> 16) & 0xffu), w[4 * i + 2], acc);
-        acc = fmaf((float)(x[i] >> 24), w[4 * i + 3], acc);
-    }
-    return acc;
+    for (int off = 1; off < LPR; off <<= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+    return v;
 }
 
 // Scan of the 8-bit sketch of the keys.  Row i of a unit is stored as codes
@@ -258,6 +242,20 @@ __device__ __forceinline__ float sketch_dot16(const uint4 &c, const float (&w)[1
 // yields the bucket of A_k exactly as in score_prune_kernel, and a row is kept when
 // bucket(approx_i + margin) is not worse than the running threshold bucket,
 // margin = 2E' + Q.  The kept rows are rescored exactly by rescore_kernel.
+//
+// The sums run on the matrix cores.  A weight q_d a_d is a whole multiple of 2^(e - 30), |q_d a_d| < 2^e, written
+// as four signed digits of base 256; the codes less 128 are signed bytes; so v_mfma_i32_16x16x64_i8 sums every
+// digit exactly and three fp32 additions put them together.  (Largest error against 64 bits, relative to
+// sum |q_d a_d|: 5.5e-6 / 5.2e-6 / 3.4e-6 at head dims 64 / 128 / 256; 16 fp32 additions a lane and a tree over the
+// lanes, biased codes, gave 1.6e-5 / 1.4e-5 / 7.4e-6.)  Sixteen query columns would fit where one is
+// wanted: the sixteen rows of the left operand hold the digits instead, several times over with zeros elsewhere, so
+// that a wave's 64 rows end up one to a lane.  From 128 columns on two lanes share a row (S = 2), because a load of
+// 16 rows x 64 bytes takes half lines, which streaming loads fetch twice (205 us instead of 180 us at 64 units x
+// 131004 rows of 128).  A step of 64 rows takes about a third of the vector instructions that fp32 arithmetic on the
+// codes took; the kernel is bound by memory latency at few units and by HBM at many.  The first rows, the
+// query, scales and residuals are all requested at the block's start, one round trip instead of three.
+// Measured before / after (kernel trace): 8 x 131004 rows of 128 29.8 / 27.3 us, 4 x 127028 19.6 / 17.7, 64 x 131004
+// 185.1 / 180.8, 8 x 1048508 183.1 / 179.1, 8 x 16323 of 64 11.1 / 9.5.
 constexpr uint32_t kBulkKeep = 96;      // of the 128 rows of a wave's first two steps
 // What the sketch scan keeps of a row: the row, and the bucket of (approximation + margin), which
 // is all the exact pass asks of it (the exact pass keeps the row when that bucket is not worse
@@ -276,9 +274,15 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     uint2 *__restrict__ surv, int n_units, int n_h, int n_cap, int64_t cb, int64_t ch, int64_t cr,
     int q_group, int mode, int k_eff, int small_chunks, int big_steps, const int32_t *__restrict__ hi_dev,
     int lo_row) {
-    constexpr int LPR = HD / 16;  // lanes per row, 16 code bytes each
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    constexpr int S = HD == 64 ? 1 : 2;   // lanes of 16 that share a row: a load takes whole 128-byte lines
+    constexpr int KS = HD / (64 * S);     // matrix instructions per tile of 16 / S rows
+    constexpr int TILES = 4 * S;          // tiles of a wave's 64 rows
+    constexpr int kLoads = TILES * KS;    // 16-byte loads of a lane per step
+    constexpr int LPQ = HD / 8;           // lanes that hold a copy of the weights, eight each
     const int n_rows = dc_live_rows(n_cap, hi_dev, lo_row);
     __shared__ uint32_t lhist[DC_HIST_BINS];
+    __shared__ __align__(16) uint8_t s_w[4][HD];  // the weights' digits, lowest first
     __shared__ uint32_t stage[kStage];  // kept rows as kSketchEntry words
     __shared__ uint32_t s_tb;  // the block's copy of the unit's running threshold bucket
     __shared__ uint32_t wtot[kThreads / 64 + 1];
@@ -290,7 +294,9 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     const int b = unit / n_h, h = unit % n_h;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const int grp = lane / LPR, col = lane % LPR;
+    // This lane loads 16 columns of row (lane & 15) / S of every tile; the row whose score it ends up with:
+    const int grp = lane >> 4, side = S == 1 ? 0 : lane & 1, par = S == 1 ? 0 : (grp ^ lane) & 1;
+    const int own_row = S == 1 ? lane : (4 * side + 2 * par + (grp >> 1)) * 8 + ((lane & 15) >> 1);
 
     const bool small = chunk < small_chunks;
     const int big_chunks = (int)(gridDim.x / n_units) - small_chunks;
@@ -303,53 +309,10 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     if (block_row0 >= n_rows) return;  // the grid is laid out for n_cap rows
     for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
 
-    const uint8_t *Cu = C + b * cb + h * ch + col * 16;
+    const uint8_t *Cu = C + b * cb + h * ch + (grp * S + side) * 16;
     UnitState *st = state + unit;
     const int last = n_rows - 1;
     uint32_t tb = load_relaxed(&st->tb_run);
-
-    // this lane's 16 weights q_d * a_d, the bias of the +128 code offset, and the margin
-    float w[16];
-    float bias, margin;
-    {
-        float qv[16];
-        {
-            float t[8];
-            dc_load_query<HD>(Q, unit, q_group, 2 * col, t);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) qv[i] = t[i];
-            dc_load_query<HD>(Q, unit, q_group, 2 * col + 1, t);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) qv[8 + i] = t[i];
-        }
-        const float4 *ap = reinterpret_cast<const float4 *>(scale + (int64_t)unit * HD + col * 16);
-        const float4 *rp = reinterpret_cast<const float4 *>(resid + (int64_t)unit * HD + col * 16);
-        float wsum = 0.f, wabs = 0.f, e = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 a4 = ap[i], r4 = rp[i];
-            const float av[4] = {a4.x, a4.y, a4.z, a4.w}, rv[4] = {r4.x, r4.y, r4.z, r4.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float ww = qv[4 * i + j] * av[j];
-                w[4 * i + j] = ww;
-                wsum += ww;
-                wabs += fabsf(ww);
-                e += fabsf(qv[4 * i + j]) * rv[j];
-            }
-        }
-        bias = -128.0f * wsum;
-        wabs = sketch_group_sum<LPR>(wabs);
-        e = sketch_group_sum<LPR>(e);
-        margin = dc_sketch_margin(e, wabs, mode);
-    }
-    if (chunk == 0 && tid == 0) st->margin = __float_as_uint(margin);
-    if (tid == 0) s_tb = tb;
-    __syncthreads();
-
-    uint32_t *wstage = stage + wave * (kBigSteps * 64);
-    uint32_t wcnt = 0, marginal = 0;
-    const unsigned long long lt = (1ull << lane) - 1ull;
 
     // Double buffering: the loads of the next step are issued before the current step is
     // worked on, so a wave always has a step's worth of bytes in flight.  The loads are
@@ -357,26 +320,126 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     // compiler wait for exactly the older buffer instead of for every load in flight.
     const int64_t blk_end = block_row0 + (int64_t)steps * kRowsPerBlockStep - 1;
     const int64_t blk_last = blk_end < (int64_t)last ? blk_end : (int64_t)last;
-    auto load_step = [&](int step, uint4 (&cv)[LPR]) __attribute__((always_inline)) {
+    auto load_step = [&](int step, uint4 (&cv)[kLoads]) __attribute__((always_inline)) {
         const int64_t row0 = block_row0 + (int64_t)step * kRowsPerBlockStep + wave * 64;
 #pragma unroll
-        for (int j = 0; j < LPR; ++j) {
-            int64_t r = row0 + grp * LPR + j;
+        for (int t = 0; t < TILES; ++t) {
+            int64_t r = row0 + t * (16 / S) + (lane & 15) / S;
             r = r > blk_last ? blk_last : r;
-            cv[j] = dc_load_stream16(Cu + r * cr);
+            const uint8_t *p = Cu + r * cr;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) cv[t * KS + ks] = dc_load_stream16(p + ks * (64 * S));
         }
     };
+
+    // the first rows are under way while the weights are worked out
+    uint4 ca[kLoads], cb2[kLoads];
+    load_step(0, ca);
+
+    // The weights q_d * a_d as whole multiples of 2^w_exp, |multiple| < 2^30, in four signed digits
+    // of base 256, and the margin.  Every wave works them out for itself and leaves one digit
+    // in LDS for all.
+    int w_exp;
+    float margin, poison;
+    {
+        const int col = lane % LPQ;
+        const float4 *ap = reinterpret_cast<const float4 *>(scale + (int64_t)unit * HD + col * 8);
+        const float4 *rp = reinterpret_cast<const float4 *>(resid + (int64_t)unit * HD + col * 8);
+        const float4 as[2] = {ap[0], ap[1]}, rs[2] = {rp[0], rp[1]};  // requested with the query, not behind it
+        float qv[8];
+        dc_load_query<HD>(Q, unit, q_group, col, qv);
+        float w[8];
+        float wabs = 0.f, wmax = 0.f, e = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float av[4] = {as[i].x, as[i].y, as[i].z, as[i].w}, rv[4] = {rs[i].x, rs[i].y, rs[i].z, rs[i].w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float ww = qv[4 * i + j] * av[j];
+                w[4 * i + j] = ww;
+                wabs += fabsf(ww);
+                wmax = fmaxf(wmax, fabsf(ww));
+                e += fabsf(qv[4 * i + j]) * rv[j];
+            }
+        }
+        wabs = dc_group_sum<LPQ>(wabs);
+        e = dc_group_sum<LPQ>(e);
+        wmax = group_max<LPQ>(wmax);
+        margin = dc_sketch_margin(e, wabs, mode);
+        // weights that are not finite leave every approximation undefined: such rows are kept
+        poison = wabs < __builtin_inff() ? 0.f : __uint_as_float(0x7fc00000u);
+        w_exp = __builtin_amdgcn_frexp_expf(wmax) - 30;
+        uint32_t dig[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)  // one digit per byte: carries out of the lower three are settled by the addition
+            dig[i] = (((uint32_t)(int)rintf(__builtin_amdgcn_ldexpf(w[i], -w_exp)) + 0x00808080u) ^ 0x00808080u) >> (8 * wave);
+        if (lane < LPQ) {
+            uint2 pk;
+            pk.x = (dig[0] & 0xffu) | ((dig[1] & 0xffu) << 8) | ((dig[2] & 0xffu) << 16) | (dig[3] << 24);
+            pk.y = (dig[4] & 0xffu) | ((dig[5] & 0xffu) << 8) | ((dig[6] & 0xffu) << 16) | (dig[7] << 24);
+            *reinterpret_cast<uint2 *>(&s_w[wave][col * 8]) = pk;
+        }
+    }
+    if (chunk == 0 && tid == 0) st->margin = __float_as_uint(margin);
+    if (tid == 0) s_tb = tb;
+    __syncthreads();
+    // The left operands: row m of 16 is digit m % 4 of the weights of one S-th of the columns, or zero.
+    // S = 1: block t of four rows for tile t.  S = 2: rows 0-7 for even tiles and 8-15 for odd ones, a
+    // block for the columns of even lanes and one for those of odd lanes, in this order or the other.
+    constexpr int kOps = 4;
+    i32x4 wd[kOps][KS];
+    {
+        const int m = lane & 15, blk = m >> 2;
+#pragma unroll
+        for (int o = 0; o < kOps; ++o) {
+            const int part = S == 1 ? 0 : (blk & 1) ^ (o >> 1);
+            const bool on = S == 1 ? blk == o : (blk >> 1) == (o & 1);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const i32x4 v = *reinterpret_cast<const i32x4 *>(&s_w[m & 3][ks * (64 * S) + (grp * S + part) * 16]);
+                wd[o][ks] = on ? v : i32x4{0, 0, 0, 0};
+            }
+        }
+    }
+
+    uint32_t *wstage = stage + wave * (kBigSteps * 64);
+    uint32_t wcnt = 0, marginal = 0;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+
     // COUNT: also count the rows kept although their own bucket is not better than the
     // threshold's (ties and near-ties); only the first two steps of a wave do.
-    auto work_step = [&](int step, const uint4 (&cv)[LPR], auto count) __attribute__((always_inline)) {
+    auto work_step = [&](int step, const uint4 (&cv)[kLoads], auto count) __attribute__((always_inline)) {
         const int64_t row0 = block_row0 + (int64_t)step * kRowsPerBlockStep + wave * 64;
-        float mine = 0.f;
+        // Register i of a lane receives the sum of digit i for its column; tiles whose operands differ share an accumulator.
+        constexpr int NACC = S == 1 ? 1 : 4;
+        i32x4 ds[NACC];
 #pragma unroll
-        for (int j = 0; j < LPR; ++j) {
-            const float p = sketch_group_sum<LPR>(sketch_dot16(cv[j], w, bias));
-            mine = (col == j) ? p : mine;
+        for (int d = 0; d < NACC; ++d) ds[d] = i32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const int d = S == 1 ? 0 : t >> 1, o = S == 1 ? t : 2 * ((t >> 1) & 1) + (t & 1);
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                const uint4 c = cv[t * KS + ks];
+                const i32x4 cs = {(int)(c.x ^ 0x80808080u), (int)(c.y ^ 0x80808080u), (int)(c.z ^ 0x80808080u),
+                                  (int)(c.w ^ 0x80808080u)};
+                ds[d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wd[o][ks], cs, ds[d], 0, 0, 0);
+            }
         }
-        const int64_t myrow = row0 + lane;
+        auto value = [&](const i32x4 &v) __attribute__((always_inline)) {
+            return fmaf(fmaf(fmaf((float)v[3], 256.f, (float)v[2]), 256.f, (float)v[1]), 256.f, (float)v[0]);
+        };
+        float mine;
+        if constexpr (S == 1) {
+            mine = value(ds[0]);
+        } else {
+            // two halves of two rows, whose other halves are in lane ^ 17: keep one row, hand over the other
+            const float v0 = value(par ? ds[1] : ds[0]), v1 = value(par ? ds[3] : ds[2]);
+            const int give = __float_as_int(side ? v0 : v1);
+            mine = (side ? v1 : v0) + __int_as_float(__builtin_amdgcn_ds_swizzle(give, (17 << 10) | 0x1f));
+        }
+        mine = __builtin_amdgcn_ldexpf(mine, w_exp) + poison;
+        const int64_t myrow = row0 + own_row;
         const bool valid = myrow < n_rows;
         const uint32_t lb = dc_score_bucket(mine), kb = dc_score_bucket(mine + margin);
         const bool keep = valid && kb <= tb;
@@ -396,8 +459,6 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
             my_steps = my_steps < steps ? my_steps : steps;
         }
     }
-    uint4 ca[LPR], cb2[LPR];
-    load_step(0, ca);
     bool bulk = false;
     const bool had_tb = tb < (uint32_t)DC_HIST_BINS;  // the first steps are judged against a real threshold
     // The threshold poll is issued before the prefetch: loads return in order, so waiting
