@@ -238,33 +238,61 @@ __global__ __launch_bounds__(kThreads) void small_layer_kernel(SmallArgs a) {
     __syncthreads();
     {
         const int grp = lane / LPR, col = lane % LPR;
-        float q[8];
-        dc_load_query<HD>(a.Q, unit, G, col, q);
         const uint16_t *Ku = Kb + (int64_t)a.n_sink * a.sr + col * 8;  // the region starts after the sinks
         const int64_t last = r1 - 1;
-        for (int64_t row0 = r0 + wave * 64; row0 < r1; row0 += kRowsPerBlockStep) {
-            float mine = 0.f;
+        // A wave takes 64 rows in NC parts of CH loads a lane.  Up to 128 columns the first part is requested before
+        // the query, so that the two share a memory round trip, and the next one before the current one is
+        // worked on (8 units x 32533 rows of 128: 37.1 -> 36.0 us).  At 256 columns, two parts a step, both only
+        // add pressure (12 units x 24615 rows: 53.0 us against 49.9 us for one part at a time behind the query).
+        // (Past the block's last row the loads repeat it.)
+        constexpr int NC = LPR / CH;
+        const int64_t first = r0 + wave * 64;
+        auto load_part = [&](int i, uint4 (&w)[CH]) __attribute__((always_inline)) {
+            const int64_t row = first + (int64_t)(i / NC) * kRowsPerBlockStep + grp * LPR + (i % NC) * CH;
 #pragma unroll
-            for (int c0 = 0; c0 < LPR; c0 += CH) {
-                uint4 w[CH];
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    int64_t r = row0 + grp * LPR + c0 + j;
-                    r = r > last ? last : r;
-                    w[j] = *reinterpret_cast<const uint4 *>(Ku + r * a.sr);
-                }
-#pragma unroll
-                for (int j = 0; j < CH; ++j) {
-                    const float p = dc_group_sum<LPR>(dc_dot8(w[j], q, 0.f));
-                    mine = (col == c0 + j) ? p : mine;
-                }
+            for (int j = 0; j < CH; ++j) {
+                const int64_t r = row + j > last ? last : row + j;
+                w[j] = *reinterpret_cast<const uint4 *>(Ku + r * a.sr);
             }
-            const int64_t myrow = row0 + lane;
+        };
+        uint4 wa[CH];
+        if (NC == 1) load_part(0, wa);
+        float q[8];
+        dc_load_query<HD>(a.Q, unit, G, col, q);
+        float mine = 0.f;
+        auto work_part = [&](int i, int part, const uint4 (&w)[CH]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const float p = dc_group_sum<LPR>(dc_dot8(w[j], q, 0.f));
+                mine = (col == part * CH + j) ? p : mine;
+            }
+            if (part != NC - 1) return;
+            const int64_t myrow = first + (int64_t)(i / NC) * kRowsPerBlockStep + lane;
             if (myrow < r1) {
                 s_scores[myrow - r0] = mine;
                 uint32_t key, bucket;
                 dc_key_bucket(mine, a.mode, key, bucket);
                 atomicAdd(&lhist[bucket], 1u);
+            }
+        };
+        const int n_parts = first < r1 ? (int)((r1 - first + kRowsPerBlockStep - 1) / kRowsPerBlockStep) * NC : 0;
+        if constexpr (NC == 1) {
+            uint4 wb[CH];
+            int i = 0;
+            for (; i + 1 < n_parts; i += 2) {
+                load_part(i + 1, wb);
+                work_part(i, 0, wa);
+                load_part(i + 2, wa);
+                work_part(i + 1, 0, wb);
+            }
+            if (i < n_parts) work_part(i, 0, wa);
+        } else {
+            for (int i = 0; i < n_parts; i += NC) {
+#pragma unroll
+                for (int part = 0; part < NC; ++part) {
+                    load_part(i + part, wa);
+                    work_part(i + part, part, wa);
+                }
             }
         }
     }
