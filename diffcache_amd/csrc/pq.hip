@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
         float half = 0.f;
 #pragma unroll
         for (int d = 0; d < DS; ++d) half = fmaf(cen[d], cen[d], half);
-        half = tid < nc ? 0.5f * half : 3.0e38f;  // a centroid that does not exist is never the nearest
+        half = tid < nc ? 0.5f * half : INFINITY;  // a centroid that does not exist is never the nearest, of no key
         if (s > 0) __syncthreads();               // the last subspace's tables are no longer read
         s_half[half_slot] = half;
 #pragma unroll

@@ -35,6 +35,25 @@ def test_pq_encode_picks_a_nearest_centroid(n, m, ds, nc):
         assert (exact != codes).float().mean() < 1e-3
 
 
+@pytest.mark.parametrize("ds,nc", [(4, 17), (8, 33), (4, 255)])
+def test_pq_encode_names_an_existing_centroid_for_any_key(ds, nc):
+    """Keys whose products leave the range of fp32, and infinite and undefined ones, get the number of a
+    centroid that exists, and leave the other keys' codes as they were."""
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(nc)
+    x = torch.randn((600, 3 * ds), generator=g, device=DEV).to(torch.bfloat16)
+    books = torch.randn((3, nc, ds), generator=g, device=DEV).abs() + 1.0
+    plain = hip.pq_encode(x, books)
+    odd = x.clone()
+    for row, value in ((0, -3.3e38), (5, 3.3e38), (17, float("inf")), (33, float("-inf")), (64, float("nan"))):
+        odd[row] = value
+        odd[row + 300, 1] = value
+    codes = hip.pq_encode(odd, books)
+    assert int(codes.max()) < nc
+    same = (odd == x).all(dim=1)
+    assert torch.equal(codes[same], plain[same])
+
+
 def test_encode_takes_what_it_took_before():
     """fp32 keys and subspace widths the kernel is not built for still go through torch's distances."""
     from diffcache_amd.pq import encode
