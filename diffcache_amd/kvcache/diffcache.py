@@ -160,12 +160,11 @@ class DiffCache:
                     for _ in range(num_layers)]
         self._ws: Optional[torch.Tensor] = None
         self._ws_rows = -1
-        # The select state inside the workspace is laid out differently by dc_decode_layer and
-        # by the stand-alone select calls, so each route keeps its own "left ready" flag and
-        # clears the other's.
-        self._ws_ready = False        # a decode_attention call has left its select state ready
-        self._ws_order = None         # ... for calls of this id order
-        self._hook_ws_ready = False   # a decode_query_kvcache call (sketch route) has
+        # The kind of call the workspace's select state was left ready for, with the sizes that its layout
+        # goes by, or None.  dc_decode_layer and the stand-alone select calls lay it out differently, and
+        # the one-kernel route's candidate slots begin behind buffers whose size goes with the
+        # region: only a call of the same kind over the same region finds it ready.
+        self._ws_state: Optional[tuple] = None
         self._attn_out: Optional[torch.Tensor] = None
         # k-check (nsw.rs:198-296): with use_k_check, decode_attention attends only to the
         # leading rows of each unit's best-first list that the check finds sufficient
@@ -219,9 +218,15 @@ class DiffCache:
                 hip.layer_workspace_bytes(n_units, cap, self.retrieval_budget, self.group,
                                           self.head_dim, attended), self.device)
             self._ws_rows = cap
-            self._ws_ready = False
-            self._hook_ws_ready = False
+            self._ws_state = None
         return self._ws
+
+    def _take_state(self, kind: tuple) -> bool:
+        """Whether the workspace's select state is ready for a call of this kind.  The caller notes the kind
+        in _ws_state again once the call is enqueued: one that raised half-way has left nothing ready."""
+        ready = self._ws_state == kind
+        self._ws_state = None
+        return ready
 
     def _set_suffix_len(self, n: int) -> None:
         """Window length and, from the host's view of the region, the whole device-side state."""
@@ -281,8 +286,6 @@ class DiffCache:
         self.kvbuf_suffix_len = keep
         hip.step_state_rollover(self._state, moved, keep)      # the device's view, in stream order
         self._store_suffix_rows = keep
-        self._ws_ready = False
-        self._hook_ws_ready = False
         self.generation += 1
         for l in range(self.num_layers):
             if self.data_layers[l] is not None:
@@ -352,15 +355,15 @@ class DiffCache:
             lo, hi = self._region()
             ws = self._ensure_workspace()
             if self.key_sketch:
+                ready = self._take_state(("select", lo, hi))
                 hip.score_select_sketch(self.kstore[layer_idx], self.sketch[layer_idx], self.qbuf, lo, hi - lo,
                                         retrieval_len, self.mode, self.hook_order, idx_out=self.idx[layer_idx],
-                                        workspace=ws, state_ready=self._hook_ws_ready)
-                self._hook_ws_ready = True
+                                        workspace=ws, state_ready=ready)
+                self._ws_state = ("select", lo, hi)
             else:
+                self._ws_state = None   # the one-shot call does not leave the state initialised
                 hip.score_select(self.kstore[layer_idx], self.qbuf, lo, hi - lo, retrieval_len, self.mode,
                                  self.hook_order, idx_out=self.idx[layer_idx], workspace=ws)
-                self._hook_ws_ready = False   # the one-shot call does not leave the state initialised
-            self._ws_ready = False
         hip.require(self.kvbuf_suffix_len < self.kvbuf_suffix_maxlen,
                     "the recent window is full (kvbuf_suffix_maxlen)")       # diffcache.py:221
         if layer_idx == self.num_layers - 1:
@@ -435,18 +438,17 @@ class DiffCache:
             # attended: [selected | prefix | the window's rows before this token | this token]
             # (a call with the region's end on the device has other launch sizes than one without:
             #  neither leaves the select state ready for the other)
-            tag = (order, dev_region)
+            tag = ("layer", order, dev_region, lo, hi)
+            ready = self._take_state(tag)
             hip.decode_layer(q, self.kstore[layer_idx], self.vstore[layer_idx], lo, hi_cap if dev_region else hi,
                              self.kvbuf_suffix_maxlen, self.retrieval_budget, None, self.idx[layer_idx], out, ws,
                              nk, nv, mode=self.mode, order=order,
-                             select_state_ready=self._ws_ready and self._ws_order == tag,
+                             select_state_ready=ready,
                              sketch=self.sketch[layer_idx], n_recent_dev=self.step_state,
                              one_kernel=self.one_kernel,
                              region_hi_dev=self._state[1:2] if dev_region else None, append=append,
                              advance=(self._state, self.kvbuf_suffix_maxlen) if last else None)
-            self._ws_ready = True
-            self._ws_order = tag        # the state is left ready for a call of the same kind only
-            self._hook_ws_ready = False
+            self._ws_state = tag
         if last and not capturing:  # a captured step is counted when it is replayed (advance_host_step)
             self.kvbuf_suffix_len += 1
             self._store_suffix_rows += 1
@@ -462,8 +464,7 @@ class DiffCache:
         if n != self._errors_seen:
             self.failed_steps += n - self._errors_seen
             self._errors_seen = n
-            self._ws_ready = False
-            self._hook_ws_ready = False
+            self._ws_state = None
             self.one_kernel = hip.ONE_KERNEL_NEVER
 
     def _decode_attention_k_check(self, layer_idx: int, q: torch.Tensor, nk: torch.Tensor, nv: torch.Tensor,
@@ -475,15 +476,15 @@ class DiffCache:
         n_units = self.batch_size * self.num_kv_heads
         ks, vs, idx = self.kstore[layer_idx], self.vstore[layer_idx], self.idx[layer_idx]
         if self.key_sketch:
+            ready = self._take_state(("select", lo, hi))
             hip.score_select_sketch(ks, self.sketch[layer_idx], q, lo, hi - lo, n_sel, self.mode,
                                     hip.ORDER_BEST, q_group=self.group, idx_out=idx, workspace=ws,
-                                    state_ready=self._hook_ws_ready)
-            self._hook_ws_ready = True
+                                    state_ready=ready)
+            self._ws_state = ("select", lo, hi)
         else:
+            self._ws_state = None
             hip.score_select(ks, q, lo, hi - lo, n_sel, self.mode, hip.ORDER_BEST, q_group=self.group,
                              idx_out=idx, workspace=ws)
-            self._hook_ws_ready = False
-        self._ws_ready = False
         hip.group_mean(q, self.group, out=self.qbuf.view(-1, self.head_dim), hd=self.head_dim)
         if self._kc_scores is None or self._kc_scores.shape[1] != n_sel:
             self._kc_scores = torch.empty((n_units, n_sel), device=self.device, dtype=torch.float32)

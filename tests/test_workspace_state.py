@@ -1,0 +1,161 @@
+"""When DiffCache tells a call that the workspace's select state is ready: only when the last call on the
+workspace was of the same kind over the same region (dc_layer_args.select_state_ready).  The native calls are
+replaced by recorders, so the rule runs without a GPU; the GPU tests below compare results."""
+import pytest
+import torch
+
+LAYERS, WINDOW = 2, 16
+
+
+class Layer:
+    """Stands in for the data layer, which needs a GPU."""
+
+    def __init__(self, **kw):
+        self.ctx_len = 0
+
+    def load(self, path, ctx_len):
+        pass
+
+    def update_r_sq(self, r_sq):
+        pass
+
+
+@pytest.fixture
+def recorded(monkeypatch):
+    """(make, calls, capture): a cache on the CPU; what its calls were told; a switch for "under capture"."""
+    from diffcache_amd.kvcache import diffcache as mod
+    calls, capture = [], []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(capture))
+    monkeypatch.setattr(mod, "DiffCacheHIP", Layer)
+    for name in ("prefill_layer", "append_kv", "step_state_advance", "step_state_rollover", "group_mean"):
+        monkeypatch.setattr(mod.hip, name, lambda *a, **k: None)
+    monkeypatch.setattr(mod.hip.Sketch, "build", lambda self, *a, **k: self)
+    monkeypatch.setattr(mod.hip, "decode_layer", lambda *a, **k: calls.append(k["select_state_ready"]))
+    monkeypatch.setattr(mod.hip, "score_select_sketch", lambda *a, **k: calls.append(k["state_ready"]))
+    monkeypatch.setattr(mod.hip, "score_select", lambda *a, **k: None)
+
+    def make(**kw):
+        return mod.DiffCache(num_layers=LAYERS, batch_size=1, max_length=4000, num_kv_heads=2, num_q_heads=4, head_dim=64,
+                             retrieval_budget=64, nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8,
+                             kvbuf_suffix_maxlen=WINDOW, attn_mass_threshold=0.9, k_check_seq=[100],
+                             r_sq=[[4.0, 4.0]] * LAYERS, device="cpu", **kw)
+    return make, calls, capture
+
+
+def prefill(cache, n):
+    k = torch.zeros((1, n, 2, 64), dtype=torch.bfloat16)
+    for l in range(LAYERS):
+        cache.prefill_update_kv_cache(k, k, l)
+
+
+def step(cache, **kw):
+    q, k = torch.zeros((1, 4, 64), dtype=torch.bfloat16), torch.zeros((1, 1, 2, 64), dtype=torch.bfloat16)
+    for l in range(LAYERS):
+        cache.decode_attention(l, q, k, k, **kw)
+
+
+def hook_step(cache):
+    for l in range(LAYERS):
+        cache.decode_query_kvcache(l)
+
+
+@pytest.mark.parametrize("one_step", [step, hook_step])
+def test_a_prompt_of_another_length_finds_no_state_ready(recorded, one_step):
+    make, calls, _ = recorded
+    cache = make()
+    for n in (3000, 700, 2000, 2000):
+        prefill(cache, n)
+        one_step(cache)
+        one_step(cache)
+    first, same = [False, True, True, True], [True] * 4
+    assert calls == first + first + first + same
+
+
+def test_a_loaded_snapshot_of_another_length_finds_no_state_ready(recorded, tmp_path):
+    import json
+    make, calls, _ = recorded
+    cache = make(key_sketch=False)
+    prefill(cache, 3000)
+    step(cache)
+    (tmp_path / "metadata.txt").write_text(json.dumps(dict(r_sq=[[1.0, 1.0]] * LAYERS, kvbuf_prefix_len=4,
+                                                           kvbuf_suffix_len=8, retrieval_region_len=500)))
+    for l in range(LAYERS):
+        for kind, rows in (("p", 4), ("s", 8)):
+            d = tmp_path / f"{kind}_l_{l:03d}"
+            d.mkdir()
+            for name in ("k.pt", "v.pt"):
+                torch.save(torch.zeros((1, 2, rows, 64), dtype=torch.bfloat16), d / name)
+    cache.load_prefill_cache(torch.zeros((1, 512)), str(tmp_path))
+    step(cache)
+    assert calls == [False, True, False, True]
+
+
+def test_routes_and_orders_and_rollovers_do_not_share_a_state(recorded):
+    from diffcache_amd import _hip as hip
+    make, calls, _ = recorded
+    cache = make()
+    prefill(cache, 1000)
+    step(cache)
+    hook_step(cache)
+    step(cache)
+    step(cache, order=hip.ORDER_BEST)
+    assert calls == [False, True] * 4
+    del calls[:]
+    while not cache.window_full():
+        step(cache, order=hip.ORDER_BEST)
+    assert all(calls)
+    del calls[:]
+    step(cache, order=hip.ORDER_BEST)       # rolls the window over first: the region grew
+    assert cache.generation == 1 and calls == [False, True]
+
+
+def test_a_call_that_raised_leaves_no_state_ready(recorded, monkeypatch):
+    make, calls, _ = recorded
+    from diffcache_amd import _hip as hip
+    cache = make()
+    prefill(cache, 1000)
+    step(cache)
+    good = hip.decode_layer
+
+    def bad(*a, **k):
+        raise hip.DiffCacheError("refused")
+    monkeypatch.setattr(hip, "decode_layer", bad)
+    with pytest.raises(hip.DiffCacheError):
+        step(cache)
+    monkeypatch.setattr(hip, "decode_layer", good)
+    step(cache)
+    assert calls == [False, True, False, True]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("route", ["one_kernel", "sketch", "stream"])
+def test_prompts_of_other_lengths_on_one_cache_equal_a_fresh_cache(route):
+    from diffcache_amd import DiffCache, _hip as hip
+    g = torch.Generator(device="cuda").manual_seed(17)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+
+    def make():
+        c = DiffCache(num_layers=LAYERS, batch_size=2, max_length=9000, num_kv_heads=4, num_q_heads=16, head_dim=128,
+                      retrieval_budget=256, nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8,
+                      kvbuf_suffix_maxlen=WINDOW, attn_mass_threshold=0.9, k_check_seq=[100],
+                      r_sq=[[4.0] * 4] * LAYERS, key_sketch=route == "sketch")
+        c.one_kernel = hip.ONE_KERNEL_EXCLUSIVE if route == "one_kernel" else hip.ONE_KERNEL_NEVER
+        return c
+    used = make()
+    # the used cache's slots begin elsewhere for every one of these regions
+    for n in (8500, 1501, 4003, 8999 - WINDOW, 700):
+        fresh = make()
+        kv = [(rnd(2, n, 4, 128), rnd(2, n, 4, 128)) for _ in range(LAYERS)]
+        for cache in (used, fresh):
+            for l, (k, v) in enumerate(kv):
+                cache.prefill_update_kv_cache(k, v, l)
+        for _ in range(2):
+            for l in range(LAYERS):
+                q, nk, nv = rnd(2, 16, 128), rnd(2, 1, 4, 128), rnd(2, 1, 4, 128)
+                x, y = (c.decode_attention(l, q, nk, nv).float() for c in (used, fresh))
+                if route == "one_kernel":
+                    assert hip.last_route() == hip.ROUTE_ONE_KERNEL
+                assert torch.equal(used.idx[l].sort(dim=1).values, fresh.idx[l].sort(dim=1).values), (n, l)
+                # rows are added in the order they were found: at most 281 terms of weight <= 1 in fp32
+                # (281 * 2^-24 * |v| < 1e-4), then one bf16 rounding (2^-8)
+                assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 1e-4).all()), (n, l)
