@@ -221,10 +221,13 @@ class DiffCache:
             self._ws_state = None
         return self._ws
 
-    def _take_state(self, kind: tuple) -> bool:
-        """Whether the workspace's select state is ready for a call of this kind.  The caller notes the kind
-        in _ws_state again once the call is enqueued: one that raised half-way has left nothing ready."""
-        ready = self._ws_state == kind
+    def _take_state(self, layer_idx: int, kind: tuple) -> bool:
+        """Whether the workspace's select state is ready for a call of this kind (its last element: under
+        capture).  The caller notes the kind in _ws_state again once the call is enqueued: one that raised
+        half-way has left nothing ready.  A captured step is replayed behind whatever used the workspace
+        meanwhile, so it sets the state up in its first layer and only its own later layers find it ready;
+        capturing it runs nothing, so an eager call behind it does not."""
+        ready = self._ws_state == kind and not (kind[-1] and layer_idx == 0)
         self._ws_state = None
         return ready
 
@@ -249,6 +252,8 @@ class DiffCache:
     def advance_host_step(self, steps: int = 1) -> None:
         """After ``steps`` replays of a captured decode step: bring the host's mirror of the
         recent-window length up to the device's counter (no synchronisation)."""
+        if steps > 0:
+            self._ws_state = None   # the replays used the workspace in their own layout
         self.kvbuf_suffix_len += steps
         self._store_suffix_rows += steps
         hip.require(self.kvbuf_suffix_len <= self.kvbuf_suffix_maxlen,
@@ -355,11 +360,12 @@ class DiffCache:
             lo, hi = self._region()
             ws = self._ensure_workspace()
             if self.key_sketch:
-                ready = self._take_state(("select", lo, hi))
+                kind = ("select", lo, hi, torch.cuda.is_current_stream_capturing())
+                ready = self._take_state(layer_idx, kind)
                 hip.score_select_sketch(self.kstore[layer_idx], self.sketch[layer_idx], self.qbuf, lo, hi - lo,
                                         retrieval_len, self.mode, self.hook_order, idx_out=self.idx[layer_idx],
                                         workspace=ws, state_ready=ready)
-                self._ws_state = ("select", lo, hi)
+                self._ws_state = kind
             else:
                 self._ws_state = None   # the one-shot call does not leave the state initialised
                 hip.score_select(self.kstore[layer_idx], self.qbuf, lo, hi - lo, retrieval_len, self.mode,
@@ -438,8 +444,8 @@ class DiffCache:
             # attended: [selected | prefix | the window's rows before this token | this token]
             # (a call with the region's end on the device has other launch sizes than one without:
             #  neither leaves the select state ready for the other)
-            tag = ("layer", order, dev_region, lo, hi)
-            ready = self._take_state(tag)
+            kind = ("layer", order, dev_region, lo, hi, capturing)
+            ready = self._take_state(layer_idx, kind)
             hip.decode_layer(q, self.kstore[layer_idx], self.vstore[layer_idx], lo, hi_cap if dev_region else hi,
                              self.kvbuf_suffix_maxlen, self.retrieval_budget, None, self.idx[layer_idx], out, ws,
                              nk, nv, mode=self.mode, order=order,
@@ -448,7 +454,7 @@ class DiffCache:
                              one_kernel=self.one_kernel,
                              region_hi_dev=self._state[1:2] if dev_region else None, append=append,
                              advance=(self._state, self.kvbuf_suffix_maxlen) if last else None)
-            self._ws_state = tag
+            self._ws_state = kind
         if last and not capturing:  # a captured step is counted when it is replayed (advance_host_step)
             self.kvbuf_suffix_len += 1
             self._store_suffix_rows += 1
@@ -476,11 +482,12 @@ class DiffCache:
         n_units = self.batch_size * self.num_kv_heads
         ks, vs, idx = self.kstore[layer_idx], self.vstore[layer_idx], self.idx[layer_idx]
         if self.key_sketch:
-            ready = self._take_state(("select", lo, hi))
+            kind = ("select", lo, hi, torch.cuda.is_current_stream_capturing())
+            ready = self._take_state(layer_idx, kind)
             hip.score_select_sketch(ks, self.sketch[layer_idx], q, lo, hi - lo, n_sel, self.mode,
                                     hip.ORDER_BEST, q_group=self.group, idx_out=idx, workspace=ws,
                                     state_ready=ready)
-            self._ws_state = ("select", lo, hi)
+            self._ws_state = kind
         else:
             self._ws_state = None
             hip.score_select(ks, q, lo, hi - lo, n_sel, self.mode, hip.ORDER_BEST, q_group=self.group,

@@ -127,6 +127,38 @@ def test_a_call_that_raised_leaves_no_state_ready(recorded, monkeypatch):
     assert calls == [False, True, False, True]
 
 
+@pytest.mark.parametrize("one_step,kw", [
+    (step, dict(key_sketch=True)),                       # the region's end on the device
+    (step, dict(use_k_check=True)), (hook_step, {}),     # and where it is a launch parameter
+])
+def test_a_captured_step_and_eager_ones_do_not_share_a_state(recorded, monkeypatch, one_step, kw):
+    from diffcache_amd import _hip as hip
+    for name in ("score_gathered", "kcheck", "gather_attn"):
+        monkeypatch.setattr(hip, name, lambda *a, **k: None)
+    make, calls, capture = recorded
+    cache = make(**kw)
+    prefill(cache, 1000)
+    for _ in range(2):              # before any eager call, and behind one
+        for _ in range(2):          # captured again: the first capture has not run either
+            del calls[:]
+            capture.append(1)
+            one_step(cache)
+            capture.clear()
+            assert calls == [False, True]   # a replay sets up what it finds, whatever ran before it
+        del calls[:]
+        one_step(cache)                     # nothing of the capture has run yet
+        assert calls == [False, True]
+    del calls[:]
+    one_step(cache)
+    assert calls == [True, True]
+    cache.kvbuf_suffix_len = 8
+    cache.advance_host_step(1)              # a replay in between, laid out its own way
+    one_step(cache)
+    cache.advance_host_step(-1)             # a token taken back: nothing ran
+    one_step(cache)
+    assert calls == [True, True, False, True, True, True]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("route", ["one_kernel", "sketch", "stream"])
 def test_prompts_of_other_lengths_on_one_cache_equal_a_fresh_cache(route):
