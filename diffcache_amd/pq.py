@@ -5,7 +5,7 @@ The reference's PQ baseline directory (evaluation/impl/pqcache) is empty, so
 this follows the benchmark configuration only: M subspaces x 256 centroids,
 8-bit codes, per-query fp32 lookup tables, 4096 candidates reranked to top-k.
 Training is one-off preparation and uses torch ops on the device around the encoding kernel;
-encoding and everything a query touches run in libdiffcache_hip.so.
+encoding (of the keys and codebooks that kernel takes) and everything a query touches run in libdiffcache_hip.so.
 """
 from __future__ import annotations
 
@@ -31,7 +31,10 @@ def train_codebooks(keys: torch.Tensor, m: int, iters: int = 8, seed: int = 0,
         c = xs[torch.randint(0, n, (n_centroids,), generator=g, device=x.device)].clone()
         cols = keys[:, j * ds:(j + 1) * ds]
         for _ in range(iters):
-            a = encode(cols, c.unsqueeze(0)).view(-1).long()
+            if hip.pq_encode_supported(cols, c.unsqueeze(0)):
+                a = hip.pq_encode(cols, c.unsqueeze(0)).view(-1).long()
+            else:       # not through encode(): its codes are bytes, and there may be more than 256 centroids
+                a = torch.cdist(xs, c).argmin(dim=1)
             sums = torch.zeros_like(c).index_add_(0, a, xs)
             cnt = torch.bincount(a, minlength=n_centroids).to(xs.dtype)
             nz = cnt > 0

@@ -1,0 +1,24 @@
+"""Codebook training and encoding for callers outside the encoding kernel's range (no GPU needed)."""
+import pytest
+import torch
+
+from diffcache_amd.pq import train_codebooks
+
+
+@pytest.mark.parametrize("n_centroids", [16, 256, 257, 600])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_training_is_lloyd_s_iteration_for_any_number_of_centroids(n_centroids, dtype):
+    n, m, ds, iters = 3000, 2, 4, 3
+    keys = torch.randn((n, m * ds), generator=torch.Generator().manual_seed(5)).to(dtype)
+    got = train_codebooks(keys, m, iters=iters, seed=7, n_centroids=n_centroids)
+    x, g = keys.float(), torch.Generator().manual_seed(7)
+    for j in range(m):
+        xs = x[:, j * ds:(j + 1) * ds].contiguous()
+        c = xs[torch.randint(0, n, (n_centroids,), generator=g)].clone()
+        for _ in range(iters):
+            a = torch.cdist(xs, c).argmin(dim=1)
+            for i in a.unique().tolist():
+                c[i] = xs[a == i].mean(dim=0)
+        # a cell's mean of at most 3000 values below 5 in fp32: 3000 * 2^-24 * 5 < 1e-3 on either side of
+        # the sum's order; a key assigned to another cell moves means by 1e-2 and more
+        assert torch.allclose(got[j], c, rtol=0.0, atol=1e-3), (got[j] - c).abs().max()
