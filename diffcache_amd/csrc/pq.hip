@@ -367,8 +367,9 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
 extern "C" int dc_pq_encode_bf16(const void *keys, int64_t key_stride, int64_t n, const float *books, uint8_t *codes,
                                  int64_t code_stride, int hd, int m, int n_centroids, void *stream) {
     const char *who = "dc_pq_encode_bf16";
-    DC_REQUIRE(keys && books && codes, "%s: null pointer", who);
     DC_REQUIRE(n >= 0 && m >= 1 && hd >= m && hd % m == 0, "%s: bad sizes", who);
+    if (n == 0) return DC_OK;  // an empty tensor has a null pointer
+    DC_REQUIRE(keys && books && codes, "%s: null pointer", who);
     const int ds = hd / m;
     DC_REQUIRE(ds == 2 || ds == 4 || ds == 8 || ds == 16, "%s: %d columns per subspace unsupported (2, 4, 8 or 16)", who, ds);
     DC_REQUIRE(n_centroids >= 1 && n_centroids <= 256, "%s: %d centroids unsupported (1 to 256)", who, n_centroids);
@@ -376,7 +377,6 @@ extern "C" int dc_pq_encode_bf16(const void *keys, int64_t key_stride, int64_t n
     DC_REQUIRE(((uintptr_t)keys) % align == 0 && key_stride >= hd && (key_stride * 2) % align == 0,
                "%s: keys must be %d-byte aligned, rows included", who, align);
     DC_REQUIRE((((uintptr_t)codes) & 3u) == 0 && code_stride >= m, "%s: codes must be 4-byte aligned, rows of at least m bytes", who);
-    if (n == 0) return DC_OK;
     const int64_t blocks = ((n + kEncKeys - 1) / kEncKeys + 7) / 8 * 8 * ((m + kEncSubs - 1) / kEncSubs);
     DC_REQUIRE(blocks < (1ll << 31), "%s: grid too large", who);
     const dim3 grid((unsigned)blocks);

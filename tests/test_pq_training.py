@@ -22,3 +22,20 @@ def test_training_is_lloyd_s_iteration_for_any_number_of_centroids(n_centroids, 
         # a cell's mean of at most 3000 values below 5 in fp32: 3000 * 2^-24 * 5 < 1e-3 on either side of
         # the sum's order; a key assigned to another cell moves means by 1e-2 and more
         assert torch.allclose(got[j], c, rtol=0.0, atol=1e-3), (got[j] - c).abs().max()
+
+
+def test_no_keys_are_encoded_to_no_codes():
+    """The C entry as well as the wrapper: an empty tensor's pointer is null, which is no error."""
+    from diffcache_amd import _hip as hip
+    assert hip.lib.dc_pq_encode_bf16(None, 128, 0, None, None, 32, 128, 32, 256, None) == 0
+    assert hip.lib.dc_pq_encode_bf16(None, 128, 1, None, None, 32, 128, 32, 256, None) == -22
+    assert hip.lib.dc_pq_encode_bf16(None, 128, 0, None, None, 32, 128, 33, 256, None) == -22
+
+
+@pytest.mark.gpu
+def test_no_keys_on_the_gpu():
+    from diffcache_amd.pq import encode
+    books = torch.zeros((32, 256, 4), device="cuda")
+    for dtype in (torch.bfloat16, torch.float32):
+        codes = encode(torch.zeros((0, 128), device="cuda", dtype=dtype), books)
+        assert codes.shape == (0, 32) and codes.dtype == torch.uint8 and codes.is_cuda
