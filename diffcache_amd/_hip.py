@@ -781,12 +781,13 @@ def pq_build_lut(q: torch.Tensor, books: torch.Tensor, n_b: int) -> torch.Tensor
 
 
 def pq_encode_supported(keys: torch.Tensor, books: torch.Tensor) -> bool:
-    """Whether dc_pq_encode_bf16 takes these: bf16 keys (n, hd) and fp32 books in GPU memory, at most 256
-    centroids, 2, 4, 8 or 16 columns per subspace, rows aligned to them."""
+    """Whether dc_pq_encode_bf16 takes these: bf16 keys (n, hd) and fp32 books in the memory of the current GPU
+    (kernels are launched there, wherever their operands are), at most 256 centroids, 2, 4, 8 or 16
+    columns per subspace, rows aligned to them."""
     m, nc, ds = books.shape
     align = min(2 * ds, 16)
-    return (keys.is_cuda and books.is_cuda and keys.dtype == torch.bfloat16 and books.dtype == torch.float32
-            and keys.dim() == 2 and keys.stride(1) == 1 and keys.shape[1] == m * ds and ds in (2, 4, 8, 16)
+    return (keys.is_cuda and keys.device == books.device and keys.device.index == torch.cuda.current_device()
+            and keys.dtype == torch.bfloat16 and books.dtype == torch.float32 and keys.dim() == 2 and keys.stride(1) == 1 and keys.shape[1] == m * ds and ds in (2, 4, 8, 16)
             and 1 <= nc <= 256 and keys.stride(0) >= m * ds
             and keys.data_ptr() % align == 0 and keys.stride(0) * 2 % align == 0)
 

@@ -32,6 +32,34 @@ def test_no_keys_are_encoded_to_no_codes():
     assert hip.lib.dc_pq_encode_bf16(None, 128, 0, None, None, 32, 128, 33, 256, None) == -22
 
 
+class Elsewhere:
+    """What pq_encode_supported looks at of a tensor on some GPU."""
+
+    def __init__(self, device, shape, dtype):
+        self.device, self.shape, self.dtype, self.is_cuda = torch.device(device), shape, dtype, True
+
+    def dim(self):
+        return len(self.shape)
+
+    def stride(self, i):
+        return (self.shape[1], 1)[i]
+
+    def data_ptr(self):
+        return 4096
+
+
+@pytest.mark.parametrize("keys_on,books_on,current,taken", [
+    ("cuda:0", "cuda:0", 0, True), ("cuda:1", "cuda:1", 1, True),
+    ("cuda:1", "cuda:1", 0, False),     # launched on GPU 0 it would work on GPU 1's memory, out of GPU 1's order
+    ("cuda:0", "cuda:1", 0, False),     # torch's error, as for any two devices
+])
+def test_the_encoding_kernel_takes_operands_of_the_current_gpu_only(monkeypatch, keys_on, books_on, current, taken):
+    from diffcache_amd import _hip as hip
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current)
+    keys, books = Elsewhere(keys_on, (100, 128), torch.bfloat16), Elsewhere(books_on, (32, 256, 4), torch.float32)
+    assert hip.pq_encode_supported(keys, books) == taken
+
+
 @pytest.mark.gpu
 def test_no_keys_on_the_gpu():
     from diffcache_amd.pq import encode
