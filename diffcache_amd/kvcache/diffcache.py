@@ -193,14 +193,14 @@ class DiffCache:
     @property
     def r_sq(self) -> List[List[float]]:
         """Largest squared key norm per layer and head (waits for the device after a prefill)."""
-        for layer_idx, value in enumerate(self._r_sq):
+        for layer_idx, value in enumerate(self._r_sq or ()):
             if isinstance(value, DeviceRSq):
                 self._r_sq[layer_idx] = value.tolist()
         return self._r_sq
 
     @r_sq.setter
     def r_sq(self, value) -> None:
-        self._r_sq = list(value)
+        self._r_sq = None if value is None else list(value)     # None: a cache that is only ever loaded
 
     def _region(self):
         lo = self.kvbuf_prefix_len

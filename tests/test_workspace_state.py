@@ -1,6 +1,7 @@
 """When DiffCache tells a call that the workspace's select state is ready: only when the last call on the
 workspace was of the same kind over the same region (dc_layer_args.select_state_ready).  The native calls are
-replaced by recorders, so the rule runs without a GPU; the GPU tests below compare results."""
+replaced by recorders, so the rule runs without a GPU; the GPU tests below compare results.  Snapshots loaded
+into such a cache are covered on the way."""
 import pytest
 import torch
 
@@ -34,11 +35,11 @@ def recorded(monkeypatch):
     monkeypatch.setattr(mod.hip, "score_select_sketch", lambda *a, **k: calls.append(k["state_ready"]))
     monkeypatch.setattr(mod.hip, "score_select", lambda *a, **k: None)
 
-    def make(**kw):
+    def make(r_sq=[[4.0, 4.0]] * LAYERS, **kw):
         return mod.DiffCache(num_layers=LAYERS, batch_size=1, max_length=4000, num_kv_heads=2, num_q_heads=4, head_dim=64,
                              retrieval_budget=64, nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8,
                              kvbuf_suffix_maxlen=WINDOW, attn_mass_threshold=0.9, k_check_seq=[100],
-                             r_sq=[[4.0, 4.0]] * LAYERS, device="cpu", **kw)
+                             r_sq=r_sq, device="cpu", **kw)
     return make, calls, capture
 
 
@@ -71,12 +72,8 @@ def test_a_prompt_of_another_length_finds_no_state_ready(recorded, one_step):
     assert calls == first + first + first + same
 
 
-def test_a_loaded_snapshot_of_another_length_finds_no_state_ready(recorded, tmp_path):
+def snapshot(tmp_path):
     import json
-    make, calls, _ = recorded
-    cache = make(key_sketch=False)
-    prefill(cache, 3000)
-    step(cache)
     (tmp_path / "metadata.txt").write_text(json.dumps(dict(r_sq=[[1.0, 1.0]] * LAYERS, kvbuf_prefix_len=4,
                                                            kvbuf_suffix_len=8, retrieval_region_len=500)))
     for l in range(LAYERS):
@@ -85,9 +82,26 @@ def test_a_loaded_snapshot_of_another_length_finds_no_state_ready(recorded, tmp_
             d.mkdir()
             for name in ("k.pt", "v.pt"):
                 torch.save(torch.zeros((1, 2, rows, 64), dtype=torch.bfloat16), d / name)
+
+
+def test_a_loaded_snapshot_of_another_length_finds_no_state_ready(recorded, tmp_path):
+    make, calls, _ = recorded
+    cache = make(key_sketch=False)
+    prefill(cache, 3000)
+    step(cache)
+    snapshot(tmp_path)
     cache.load_prefill_cache(torch.zeros((1, 512)), str(tmp_path))
     step(cache)
     assert calls == [False, True, False, True]
+
+
+def test_a_cache_that_is_only_loaded_needs_no_r_sq(recorded, tmp_path):
+    make, _, _ = recorded
+    cache = make(r_sq=None)
+    assert cache.r_sq is None
+    snapshot(tmp_path)
+    cache.load_prefill_cache(torch.zeros((1, 512)), str(tmp_path))
+    assert cache.r_sq == [[1.0, 1.0]] * LAYERS
 
 
 def test_routes_and_orders_and_rollovers_do_not_share_a_state(recorded):
