@@ -78,7 +78,7 @@ class PQIndex:
         nu = b * h
         self.ids = torch.empty((nu, self.topk), dtype=torch.int32, device=dev)
         self.ws = hip.alloc_workspace(hip.lib.dc_pq_search_workspace_bytes(nu, n, self.n_cand), dev)
-        self._ws_ready = False      # every search leaves the workspace ready for the next one
+        self._ws_ready = False      # every search that runs leaves the workspace ready for the next one
 
     @classmethod
     def build(cls, store_k: torch.Tensor, m: int = 32, sample: int = 65536, iters: int = 8,
@@ -95,7 +95,8 @@ class PQIndex:
         lut = hip.pq_build_lut(q, self.books, self.b)
         ids = hip.pq_search(self.store_k, self.codes, lut, q, self.n_cand, self.topk,
                             idx_out=self.ids, workspace=self.ws, state_ready=self._ws_ready)
-        self._ws_ready = True
+        if not self._ws_ready:      # capturing a search runs nothing: only an eager one leaves it ready
+            self._ws_ready = not torch.cuda.is_current_stream_capturing()
         return ids
 
     def search_stepwise(self, q: torch.Tensor) -> torch.Tensor:

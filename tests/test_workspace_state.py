@@ -173,6 +173,22 @@ def test_a_captured_step_and_eager_ones_do_not_share_a_state(recorded, monkeypat
     assert calls == [True, True, False, True, True, True]
 
 
+def test_a_captured_search_does_not_ready_the_workspace_of_an_eager_one(monkeypatch):
+    from diffcache_amd import pq
+    calls, capture = [], [1]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(capture))
+    monkeypatch.setattr(pq.hip, "pq_build_lut", lambda *a: None)
+    monkeypatch.setattr(pq.hip, "pq_search", lambda *a, **k: calls.append(k["state_ready"]))
+    index = pq.PQIndex(torch.zeros((1, 1, 100, 64), dtype=torch.bfloat16), torch.zeros((1, 16, 256, 4)),
+                       torch.zeros((1, 100, 16), dtype=torch.uint8))
+    index.search(None)
+    index.search(None)
+    capture.clear()
+    for _ in range(3):
+        index.search(None)
+    assert calls == [False, False, False, True, True]
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("route", ["one_kernel", "sketch", "stream"])
 def test_prompts_of_other_lengths_on_one_cache_equal_a_fresh_cache(route):
