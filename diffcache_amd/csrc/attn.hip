@@ -44,12 +44,13 @@ __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, 
     dc_attn_split_mfma<HD>(a, group, blockIdx.x % n_units, blockIdx.x / n_units, s_dyn);
 }
 
-// out[u, g, :] = sum_s w_s acc_s / sum_s w_s l_s with w_s = exp(m_s - max m): one block
-// per (unit, head), one thread per output column.
-// The splits of one query head, combined.  A few KB per block, so what bounds it is the chain of memory round
-// trips: the block's threads share the splits out (HD/4 threads to a row of 16-byte pieces) and request their
-// rows together with every (m, l) they need, before any weight is known, so that there is one round trip up
-// to 256 / (HD/4) * kMergeBatch splits (64 of 128 columns: a budget of 8192 rows) and one for as many more.
+// The splits of one query head, combined: out[u, g, :] = sum_s w_s acc_s / sum_s w_s l_s with
+// w_s = exp(m_s - max m), one block per (unit, head).  A few KB per block, so what bounds it is the chain of
+// memory round trips: the block's threads share the splits out (HD/4 threads to a row of 16-byte pieces) and
+// request their rows together with the (m, l) of the first 64 splits, before any weight is known: one round trip up
+// to min(64, 256 / (HD/4) * kMergeBatch) splits, that is 64 up to 128 columns (8192 attended rows) and 32 at 256
+// (2048 rows).  From 65 on the maximum and then the sum fetch the other (m, l), and every further batch of
+// rows is a trip of its own.
 // Every wave derives the largest m and the sum by itself; the only barrier is that of the last sum.
 // 8 units, group 4, 128 columns: 18 splits 4.8 -> 3.7 us, 33 splits 5.5 -> 4.7 us (one thread per column before,
 // its rows eight at a time behind the weights).

@@ -251,8 +251,8 @@ __device__ __forceinline__ float group_max(float v) {
 // wanted: the sixteen rows of the left operand hold the digits instead, several times over with zeros elsewhere, so
 // that a wave's 64 rows end up one to a lane.  From 128 columns on two lanes share a row (S = 2), because a load of
 // 16 rows x 64 bytes takes half lines, which streaming loads fetch twice (205 us instead of 180 us at 64 units x
-// 131004 rows of 128).  A step of 64 rows takes about a third of the vector instructions that fp32 arithmetic on the
-// codes took; the kernel is bound by memory latency at few units and by HBM at many.  The first rows, the
+// 131004 rows of 128).  A step of 64 rows of 128 takes 284 vector instructions in all, 532 with fp32 arithmetic on the
+// codes; the kernel is bound by memory latency at few units and by HBM at many.  The first rows, the
 // query, scales and residuals are all requested at the block's start, one round trip instead of three.
 // Measured before / after (kernel trace): 8 x 131004 rows of 128 29.8 / 27.3 us, 4 x 127028 19.6 / 17.7, 64 x 131004
 // 185.1 / 180.8, 8 x 1048508 183.1 / 179.1, 8 x 16323 of 64 11.1 / 9.5.

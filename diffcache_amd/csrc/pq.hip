@@ -95,9 +95,10 @@ __global__ __launch_bounds__(kThreads) void pq_adc_kernel(
 // v_min3, a compare, a select).  At the end the four lanes of a key settle its octet, each lane
 // for the key of one of the wave's four groups (an exchange that halves twice), and that lane takes
 // the least of the eight in fp32.  200003 keys of 128 columns, 32
-// subspaces: 97 us, the vector ALUs busy 82 % of it (torch's distance matrices, written to and read
-// from HBM four times over, took 11.8 ms).  With the tables in plain order the LDS was busy 87 % of
-// 115 us, three quarters of that in bank conflicts; a search of four values at a time 120 us.
+// subspaces: 94-98 us, the vector ALUs issuing 88 % of the kernel's time and the matrix cores busy 46 %
+// (SQ counters); torch's distance matrices, written to and read from HBM four times over, took 11.8 ms.
+// With the tables in plain order (bank conflicts where an octet is settled) it took 115 us, with a search
+// of four values at a time 120 us.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));

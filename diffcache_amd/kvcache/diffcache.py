@@ -95,7 +95,7 @@ class DiffCache:
         # hook_order: order of the ids that decode_query_kvcache selects, hence of the rows that
         # decode_post_query_operation gathers into kbuf/vbuf.  ORDER_BEST is the reference's
         # (best first, nsw.rs:592-630); attention over the buffer does not depend on the order, so
-        # a caller that only attends may pass hip.ORDER_ANY and save the sort.
+        # a caller that only attends may pass hip.ORDER_ANY and, above 4096 ids, save a sort.
         # exclusive_gpu: the caller vouches that nothing else keeps CUs of this GPU busy while this
         # cache decodes (no second cache decoding on another stream, no long-lived kernels).  Short
         # contexts then run as one kernel under graph capture too; without it a captured step takes
@@ -251,7 +251,8 @@ class DiffCache:
 
     def advance_host_step(self, steps: int = 1) -> None:
         """After ``steps`` replays of a captured decode step: bring the host's mirror of the
-        recent-window length up to the device's counter (no synchronisation)."""
+        recent-window length up to the device's counter (no synchronisation).  Negative: tokens taken
+        back, which hip.step_state_advance takes off the device's words (append position included)."""
         if steps > 0:
             self._ws_state = None   # the replays used the workspace in their own layout
         self.kvbuf_suffix_len += steps

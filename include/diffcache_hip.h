@@ -436,8 +436,7 @@ typedef struct dc_step_args {
 int dc_decode_layer_step(const dc_layer_args *args, const dc_step_args *step, void *stream);
 /*
  * Short contexts.  With scores == NULL, order == DC_ORDER_ANY and at most 640 Ki region rows
- * over all units (and, when a sketch is passed, whose chain of kernels is the faster one, at most
- * 40 Ki region rows per unit), dc_decode_layer runs the layer as ONE kernel whose blocks are all resident
+ * over all units (and, when a sketch is passed, at most 40 Ki region rows per unit), dc_decode_layer runs the layer as ONE kernel whose blocks are all resident
  * (two per CU) and hand their phases over through the workspace (same results; the event pair
  * then brackets that kernel).  No counterpart in the reference, whose layers run on the CPU pool
  * (lib.rs:352-369); what it has to match is that one layer call is always right

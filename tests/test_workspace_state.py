@@ -221,3 +221,74 @@ def test_prompts_of_other_lengths_on_one_cache_equal_a_fresh_cache(route):
                 # rows are added in the order they were found: at most 281 terms of weight <= 1 in fp32
                 # (281 * 2^-24 * |v| < 1e-4), then one bf16 rounding (2^-8)
                 assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 1e-4).all()), (n, l)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("length", [6000, 100])     # with the region's end on the device, and as a launch parameter
+def test_eager_steps_between_replays_and_tokens_taken_back(length):
+    """One cache alternates eager steps, hook calls, replays of a captured step and tokens taken back; every step's
+    ids, output and appended rows equal those of a cache that only steps eagerly."""
+    from diffcache_amd import DiffCache, _hip as hip
+    g = torch.Generator(device="cuda").manual_seed(23)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)
+    used, plain = (DiffCache(num_layers=LAYERS, batch_size=2, max_length=9000, num_kv_heads=4, num_q_heads=16, head_dim=128,
+                             retrieval_budget=256, nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8,
+                             kvbuf_suffix_maxlen=40, attn_mass_threshold=0.9, k_check_seq=[100],
+                             r_sq=[[4.0] * 4] * LAYERS) for _ in range(2))
+    for l in range(LAYERS):
+        k, v = rnd(2, length, 4, 128), rnd(2, length, 4, 128)
+        for cache in (used, plain):
+            cache.prefill_update_kv_cache(k, v, l)
+    q, nk, nv, out = ([torch.zeros(s, device="cuda", dtype=torch.bfloat16) for _ in range(LAYERS)]
+                      for s in ((2, 16, 128), (2, 1, 4, 128), (2, 1, 4, 128), (2, 16, 128)))
+    for t in (*q, *nk, *nv):
+        t.normal_(generator=g)
+
+    def step(cache):
+        for l in range(LAYERS):
+            cache.decode_attention(l, q[l], nk[l], nv[l], out=out[l])
+
+    def replay(cache):
+        graph.replay()
+        cache.advance_host_step()
+
+    def take_back(cache):
+        cache.advance_host_step(-1)
+        hip.step_state_advance(cache._state, -1, cache.kvbuf_suffix_maxlen)
+
+    used._ensure_workspace()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(used)
+    lo, hi = used._region()
+    # the first eager step comes behind a capture that has not run
+    for i, how in enumerate((step, replay, step, step, replay, "hooks", replay, step, "back", replay, "back", step, replay)):
+        if how == "hooks":      # (only their use of the workspace matters here: the step they count is taken back)
+            for l in range(LAYERS):
+                used.decode_pre_query_operation(q[l])
+                used.decode_query_kvcache(l)
+            used.kvbuf_suffix_len -= 1
+            hip.step_state_advance(used._state, -1, used.kvbuf_suffix_maxlen)
+            continue
+        if how == "back":
+            for cache in (used, plain):
+                take_back(cache)
+                for store in (*cache.kstore, *cache.vstore):
+                    store[:, :, hi + cache.kvbuf_suffix_len].fill_(7.0)     # a row that is not written again would show
+            continue
+        for t in (*q, *nk, *nv):
+            t.normal_(generator=g)
+        how(used)
+        got, ids = [t.clone() for t in out], [t.clone() for t in used.idx]
+        step(plain)
+        n = hi + used.kvbuf_suffix_len
+        assert used._state.tolist() == plain._state.tolist() == [n - hi, hi, n, 0], (i, how)
+        for l in range(LAYERS):
+            assert torch.equal(ids[l].sort(dim=1).values, plain.idx[l].sort(dim=1).values), (i, l)
+            x, y = got[l].float(), out[l].float()
+            # rows are added in another order on another route: at most 301 terms of weight <= 1 in fp32
+            # (301 * 2^-24 * |v| < 1e-4), then one bf16 rounding (2^-8) on either side
+            assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 1e-4).all()), (i, l)
+            assert torch.equal(used.kstore[l][:, :, :n], plain.kstore[l][:, :, :n]), (i, l)
+            assert torch.equal(used.vstore[l][:, :, :n], plain.vstore[l][:, :, :n]), (i, l)
