@@ -200,9 +200,10 @@ def _counter(t: Optional[torch.Tensor]):
 
 def _store_strides(store: torch.Tensor) -> Tuple[int, int, int]:
     """(batch, head, row) element strides of a (b, h, n, hd) bf16 store."""
-    if store.dim() != 4 or store.dtype != torch.bfloat16 or store.stride(3) != 1:
+    strides = store.stride()
+    if len(strides) != 4 or store.dtype != torch.bfloat16 or strides[3] != 1:
         raise DiffCacheError("a K/V store must be a (b, h, n, hd) bfloat16 tensor with contiguous rows")
-    return store.stride(0), store.stride(1), store.stride(2)
+    return strides[:3]
 
 
 def require(cond: bool, msg: str = "") -> None:
@@ -370,10 +371,11 @@ def score_select_sketch(store_k: torch.Tensor, sketch: Sketch, q: torch.Tensor, 
                         budget: int, mode: int = MODE_REF_DIST, order: int = ORDER_ANY, q_group: int = 1,
                         idx_out: Optional[torch.Tensor] = None, workspace: Optional[torch.Tensor] = None,
                         state_ready: bool = False,
-                        scan_events: Optional[Tuple[torch.cuda.Event, torch.cuda.Event]] = None
-                        ) -> torch.Tensor:
+                        scan_events: Optional[Tuple[torch.cuda.Event, torch.cuda.Event]] = None,
+                        whole: bool = False) -> torch.Tensor:
     """The ids of ``score_select`` (exact top-k of the bf16 keys), found by scanning the
-    8-bit sketch and rescoring the rows that can still matter."""
+    8-bit sketch and rescoring the rows that can still matter.  ``whole``: return idx_out as it is
+    instead of a view of its first ids."""
     kptr, b, h, hd, sb, sh, sr = _score_select_args(store_k, q, lo, n_rows, q_group)
     k_eff = min(budget, n_rows)
     if idx_out is None:
@@ -381,21 +383,22 @@ def score_select_sketch(store_k: torch.Tensor, sketch: Sketch, q: torch.Tensor, 
     if workspace is None:
         workspace = alloc_workspace(sketch_select_workspace_bytes(b * h, n_rows, budget), store_k.device)
     c = sketch.codes
+    cb, ch, cr, _ = c.stride()
     ev0 = ev1 = None
     if scan_events is not None:
         ev0, ev1 = scan_events[0].cuda_event, scan_events[1].cuda_event
     _check(lib.dc_score_select_sketch_bf16(
-        kptr, _dev(c, "codes") + lo * c.stride(2), _dev(sketch.scale, "scale"), _dev(sketch.resid, "resid"),
+        kptr, _dev(c, "codes") + lo * cr, _dev(sketch.scale, "scale"), _dev(sketch.resid, "resid"),
         _dev(q, "q"), _dev(idx_out, "idx_out"), idx_out.stride(0), b, h, n_rows, hd, sb, sh, sr,
-        c.stride(0), c.stride(1), c.stride(2), q_group, budget, mode, order, int(state_ready),
+        cb, ch, cr, q_group, budget, mode, order, int(state_ready),
         _dev(workspace, "workspace"), workspace.numel(), ev0, ev1, _stream()))
-    return idx_out[:, :k_eff]
+    return idx_out if whole else idx_out[:, :k_eff]
 
 
 def gather_rows(store_k: Optional[torch.Tensor], store_v: Optional[torch.Tensor], idx: torch.Tensor,
                 out_k: Optional[torch.Tensor], out_v: Optional[torch.Tensor], row_offset: int = 0,
-                n_idx: Optional[int] = None) -> None:
-    """out[b, h, j, :] = store[b, h, row_offset + idx[b*H + h, j], :] for j < n_idx."""
+                n_idx: Optional[int] = None, out_row: int = 0) -> None:
+    """out[b, h, out_row + j, :] = store[b, h, row_offset + idx[b*H + h, j], :] for j < n_idx."""
     ref = store_k if store_k is not None else store_v
     sb, sh, sr = _store_strides(ref)
     b, h, _, hd = ref.shape
@@ -404,11 +407,17 @@ def gather_rows(store_k: Optional[torch.Tensor], store_v: Optional[torch.Tensor]
     n_idx = idx.shape[1] if n_idx is None else n_idx
     require(idx.dim() == 2 and idx.shape[0] == b * h and idx.shape[1] >= n_idx and idx.element_size() == 4,
             "idx must be a 32-bit (bsz * kv_heads, >= n_idx) tensor")
-    for o in (out_k, out_v):
-        require(o is None or (o.shape[0] == b and o.shape[1] == h and o.shape[2] >= n_idx and o.shape[3] == hd),
+    ptrs = []
+    for o, name in ((out_k, "out_k"), (out_v, "out_v")):
+        if o is None:
+            ptrs.append(None)
+            continue
+        ob, oh, on, od = o.shape
+        require(ob == b and oh == h and out_row >= 0 and on - out_row >= n_idx and od == hd,
                 "out_k / out_v must be (bsz, kv_heads, >= n_idx, head_dim)")
+        ptrs.append(_dev(o, name) + out_row * dr * 2)
     _check(lib.dc_gather_rows_bf16(_opt(store_k, "store_k"), _opt(store_v, "store_v"), _dev(idx, "idx"),
-                                   _opt(out_k, "out_k"), _opt(out_v, "out_v"), b, h, n_idx,
+                                   ptrs[0], ptrs[1], b, h, n_idx,
                                    idx.stride(0), hd, row_offset, sb, sh, sr, db, dh, dr, _stream()))
 
 
@@ -664,6 +673,31 @@ def _layer_args(q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores
     return a
 
 
+def _new_rows(new_k, new_v, numel: int) -> None:
+    for t in (new_k, new_v):
+        if t is None or t.numel() != numel or not t.is_contiguous():
+            raise DiffCacheError("new_k/new_v must be contiguous and hold (b, h, hd) values")
+
+
+def _step_args(s: StepArgs, store_k, new_k, new_v, append, advance) -> None:
+    """struct dc_step_args from the ``append`` and ``advance`` of decode_layer, with their checks."""
+    if append is not None:
+        b, h, n_max, hd = store_k.shape
+        if not 0 <= append[0] < n_max:
+            raise DiffCacheError(f"append position {append[0]} outside the store of {n_max} rows")
+        _new_rows(new_k, new_v, b * h * hd)
+        s.append, s.pos, s.pos_end = 1, append[0], min(append[2], n_max)
+        s.pos_dev = _counter(append[1])
+    else:
+        s.append = 0
+    s.advance_state = None
+    if advance is not None:
+        state, s.advance_limit = advance
+        if not state.is_cuda or state.dtype != torch.int32 or state.numel() < 4 or not state.is_contiguous():
+            raise DiffCacheError("the step state must be a contiguous int32 tensor of 4 elements in GPU memory")
+        s.advance_state = state.data_ptr()
+
+
 def decode_layer(q: torch.Tensor, store_k: torch.Tensor, store_v: torch.Tensor, n_sink: int,
                  recent_lo: int, n_recent: int, budget: int, scores: Optional[torch.Tensor],
                  idx_out: torch.Tensor, out: torch.Tensor, workspace: torch.Tensor,
@@ -677,8 +711,10 @@ def decode_layer(q: torch.Tensor, store_k: torch.Tensor, store_v: torch.Tensor, 
                  one_kernel: int = ONE_KERNEL_AUTO,
                  region_hi_dev: Optional[torch.Tensor] = None,
                  append: Optional[Tuple[int, Optional[torch.Tensor], int]] = None,
-                 advance: Optional[Tuple[torch.Tensor, int]] = None) -> torch.Tensor:
+                 advance: Optional[Tuple[torch.Tensor, int]] = None,
+                 kept: Optional["LayerStep"] = None) -> torch.Tensor:
     """score -> select -> attend for one layer, enqueued on the current stream.
+    ``kept``: the layer's LayerStep, for callers that come back every step with the same stores.
     ``n_recent_dev``: the suffix length as a device-side int32 (``n_recent`` = capacity).
     ``select_state_ready``: see dc_layer_args in the header (skips the init kernel).
     ``sketch``: scan the 8-bit sketch of the keys instead of the keys (same result).
@@ -688,6 +724,11 @@ def decode_layer(q: torch.Tensor, store_k: torch.Tensor, store_v: torch.Tensor, 
     ``append`` (pos, pos_dev, pos_end): new_k / new_v also go to that row of the store, as append_kv
     puts them there; ``advance`` (state, limit): step_state_advance by one behind the layer.  Both ride
     in the layer's own launches."""
+    if kept is not None:
+        kept(q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores, idx_out, out, workspace, new_k, new_v, lse,
+             mode, order, scale, select_state_ready, scan_events, sketch, n_recent_dev, one_kernel, region_hi_dev, append,
+             advance)
+        return out
     a = _layer_args(q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores, idx_out, out, workspace,
                     new_k, new_v, lse, mode, order, scale, select_state_ready, scan_events, sketch, n_recent_dev,
                     one_kernel, region_hi_dev)
@@ -695,22 +736,64 @@ def decode_layer(q: torch.Tensor, store_k: torch.Tensor, store_v: torch.Tensor, 
         _check(lib.dc_decode_layer(C.byref(a), _stream()))
         return out
     s = StepArgs()
-    if append is not None:
-        b, h, n_max, hd = store_k.shape
-        if not 0 <= append[0] < n_max:
-            raise DiffCacheError(f"append position {append[0]} outside the store of {n_max} rows")
-        for t in (new_k, new_v):
-            if t is None or t.numel() != b * h * hd or not t.is_contiguous():
-                raise DiffCacheError("new_k/new_v must be contiguous and hold (b, h, hd) values")
-        s.append, s.pos, s.pos_end = 1, append[0], min(append[2], n_max)
-        s.pos_dev = _counter(append[1])
-    if advance is not None:
-        state, s.advance_limit = advance
-        if not state.is_cuda or state.dtype != torch.int32 or state.numel() < 4 or not state.is_contiguous():
-            raise DiffCacheError("the step state must be a contiguous int32 tensor of 4 elements in GPU memory")
-        s.advance_state = state.data_ptr()
+    _step_args(s, store_k, new_k, new_v, append, advance)
     _check(lib.dc_decode_layer_step(C.byref(a), C.byref(s), _stream()))
     return out
+
+
+class LayerStep:
+    """decode_layer for a caller that keeps the stores, ids, workspace, sketch and counters of a layer from step to
+    step, as DiffCache does.  Filling and checking dc_layer_args anew in every call was a third of a layer's host time
+    (16.1 us of it per layer of eight one-kernel layers, launch included; 10.7 us now).  The struct is
+    filled and checked again whenever any pointer, shape, stride, type or size of them differs from the last
+    call's; what is new in every call (q, new_k, new_v, out) is checked in every call."""
+
+    def __init__(self) -> None:
+        self._key: Optional[tuple] = None
+        self._args: Optional[LayerArgs] = None
+        self._step = StepArgs()
+
+    def __call__(self, q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores, idx_out, out, workspace, new_k, new_v,
+                 lse, mode, order, scale, select_state_ready, scan_events, sketch, n_recent_dev, one_kernel, region_hi_dev,
+                 append, advance) -> None:
+        """The arguments of decode_layer."""
+        n = q.numel()
+        key = None
+        if scores is None and lse is None and scan_events is None and append is not None:
+            key = (store_k.data_ptr(), store_k.shape, store_k.stride(), store_k.dtype, store_v.data_ptr(), store_v.stride(),
+                   store_v.dtype, idx_out.data_ptr(), idx_out.shape, idx_out.stride(), workspace.data_ptr(),
+                   workspace.numel(), n_sink, recent_lo, n_recent, budget, mode, order, scale, n, append[0], append[2])
+            if sketch is not None:
+                c = sketch.codes
+                key += (c.data_ptr(), c.shape, c.stride(), sketch.scale.data_ptr(), sketch.resid.data_ptr())
+            pos_dev = append[1]
+            for t in (n_recent_dev, region_hi_dev, None if pos_dev is n_recent_dev else pos_dev, advance and advance[0]):
+                if t is not None:
+                    key += (t.data_ptr(), t.numel(), t.dtype)
+                else:
+                    key += (None,)
+        s = self._step
+        if key is None or key != self._key:
+            self._key = None
+            a = _layer_args(q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores, idx_out, out, workspace,
+                            new_k, new_v, lse, mode, order, scale, select_state_ready, scan_events, sketch, n_recent_dev,
+                            one_kernel, region_hi_dev)
+            _step_args(s, store_k, new_k, new_v, append, advance)
+            a._keep = None      # the caller keeps them
+            self._new_numel = a.n_b * a.n_h * a.hd
+            self._args, self._key = a, key
+        else:
+            a = self._args
+            if not q.is_contiguous():
+                raise DiffCacheError("q must be contiguous")
+            if out.numel() < n or out.dtype != torch.bfloat16 or not out.is_contiguous():
+                raise DiffCacheError("out must be a contiguous bf16 tensor of the size of q")
+            _new_rows(new_k, new_v, self._new_numel)
+            a.q, a.new_k, a.new_v, a.out = _dev(q, "q"), _dev(new_k, "new_k"), _dev(new_v, "new_v"), _dev(out, "out")
+            a.select_state_ready, a.one_kernel = 1 if select_state_ready else 0, one_kernel
+            if advance is not None:
+                s.advance_limit = advance[1]
+        _check(lib.dc_decode_layer_step(C.byref(a), C.byref(s), _stream()))
 
 
 class LayerCall:

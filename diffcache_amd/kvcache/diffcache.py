@@ -158,6 +158,7 @@ class DiffCache:
         # selected node ids of every layer, relative to the retrieval region, best first
         self.idx = [torch.zeros((n_units, max(retrieval_budget, 1)), device=self.device, dtype=torch.int32)
                     for _ in range(num_layers)]
+        self._layer_step = [hip.LayerStep() for _ in range(num_layers)]
         self._ws: Optional[torch.Tensor] = None
         self._ws_rows = -1
         # The kind of call the workspace's select state was left ready for, with the sizes that its layout
@@ -349,7 +350,7 @@ class DiffCache:
     # ------------------------------------------------------------------ decode hooks
     def decode_pre_query_operation(self, queries: torch.Tensor) -> None:
         """GQA-group mean of the layer's queries (diffcache.py:191-194), kept on the device."""
-        hip.group_mean(queries, self.group, out=self.qbuf.view(-1, self.head_dim), hd=self.head_dim)
+        hip.group_mean(queries, self.group, out=self.qbuf, hd=self.head_dim)
 
     def decode_query_kvcache(self, layer_idx: int) -> None:
         """Exact scan + top-k of the retrieval region with the mean query
@@ -365,7 +366,7 @@ class DiffCache:
                 ready = self._take_state(layer_idx, kind)
                 hip.score_select_sketch(self.kstore[layer_idx], self.sketch[layer_idx], self.qbuf, lo, hi - lo,
                                         retrieval_len, self.mode, self.hook_order, idx_out=self.idx[layer_idx],
-                                        workspace=ws, state_ready=ready)
+                                        workspace=ws, state_ready=ready, whole=True)
                 self._ws_state = kind
             else:
                 self._ws_state = None   # the one-shot call does not leave the state initialised
@@ -384,9 +385,8 @@ class DiffCache:
             return
         lo, _ = self._region()
         b0 = self.retrieval_budget
-        hip.gather_rows(self.kstore[layer_idx], self.vstore[layer_idx], self.idx[layer_idx],
-                        self.kbuf[layer_idx][:, :, b0 - retrieval_len:b0],
-                        self.vbuf[layer_idx][:, :, b0 - retrieval_len:b0], row_offset=lo, n_idx=retrieval_len)
+        hip.gather_rows(self.kstore[layer_idx], self.vstore[layer_idx], self.idx[layer_idx], self.kbuf[layer_idx],
+                        self.vbuf[layer_idx], row_offset=lo, n_idx=retrieval_len, out_row=b0 - retrieval_len)
 
     # ------------------------------------------------------------------ native decode path
     def decode_attention(self, layer_idx: int, queries: torch.Tensor, key_states: torch.Tensor,
@@ -408,14 +408,14 @@ class DiffCache:
                     "the recent window is full (kvbuf_suffix_maxlen): call rollover() between steps")
         lo, hi = self._region()
         hip.require(hi + self.kvbuf_suffix_len < self.max_length, "store is full")
-        q = queries.reshape(b, hq, hd)
-        if not q.is_contiguous():
-            q = q.contiguous()
-        nk, nv = key_states.reshape(b, hkv, hd), value_states.reshape(b, hkv, hd)
-        if not nk.is_contiguous():
-            nk = nk.contiguous()
-        if not nv.is_contiguous():
-            nv = nv.contiguous()
+        # (their values in this order are what is asked for: a contiguous tensor of that many is passed as it is)
+        q, nk, nv = queries, key_states, value_states
+        if q.numel() != b * hq * hd or not q.is_contiguous():
+            q = q.reshape(b, hq, hd).contiguous()
+        if nk.numel() != b * hkv * hd or not nk.is_contiguous():
+            nk = nk.reshape(b, hkv, hd).contiguous()
+        if nv.numel() != b * hkv * hd or not nv.is_contiguous():
+            nv = nv.reshape(b, hkv, hd).contiguous()
         # Under capture the region's end is read from the device wherever the path allows it (a
         # region of at least `budget` rows, no k-check), so that the graph outlives a rollover:
         # launches and workspace are then laid out for the longest region the store can hold.
@@ -454,7 +454,8 @@ class DiffCache:
                              sketch=self.sketch[layer_idx], n_recent_dev=self.step_state,
                              one_kernel=self.one_kernel,
                              region_hi_dev=self._state[1:2] if dev_region else None, append=append,
-                             advance=(self._state, self.kvbuf_suffix_maxlen) if last else None)
+                             advance=(self._state, self.kvbuf_suffix_maxlen) if last else None,
+                             kept=self._layer_step[layer_idx])
             self._ws_state = kind
         if last and not capturing:  # a captured step is counted when it is replayed (advance_host_step)
             self.kvbuf_suffix_len += 1
