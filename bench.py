@@ -356,6 +356,11 @@ class DecodeWorkload:
             call_path = "dc_decode_layer (short context: one kernel)"
             path_bytes = step_bytes
             scan_bytes = unit_bytes * nu
+        elif self.calls[(0, scan, mode)].is_short():
+            # short context: scores of every bf16 key row (with or without a sketch), selection and attention, merge
+            kernel = "short_score_kernel<%d>" % hd
+            call_path = "dc_decode_layer (short context: three kernels)"
+            path_bytes, scan_bytes = step_bytes, rows_bytes_8d
         ach = scan_bytes / (scan_ms * 1e-3) / 1e9
         roofline = {
             "bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBPS,
@@ -367,8 +372,8 @@ class DecodeWorkload:
             "achieved_8d": rows_bytes_8d / (scan_ms * 1e-3) / 1e9,
             "frac_8d": rows_bytes_8d / (scan_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,
         }
-        one_kernel = kernel.startswith("small_layer_kernel")
-        key = "c2.one_kernel" if (self.name == "c2" and one_kernel) else f"{self.name}.{scan}"
+        one_kernel, short = kernel.startswith("small_layer_kernel"), kernel.startswith("short_score_kernel")
+        key = f"{self.name}.{'one_kernel' if one_kernel else 'short' if short else scan}"
         roofline["traffic"] = profiled_traffic(key)
         if roofline["traffic"] is not None:
             roofline["traffic_source"] = "profiles/hbm_traffic.json: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE when " \
@@ -384,7 +389,7 @@ class DecodeWorkload:
             "workload": cfg["desc"], "scan": scan,
             # the arithmetic the route computes in: the sketch scan reads one byte per key element
             # and the rows that survive are rescored from the bf16 keys in fp32
-            "dtype": "bf16" if (one_kernel or scan != "sketch") else "u8 sketch scan + bf16 exact rescoring",
+            "dtype": "bf16" if (one_kernel or short or scan != "sketch") else "u8 sketch scan + bf16 exact rescoring",
             "level": level,
             "device_state": {"before": state_before, "after": state_after},
             "call_path": call_path,

@@ -32,7 +32,7 @@ SYMBOLS = (
     "dc_step_advance", "dc_step_state_advance", "dc_step_state_rollover", "dc_ingest_kv_bf16",
     "dc_prefill_workspace_bytes", "dc_prefill_layer_bf16", "dc_layer_workspace_bytes", "dc_decode_layer",
     "dc_decode_layer_step", "dc_decode_layer_status", "dc_set_wait_limit", "dc_decode_layer_route", "dc_last_route",
-    "dc_decode_layer_errors", "dc_one_kernel_guard",
+    "dc_decode_layer_errors", "dc_one_kernel_guard", "dc_decode_layer_is_short",
     "dc_pq_build_lut", "dc_pq_adc_scan", "dc_score_gathered_bf16", "dc_compose_idx",
     "dc_score_select_workspace_bytes", "dc_select_state_init", "dc_score_prune_bf16",
     "dc_sparse_select", "dc_score_select_bf16",
@@ -125,6 +125,7 @@ def _load() -> C.CDLL:
         "dc_set_wait_limit": (None, [i]),
         "dc_decode_layer_route": (i, [C.POINTER(LayerArgs)]),
         "dc_last_route": (i, []),
+        "dc_decode_layer_is_short": (i, [C.POINTER(LayerArgs)]),
         "dc_decode_layer_errors": (C.c_uint, []),
         "dc_one_kernel_guard": (i, [i, i, i, i, i]),
         "dc_pq_build_lut": (i, [p, p, p, i, i, i, i, p]),
@@ -818,6 +819,9 @@ class LayerCall:
     def route(self) -> int:
         return int(lib.dc_decode_layer_route(C.byref(self.args)))
 
+    def is_short(self) -> bool:
+        return lib.dc_decode_layer_is_short(C.byref(self.args)) == 1
+
 
 ROUTE_ATTEND_ONLY, ROUTE_DENSE, ROUTE_STREAM, ROUTE_SKETCH, ROUTE_ONE_KERNEL = range(5)
 
@@ -839,6 +843,15 @@ def decode_layer_route(*args, **kwargs) -> int:
     if rc < 0:
         _check(rc)
     return rc
+
+
+def decode_layer_is_short(*args, **kwargs) -> bool:
+    """Whether a decode_layer call with these arguments that does not run as one kernel takes the chain of
+    three kernels for short contexts, which reads the bf16 keys with or without a sketch."""
+    rc = lib.dc_decode_layer_is_short(C.byref(_layer_args(*args, **kwargs)))
+    if rc < 0:
+        _check(rc)
+    return rc == 1
 
 
 def decode_layer_status(*args, **kwargs) -> None:

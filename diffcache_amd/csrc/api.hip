@@ -116,13 +116,14 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
                               : (a->scores ? DC_ROUTE_DENSE
                                            : (a->sketch_codes && region <= DC_SKETCH_MAX_ROWS ? DC_ROUTE_SKETCH
                                                                                              : DC_ROUTE_STREAM));
+    const bool short_ok = dc_short_supported(a, region, k_eff);
     if (k_eff > 0 && !a->scores && a->order == DC_ORDER_ANY && !a->region_hi_dev &&
         dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr)) {
         // short context: the whole layer in one kernel whose blocks are all resident (ids in no
         // particular order); reads the bf16 keys, with or without a sketch.  The state is set up
-        // for this route even when the call is sent down the chain below (another launch of the
-        // kernel is in flight on another stream, or the stream is being captured): the next call
-        // with these sizes may take the kernel and be told that the state is ready.
+        // for this route even when the call is sent down a chain below (which is faster at these sizes, or
+        // another launch of the kernel is in flight on another stream, or the stream is being captured): the next
+        // call with these sizes may take the kernel and be told that the state is ready.
         if (!ready) {
             rc = dc_select_state_init(n_units, region, a->budget, w.topk, w.topk_bytes, stream);
             if (rc) return rc;
@@ -130,8 +131,11 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
             if (rc) return rc;
             ready = 1;
         }
-        if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
-        rc = dc_small_try(a, region, k_eff, w.topk, w.small_cand, w.attn, w.attn_bytes, stream, step);
+        rc = 0;
+        if (!short_ok || !dc_short_first(a, region)) {
+            if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
+            rc = dc_small_try(a, region, k_eff, w.topk, w.small_cand, w.attn, w.attn_bytes, stream, step);
+        }
         if (rc < 0) return rc;
         if (rc == 1) {
             if (a->ev_scan_end) (void)hipEventRecord((hipEvent_t)a->ev_scan_end, st);
@@ -139,6 +143,13 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
             // (every block of that kernel reads the state at a time of its own)
             return adv ? dc_step_state_advance(adv, 1, step->advance_limit, stream) : DC_OK;
         }
+    }
+    if (short_ok) {
+        if (!ready) {
+            rc = dc_select_state_init(n_units, region, a->budget, w.topk, w.topk_bytes, stream);
+            if (rc) return rc;
+        }
+        return dc_short_layer(a, region, k_eff, w.topk, w.attn, w.attn_bytes, stream, step);
     }
     if (k_eff > 0 && !a->scores && a->sketch_codes && region <= DC_SKETCH_MAX_ROWS) {
         // streaming select over the 8-bit sketch, exact rescoring of the kept rows
@@ -198,9 +209,17 @@ extern "C" int dc_decode_layer_route(const dc_layer_args *a) {
     if (n_units == 0 || k_eff <= 0) return DC_ROUTE_ATTEND_ONLY;
     if (a->scores) return DC_ROUTE_DENSE;
     if (a->order == DC_ORDER_ANY && a->one_kernel != DC_ONE_KERNEL_NEVER && !a->region_hi_dev &&
+        !(dc_short_supported(a, region, k_eff) && dc_short_first(a, region)) &&
         dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr))
         return DC_ROUTE_ONE_KERNEL;
     return a->sketch_codes && region <= DC_SKETCH_MAX_ROWS ? DC_ROUTE_SKETCH : DC_ROUTE_STREAM;
+}
+
+extern "C" int dc_decode_layer_is_short(const dc_layer_args *a) {
+    const int route = dc_decode_layer_route(a);
+    if (route != DC_ROUTE_SKETCH && route != DC_ROUTE_STREAM) return route < 0 ? route : 0;
+    const int region = (int)(a->recent_lo - a->n_sink);
+    return dc_short_supported(a, region, a->budget < region ? a->budget : region) ? 1 : 0;
 }
 
 extern "C" int dc_decode_layer_status(const dc_layer_args *a, void *stream) {

@@ -41,7 +41,11 @@ __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, 
     // blocks on 1024 places) then ends on every unit's last, partial split instead of on the last
     // units' full ones.
     const int n_units = (int)(gridDim.x / (unsigned)a.n_splits);
-    dc_attn_split_mfma<HD>(a, group, blockIdx.x % n_units, blockIdx.x / n_units, s_dyn);
+    const int unit = blockIdx.x % n_units, split = blockIdx.x / n_units;
+    AttnFrame<HD> f;
+    f.load(a, group, unit);
+    const uint32_t *ids = a.idx + (int64_t)unit * a.idx_stride;
+    dc_attn_split_mfma<HD, kAttnWaves, mfma_tiles(HD)>(a, f, group, unit, split, s_dyn, [ids](int p) { return ids[p]; });
 }
 
 // The splits of one query head, combined: out[u, g, :] = sum_s w_s acc_s / sum_s w_s l_s with
@@ -55,13 +59,15 @@ __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, 
 // 8 units, group 4, 128 columns: 18 splits 4.8 -> 3.7 us, 33 splits 5.5 -> 4.7 us (one thread per column before,
 // its rows eight at a time behind the weights).
 constexpr int kMergeBatch = 8;
+static_assert(DC_HIST_BINS == 4 * 256, "a thread clears four bins");
 
 template <int HD>
 __global__ __launch_bounds__(256) void merge_kernel(const float *__restrict__ ws_acc,
                                                     const float *__restrict__ ws_ml,
                                                     uint16_t *__restrict__ out, float *__restrict__ lse,
                                                     int group, int n_splits,
-                                                    int32_t *__restrict__ adv_state, int adv_limit) {
+                                                    int32_t *__restrict__ adv_state, int adv_limit,
+                                                    uint32_t *__restrict__ clear_hist) {
     constexpr int kLanes = HD / 4, kParts = 256 / kLanes;
     __shared__ float4 s_acc[256];
     const int ug = blockIdx.x;  // unit * group + g
@@ -94,6 +100,8 @@ __global__ __launch_bounds__(256) void merge_kernel(const float *__restrict__ ws
     load_rows(0);
     // the step is counted here because no block of this kernel reads the state
     if (adv_state && blockIdx.x == 0 && tid == 255) dc_state_advance(adv_state, 1, adv_limit);
+    if (clear_hist && g == 0)
+        reinterpret_cast<uint4 *>(clear_hist + (int64_t)unit * DC_HIST_BINS)[tid] = make_uint4(0u, 0u, 0u, 0u);
     float M = own.x;
     for (int sp = lane + 64; sp < n_splits; sp += 64) M = fmaxf(M, load_ml(sp).x);
 #pragma unroll
@@ -270,7 +278,6 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
     aa.ksb = ksb, aa.ksh = ksh, aa.ksr = ksr, aa.vsb = vsb, aa.vsh = vsh, aa.vsr = vsr;
     aa.scale = scale;
     aa.app = dc_append_of(step, k, v);
-    uint16_t *o16 = (uint16_t *)out;
     int rc = 0;
     if (mfma) {
         const size_t lds = mfma_shared_bytes(hd, group);
@@ -282,9 +289,16 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
     else rc = launch_attn<256>(group, grid, st, aa);
     DC_REQUIRE(rc == 0, "%s: unsupported group %d", who, group);
     DC_CHECK_LAUNCH(who);
+    return dc_merge_launch(who, w.acc, w.ml, out, lse, n_units, group, hd, plan.n_splits, step, nullptr, stream);
+}
+
+// merge_kernel over every unit and head; clear_hist: null, or the units' histograms, which it leaves zero.
+int dc_merge_launch(const char *who, const float *acc, const float *ml, void *out, float *lse, int n_units, int group, int hd,
+                    int n_splits, const dc_step_args *step, uint32_t *clear_hist, void *stream) {
 #define DC_LAUNCH_MERGE(HD)                                                                                              \
-    hipLaunchKernelGGL(merge_kernel<HD>, dim3((unsigned)(n_units * group)), dim3(256), 0, st, w.acc, w.ml, o16, lse, group, \
-                       plan.n_splits, step ? step->advance_state : nullptr, step ? step->advance_limit : 0)
+    hipLaunchKernelGGL(merge_kernel<HD>, dim3((unsigned)(n_units * group)), dim3(256), 0, (hipStream_t)stream, acc, ml,   \
+                       (uint16_t *)out, lse, group, n_splits, step ? step->advance_state : nullptr,                       \
+                       step ? step->advance_limit : 0, clear_hist)
     if (hd == 64) DC_LAUNCH_MERGE(64);
     else if (hd == 128) DC_LAUNCH_MERGE(128);
     else DC_LAUNCH_MERGE(256);

@@ -313,10 +313,9 @@ typedef uint32_t dc_u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kMfmaMaxGroup = 16;
 __host__ __device__ constexpr int mfma_tiles(int hd) { return hd <= 128 ? 2 : 1; }
-__host__ __device__ constexpr int mfma_rows_per_split(int hd) { return kAttnWaves * 16 * mfma_tiles(hd); }
-// floats of LDS: per-wave maxima and sums of 16 heads, per-wave partial outputs of G heads
-inline size_t mfma_shared_bytes(int hd, int group) {
-    return (size_t)(2 * kAttnWaves * 16 + kAttnWaves * group * hd) * sizeof(float);
+// bytes of LDS: per-wave maxima and sums of 16 heads, per-wave partial outputs of G heads
+inline size_t mfma_shared_bytes(int hd, int group, int waves = kAttnWaves) {
+    return (size_t)(2 * waves * 16 + waves * group * hd) * sizeof(float);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t dc_rows_rsrc(const void *base) {
@@ -330,38 +329,57 @@ __device__ __forceinline__ uint32_t dc_pack_bf16(float lo, float hi) {
     return __builtin_amdgcn_perm(rb, ra, 0x07060302u);  // (rb & 0xffff0000) | (ra >> 16)
 }
 
+// What a split needs besides the rows: the lengths of the unit's attended list (some of them device words) and
+// the query heads as the B operand (head c, columns 32 ch + 8 q .. + 7).  Read ahead of the row ids.
 template <int HD>
-__device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int unit, int split, float *s_mem) {
-    constexpr int TILES = mfma_tiles(HD);
+struct AttnFrame {
+    static constexpr int CH = HD / 32;  // instructions of one tile's QK^T
+    int n_recent, n_total, n_eff;
+    int64_t recent_lo;
+    dc_u32x4 bq[CH];
+    __device__ __forceinline__ void load(const AttnArgs &a, int G, int unit) {
+        const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+        n_recent = a.n_recent, n_total = a.n_total;
+        recent_lo = a.recent_lo_dev ? (int64_t)*a.recent_lo_dev : a.recent_lo;
+        if (a.n_recent_dev) {  // the window's length may live on the device (cache_seqlens, base.py:134-142)
+            int cur = *a.n_recent_dev;
+            cur = cur < 0 ? 0 : (cur < n_recent ? cur : n_recent);
+            n_total -= n_recent - cur;
+            n_recent = cur;
+        }
+        n_eff = a.n_idx;  // only the first n_eff selected ids of the unit count when per-unit sizes are given
+        if (a.n_idx_unit) {
+            const uint32_t ne = a.n_idx_unit[unit];
+            n_eff = ne < (uint32_t)a.n_idx ? (int)ne : a.n_idx;
+        }
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) {
+            bq[ch] = dc_u32x4{0u, 0u, 0u, 0u};
+            if (c < G) bq[ch] = *reinterpret_cast<const dc_u32x4 *>(a.Q + ((int64_t)unit * G + c) * HD + ch * 32 + q * 8);
+        }
+    }
+};
+
+// id_of(p): the selected id at position p < n_idx of the unit's list (relative to the region).
+template <int HD, int WAVES, int TILES, typename Ids>
+__device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, const AttnFrame<HD> &f, int G, int unit, int split,
+                                                   float *s_mem, Ids id_of) {
     constexpr int EPL = HD / 16;   // columns of a V row per lane
     constexpr int VW = EPL / 2;    // the same in 32-bit words
     constexpr int CH = HD / 32;    // instructions of one tile's QK^T
     constexpr int ROWS_W = 16 * TILES;
-    constexpr int ROWS = kAttnWaves * ROWS_W;
+    constexpr int ROWS = WAVES * ROWS_W;
     static_assert(HD == 64 || HD == 128 || HD == 256, "head_dim");
-    float *s_red = s_mem;                          // [kAttnWaves][16]
-    float *s_l = s_mem + kAttnWaves * 16;          // [kAttnWaves][16]
-    float *s_acc = s_mem + 2 * kAttnWaves * 16;    // [kAttnWaves][G * HD]
+    float *s_red = s_mem;                     // [WAVES][16]
+    float *s_l = s_mem + WAVES * 16;          // [WAVES][16]
+    float *s_acc = s_mem + 2 * WAVES * 16;    // [WAVES][G * HD]
 
     const int b = unit / a.n_h, h = unit % a.n_h;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int q = lane >> 4, c = lane & 15;
-    const int n_idx = a.n_idx, n_sink = a.n_sink;
-    int n_recent = a.n_recent, n_total = a.n_total;
-    const int64_t recent_lo = a.recent_lo_dev ? (int64_t)*a.recent_lo_dev : a.recent_lo;
-    if (a.n_recent_dev) {  // the window's length may live on the device (cache_seqlens, base.py:134-142)
-        int cur = *a.n_recent_dev;
-        cur = cur < 0 ? 0 : (cur < n_recent ? cur : n_recent);
-        n_total -= n_recent - cur;
-        n_recent = cur;
-    }
-    int n_eff = n_idx;  // only the first n_eff selected ids of the unit count when per-unit sizes are given
-    if (a.n_idx_unit) {
-        const uint32_t ne = a.n_idx_unit[unit];
-        n_eff = ne < (uint32_t)n_idx ? (int)ne : n_idx;
-    }
+    const int n_idx = a.n_idx, n_sink = a.n_sink, n_recent = f.n_recent;
     const int p0 = split * ROWS + wave * ROWS_W;
-    auto live = [&](int vj) { return vj < n_total && (vj < n_eff || vj >= n_idx); };
+    auto live = [&](int vj) { return vj < f.n_total && (vj < f.n_eff || vj >= n_idx); };
 
     // the store row of this lane's K position of every tile (row 0 for positions that do not count)
     uint32_t rowk[TILES];
@@ -370,19 +388,12 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int
         const int vj = p0 + t * 16 + c;
         uint32_t r = 0;
         if (live(vj)) {
-            if (vj < n_idx) r = (uint32_t)(a.region_lo + a.idx[(int64_t)unit * a.idx_stride + vj]);
+            if (vj < n_idx) r = (uint32_t)(a.region_lo + id_of(vj));
             else if (vj < n_idx + n_sink) r = (uint32_t)(vj - n_idx);
-            else if (vj < n_idx + n_sink + n_recent) r = (uint32_t)(recent_lo + (vj - n_idx - n_sink));
+            else if (vj < n_idx + n_sink + n_recent) r = (uint32_t)(f.recent_lo + (vj - n_idx - n_sink));
             else r = kNewToken;
         }
         rowk[t] = r;
-    }
-    // the query heads as the B operand: head c, columns 32 ch + 8 q .. + 7
-    dc_u32x4 bq[CH];
-#pragma unroll
-    for (int ch = 0; ch < CH; ++ch) {
-        bq[ch] = dc_u32x4{0u, 0u, 0u, 0u};
-        if (c < G) bq[ch] = *reinterpret_cast<const dc_u32x4 *>(a.Q + ((int64_t)unit * G + c) * HD + ch * 32 + q * 8);
     }
     const __amdgpu_buffer_rsrc_t rk = dc_rows_rsrc(a.K + b * a.ksb + h * a.ksh);
     const __amdgpu_buffer_rsrc_t rv = dc_rows_rsrc(a.V + b * a.vsb + h * a.vsh);
@@ -438,7 +449,7 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int
 #pragma unroll
         for (int ch = 0; ch < CH; ++ch)
             s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, kw[t][ch]),
-                                                        __builtin_bit_cast(dc_bf16x8, bq[ch]), s, 0, 0, 0);
+                                                        __builtin_bit_cast(dc_bf16x8, f.bq[ch]), s, 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             x[t][i] = live(p0 + t * 16 + 4 * q + i) ? s[i] * a.scale : -INFINITY;
@@ -452,7 +463,7 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int
     __syncthreads();
     float m = s_red[c];
 #pragma unroll
-    for (int w2 = 1; w2 < kAttnWaves; ++w2) m = fmaxf(m, s_red[w2 * 16 + c]);
+    for (int w2 = 1; w2 < WAVES; ++w2) m = fmaxf(m, s_red[w2 * 16 + c]);
 
     // P = exp(S - m): this lane's part of the A operand of P V, as the sum of two bf16 values
     // (p = hi + lo to 2^-17 of p: with P rounded to one bf16 a slice of a few rows misses the
@@ -511,16 +522,16 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, int G, int
     }
     __syncthreads();
     const int64_t slot = (int64_t)unit * a.n_splits + split;
-    for (int o = tid; o < G * HD; o += kAttnThreads) {
+    for (int o = tid; o < G * HD; o += WAVES * 64) {
         float s = s_acc[o];
 #pragma unroll
-        for (int w2 = 1; w2 < kAttnWaves; ++w2) s += s_acc[w2 * G * HD + o];
+        for (int w2 = 1; w2 < WAVES; ++w2) s += s_acc[w2 * G * HD + o];
         a.ws_acc[slot * (G * HD) + o] = s;
     }
     if (tid < G) {
         float l = s_l[tid], mm = s_red[tid];
 #pragma unroll
-        for (int w2 = 1; w2 < kAttnWaves; ++w2) {
+        for (int w2 = 1; w2 < WAVES; ++w2) {
             l += s_l[w2 * 16 + tid];
             mm = fmaxf(mm, s_red[w2 * 16 + tid]);
         }

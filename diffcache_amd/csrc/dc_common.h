@@ -59,6 +59,13 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
                           int64_t ksh, int64_t ksr, int64_t vsb, int64_t vsh, int64_t vsr, float scale,
                           void *workspace, size_t workspace_bytes, void *stream, const int32_t *recent_lo_dev,
                           const dc_step_args *step = nullptr);
+int dc_merge_launch(const char *who, const float *acc, const float *ml, void *out, float *lse, int n_units, int group, int hd,
+                    int n_splits, const dc_step_args *step, uint32_t *clear_hist, void *stream);
+// short.hip: a decode layer in three kernels, for short contexts
+bool dc_short_supported(const dc_layer_args *a, int region, int k_eff);
+bool dc_short_first(const dc_layer_args *a, int region);
+int dc_short_layer(const dc_layer_args *a, int region, int k_eff, void *sel_ws, void *attn_ws, size_t attn_ws_bytes,
+                   void *stream, const dc_step_args *step);
 // sketch.hip: the quantising pass of dc_sketch_build_bf16
 int dc_sketch_quantise_launch(const char *who, const void *k, uint8_t *codes, const float *scale, float *resid,
                               int n_units, int n_h, int n_rows, int hd, int64_t sb, int64_t sh, int64_t sr, int64_t cb,

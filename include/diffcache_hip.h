@@ -435,10 +435,18 @@ typedef struct dc_step_args {
 } dc_step_args;
 int dc_decode_layer_step(const dc_layer_args *args, const dc_step_args *step, void *stream);
 /*
- * Short contexts.  With scores == NULL, order == DC_ORDER_ANY and at most 640 Ki region rows
- * over all units (and, when a sketch is passed, at most 40 Ki region rows per unit), dc_decode_layer runs the layer as ONE kernel whose blocks are all resident
+ * Short contexts.  With scores == NULL, order == DC_ORDER_ANY, at most 32 Ki region rows per unit and 64 MiB of
+ * keys in the regions of all units, a layer runs as a chain of THREE kernels over the bf16 keys, with or without a
+ * sketch (scores; selection and attention in one; merge), on any stream, also under capture and with
+ * region_hi_dev; the event pair brackets the first.  dc_decode_layer_is_short says whether a call that does not
+ * run as one kernel is of that kind; its route is named DC_ROUTE_SKETCH or DC_ROUTE_STREAM like any chain's.
+ *
+ * With at most 640 Ki region rows over all units (and, when a sketch is passed, at most 40 Ki region rows per
+ * unit), dc_decode_layer can run the layer as ONE kernel whose blocks are all resident
  * (two per CU) and hand their phases over through the workspace (same results; the event pair
- * then brackets that kernel).  No counterpart in the reference, whose layers run on the CPU pool
+ * then brackets that kernel).  It does so where the chain of three does not apply; with DC_ONE_KERNEL_EXCLUSIVE; for
+ * callers without a sketch, up to 12 Ki rows per unit or two units; and with a sketch, for two units of more than
+ * 16 Ki rows.  No counterpart in the reference, whose layers run on the CPU pool
  * (lib.rs:352-369); what it has to match is that one layer call is always right
  * (src/diffcache/base.py:150-155).
  *
@@ -485,10 +493,11 @@ unsigned dc_decode_layer_errors(void);
  */
 #define DC_ROUTE_ATTEND_ONLY 0 /* nothing to select (empty region or budget 0) */
 #define DC_ROUTE_DENSE 1       /* fp32 scores materialised: dc_score_bf16 + dc_topk_select */
-#define DC_ROUTE_STREAM 2      /* dc_score_prune_bf16 + dc_sparse_select */
-#define DC_ROUTE_SKETCH 3      /* dc_score_select_sketch_bf16 */
+#define DC_ROUTE_STREAM 2      /* a chain without a sketch: dc_score_prune_bf16 + dc_sparse_select, or the short one */
+#define DC_ROUTE_SKETCH 3      /* a chain with one: dc_score_select_sketch_bf16, or the short one */
 #define DC_ROUTE_ONE_KERNEL 4  /* short context: the whole layer in one kernel */
 int dc_decode_layer_route(const dc_layer_args *args);
+int dc_decode_layer_is_short(const dc_layer_args *args); /* 1, 0 or a negative DC_E* code; see "Short contexts" */
 int dc_last_route(void);
 /*
  * The rule by which a call is kept off the one-kernel route, as a function of what the library
