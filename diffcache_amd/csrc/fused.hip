@@ -266,8 +266,15 @@ constexpr int kSketchRowBits = 22;
 constexpr int kSketchMaxRows = 1 << kSketchRowBits;
 static_assert(kSketchMaxRows == DC_SKETCH_MAX_ROWS && DC_HIST_BINS <= (1 << (32 - kSketchRowBits)), "row and bucket share a word");
 __device__ __forceinline__ uint32_t sketch_entry(uint32_t bucket, uint32_t row) { return (bucket << kSketchRowBits) | row; }
+// words of two bytes between the units of a dense scan's buckets (16-byte rows of them)
+__host__ __device__ __forceinline__ int64_t dense_stride(int n_cap) { return ((int64_t)n_cap + 7) & ~7ll; }
 
-template <int HD, bool SHARED_POLL>
+// DENSE: for scans whose blocks all run at the same time.  There a threshold never comes early enough to drop a row
+// worth its poll, so nothing is polled or listed: every row's bucket of (approximation + margin) goes to the row's
+// own place, two bytes, and the exact pass reads them all.  That leaves out the block's closing round trip (the returning
+// atomic that reserves its list slots) and the refresh of the threshold behind it, and the grid can be one of equal
+// shares (sizes and times: plan_dense).
+template <int HD, bool SHARED_POLL, bool DENSE>
 __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kernel(
     const uint8_t *__restrict__ C, const uint16_t *__restrict__ Q, const float *__restrict__ scale,
     const float *__restrict__ resid, uint32_t *__restrict__ hist, UnitState *__restrict__ state,
@@ -283,7 +290,7 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     const int n_rows = dc_live_rows(n_cap, hi_dev, lo_row);
     __shared__ uint32_t lhist[DC_HIST_BINS];
     __shared__ __align__(16) uint8_t s_w[4][HD];  // the weights' digits, lowest first
-    __shared__ uint32_t stage[kStage];  // kept rows as kSketchEntry words
+    __shared__ uint32_t stage[DENSE ? 1 : kStage];  // kept rows as kSketchEntry words
     __shared__ uint32_t s_tb;  // the block's copy of the unit's running threshold bucket
     __shared__ uint32_t wtot[kThreads / 64 + 1];
     __shared__ uint32_t s_wcnt[kThreads / 64];
@@ -312,7 +319,8 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     const uint8_t *Cu = C + b * cb + h * ch + (grp * S + side) * 16;
     UnitState *st = state + unit;
     const int last = n_rows - 1;
-    uint32_t tb = load_relaxed(&st->tb_run);
+    uint32_t tb = DENSE ? (uint32_t)DC_HIST_BINS : load_relaxed(&st->tb_run);
+    uint16_t *du = reinterpret_cast<uint16_t *>(surv) + (int64_t)unit * dense_stride(n_cap);
 
     // Double buffering: the loads of the next step are issued before the current step is
     // worked on, so a wave always has a step's worth of bytes in flight.  The loads are
@@ -442,6 +450,13 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
         const int64_t myrow = row0 + own_row;
         const bool valid = myrow < n_rows;
         const uint32_t lb = dc_score_bucket(mine), kb = dc_score_bucket(mine + margin);
+        if constexpr (DENSE) {
+            if (valid) {
+                du[myrow] = (uint16_t)kb;
+                atomicAdd(&lhist[lb], 1u);
+            }
+            return;
+        }
         const bool keep = valid && kb <= tb;
         if (keep) atomicAdd(&lhist[lb], 1u);
         const unsigned long long mask = __ballot(keep);
@@ -469,6 +484,22 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     // polls and passes the value on through LDS.  With many units every wave polls for
     // itself, which keeps its threshold one step fresher.
     // (SHARED_POLL is a template parameter: as a run-time choice it costs registers.)
+    if constexpr (DENSE) {
+        for (; step + 1 < my_steps; step += 2) {
+            load_step(step + 1, cb2);
+            work_step(step, ca, std::false_type{});
+            load_step(step + 2, ca);
+            work_step(step + 1, cb2, std::false_type{});
+        }
+        if (step < my_steps) work_step(step, ca, std::false_type{});
+        __syncthreads();
+        uint32_t *hu = hist + (int64_t)unit * DC_HIST_BINS;
+        for (int i = tid; i < DC_HIST_BINS; i += kThreads) {
+            const uint32_t c = lhist[i];
+            if (c) atomicAdd(&hu[i], c);
+        }
+        return;
+    }
     auto two_steps = [&](auto count) __attribute__((always_inline)) {
         uint32_t tb_next = tb;
         if (!SHARED_POLL || wave == 0) tb_next = load_relaxed(&st->tb_run);
@@ -729,15 +760,20 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(
 // holds every member of the top-k).
 constexpr int kRescoreBatch = 4;
 
-template <int HD>
+// DENSE: the scan left a bucket for every row (sketch_prune_kernel); a block takes kDensePer rows of a thread at a time, side
+// by side, and the tiles of a unit are dealt to its blocks as they come.
+constexpr int kDensePer = 8;
+
+template <int HD, bool DENSE>
 __global__ __launch_bounds__(kThreads) void rescore_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, const uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, const uint2 *__restrict__ surv, uint32_t *__restrict__ cand_key,
     uint32_t *__restrict__ cand_idx, int n_units, int n_h, int n_rows, int64_t sb, int64_t sh,
-    int64_t sr, int q_group, int mode, int k_eff, int nblk) {
+    int64_t sr, int q_group, int mode, int k_eff, int nblk, const int32_t *__restrict__ hi_dev, int lo_row) {
     constexpr int LPR = HD / 8;
     constexpr int GROUPS = kThreads / LPR;
-    constexpr uint32_t kPer = kRescoreBatch * kThreads;
+    constexpr int kOwn = DENSE ? kDensePer : kRescoreBatch;  // entries of a thread per batch
+    constexpr uint32_t kPer = kOwn * kThreads;
     __shared__ uint32_t cid[kPer];
     __shared__ uint32_t ckey[kPer];
     __shared__ uint32_t wtot[kThreads / 64 + 1];
@@ -761,20 +797,34 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
     // beyond the length is stale and is masked below), together with the length, the histogram
     // and the query: one memory round trip for all of them.
     const uint32_t *su = reinterpret_cast<const uint32_t *>(surv) + (int64_t)unit * n_rows;
-    uint32_t p[kRescoreBatch];
+    const uint16_t *du = reinterpret_cast<const uint16_t *>(surv) + (int64_t)unit * dense_stride(n_rows);
+    uint32_t p[4];
+    auto load_dense = [&](uint32_t t) __attribute__((always_inline)) {
+        const uint32_t i = (((uint32_t)blk + t * (uint32_t)nblk) * kThreads + (uint32_t)tid) * kDensePer;
+        uint4 v = make_uint4(~0u, ~0u, ~0u, ~0u);
+        if (i < (uint32_t)n_rows) v = *reinterpret_cast<const uint4 *>(du + i);
+        p[0] = v.x, p[1] = v.y, p[2] = v.z, p[3] = v.w;
+    };
+    uint32_t n_s;
+    if constexpr (DENSE) {
+        load_dense(0u);
+        n_s = (uint32_t)dc_live_rows(n_rows, hi_dev, lo_row);
+    } else {
 #pragma unroll
-    for (int j = 0; j < kRescoreBatch; ++j) {
-        const uint32_t i = entry((uint32_t)j);
-        p[j] = 0xffffffffu;
-        if (i < (uint32_t)n_rows) p[j] = su[i];
+        for (int j = 0; j < kRescoreBatch; ++j) {
+            const uint32_t i = entry((uint32_t)j);
+            p[j] = 0xffffffffu;
+            if (i < (uint32_t)n_rows) p[j] = su[i];
+        }
+        n_s = st->surv_cnt;
     }
-    uint32_t n_s = st->surv_cnt;
     float q[8];
     dc_load_query<HD>(Q, unit, q_group, col, q);
     uint32_t tb, c_less;
     unit_threshold(hist + (int64_t)unit * DC_HIST_BINS, (uint32_t)k_eff, wtot, sres, tb, c_less);
     if (n_s > (uint32_t)n_rows) n_s = n_rows;
-    const uint32_t n_tiles = (n_s + kThreads - 1) / kThreads;
+    constexpr uint32_t kTile = DENSE ? kPer : (uint32_t)kThreads;
+    const uint32_t n_tiles = (n_s + kTile - 1) / kTile;
     if ((uint32_t)blk >= n_tiles) return;
     const uint32_t my_tiles = (n_tiles - (uint32_t)blk + (uint32_t)nblk - 1) / (uint32_t)nblk;
     if (blk == 0 && tid == 0) st->c_less = 0;
@@ -782,24 +832,34 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
     uint32_t *ck = cand_key + (int64_t)unit * n_rows;
     uint32_t *ci = cand_idx + (int64_t)unit * n_rows;
 
-    for (uint32_t t0 = 0; t0 < my_tiles; t0 += kRescoreBatch) {
+    for (uint32_t t0 = 0; t0 < my_tiles; t0 += DENSE ? 1 : kRescoreBatch) {
         uint32_t pass = 0;
+        const uint32_t row0 = (((uint32_t)blk + t0 * (uint32_t)nblk) * kThreads + (uint32_t)tid) * kDensePer;  // DENSE
+        if constexpr (DENSE) {
+            if (t0 != 0) load_dense(t0);
 #pragma unroll
-        for (int j = 0; j < kRescoreBatch; ++j) {
-            const uint32_t t = t0 + (uint32_t)j;
-            const uint32_t i = entry(t);
-            const bool in = t < my_tiles && i < n_s;
-            if (t0 != 0) {
-                p[j] = 0xffffffffu;
-                if (in) p[j] = su[i];
+            for (int j = 0; j < kDensePer; ++j) {
+                const uint32_t kb = j & 1 ? p[j / 2] >> 16 : p[j / 2] & 0xffffu;
+                if (row0 + j < n_s && kb <= tb) pass |= 1u << j;
             }
-            if (in && (p[j] >> kSketchRowBits) <= tb) pass |= 1u << j;
+        } else {
+#pragma unroll
+            for (int j = 0; j < kRescoreBatch; ++j) {
+                const uint32_t t = t0 + (uint32_t)j;
+                const uint32_t i = entry(t);
+                const bool in = t < my_tiles && i < n_s;
+                if (t0 != 0) {
+                    p[j] = 0xffffffffu;
+                    if (in) p[j] = su[i];
+                }
+                if (in && (p[j] >> kSketchRowBits) <= tb) pass |= 1u << j;
+            }
         }
         uint32_t n_c;
         uint32_t pos = block_excl_scan<kThreads>(__popc(pass), wtot, &n_c);
 #pragma unroll
-        for (int j = 0; j < kRescoreBatch; ++j)
-            if (pass & (1u << j)) cid[pos++] = p[j] & (uint32_t)(kSketchMaxRows - 1);
+        for (int j = 0; j < kOwn; ++j)
+            if (pass & (1u << j)) cid[pos++] = DENSE ? row0 + j : p[j] & (uint32_t)(kSketchMaxRows - 1);
         // The list slot is reserved now and looked at after the rows are scored.  (Through an address
         // the compiler cannot prove uniform: it turns an atomic on a uniform address into one atomic
         // per wave plus a broadcast of the result and waits for that on the spot, a memory round
@@ -1103,6 +1163,25 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
     return DC_OK;
 }
 
+// Whether the sketch scan of these sizes is a dense one, and its grid: blocks of equal shares, all running at once
+// (four per CU at 64 columns, three at 128, two at 256).  Per layer, us, listed / dense: 8 units x 131004 rows of 128 columns
+// 48.9 / 45.1, x 65468 38.5 / 35.5, 16 x 131004 75.0 / 69.5, 32 x 131004 125.4 / 121.5, 4 x 1048508 135.5 / 121.8, 128 x 32700 138.6 /
+// 135; 8 x 131004 of 64 38.4 / 32.0, 12 x 24615 of 256 44.7 / 41.4.  Beyond 4 Mi rows in all equal shares end at unequal times
+// and the two bytes a row outweigh the list: 64 x 131004 225.8 / 237.7, 8 x 1048508 221.7 / 235.3.
+constexpr int64_t kDenseMostTiles = (4ll << 20) / kRowsPerBlockStep;
+
+bool plan_dense(int64_t n_units, int n_rows, int hd, FusedPlan *p) {
+    const int64_t tiles = ((int64_t)n_rows + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
+    if (n_units * tiles > kDenseMostTiles) return false;
+    if (p) {
+        const int64_t most = 256 * (hd == 64 ? 4 : (hd == 128 ? 3 : 2)), steps = (n_units * tiles + most - 1) / most;
+        p->small_chunks = 0;
+        p->big_steps = (int)steps;
+        p->blocks = n_units * ((tiles + steps - 1) / steps);
+    }
+    return true;
+}
+
 int check_ws(const char *who, void *workspace, size_t workspace_bytes, int n_units, int n_rows,
              int budget, FusedWs *w) {
     DC_REQUIRE(workspace && (((uintptr_t)workspace) & 255u) == 0,
@@ -1278,6 +1357,7 @@ int dc_sketch_scan_launch(const char *who, const void *k, const uint8_t *codes, 
     FusedPlan p;
     int rc = plan_fused(who, n_b, n_h, n_rows, budget, &p, kBigSteps, kRowsPerBlockStep, kSketchFillBlocks);
     if (rc) return rc;
+    const bool dense = plan_dense(p.n_units, n_rows, hd, &p);
     if (p.n_units == 0 || p.k_eff == 0) return DC_OK;
     DC_REQUIRE(workspace && (((uintptr_t)workspace) & 255u) == 0,
                "%s: workspace must be non-null and 256-byte aligned", who);
@@ -1292,17 +1372,21 @@ int dc_sketch_scan_launch(const char *who, const void *k, const uint8_t *codes, 
         if (rc) return rc;
     }
     if (ev_scan_begin) (void)hipEventRecord((hipEvent_t)ev_scan_begin, st);
-#define DC_LAUNCH_SK(HD, SP)                                                                        \
-    hipLaunchKernelGGL((sketch_prune_kernel<HD, SP>), dim3((unsigned)p.blocks), dim3(kThreads), 0, st,  \
+#define DC_LAUNCH_SK(HD, SP, DN)                                                                    \
+    hipLaunchKernelGGL((sketch_prune_kernel<HD, SP, DN>), dim3((unsigned)p.blocks), dim3(kThreads), 0, st,  \
                        codes, (const uint16_t *)q, scale, resid, w.hist, w.state, w.surv, p.n_units,    \
                        n_h, n_rows, cb, ch, cr, q_group, mode, p.k_eff, p.small_chunks, p.big_steps, hi_dev, lo_row)
     const bool shared_poll = p.n_units <= kSharedPollUnits;
-    if (hd == 64 && shared_poll) DC_LAUNCH_SK(64, true);
-    else if (hd == 64) DC_LAUNCH_SK(64, false);
-    else if (hd == 128 && shared_poll) DC_LAUNCH_SK(128, true);
-    else if (hd == 128) DC_LAUNCH_SK(128, false);
-    else if (shared_poll) DC_LAUNCH_SK(256, true);
-    else DC_LAUNCH_SK(256, false);
+#define DC_LAUNCH_SKH(HD)                                  \
+    do {                                                   \
+        if (dense) DC_LAUNCH_SK(HD, false, true);          \
+        else if (shared_poll) DC_LAUNCH_SK(HD, true, false); \
+        else DC_LAUNCH_SK(HD, false, false);               \
+    } while (0)
+    if (hd == 64) DC_LAUNCH_SKH(64);
+    else if (hd == 128) DC_LAUNCH_SKH(128);
+    else DC_LAUNCH_SKH(256);
+#undef DC_LAUNCH_SKH
 #undef DC_LAUNCH_SK
     DC_CHECK_LAUNCH(who);
     if (ev_scan_end) (void)hipEventRecord((hipEvent_t)ev_scan_end, st);
@@ -1351,14 +1435,25 @@ int dc_sketch_select_impl(const void *k, const uint8_t *codes, const float *scal
     const int cap = p.n_units >= grid ? 1 : grid / p.n_units;
     if (nblk > cap) nblk = cap;
     if (nblk < 1) nblk = 1;
-#define DC_LAUNCH_RS(HD)                                                                              \
-    hipLaunchKernelGGL(rescore_kernel<HD>, dim3((unsigned)p.n_units * (unsigned)nblk), dim3(kThreads), 0, \
+    const bool dense = plan_dense(p.n_units, n_rows, hd, nullptr);
+    if (dense) {
+        const int tiles = (n_rows + kThreads * kDensePer - 1) / (kThreads * kDensePer);
+        if (nblk > tiles) nblk = tiles;
+    }
+#define DC_LAUNCH_RSD(HD, DN)                                                                         \
+    hipLaunchKernelGGL((rescore_kernel<HD, DN>), dim3((unsigned)p.n_units * (unsigned)nblk), dim3(kThreads), 0, \
                        st, (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv, w.cand_key, \
-                       w.cand_idx, p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, nblk)
+                       w.cand_idx, p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, nblk, hi_dev, lo_row)
+#define DC_LAUNCH_RS(HD)                     \
+    do {                                     \
+        if (dense) DC_LAUNCH_RSD(HD, true);  \
+        else DC_LAUNCH_RSD(HD, false);       \
+    } while (0)
     if (hd == 64) DC_LAUNCH_RS(64);
     else if (hd == 128) DC_LAUNCH_RS(128);
     else DC_LAUNCH_RS(256);
 #undef DC_LAUNCH_RS
+#undef DC_LAUNCH_RSD
     DC_CHECK_LAUNCH(who);
     return launch_finish(who, w, idx_out, idx_unit_stride, p.n_units, n_rows, p.k_eff, mode, order, 1, st);
 }
