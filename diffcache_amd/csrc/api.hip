@@ -132,7 +132,7 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
             ready = 1;
         }
         rc = 0;
-        if (!short_ok || !dc_short_first(a, region)) {
+        if (dc_one_kernel_first(a, region, k_eff)) {
             if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
             rc = dc_small_try(a, region, k_eff, w.topk, w.small_cand, w.attn, w.attn_bytes, stream, step);
         }
@@ -209,7 +209,7 @@ extern "C" int dc_decode_layer_route(const dc_layer_args *a) {
     if (n_units == 0 || k_eff <= 0) return DC_ROUTE_ATTEND_ONLY;
     if (a->scores) return DC_ROUTE_DENSE;
     if (a->order == DC_ORDER_ANY && a->one_kernel != DC_ONE_KERNEL_NEVER && !a->region_hi_dev &&
-        !(dc_short_supported(a, region, k_eff) && dc_short_first(a, region)) &&
+        dc_one_kernel_first(a, region, k_eff) &&
         dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr))
         return DC_ROUTE_ONE_KERNEL;
     return a->sketch_codes && region <= DC_SKETCH_MAX_ROWS ? DC_ROUTE_SKETCH : DC_ROUTE_STREAM;

@@ -63,7 +63,7 @@ int dc_merge_launch(const char *who, const float *acc, const float *ml, void *ou
                     int n_splits, const dc_step_args *step, uint32_t *clear_hist, void *stream);
 // short.hip: a decode layer in three kernels, for short contexts
 bool dc_short_supported(const dc_layer_args *a, int region, int k_eff);
-bool dc_short_first(const dc_layer_args *a, int region);
+bool dc_one_kernel_first(const dc_layer_args *a, int region, int k_eff);
 int dc_short_layer(const dc_layer_args *a, int region, int k_eff, void *sel_ws, void *attn_ws, size_t attn_ws_bytes,
                    void *stream, const dc_step_args *step);
 // sketch.hip: the quantising pass of dc_sketch_build_bf16

@@ -433,8 +433,10 @@ constexpr int kScoreBlocks = 512;
 // that and another two kernels' worth of hand-overs.  Per layer, this chain / sketch chain, us: 8 units x 16316
 // rows of 128 columns (33 MB) 21.9 / 27.3, x 24616 (50 MB) 26.4 / 28.8, x 32533 (67 MB) 30.1 / 29.9; 32 x 8124 (67 MB)
 // 27.9 / 32.1, x 16316 (134 MB) 43.5 / 40.9; 64 x 4028 (66 MB) 28.4 / 33.5; 12 x 24615 of 256 (151 MB) 50.0 / 44.0;
-// 8 x 16323 of 64 (17 MB) 19.2 / 24.8.
-constexpr int64_t kShortBytes = 64ll << 20;
+// 8 x 16323 of 64 (17 MB) 19.2 / 24.8.  (With the dense scan of later the sketch chain takes 26.2, 27.7, 28.4; 29.7, 35.8; 32.5; 40.3;
+// 22.7.)  It goes with k, 8 x 32533 x 128 with 4096 ids: 31.4 / 35.5, so long regions of which few rows are selected
+// leave at kShortBytesFew.
+constexpr int64_t kShortBytes = 64ll << 20, kShortBytesFew = 56ll << 20;
 
 }  // namespace
 
@@ -443,20 +445,27 @@ constexpr int64_t kShortBytes = 64ll << 20;
 bool dc_short_supported(const dc_layer_args *a, int region, int k_eff) {
     const int64_t n_units = (int64_t)a->n_b * a->n_h;
     return a->order == DC_ORDER_ANY && !a->scores && k_eff > 0 && n_units > 0 && region >= 64 && region <= kShortMaxRows &&
-           n_units * region * a->hd * 2 <= kShortBytes && a->group >= 1 && a->group * a->hd <= 1024 &&
+           n_units * region * a->hd * 2 <=
+               (a->sketch_codes && region > 16 * 1024 && k_eff < region / 12 ? kShortBytesFew : kShortBytes) && a->group >= 1 && a->group * a->hd <= 1024 &&
            (a->hd == 64 || a->hd == 128 || a->hd == 256) && a->kv_row_stride > 0 &&
            (a->recent_lo + a->n_recent + 1) * a->kv_row_stride * 2 <= 0xffffffffll;
 }
 
-// Whether it is preferred to the one kernel where both can be taken.  It is the faster one at every size measured
-// (us, one kernel / this chain): 2 units x 4028 rows of 128 columns 18.1 / 15.4, x 16316 22.8 / 19.0; 8 x 4028 19.2 /
-// 17.3, x 16316 30.4 / 21.9, x 32533 35.1 / 30.1; 64 x 4028 32.2 / 28.4; 8 x 16323 of 64 33.1 / 19.2.  Two units of more than
-// 16 Ki rows, callers without a sketch up to 12 Ki, and callers who vouch for an exclusive GPU stay with the one
-// kernel all the same: that is the route they are told of (dc_decode_layer_route) and rely on.
-bool dc_short_first(const dc_layer_args *a, int region) {
+// Whether a layer that can run as one kernel (small.hip) does.  With a sketch the chains are the faster ones at every
+// size measured (us, one kernel / this chain / sketch chain): 2 units x 4028 rows of 128 columns 18.1 / 15.4, x 16316
+// 22.8 / 19.0; 8 x 4028 19.2 / 17.3, x 16316 30.4 / 21.9, x 32533 35.1 / 30.1 / 28.4; 64 x 4028 32.2 / 28.4; 8 x 16323 of 64 33.1 / 19.2;
+// 32 x 16316 44.7 / - / 35.8; 12 x 24615 of 256 51.0 / - / 40.3; 8 x 39932 of 128 39.5 / - / 31.4 (with the longer sketch chain of
+// then).  What is left to it: groups too large for this chain's attention, as long as it takes less than the sketch
+// chain (8 x 4028 of 256 22.5 / - / 31.6, x 16316 38.7 / - / 33.0).  Two units of more than 16 Ki rows, callers
+// without a sketch up to 12 Ki rows or two units, and callers who vouch for an exclusive GPU stay with it all the same:
+// that is the route they are told of (dc_decode_layer_route) and rely on.
+bool dc_one_kernel_first(const dc_layer_args *a, int region, int k_eff) {
     const int64_t n_units = (int64_t)a->n_b * a->n_h;
-    if (a->one_kernel == DC_ONE_KERNEL_EXCLUSIVE) return false;
-    return a->sketch_codes ? n_units > 2 || region <= 16 * 1024 : n_units > 2 && region > 12 * 1024;
+    const bool short_ok = dc_short_supported(a, region, k_eff);
+    if (a->one_kernel == DC_ONE_KERNEL_EXCLUSIVE) return true;
+    if (!a->sketch_codes) return !short_ok || n_units <= 2 || region <= 12 * 1024;
+    if (n_units <= 2 && region > 16 * 1024) return true;
+    return !short_ok && region <= 16 * 1024 && n_units * region * a->hd * 2 <= (32ll << 20);
 }
 
 // The layer on `stream`.  sel_ws: the select part of the workspace, its histograms zero (and left so).

@@ -46,11 +46,7 @@ constexpr int kSmallRows = 4096;     // rows a block scores at most (their score
 constexpr int kSmallCand = 4096;     // candidates of a unit that are ranked in LDS
 constexpr int kSmallBlocks = 512;    // blocks of a launch at most: two per CU
 constexpr int64_t kSmallTotalRows = 640 * 1024;  // rows of all units that the route takes on (measured crossover)
-// ... and rows per unit when the caller brings a sketch.  The line was drawn where the sketch chain won then (8 units,
-// 128 columns: 43.3 us against 41.6 us for the chain at 49152 rows, 37.3 against 40.6 at 32768; 16 units: 53.4
-// against 50.8 at 40960).  The chain has become faster since and wins well below it: at 8 units of 128
-// columns 22.9 against 27.5 us at 8124 rows, but 32.1 against 27.7 at 16316 and 36.4 against 30.4 at 32533; 16
-// units 28.7 / 26.9 at 8124; 12 units of 256 columns 51.1 / 43.5 at 24615.
+// ... and rows per unit when the caller brings a sketch (where it is preferred to the chains: dc_one_kernel_first).
 constexpr int kSmallSketchRows = 40 * 1024;
 constexpr int kSmallMl = 2048;       // floats of (m, l) the merge keeps in LDS: blocks per unit * G * 2
 

@@ -144,7 +144,29 @@ def test_which_calls_take_the_short_chain():
     assert short() == short(sketch=None) == 1
     assert short(rows=64) == 1 and short(rows=63) == 0
     assert short(units=1, rows=32768) == 1 and short(units=1, rows=32769) == 0
-    assert short(units=8, rows=32768) == 1 and short(units=9, rows=32768) == 0      # 64 MiB of keys
+    assert short(units=8, rows=32768, budget=4096) == 1 and short(units=9, rows=32768, budget=4096) == 0    # 64 MiB of keys
+    assert short(units=7, rows=32768) == 1 and short(units=8, rows=32768) == 0      # 56 MiB, few rows selected
+    assert short(units=8, rows=32768, sketch=None) == short(units=16, rows=16384) == 1
     assert short(hd=256, group=4) == 1 and short(hd=256, group=5) == 0 and short(group=8) == 1 and short(group=9) == 0
     assert short(order=hip.ORDER_BEST) == short(order=hip.ORDER_INDEX) == short(budget=0) == short(scores=0x1000) == 0
     assert short(kv_row_stride=1 << 20) == 0                                        # rows beyond 4 GiB of the unit's first
+
+
+@pytest.mark.gpu
+def test_which_calls_run_as_one_kernel():
+    from diffcache_amd import _hip as hip
+
+    def route(units, rows, hd=128, group=4, sketch=0x1000, policy=hip.ONE_KERNEL_AUTO, region_hi_dev=None):
+        a = hip.LayerArgs()
+        a.n_b, a.n_h, a.group, a.hd, a.budget, a.n_sink = 1, units, group, hd, 512, 4
+        a.recent_lo, a.n_recent, a.kv_row_stride, a.sketch_codes, a.one_kernel = 4 + rows, 64, hd, sketch, policy
+        a.region_hi_dev = region_hi_dev
+        return hip.lib.dc_decode_layer_route(ctypes.byref(a))
+    one, chain, stream = hip.ROUTE_ONE_KERNEL, hip.ROUTE_SKETCH, hip.ROUTE_STREAM
+    assert [route(8, n) for n in (4028, 16384, 32768, 40960)] == [chain] * 4
+    assert [route(2, n) for n in (4028, 16384, 16385, 40960, 40961)] == [chain, chain, one, one, chain]
+    assert [route(8, n, sketch=None) for n in (4028, 12288, 12289, 32768, 40960)] == [one, one, stream, stream, one]
+    assert [route(2, n, sketch=None) for n in (4028, 40960)] == [one, one]
+    assert [route(8, n, policy=hip.ONE_KERNEL_EXCLUSIVE) for n in (4028, 32768)] == [one, one]
+    assert route(8, 4028, policy=hip.ONE_KERNEL_NEVER) == chain and route(8, 4028, region_hi_dev=0x1000) == chain
+    assert [route(8, n, hd=256, group=6) for n in (4028, 8192, 8193)] == [one, one, chain]
