@@ -83,25 +83,25 @@ __global__ __launch_bounds__(kThreads) void pq_adc_kernel(
 //
 // The distance that decides, |c|^2 / 2 - x.c, is a contraction over the few columns of a subspace,
 // so it runs on the matrix cores: keys are bf16 already, a centroid's fp32 value is the exact
-// sum of three bf16 values, and |c|^2 / 2 is three more with a factor of one, so the distances of 16
-// keys to 16 centroids are one v_mfma_f32_16x16x16_bf16 (16x16x32 from 8 columns on, two of them for
-// 16) of exact products with fp32 accumulation.  M = centroids and N = keys, so that a lane holds distances
-// of ONE key: lane (q, c) = (lane / 16, lane % 16) supplies part q of a centroid (the three terms,
-// then the bias) and the columns of key c (q < 3) or ones (q = 3).  Row 4 q + i of tile 2 p + h is
-// centroid 32 p + 8 q + 4 h + i: a lane's eight results of two tiles are eight neighbours, an "octet".
+// sum of three bf16 values, and |c|^2 / 2 is three more with a factor of one, so the distances of 32
+// keys to 32 centroids are one v_mfma_f32_32x32x16_bf16 (two at 8 columns, four at 16)
+// of exact products with fp32 accumulation.  M = centroids and N = keys, so that a lane holds distances
+// of ONE key: lane (h, c) = (lane / 32, lane % 32) supplies the first two parts of centroid c (h = 0), or the third and
+// the bias (from 8 columns on one part per instruction), and the columns of key c, or ones against the bias.  Row
+// 16 j + 8 u + 4 h + t of tile p is centroid 32 p + 16 j + 8 h + 4 u + t: a lane's sixteen results of a tile are two times
+// eight neighbours, two "octets".
 //
-// What bounds the kernel is the search for the minimum on the vector ALUs: 256 values per key and
-// subspace.  Six instructions per eight values keep the least value and the octet it came from (four
-// v_min3, a compare, a select).  At the end the four lanes of a key settle its octet, each lane
-// for the key of one of the wave's four groups (an exchange that halves twice), and that lane takes
-// the least of the eight in fp32.  200003 keys of 128 columns, 32
-// subspaces: 94-98 us, the vector ALUs issuing 88 % of the kernel's time and the matrix cores busy 46 %
-// (SQ counters); torch's distance matrices, written to and read from HBM four times over, took 11.8 ms.
-// With the tables in plain order (bank conflicts where an octet is settled) it took 115 us, with a search
-// of four values at a time 120 us.
+// What bounds the kernel is instruction issue on the vector ALUs, most of it the search for the minimum: 256 values per key
+// and subspace.  Six instructions per eight values keep the least value and the octet it came from (four
+// v_min3, a compare, a select).  At the end the two lanes of a key settle its octet, each lane
+// for the key of one of the wave's two groups (v_permlane32_swap exchanges the halves), and that lane takes
+// the least of the eight in fp32, from tables whose octets are padded apart so that lanes that look at the same place of
+// different octets read different banks at fixed offsets.  200003 keys of 128 columns, 32 subspaces: 75 us, the vector ALUs issuing 95 % of
+// the kernel's time (347 instructions per wave and subspace, 192 of them the search); with tiles of 16 x 16 x 16 (half the rate of
+// the wider ones, four lanes to settle a key through LDS shuffles; 488 instructions) 96, with 32 x 32 x 8 90; torch's
+// distance matrices, written to and read from HBM four times over, took 11.8 ms.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // The upper halves of the three words sum up to x: 8 + 8 + 8 bits of its mantissa.
 __device__ __forceinline__ void split3(float x, uint32_t &a, uint32_t &b, uint32_t &c) {
@@ -111,9 +111,10 @@ __device__ __forceinline__ void split3(float x, uint32_t &a, uint32_t &b, uint32
     c = __float_as_uint(r - __uint_as_float(b));
 }
 
-constexpr int kEncGroups = 4;                              // groups of 16 keys per wave: one per quarter of its lanes
-constexpr int kEncKeys = kThreads / 64 * 16 * kEncGroups;  // keys per block
+constexpr int kEncGroups = 2;                              // groups of 32 keys per wave: one per half of its lanes
+constexpr int kEncKeys = kThreads / 64 * 32 * kEncGroups;  // keys per block
 constexpr int kEncSubs = 4;                                // subspaces per block: their codes leave as one word
+constexpr int kEncHalf = 12;                               // words of an octet's half norms, padded
 
 // (At least two waves per SIMD asked for: with up to 256 registers the compiler leaves the results of the
 // matrix instructions in vector registers; with more it moves each through an accumulation register,
@@ -122,18 +123,18 @@ template <int DS>
 __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
     const uint16_t *__restrict__ keys, int64_t key_stride, int64_t n, const float *__restrict__ books,
     uint8_t *__restrict__ codes, int64_t code_stride, int m, int nc) {
-    constexpr int KL = DS <= 4 ? 4 : 8;         // operand elements per lane and instruction
-    constexpr int KW = KL / 2;                   // the same in words
-    constexpr int PARTS = DS <= 8 ? 1 : DS / 8;  // instructions per tile
+    constexpr int KW = 4;                        // operand words per lane and instruction
+    constexpr int NI = DS <= 4 ? 1 : 2;          // instructions per tile and eight columns (four, where there are no more)
+    constexpr int KL = DS <= 4 ? 4 : 8;          // columns of a part of the centroid per lane and instruction
+    constexpr int PARTS = DS <= 8 ? 1 : DS / 8;  // eights of columns
     constexpr int XW = (DS + 1) / 2;             // words of a key's columns
-    // [tile][q][row][word]: a wave's operand is one stretch
-    __shared__ __align__(16) uint32_t s_a[PARTS][256 * 4 * KW];
-    // Centroid i of an octet sits at place i ^ (octet & 7) of it, its half norm at i ^ 2 (octet / 8): lanes that
-    // look at the same i of different octets read different banks.
-    __shared__ __align__(16) float s_c[256 * DS];
-    __shared__ __align__(16) float s_half[256];
+    constexpr int kOctet = 8 * DS + (DS < 4 ? DS : 4);  // words of an octet's centroids, padded
+    // [tile][instruction][lane][word]: a wave's operand is one stretch
+    __shared__ __align__(16) uint32_t s_a[PARTS][8 * NI * 64 * KW];
+    __shared__ __align__(16) float s_c[32 * kOctet];
+    __shared__ __align__(16) float s_half[32 * kEncHalf];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int q = lane >> 4, c = lane & 15;
+    const int h = lane >> 5, c = lane & 31;
     // The blocks that read the same keys (a few columns each, of lines they share) are numbered 8 apart:
     // they run on one XCD at about the same time and find the lines in its L2.
     const int n_y = (m + kEncSubs - 1) / kEncSubs;
@@ -141,12 +142,12 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
     const int64_t kblk = (int64_t)(turn / n_y) * 8 + xcd;
     const int sub0 = (turn % n_y) * kEncSubs;
     const int n_sub = m - sub0 < kEncSubs ? m - sub0 : kEncSubs;
-    const int64_t key0 = kblk * kEncKeys + wave * (16 * kEncGroups);
+    const int64_t key0 = kblk * kEncKeys + wave * (32 * kEncGroups);
     if (kblk * kEncKeys >= n) return;  // the grid is a whole number of eights
     const uint16_t *kp[kEncGroups];
 #pragma unroll
     for (int g = 0; g < kEncGroups; ++g) {
-        int64_t k = key0 + g * 16 + c;
+        int64_t k = key0 + g * 32 + c;
         k = k < n ? k : n - 1;
         kp[g] = keys + k * key_stride;
     }
@@ -180,8 +181,7 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
         }
     };
     // where this thread's centroid sits among the tiles' rows
-    const int tile = 2 * (tid >> 5) + ((tid >> 2) & 1), row = 4 * ((tid >> 3) & 3) + (tid & 3);
-    const int c_slot = (tid & ~7) | ((tid ^ (tid >> 3)) & 7), half_slot = (tid & ~7) | ((tid ^ (2 * (tid >> 6))) & 7);
+    const int row = 16 * ((tid >> 4) & 1) + 8 * ((tid >> 2) & 1) + 4 * ((tid >> 3) & 1) + (tid & 3);
     uint32_t word = 0u;  // the codes of key key0 + lane
     load_centroid(sub0);
     load_keys(sub0, xw);
@@ -192,12 +192,12 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
         for (int d = 0; d < DS; ++d) half = fmaf(cen[d], cen[d], half);
         half = tid < nc ? 0.5f * half : INFINITY;  // a centroid that does not exist is never the nearest, of no key
         if (s > 0) __syncthreads();               // the last subspace's tables are no longer read
-        s_half[half_slot] = half;
+        s_half[(tid >> 3) * kEncHalf + (tid & 7)] = half;
 #pragma unroll
-        for (int d = 0; d < DS; ++d) s_c[c_slot * DS + d] = cen[d];
+        for (int d = 0; d < DS; ++d) s_c[(tid >> 3) * kOctet + (tid & 7) * DS + d] = cen[d];
 #pragma unroll
         for (int p = 0; p < PARTS; ++p) {
-            uint32_t e[4][KL];  // bf16 values in the upper halves
+            uint32_t e[4][KL];  // bf16 values in the upper halves: the three parts, the bias
 #pragma unroll
             for (int j = 0; j < KL; ++j) {
                 e[0][j] = e[1][j] = e[2][j] = e[3][j] = 0u;
@@ -205,146 +205,135 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
             }
             if (p == 0) split3(half, e[3][0], e[3][1], e[3][2]);
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+            for (int r = 0; r < 4; ++r)  // two instructions: r in lane 32 (r % 2) of number r / 2; one: parts 2 l and 2 l + 1 in half l
 #pragma unroll
-                for (int w = 0; w < KW; ++w)
-                    s_a[p][((tile * 4 + r) * 16 + row) * KW + w] = __builtin_amdgcn_perm(e[r][2 * w + 1], e[r][2 * w], 0x07060302u);
+                for (int w = 0; w < KL / 2; ++w) {
+                    const int at = NI == 2 ? ((tid >> 5) * 128 + r * 32 + row) * KW + w : ((tid >> 5) * 64 + (r / 2) * 32 + row) * KW + 2 * (r % 2) + w;
+                    s_a[p][at] = __builtin_amdgcn_perm(e[r][2 * w + 1], e[r][2 * w], 0x07060302u);
+                }
         }
         __syncthreads();
-        // the keys' operands: the columns for the lanes of the centroid's parts, ones for the bias
-        uint32_t b[kEncGroups][PARTS][KW];
+        // the keys' operands: the columns, and ones against the bias
+        uint32_t b[kEncGroups][PARTS][NI][KW];
 #pragma unroll
         for (int g = 0; g < kEncGroups; ++g)
 #pragma unroll
             for (int p = 0; p < PARTS; ++p)
 #pragma unroll
                 for (int w = 0; w < KW; ++w) {
-                    const int xi = p * KW + w;
+                    const int xi = NI == 2 ? p * KW + w : w % 2, wb = NI == 2 ? w : w - 2;
                     const uint32_t x = xi < XW ? xw[g][xi < XW ? xi : 0] : 0u;
-                    const uint32_t one = p != 0 ? 0u : (w == 0 ? 0x3f803f80u : (w == 1 ? 0x00003f80u : 0u));
-                    b[g][p][w] = q < 3 ? x : one;
+                    const uint32_t one = p != 0 ? 0u : (wb == 0 ? 0x3f803f80u : (wb == 1 ? 0x00003f80u : 0u));
+                    b[g][p][0][w] = x;
+                    if (NI == 2 || w >= 2) b[g][p][NI - 1][w] = h == 0 ? x : one;
                 }
         if (s + 1 < n_sub) {  // the next subspace's centroids and columns are on the way meanwhile
             load_centroid(sub0 + s + 1);
             load_keys(sub0 + s + 1, xn);
         }
         float best[kEncGroups];
-        uint32_t pair[kEncGroups];
+        uint32_t from[kEncGroups];  // 2 * tile + which of its octets
 #pragma unroll
         for (int g = 0; g < kEncGroups; ++g) {
             best[g] = INFINITY;
-            pair[g] = 0u;
+            from[g] = 0u;
         }
-        uint32_t aw[2][PARTS][KW], an[2][PARTS][KW];
-        auto load_pair = [&](int t2, uint32_t(&dst)[2][PARTS][KW]) __attribute__((always_inline)) {
+        uint32_t aw[PARTS][NI][KW], an[PARTS][NI][KW];
+        auto load_tile = [&](int t, uint32_t(&dst)[PARTS][NI][KW]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int p = 0; p < PARTS; ++p)
 #pragma unroll
-                for (int p = 0; p < PARTS; ++p) {
-                    const uint32_t *src = &s_a[p][(((2 * t2 + h) * 4 + q) * 16 + c) * KW];
-                    if constexpr (KW == 2) {
-                        const uint2 v = *reinterpret_cast<const uint2 *>(src);
-                        dst[h][p][0] = v.x, dst[h][p][1] = v.y;
-                    } else {
-                        const uint4 v = *reinterpret_cast<const uint4 *>(src);
-                        dst[h][p][0] = v.x, dst[h][p][1] = v.y, dst[h][p][2] = v.z, dst[h][p][3] = v.w;
-                    }
+                for (int i = 0; i < NI; ++i) {
+                    const uint4 v = *reinterpret_cast<const uint4 *>(&s_a[p][((NI * t + i) * 64 + lane) * KW]);
+                    dst[p][i][0] = v.x, dst[p][i][1] = v.y, dst[p][i][2] = v.z, dst[p][i][3] = v.w;
                 }
         };
-        load_pair(0, an);
-#pragma unroll 2
-        for (int t2 = 0; t2 < 8; ++t2) {
+        load_tile(0, an);
+#pragma unroll  // (whole: the octets' numbers are constants of their instructions then, and so are the tiles' addresses)
+        for (int t = 0; t < 8; ++t) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int p = 0; p < PARTS; ++p)
 #pragma unroll
-                for (int p = 0; p < PARTS; ++p)
+                for (int i = 0; i < NI; ++i)
 #pragma unroll
-                    for (int w = 0; w < KW; ++w) aw[h][p][w] = an[h][p][w];
-            load_pair((t2 + 1) & 7, an);  // the next pair of tiles is on the way
-            // all products first, then each step of the search for all groups: a result is a dozen
+                    for (int w = 0; w < KW; ++w) aw[p][i][w] = an[p][i][w];
+            if (t < 7) load_tile(t + 1, an);  // the next tile is on the way
+            // all products first, then each step of the search for all groups: a result is some dozen
             // cycles away from its instruction, a compare's mask two from its reader
-            f32x4 d[kEncGroups][2];
+            f32x16 d[kEncGroups];
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int g = 0; g < kEncGroups; ++g)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) d[g][i] = 0.f;
+#pragma unroll
+            for (int p = 0; p < PARTS; ++p)
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+#pragma unroll
+                    for (int g = 0; g < kEncGroups; ++g) {
+                        const uint4 av = make_uint4(aw[p][i][0], aw[p][i][1], aw[p][i][2], aw[p][i][3]);
+                        const uint4 bv = make_uint4(b[g][p][i][0], b[g][p][i][1], b[g][p][i][2], b[g][p][i][3]);
+                        d[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
+                                                                       __builtin_bit_cast(bf16x8, bv), d[g], 0, 0, 0);
+                    }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int o = 0; o < 2; ++o) {
+                float v[kEncGroups];
+                bool less[kEncGroups];
+#pragma unroll
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(d[g][8 * o], d[g][8 * o + 1]), d[g][8 * o + 2]);
+#pragma unroll
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][8 * o + 3]), d[g][8 * o + 4]);
+#pragma unroll
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][8 * o + 5]), d[g][8 * o + 6]);
+#pragma unroll
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][8 * o + 7]), best[g]);
+#pragma unroll
+                for (int g = 0; g < kEncGroups; ++g) less[g] = v[g] < best[g];
 #pragma unroll
                 for (int g = 0; g < kEncGroups; ++g) {
-                    d[g][h] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int p = 0; p < PARTS; ++p) {
-                        if constexpr (KW == 2) {
-                            const uint2 av = make_uint2(aw[h][p][0], aw[h][p][1]), bv = make_uint2(b[g][p][0], b[g][p][1]);
-                            d[g][h] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, av),
-                                                                                __builtin_bit_cast(s16x4, bv), d[g][h], 0, 0, 0);
-                        } else {
-                            const uint4 av = make_uint4(aw[h][p][0], aw[h][p][1], aw[h][p][2], aw[h][p][3]);
-                            const uint4 bv = make_uint4(b[g][p][0], b[g][p][1], b[g][p][2], b[g][p][3]);
-                            d[g][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av),
-                                                                              __builtin_bit_cast(bf16x8, bv), d[g][h], 0, 0, 0);
-                        }
-                    }
+                    from[g] = less[g] ? (uint32_t)(2 * t + o) : from[g];
+                    best[g] = v[g];
                 }
-            __builtin_amdgcn_sched_barrier(0);
-            float v[kEncGroups];
-            bool less[kEncGroups];
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(d[g][0][0], d[g][0][1]), d[g][0][2]);
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][0][3]), d[g][1][0]);
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][1][1]), d[g][1][2]);
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][1][3]), best[g]);
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g) less[g] = v[g] < best[g];
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g) {
-                pair[g] = less[g] ? (uint32_t)t2 : pair[g];
-                best[g] = v[g];
             }
             __builtin_amdgcn_sched_barrier(0);
         }
-        // The four lanes of a key hold its least value over their octets each.  Lanes q and q ^ 2 exchange
-        // two groups, then q and q ^ 1 one of the two that are left: lane q ends with group q.
-        // (Equal values: the lower octet.)
-        auto lesser = [](float &v, uint32_t &o, float v2, uint32_t o2) __attribute__((always_inline)) {
-            const bool take = v2 < v || (v2 == v && o2 < o);
-            v = take ? v2 : v;
-            o = take ? o2 : o;
-        };
-        const bool up2 = (q & 2) != 0, up1 = (q & 1) != 0;
-        float v2[2];
-        uint32_t o2[2];
+        // The two lanes of a key hold its least value over their octets each.  The halves of the wave exchange a
+        // group: half h ends with both lanes' values for group h.  (Equal values: the lower octet.)
+        uint32_t oct[kEncGroups];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            v2[i] = up2 ? best[2 + i] : best[i];
-            o2[i] = (up2 ? pair[2 + i] : pair[i]) * 4u + (uint32_t)q;
-            const float vs = up2 ? best[i] : best[2 + i];
-            const uint32_t os = (up2 ? pair[i] : pair[2 + i]) * 4u + (uint32_t)q;
-            lesser(v2[i], o2[i], __shfl_xor(vs, 32, 64), (uint32_t)__shfl_xor((int)os, 32, 64));
-        }
-        float v1 = up1 ? v2[1] : v2[0];
-        uint32_t octet = up1 ? o2[1] : o2[0];
-        lesser(v1, octet, __shfl_xor(up1 ? v2[0] : v2[1], 16, 64), (uint32_t)__shfl_xor((int)(up1 ? o2[0] : o2[1]), 16, 64));
+        for (int g = 0; g < kEncGroups; ++g) oct[g] = 2u * from[g] + (uint32_t)h;
+        const auto bv = __builtin_amdgcn_permlane32_swap(__float_as_uint(best[0]), __float_as_uint(best[1]), false, false);
+        const auto ov = __builtin_amdgcn_permlane32_swap(oct[0], oct[1], false, false);
+        const float v0 = __uint_as_float(bv[0]), v1 = __uint_as_float(bv[1]);
+        const bool second = v1 < v0 || (v1 == v0 && ov[1] < ov[0]);
+        const uint32_t octet = second ? ov[1] : ov[0];
         // the least of the octet, in fp32, for key key0 + lane
-        uint32_t x[XW];
+        float xf[2 * XW];
 #pragma unroll
         for (int w = 0; w < XW; ++w) {
-            const uint32_t x0 = up1 ? xw[1][w] : xw[0][w], x1 = up1 ? xw[3][w] : xw[2][w];
-            x[w] = up2 ? x1 : x0;
+            const uint32_t x = h ? xw[1][w] : xw[0][w];
+            xf[2 * w] = dc_bf16_lo(x);
+            xf[2 * w + 1] = dc_bf16_hi(x);
         }
-        float least = 0.f;
-        uint32_t id = 0u;
+        const float4 *hp = reinterpret_cast<const float4 *>(s_half + octet * kEncHalf);
+        const float4 h0 = hp[0], h1 = hp[1];
+        const float hs[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+        const float *cp = s_c + octet * kOctet;
+        float dist[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            float dist = s_half[octet * 8u + ((uint32_t)i ^ (2u * (octet >> 3)))];
-            const float *cp = s_c + (octet * 8u + ((uint32_t)i ^ (octet & 7u))) * DS;
+            dist[i] = hs[i];
 #pragma unroll
-            for (int w = 0; w < XW; ++w) {
-                dist = fmaf(-dc_bf16_lo(x[w]), cp[2 * w], dist);
-                dist = fmaf(-dc_bf16_hi(x[w]), cp[2 * w + 1], dist);
-            }
-            const bool take = i == 0 || dist < least;
-            least = take ? dist : least;
+            for (int k = 0; k < DS; ++k) dist[i] = fmaf(-xf[k], cp[i * DS + k], dist[i]);
+        }
+        float least = dist[0];
+        uint32_t id = 0u;
+#pragma unroll
+        for (int i = 1; i < 8; ++i) {
+            const bool take = dist[i] < least;
+            least = take ? dist[i] : least;
             id = take ? (uint32_t)i : id;
         }
         word |= (octet * 8u + id) << (8 * s);
