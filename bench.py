@@ -460,7 +460,7 @@ def measure_pq(torch, hip, dev, steps: int, warmup: int, stepwise: bool = False,
         "call_path": "dc_pq_build_lut + " + ("the stepwise entry points" if stepwise else "dc_pq_search_bf16"),
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBPS, "traffic": None,
-                     "kernel": "pq_adc_kernel<32>" if stepwise else "pq_prune_kernel<32>",
+                     "kernel": "pq_adc_kernel<32>" if stepwise else "pq_scan_kernel<32>",
                      "algorithmic_bytes_per_launch": scan_bytes, "avg_launch_us": scan_ms * 1e3,
                      "timed_launches": len(ev)},
         "step_8d_bytes": algo, "step_8d_frac": algo / (ms * 1e-3) / 1e9 / HBM_PEAK_GBPS,

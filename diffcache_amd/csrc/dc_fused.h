@@ -12,8 +12,7 @@ constexpr int kSmallChunks = 16;   // leading 256-row blocks per unit
 constexpr int kStage = kBigSteps * kRowsPerBlockStep;
 constexpr int kCandLds = 16384;    // candidates the finish kernel keeps in LDS (128 KB of the CU's 160)
 constexpr int kSharedPollUnits = 8;   // sketch scan: up to this many units, one wave per block polls
-constexpr int kPqThreads = 512;    // PQ scan: threads per block = keys per step
-constexpr int kPqBigSteps = 8;     // PQ scan: 4096 keys per large block
+constexpr int kPqThreads = 1024;   // PQ scan: threads per block = keys per step
 constexpr int kBinsPerThread = DC_HIST_BINS / kThreads;  // bins a thread owns when a block scans a histogram
 static_assert(kBinsPerThread % 4 == 0 && kBinsPerThread * kThreads == DC_HIST_BINS, "bin split");
 

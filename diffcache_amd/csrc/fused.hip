@@ -28,6 +28,7 @@
 // sketch.hip) with a margin that makes its pruning safe, rescore_kernel computes
 // the exact scores of the rows that survive it and lists them as candidates, and
 // select_finish_kernel picks the k best of that list.
+#include <stddef.h>
 #include <type_traits>
 #include "dc_common.h"
 #include "dc_select.h"
@@ -68,7 +69,7 @@ __device__ __forceinline__ void lds_store_relaxed(uint32_t *p, uint32_t v) {
 // the unit's list with one returning atomic, flush the block's histogram, and in
 // the blocks chosen by the caller refresh the unit's running threshold from
 // whatever part of the histogram is visible.  Staleness only loosens the bound.
-template <int kT = kThreads, typename E = uint2>
+template <typename E = uint2>
 __device__ __forceinline__ void prune_block_finish(uint32_t *lhist, const E *wstage, uint32_t wcnt,
                                                    uint32_t *s_wcnt, uint32_t *s_base, uint32_t *wtot,
                                                    UnitState *st, uint32_t *hu, E *surv_unit,
@@ -81,12 +82,12 @@ __device__ __forceinline__ void prune_block_finish(uint32_t *lhist, const E *wst
     // the atomic is in flight while the histogram is flushed
     uint32_t wbase = 0, cnt = 0;
 #pragma unroll
-    for (int w2 = 0; w2 < kT / 64; ++w2) {
+    for (int w2 = 0; w2 < kThreads / 64; ++w2) {
         if (w2 < wave) wbase += s_wcnt[w2];
         cnt += s_wcnt[w2];
     }
     if (tid == 0) *s_base = cnt ? atomicAdd(&st->surv_cnt, cnt) : 0;
-    for (int i = tid; i < DC_HIST_BINS; i += kT) {
+    for (int i = tid; i < DC_HIST_BINS; i += kThreads) {
         const uint32_t c = lhist[i];
         if (c) atomicAdd(&hu[i], c);
     }
@@ -102,12 +103,12 @@ __device__ __forceinline__ void prune_block_finish(uint32_t *lhist, const E *wst
     {
         const unsigned long long *h64 = reinterpret_cast<const unsigned long long *>(hu);
         unsigned long long *l64 = reinterpret_cast<unsigned long long *>(lhist);
-        for (int i = tid; i < DC_HIST_BINS / 2; i += kT)
+        for (int i = tid; i < DC_HIST_BINS / 2; i += kThreads)
             l64[i] = __hip_atomic_load(h64 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    constexpr int kBins = DC_HIST_BINS / kT;  // adjacent bins a thread owns
-    static_assert(kBins * kT == DC_HIST_BINS, "bin split");
+    constexpr int kBins = DC_HIST_BINS / kThreads;  // adjacent bins a thread owns
+    static_assert(kBins * kThreads == DC_HIST_BINS, "bin split");
     uint32_t bins[kBins];
     uint32_t sum = 0;
 #pragma unroll
@@ -116,7 +117,7 @@ __device__ __forceinline__ void prune_block_finish(uint32_t *lhist, const E *wst
         sum += bins[i];
     }
     uint32_t total;
-    const uint32_t excl = block_excl_scan<kT>(sum, wtot, &total);
+    const uint32_t excl = block_excl_scan<kThreads>(sum, wtot, &total);
     if (excl < kk && kk <= excl + sum) {
         uint32_t run = excl;
         bool done = false;
@@ -545,54 +546,43 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
         work_step(step, ca, std::false_type{});  // an odd last step; its rows are already on the way
     }
     const bool refresh = small ? (chunk & 3) == 3 : ((chunk - small_chunks) & 7) == 7;
-    prune_block_finish<kThreads, uint32_t>(lhist, wstage, wcnt, s_wcnt, &s_base, wtot, st,
+    prune_block_finish<uint32_t>(lhist, wstage, wcnt, s_wcnt, &s_base, wtot, st,
                                            hist + (int64_t)unit * DC_HIST_BINS,
                                            reinterpret_cast<uint32_t *>(surv) + (int64_t)unit * n_cap, refresh,
                                            (uint32_t)k_eff);
 }
 
-// The same scan for the PQ baseline: a key's score is its ADC score (dc_pq.h), read
-// from M code bytes per key, in DC_MODE_IP order.  One key per lane.  The unit's
-// tables are staged per block, so blocks are large: 512 threads, 512 keys per step.
-template <int M>
-__global__ __launch_bounds__(kPqThreads) void pq_prune_kernel(
-    const uint8_t *__restrict__ codes, const float *__restrict__ lut, uint32_t *__restrict__ hist,
-    UnitState *__restrict__ state, uint2 *__restrict__ surv, int n_units, int n_rows, int k_eff,
-    int small_chunks, int big_steps) {
-    constexpr int NW = M / 4;
-    constexpr int kWaves = kPqThreads / 64;
-    __shared__ float s_lut[kPqLutWords];
-    __shared__ uint32_t lhist[DC_HIST_BINS];
-    __shared__ uint2 stage[kWaves * kPqBigSteps * 64];
-    __shared__ uint32_t s_tb;  // the block's copy of the unit's running threshold bucket
-    __shared__ uint32_t wtot[kWaves + 1];
-    __shared__ uint32_t s_wcnt[kWaves];
-    __shared__ uint32_t s_base;
+// The scan of the PQ baseline: a key's score is its ADC score (dc_pq.h), read from M code bytes per key, in DC_MODE_IP
+// order.  One key per lane.  A block stages its unit's tables once and scans an equal share of the unit's keys; like the
+// dense sketch scan it leaves every key's bucket at the key's own place, and the histogram.  Nothing is polled, listed
+// or handed over before the block's end.
+//
+// Bound by instruction issue and HBM together (some 130 vector instructions per 64 keys, 32 of them the additions, 32 the
+// addresses of the tables; 268 MB of codes in 46 us = 5.8 TB/s).  8 x 1048576 codes of 32 bytes: 46 us.  Listed, in blocks of
+// 4096 keys, half of a block's life went into staging the tables and closing (76 us; 70 with the wide tables, sixteen
+// waves per block).  One block of 1024 threads per CU: two 46.2, four 51; three steps of codes ahead 48.9, one 47.6;
+// blocks of 512 threads 46.1, two of them 51.5.
+constexpr int kPqBlocks = 256;
 
+template <int M>
+__global__ __launch_bounds__(kPqThreads, 4) void pq_scan_kernel(
+    const uint8_t *__restrict__ codes, const float *__restrict__ lut, uint32_t *__restrict__ hist,
+    uint2 *__restrict__ surv, int n_units, int n_rows, int steps) {
+    constexpr int NW = M / 4;
+    __shared__ float s_lut[kPqWideWords];
+    __shared__ uint32_t lhist[DC_HIST_BINS];
     const int unit = blockIdx.x % n_units;
     const int chunk = blockIdx.x / n_units;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    const bool small = chunk < small_chunks;
-    const int big_chunks = (int)(gridDim.x / n_units) - small_chunks;
-    const int big_id = small ? 0 : (int)(((int64_t)(chunk - small_chunks) + (int64_t)unit * 7) % big_chunks);
-    const int64_t block_row0 =
-        small ? (int64_t)chunk * kPqThreads
-              : (int64_t)small_chunks * kPqThreads + (int64_t)big_id * big_steps * kPqThreads;
-    const int steps = small ? 1 : big_steps;
-
-    for (int i = tid; i < DC_HIST_BINS; i += kPqThreads) lhist[i] = 0;
-    pq_stage_lut<M>(s_lut, lut + (int64_t)unit * M * 256, tid, kPqThreads);
-    PqLane<M> ln;
-    ln.init(lane);
-    UnitState *st = state + unit;
-    const int64_t last = n_rows - 1;
-    uint32_t tb = load_relaxed(&st->tb_run);
-    const uint8_t *cu = codes + (int64_t)unit * n_rows * M;
-    // rows are a multiple of 64 from the start of the unit: lane = key mod 64, as pq_adc_score expects
+    const int64_t block_row0 = (int64_t)chunk * steps * kPqThreads;
     const int64_t blk_end = block_row0 + (int64_t)steps * kPqThreads - 1;
-    const int64_t blk_last = blk_end < last ? blk_end : last;
-    auto load_row = [&](int64_t row0, uint32_t(&w)[NW]) {
+    const int64_t blk_last = blk_end < (int64_t)n_rows - 1 ? blk_end : (int64_t)n_rows - 1;
+    if (block_row0 >= n_rows) return;
+    const uint8_t *cu = codes + (int64_t)unit * n_rows * M;
+    uint16_t *du = reinterpret_cast<uint16_t *>(surv) + (int64_t)unit * dense_stride(n_rows);
+    // rows are a multiple of 64 from the start of the unit: lane = key mod 64, as pq_adc_score expects
+    auto load_row = [&](int64_t row0, uint32_t(&w)[NW]) __attribute__((always_inline)) {
         int64_t r = row0 + lane;
         r = r > blk_last ? blk_last : r;
         // plain loads: the two halves of a 32-byte row come from the same cache line
@@ -606,61 +596,146 @@ __global__ __launch_bounds__(kPqThreads) void pq_prune_kernel(
             w[4 * i + 3] = t.w;
         }
     };
-    // A wave keeps the codes of kAhead steps in flight beyond the one it scores: 32 bytes
-    // per lane and step are too few to cover the memory latency otherwise.  Loads return
-    // in order, so the threshold polled before the rows of step s + kAhead is first looked
-    // at when those rows are, and never makes the wave wait for younger loads.  The
-    // requests are issued unconditionally (past the block's end they repeat its last
-    // row) so that the number of loads in flight is the same on every path.
-    constexpr int kAhead = 3, kRing = kAhead + 1;
+    // The codes of kAhead steps are in flight beyond the one that is scored; requests past the
+    // block's end repeat its last row, so that their number is the same on every path.
+    constexpr int kAhead = 2, kRing = kAhead + 1;
     uint32_t buf[kRing][NW];
     const int64_t wave_row0 = block_row0 + wave * 64;
-    const int64_t rows_left = (int64_t)n_rows - wave_row0;
-    const int64_t steps_left = (rows_left + kPqThreads - 1) / kPqThreads;
-    const int my_steps = rows_left <= 0 ? 0 : (int)(steps_left < steps ? steps_left : steps);
-    uint32_t tb_polled = tb;
-    if (tid == 0) s_tb = tb;
+    const int64_t rows_left = blk_last + 1 - wave_row0;
+    const int my_steps = rows_left <= 0 ? 0 : (int)((rows_left + kPqThreads - 1) / kPqThreads);
 #pragma unroll
     for (int j = 0; j < kAhead; ++j) load_row(wave_row0 + (int64_t)j * kPqThreads, buf[j]);
+    for (int i = tid; i < DC_HIST_BINS; i += kPqThreads) lhist[i] = 0;
+    pq_stage_lut_wide<M>(s_lut, lut + (int64_t)unit * M * 256, tid, kPqThreads);
+    PqWideLane<M> ln;
+    ln.init(lane);
     __syncthreads();
-
-    // each wave stages its survivors in its own slice (at most 64 per step)
-    uint2 *wstage = stage + wave * (kPqBigSteps * 64);
-    uint32_t wcnt = 0;
-    const unsigned long long lt = (1ull << lane) - 1ull;
-
     for (int s0 = 0; s0 < my_steps; s0 += kRing) {
 #pragma unroll
         for (int j = 0; j < kRing; ++j) {
             const int step = s0 + j;
             const int64_t row0 = wave_row0 + (int64_t)step * kPqThreads;
-            // The poll crosses the chip (agent scope) and every younger load of the wave
-            // queues behind it, so only wave 0 polls, once per kRing steps, and hands the
-            // value to the other waves through LDS when it has arrived.
-            if (wave == 0 && j == 0) tb_polled = load_relaxed(&st->tb_run);
             load_row(row0 + (int64_t)kAhead * kPqThreads, buf[(j + kAhead) % kRing]);
-            if (wave == 0 && j == kAhead && lane == 0) lds_store_relaxed(&s_tb, tb_polled);
-            if (step < my_steps) {  // wave-uniform; no barrier inside the loop
-                const float mine = pq_adc_score<M>(buf[j], s_lut, ln);
-                tb = lds_load_relaxed(&s_tb);
-                const int64_t myrow = row0 + lane;
-                const bool valid = myrow < n_rows;
-                uint32_t key = 0, bucket = 0xffffffffu;
-                if (valid) dc_key_bucket(mine, DC_MODE_IP, key, bucket);
-                const bool keep = valid && bucket <= tb;
-                if (keep) atomicAdd(&lhist[bucket], 1u);
-                const unsigned long long mask = __ballot(keep);
-                if (keep)
-                    wstage[wcnt + __popcll(mask & lt)] = make_uint2((uint32_t)myrow, __float_as_uint(mine));
-                wcnt += (uint32_t)__popcll(mask);
+            if (step < my_steps) {  // wave-uniform
+                const float mine = pq_adc_score_wide<M>(buf[j], s_lut, ln);
+                uint32_t key, bucket;
+                dc_key_bucket(mine, DC_MODE_IP, key, bucket);
+                if (row0 + lane <= blk_last) {
+                    du[row0 + lane] = (uint16_t)bucket;
+                    atomicAdd(&lhist[bucket], 1u);
+                }
             }
         }
     }
-    // every 4th small block and every 2nd large one refresh the running threshold
-    const bool refresh = small ? (chunk & 3) == 3 : ((chunk - small_chunks) & 1) == 1;
-    prune_block_finish<kPqThreads>(lhist, wstage, wcnt, s_wcnt, &s_base, wtot, st,
-                                   hist + (int64_t)unit * DC_HIST_BINS, surv + (int64_t)unit * n_rows,
-                                   refresh, (uint32_t)k_eff);
+    __syncthreads();
+    uint32_t *hu = hist + (int64_t)unit * DC_HIST_BINS;
+    for (int i = tid; i < DC_HIST_BINS; i += kPqThreads) {
+        const uint32_t c = lhist[i];
+        if (c) atomicAdd(&hu[i], c);
+    }
+}
+
+// classify_kernel for the buckets that pq_scan_kernel left: keys in buckets better than the threshold bucket are certain
+// members, keys in it become candidates, whose scores are worked out once more (the additions of pq_adc_score).  A block
+// takes kPqClassRows keys and reserves its places in both lists with one returning atomic.
+constexpr int kPqClassRows = 8192;
+static_assert(offsetof(UnitState, win_cnt) == offsetof(UnitState, surv_cnt) + 4 && offsetof(UnitState, surv_cnt) % 8 == 0, "one word");
+
+template <int M>
+__global__ __launch_bounds__(kThreads) void pq_classify_kernel(
+    const uint8_t *__restrict__ codes, const float *__restrict__ lut, const uint32_t *__restrict__ hist,
+    UnitState *__restrict__ state, const uint2 *__restrict__ surv, uint32_t *__restrict__ cand_key,
+    uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride, int n_units, int n_rows, int k_eff) {
+    constexpr int kVec = kPqClassRows / kThreads / 8;  // vectors of eight buckets per thread
+    constexpr int NW = M / 4;
+    __shared__ uint16_t s_sure[kPqClassRows], s_cand[kPqClassRows];
+    __shared__ uint32_t wtot[kThreads / 64 + 1];
+    __shared__ uint32_t sres[2];
+    __shared__ uint32_t sbase[2];
+    const int unit = blockIdx.x % n_units, blk = blockIdx.x / n_units;
+    const int tid = threadIdx.x;
+    const int row0 = blk * kPqClassRows;
+    UnitState *st = state + unit;
+    const uint16_t *du = reinterpret_cast<const uint16_t *>(surv) + (int64_t)unit * dense_stride(n_rows);
+    uint4 v[kVec];
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) {
+        const int64_t r = (int64_t)row0 + (i * kThreads + tid) * 8;
+        v[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        if (r < n_rows) v[i] = *reinterpret_cast<const uint4 *>(du + r);
+    }
+    const uint32_t kk = (uint32_t)k_eff;
+    uint32_t tb, c_less;
+    unit_threshold(hist + (int64_t)unit * DC_HIST_BINS, kk, wtot, sres, tb, c_less);
+    if (blk == 0 && tid == 0) {
+        st->c_less = c_less;
+        st->cand_cnt = tb < (uint32_t)DC_HIST_BINS ? hist[(int64_t)unit * DC_HIST_BINS + tb] : 0u;  // every key is counted
+    }
+    uint32_t sure = 0, cand = 0;  // a bit per key
+    static_assert(kVec * 8 <= 32, "bits of a thread's keys");
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) {
+        const uint32_t w4[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t bucket = j & 1 ? w4[j / 2] >> 16 : w4[j / 2] & 0xffffu;
+            const bool live = row0 + (i * kThreads + tid) * 8 + j < n_rows;
+            sure |= live && bucket < tb ? 1u << (8 * i + j) : 0u;
+            cand |= live && bucket == tb ? 1u << (8 * i + j) : 0u;
+        }
+    }
+    uint32_t tot;
+    const uint32_t ex = block_excl_scan<kThreads>(__popc(sure) | __popc(cand) << 16, wtot, &tot);
+    const uint32_t n_sure = tot & 0xffffu, n_cand = tot >> 16;
+    // (both lists with one addition: their cursors are the halves of one word, additions to which are served one after
+    // the other, 128 of them per unit at a million keys)
+    if (tid == 0) {
+        unsigned long long at = 0ull;
+        if (tot) at = atomicAdd(reinterpret_cast<unsigned long long *>(&st->surv_cnt), (unsigned long long)n_sure << 32 | n_cand);
+        sbase[0] = (uint32_t)(at >> 32);
+        sbase[1] = (uint32_t)at;
+    }
+    auto list = [&](uint32_t bits, uint32_t at, uint16_t *dst) __attribute__((always_inline)) {
+        while (bits) {
+            const int b = __ffs(bits) - 1;
+            bits &= bits - 1u;
+            dst[at++] = (uint16_t)(((b >> 3) * kThreads + tid) * 8 + (b & 7));
+        }
+    };
+    list(sure, ex & 0xffffu, s_sure);
+    list(cand, ex >> 16, s_cand);
+    __syncthreads();
+    uint32_t *io = idx_out + (int64_t)unit * idx_stride;
+    for (uint32_t i = tid; i < n_sure; i += kThreads) {
+        const uint32_t at = sbase[0] + i;
+        if (at < kk) io[at] = (uint32_t)row0 + s_sure[i];
+    }
+    const uint8_t *cu = codes + (int64_t)unit * n_rows * M;
+    const float *lu = lut + (int64_t)unit * M * 256;
+    for (uint32_t i = tid; i < n_cand; i += kThreads) {
+        const uint32_t row = (uint32_t)row0 + s_cand[i], at = sbase[1] + i;
+        const uint4 *cp = reinterpret_cast<const uint4 *>(cu + (int64_t)row * M);
+        uint32_t w[NW], rw[NW];
+#pragma unroll
+        for (int x = 0; x < NW / 4; ++x) {
+            const uint4 t = cp[x];
+            w[4 * x] = t.x, w[4 * x + 1] = t.y, w[4 * x + 2] = t.z, w[4 * x + 3] = t.w;
+        }
+        PqWideLane<M> ln;
+        ln.init((int)(row & 63u));
+        pq_rotate<M>(w, ln.rot, ln.sh, rw);
+        float e[M], acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < M; ++j) e[j] = lu[((row + j) % M) * 256 + ((rw[j / 4] >> (8 * (j % 4))) & 0xffu)];
+#pragma unroll
+        for (int j = 0; j < M; ++j) acc += e[j];
+        uint32_t key, bucket;
+        dc_key_bucket(acc, DC_MODE_IP, key, bucket);
+        if (at < (uint32_t)n_rows) {
+            cand_key[(int64_t)unit * n_rows + at] = key;
+            cand_idx[(int64_t)unit * n_rows + at] = row;
+        }
+    }
 }
 
 // Several blocks per unit split the unit's survivor list: rows in buckets better
@@ -1147,7 +1222,7 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
     // chunks per unit: up to kSmallChunks blocks of one step, then blocks of big_steps steps.
     // Short scans take fewer steps per block so that the grid still has fill_div blocks or
     // more: a block's steps run one after the other, and with few blocks the kernel
-    // lasts as long as its longest block.  (2048 for the bf16 and PQ scans; the sketch scan,
+    // lasts as long as its longest block.  (2048 for the bf16 scan; the listed sketch scan,
     // whose blocks cost more to start and to end than their steps cost, does better with 512:
     // 34 against 42 us at 8 units x 131072 rows, 37 against 46 us at 32 units x 32768 rows.)
     const int64_t tiles = ((int64_t)n_rows + rows_per_step - 1) / rows_per_step;
@@ -1480,7 +1555,7 @@ extern "C" int dc_pq_search_bf16(const void *k, const uint8_t *codes, const floa
     DC_REQUIRE(sb % 8 == 0 && sh % 8 == 0 && sr % 8 == 0 && sr >= hd,
                "%s: key strides must be multiples of 8 elements and row_stride >= hd", who);
     FusedPlan p;
-    int rc = plan_fused(who, n_b, n_h, n_rows, n_cand, &p, kPqBigSteps, kPqThreads);
+    int rc = plan_fused(who, n_b, n_h, n_rows, n_cand, &p);
     if (rc) return rc;
     const int k1 = p.k_eff;                   // candidates per unit
     const int k2 = topk < k1 ? topk : k1;     // results per unit
@@ -1500,17 +1575,30 @@ extern "C" int dc_pq_search_bf16(const void *k, const uint8_t *codes, const floa
         rc = dc_select_state_init(p.n_units, n_rows, n_cand, workspace, workspace_bytes, stream);
         if (rc) return rc;
     }
+    // equal shares for as many blocks as run at once
+    const int64_t tiles = ((int64_t)n_rows + kPqThreads - 1) / kPqThreads;
+    const int64_t steps = (p.n_units * tiles + kPqBlocks - 1) / kPqBlocks;
+    const int64_t blocks = p.n_units * ((tiles + steps - 1) / steps);
+    const int64_t class_blocks = p.n_units * (((int64_t)n_rows + kPqClassRows - 1) / kPqClassRows);
+    DC_REQUIRE(blocks < (1ll << 31) && class_blocks < (1ll << 31), "%s: grid too large", who);
     if (ev_scan_begin) (void)hipEventRecord((hipEvent_t)ev_scan_begin, st);
     if (m == 16)
-        hipLaunchKernelGGL(pq_prune_kernel<16>, dim3((unsigned)p.blocks), dim3(kPqThreads), 0, st, codes, lut,
-                           w.hist, w.state, w.surv, p.n_units, n_rows, k1, p.small_chunks, p.big_steps);
+        hipLaunchKernelGGL(pq_scan_kernel<16>, dim3((unsigned)blocks), dim3(kPqThreads), 0, st, codes, lut, w.hist, w.surv,
+                           p.n_units, n_rows, (int)steps);
     else
-        hipLaunchKernelGGL(pq_prune_kernel<32>, dim3((unsigned)p.blocks), dim3(kPqThreads), 0, st, codes, lut,
-                           w.hist, w.state, w.surv, p.n_units, n_rows, k1, p.small_chunks, p.big_steps);
+        hipLaunchKernelGGL(pq_scan_kernel<32>, dim3((unsigned)blocks), dim3(kPqThreads), 0, st, codes, lut, w.hist, w.surv,
+                           p.n_units, n_rows, (int)steps);
     DC_CHECK_LAUNCH(who);
     if (ev_scan_end) (void)hipEventRecord((hipEvent_t)ev_scan_end, st);
     // the k1 best ADC scores of every unit, in no particular order
-    rc = launch_select(who, w, cand, k1, p.n_units, n_rows, k1, DC_MODE_IP, DC_ORDER_ANY, 1, st);
+    if (m == 16)
+        hipLaunchKernelGGL(pq_classify_kernel<16>, dim3((unsigned)class_blocks), dim3(kThreads), 0, st, codes, lut, w.hist, w.state,
+                           w.surv, w.cand_key, w.cand_idx, cand, (int64_t)k1, p.n_units, n_rows, k1);
+    else
+        hipLaunchKernelGGL(pq_classify_kernel<32>, dim3((unsigned)class_blocks), dim3(kThreads), 0, st, codes, lut, w.hist, w.state,
+                           w.surv, w.cand_key, w.cand_idx, cand, (int64_t)k1, p.n_units, n_rows, k1);
+    DC_CHECK_LAUNCH(who);
+    rc = launch_finish(who, w, cand, k1, p.n_units, n_rows, k1, DC_MODE_IP, DC_ORDER_ANY, 1, st);
     if (rc) return rc;
     const int lpr = hd / 8, groups = kThreads / lpr;
     const int64_t bpu = ((int64_t)k1 + groups - 1) / groups;
