@@ -25,20 +25,49 @@ constexpr int kSplitWaves = 8;                     // of a block of short_attend
 constexpr int kSplitThreads = kSplitWaves * 64;
 constexpr int kSplitRows = kSplitWaves * 16;       // list positions of a split: one tile of 16 per wave
 constexpr int kShortMaxRows = 16 * 4 * kSplitThreads;  // 16 vectors of four keys per thread; places fit 16 bits
+constexpr int kRankMost = 128;                     // rows of the threshold bucket that are ranked straight away
 constexpr int kListMost = 2048;                    // rows of the threshold bucket that are listed
 constexpr uint32_t kNoKey = 0xffffffffu;           // the key of no row
 
-// The worst key a row can have; rows without a number go to either end of the order, as their bucket says.
+// The buckets of a histogram: those of dc_score_bucket, or, FINE, of half their width for positive scores (16 per binade
+// from 2^-12 to 2^20).  Half as many candidates spare regions of up to 4 Ki rows a pass of the cutoff (8 units x 4028 rows:
+// 17.1 -> 16.7 us, 2 x 4028 15.4 -> 14.8); in longer ones they cost as much in counts (8 x 16323 of 64 19.0 -> 19.5).
+template <bool FINE>
+struct ShortBuckets {
+    static constexpr uint32_t kGrain = FINE ? 4u : kSubBits, kPos = FINE ? 512u : kPosBuckets;
+    static constexpr uint32_t kLo = FINE ? (127u - 12u) << 23 : (127u - 20u) << 23;  // the least positive score told apart
+    static_assert(kPos + 512u <= DC_HIST_BINS, "positive and negative buckets");
+    static __device__ __forceinline__ uint32_t of(float s) {
+        if (!FINE) return dc_score_bucket(s);
+        const uint32_t b = __float_as_uint(s + 0.0f);  // -0 -> +0
+        const uint32_t mag = b & 0x7fffffffu;
+        if (b & 0x80000000u) return kPos + (mag >> 22);
+        constexpr uint32_t hi = kLo + (kPos << (23u - kGrain)) - 1u;
+        const uint32_t m = mag < kLo ? kLo : (mag > hi ? hi : mag);
+        return (kPos - 1u) - ((m - kLo) >> (23u - kGrain));
+    }
+};
+
+// Key (as dc_key_bucket) and bucket of a row; rows without a number go to either end of the order, as their bucket says.
+template <bool FINE>
 __device__ __forceinline__ void short_key(float s, int mode, uint32_t &key, uint32_t &bucket) {
-    dc_key_bucket(s, mode, key, bucket);
-    if (mode == DC_MODE_REF_DIST && !(s == s)) key = bucket < kPosBuckets ? 0u : kNoKey;
+    using B = ShortBuckets<FINE>;
+    if (mode == DC_MODE_REF_DIST) {
+        const float d = 65536.0f - s;
+        key = dc_f2ord(d);
+        bucket = B::of(65536.0f - d);
+        if (!(s == s)) key = bucket < B::kPos ? 0u : kNoKey;
+    } else {
+        key = dc_f2ord(-(s + 0.0f));
+        bucket = B::of(s);
+    }
     key = key < kNoKey ? key : kNoKey - 1u;
 }
 
 // Bound by memory latency up to some 30 MB of keys (5 us at 8 units x 4028 rows of 128 columns, 7 at 8 x 16323 of 64,
 // of which 2 are the launch), then by bandwidth (14.6 us at 8 x 32533 of 128: 4.6 TB/s).  A wave takes eight loads of 64 / LPR rows
 // each at a time, two such parts in flight, the first of them on the way before the query is there.
-template <int HD>
+template <int HD, bool FINE>
 __global__ __launch_bounds__(kThreads) void short_score_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, uint32_t *__restrict__ hist,
     uint32_t *__restrict__ keys, int64_t key_stride, int n_units, int n_h, int n_cap, int64_t sb, int64_t sh, int64_t sr,
@@ -82,7 +111,7 @@ __global__ __launch_bounds__(kThreads) void short_score_kernel(
         const int64_t row = block_row0 + (int64_t)(i * WAVES + wave) * PART + grp * NL + col;
         if (col < NL && row < n_rows) {
             uint32_t key, bucket;
-            short_key(mine, mode, key, bucket);
+            short_key<FINE>(mine, mode, key, bucket);
             ku[row] = key;
             atomicAdd(&lhist[bucket], 1u);
         }
@@ -109,43 +138,45 @@ __global__ __launch_bounds__(kThreads) void short_score_kernel(
 // a value that is the same in all lanes, in a scalar register
 __device__ __forceinline__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 
-// Whether a key's bucket is `b` or worse (the buckets of dc_key_bucket, from the key alone).
+// Whether a key's bucket is `b` or worse (from the key alone).
+template <bool FINE>
 __device__ __forceinline__ bool key_reaches(uint32_t key, uint32_t b, int mode) {
     const float x = __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);  // dc_f2ord, inverted
-    return dc_score_bucket(mode == DC_MODE_REF_DIST ? 65536.0f - x : -x) >= b;
+    return ShortBuckets<FINE>::of(mode == DC_MODE_REF_DIST ? 65536.0f - x : -x) >= b;
 }
 
 // The smallest key whose bucket is lane % 2 + bin or worse, in every lane of that parity: the ends of
 // a bucket.  DC_MODE_IP: the map inverted.  DC_MODE_REF_DIST: the map inverted up to the rounding of d, the 32 keys
 // around tried at once; scores beyond 32768, whose d has another grid than the score, may miss that window and
 // are bisected.
+template <bool FINE>
 __device__ __forceinline__ uint32_t bucket_first_key(uint32_t bin, int mode) {
-    constexpr uint32_t kLoMag = (127u - 20u) << 23;
+    constexpr uint32_t kLoMag = ShortBuckets<FINE>::kLo, kPos = ShortBuckets<FINE>::kPos, kGrain = ShortBuckets<FINE>::kGrain;
     constexpr uint32_t kFirst = 0x007fffffu, kLast = 0xff800000u;  // the keys of -inf and +inf
     const int lane = threadIdx.x & 63;
     const uint32_t b = bin + (uint32_t)(lane & 1);
     // the largest score in bucket b or a worse one
-    const uint32_t mag = b < kPosBuckets ? kLoMag + ((kPosBuckets - b) << (23u - kSubBits)) - 1u : (b - kPosBuckets) << 22;
+    const uint32_t mag = b < kPos ? kLoMag + ((kPos - b) << (23u - kGrain)) - 1u : (b - kPos) << 22;
     if (mode == DC_MODE_IP) {
         if (b == 0u) return 0u;
-        if (b < kPosBuckets) return 0x7fffffffu - mag;
-        return b - kPosBuckets < 512u ? 0x80000000u | mag : kNoKey;
+        if (b < kPos) return 0x7fffffffu - mag;
+        return b - kPos < 512u ? 0x80000000u | mag : kNoKey;
     }
-    const float s = __uint_as_float(b < kPosBuckets ? mag : 0x80000000u | mag);
-    const uint32_t guess = dc_f2ord(65536.0f - (b < kPosBuckets + 511u ? s : -__builtin_inff()));
+    const float s = __uint_as_float(b < kPos ? mag : 0x80000000u | mag);
+    const uint32_t guess = dc_f2ord(65536.0f - (b < kPos + 511u ? s : -__builtin_inff()));
     uint32_t c = guess - 16u + (uint32_t)(lane >> 1);
     c = c < kFirst ? kFirst : (c > kLast ? kLast : c);
-    unsigned long long hits = __ballot(key_reaches(c, b, mode)) >> (lane & 1) & 0x5555555555555555ull;
+    unsigned long long hits = __ballot(key_reaches<FINE>(c, b, mode)) >> (lane & 1) & 0x5555555555555555ull;
     const int first = hits ? (int)__builtin_ctzll(hits) : 64;  // 2 * place in the window
     uint32_t out = guess - 16u + (uint32_t)(first >> 1);
     bool sure = first > 0 && first < 64;
     if (b == 0u) out = 0u, sure = true;
-    if (b >= kPosBuckets + 511u) out = b == kPosBuckets + 511u ? kLast + 1u : kNoKey, sure = true;  // rows without a number
+    if (b >= kPos + 511u) out = b == kPos + 511u ? kLast + 1u : kNoKey, sure = true;  // rows without a number
     if (__ballot(!sure)) {
-        uint32_t lo = kFirst, hi = kLast;  // lo does not reach b > 0, hi does reach every b <= kPosBuckets + 510
+        uint32_t lo = kFirst, hi = kLast;  // lo does not reach b > 0, hi does reach every b <= kPos + 510
         while (hi - lo > 1u) {
             const uint32_t mid = lo + (hi - lo) / 2u;
-            if (key_reaches(mid, b, mode)) hi = mid;
+            if (key_reaches<FINE>(mid, b, mode)) hi = mid;
             else lo = mid;
         }
         if (!sure) out = hi;
@@ -163,7 +194,7 @@ struct ShortArgs {
 
 struct ShortShared {
     uint32_t lh[256];
-    unsigned long long tie[64];
+    unsigned long long tie[kRankMost];
     uint32_t own[kSplitRows];  // the split's selected ids
     uint32_t wtot[kSplitWaves + 1];
     uint32_t n_tie;
@@ -317,7 +348,7 @@ __global__ __launch_bounds__(kSplitThreads) void short_attend_kernel(AttnArgs a,
         f.load(a, group, unit);
         uint32_t lo = kNoKey, hi = kNoKey - 1u;  // fewer rows than k: all are certain
         if (bin < (uint32_t)DC_HIST_BINS) {
-            const uint32_t ends = bucket_first_key(bin, s.mode);
+            const uint32_t ends = bucket_first_key<NV <= 2>(bin, s.mode);
             lo = (uint32_t)__builtin_amdgcn_readlane((int)ends, 0);
             hi = (uint32_t)__builtin_amdgcn_readlane((int)ends, 1) - 1u;
         }
@@ -326,6 +357,7 @@ __global__ __launch_bounds__(kSplitThreads) void short_attend_kernel(AttnArgs a,
         for (int w = 0; w < MW; ++w) sure[w] = cand[w] = 0u;
 #pragma unroll
         for (int i = NV - 1; i >= 0; --i) {
+            if (4 * i * kSplitThreads >= n_rows) continue;  // (the vectors go by the largest region)
             const uint32_t k4[4] = {kv[i].x, kv[i].y, kv[i].z, kv[i].w};
 #pragma unroll
             for (int j = 3; j >= 0; --j) {
@@ -364,6 +396,35 @@ __global__ __launch_bounds__(kSplitThreads) void short_attend_kernel(AttnArgs a,
         if (slot0 + kSplitRows > n_sure && n_sure < kk) {
             if (rem >= n_cand) {
                 each_bit(cand, n_sure + p_cand, own);
+            } else if (n_cand <= (uint32_t)kRankMost) {
+                // few: the rank among them is the place
+                if (NV <= 4) {
+                    uint32_t e = p_cand;
+#pragma unroll
+                    for (int i = 0; i < NV; ++i) {
+                        const uint32_t k4[4] = {kv[i].x, kv[i].y, kv[i].z, kv[i].w};
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if (cand[0] >> (4 * i + j) & 1u)
+                                sh.tie[e++] = ((unsigned long long)k4[j] << 32) | (uint32_t)(4 * (i * kSplitThreads + tid) + j);
+                    }
+                } else {
+                    each_bit(cand, p_cand, [&](uint32_t place, uint32_t row) __attribute__((always_inline)) { sh.list[place] = (uint16_t)row; });
+                    __syncthreads();
+                    if (tid < (int)n_cand) {
+                        const uint32_t row = sh.list[tid];
+                        sh.tie[tid] = ((unsigned long long)ku[row] << 32) | row;
+                    }
+                }
+                __syncthreads();
+                constexpr int kLanes = kSplitThreads / kRankMost;  // lanes to an entry
+                const uint32_t e = (uint32_t)(tid / kLanes);
+                const unsigned long long mine = e < n_cand ? sh.tie[e] : ~0ull;
+                uint32_t rank = 0u;
+                for (uint32_t j = (uint32_t)(tid % kLanes); j < n_cand; j += kLanes) rank += sh.tie[j] < mine ? 1u : 0u;
+#pragma unroll
+                for (int d = 1; d < kLanes; d <<= 1) rank += (uint32_t)__shfl_xor((int)rank, d, 64);
+                if (tid % kLanes == 0 && e < n_cand && rank < rem) own(n_sure + rank, (uint32_t)mine);
             } else if (n_cand <= (uint32_t)kListMost) {
                 each_bit(cand, p_cand, [&](uint32_t place, uint32_t row) __attribute__((always_inline)) { sh.list[place] = (uint16_t)row; });
                 __syncthreads();
@@ -502,15 +563,22 @@ int dc_short_layer(const dc_layer_args *a, int region, int k_eff, void *sel_ws, 
     const int64_t all_parts = (region + part_rows - 1) / part_rows;
     const int64_t parts = (n_units * all_parts + kScoreBlocks - 1) / kScoreBlocks;
     const int64_t bpu = (all_parts + parts - 1) / parts;
+    const bool fine = region <= 2 * 4 * kSplitThreads;  // NV <= 2 of short_attend_kernel
     if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
-#define DC_LAUNCH_SS(HD)                                                                                              \
-    hipLaunchKernelGGL(short_score_kernel<HD>, dim3((unsigned)(n_units * bpu)), dim3(kThreads), 0, st, k_region,       \
+#define DC_LAUNCH_SSF(HD, FN)                                                                                         \
+    hipLaunchKernelGGL((short_score_kernel<HD, FN>), dim3((unsigned)(n_units * bpu)), dim3(kThreads), 0, st, k_region,       \
                        (const uint16_t *)a->q, w.hist, keys, key_stride, n_units, a->n_h, region, a->kv_batch_stride,  \
                        a->kv_head_stride, a->kv_row_stride, a->group, a->mode, (int)parts, a->region_hi_dev, a->n_sink)
+#define DC_LAUNCH_SS(HD)                    \
+    do {                                    \
+        if (fine) DC_LAUNCH_SSF(HD, true);  \
+        else DC_LAUNCH_SSF(HD, false);      \
+    } while (0)
     if (hd == 64) DC_LAUNCH_SS(64);
     else if (hd == 128) DC_LAUNCH_SS(128);
     else DC_LAUNCH_SS(256);
 #undef DC_LAUNCH_SS
+#undef DC_LAUNCH_SSF
     DC_CHECK_LAUNCH(who);
     if (a->ev_scan_end) (void)hipEventRecord((hipEvent_t)a->ev_scan_end, st);
 

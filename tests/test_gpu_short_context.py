@@ -101,7 +101,7 @@ def test_rows_without_a_number_are_chosen_as_by_the_long_chain(mode):
 @pytest.mark.gpu
 def test_the_live_end_of_the_region_comes_from_the_device():
     """Launches laid out for the largest region: shorter ends, the split's places and the padding of the last four keys
-    move with the device word; every replay equals an eager call that passes the end as a size."""
+    move with the device word; every replay agrees with an eager call that passes the end as a size."""
     from diffcache_amd import _hip as hip
     g = torch.Generator(device=DEV).manual_seed(5)
     b, hkv, group, hd, cap, budget, sink, window = 2, 2, 4, 128, 9001, 200, 4, 16
@@ -127,7 +127,11 @@ def test_the_live_end_of_the_region_comes_from_the_device():
         graph.replay()
         call(1, sink + region, False)
         torch.cuda.synchronize()
-        assert torch.equal(idx[0], idx[1]) and torch.equal(out[0], out[1]), region
+        # launches laid out for 4 Ki rows count in finer buckets, so the rows may come in another order: sums of at
+        # most 221 terms of weight <= 1 in fp32 (221 * 2^-24 * |v| < 1e-4), then one bf16 rounding (2^-8) on either side
+        assert torch.equal(idx[0].sort(dim=1).values, idx[1].sort(dim=1).values), region
+        x, y = out[0].float(), out[1].float()
+        assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 1e-4).all()), region
         torch.randn(1000, device=DEV).sum().item()      # eager work between replays
 
 
