@@ -747,9 +747,11 @@ class LayerStep:
     step, as DiffCache does.  Filling and checking dc_layer_args anew in every call was a third of a layer's host time
     (16.1 us of it per layer of eight one-kernel layers, launch included; 10.7 us now).  The struct is
     filled and checked again whenever any pointer, shape, stride, type or size of them differs from the last
-    call's; what is new in every call (q, new_k, new_v, out) is checked in every call."""
+    call's; what is new in every call (q, new_k, new_v, out) is checked in every call.  The first call keeps
+    nothing: comparing costs it 3 us, which only a second call can win back."""
 
     def __init__(self) -> None:
+        self._again = False
         self._key: Optional[tuple] = None
         self._args: Optional[LayerArgs] = None
         self._step = StepArgs()
@@ -759,8 +761,8 @@ class LayerStep:
                  append, advance) -> None:
         """The arguments of decode_layer."""
         n = q.numel()
-        key = None
-        if scores is None and lse is None and scan_events is None and append is not None:
+        key, again, self._again = None, self._again, True
+        if again and scores is None and lse is None and scan_events is None and append is not None:
             key = (store_k.data_ptr(), store_k.shape, store_k.stride(), store_k.dtype, store_v.data_ptr(), store_v.stride(),
                    store_v.dtype, idx_out.data_ptr(), idx_out.shape, idx_out.stride(), workspace.data_ptr(),
                    workspace.numel(), n_sink, recent_lo, n_recent, budget, mode, order, scale, n, append[0], append[2])

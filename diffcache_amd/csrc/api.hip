@@ -117,7 +117,8 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
                                            : (a->sketch_codes && region <= DC_SKETCH_MAX_ROWS ? DC_ROUTE_SKETCH
                                                                                              : DC_ROUTE_STREAM));
     const bool short_ok = dc_short_supported(a, region, k_eff);
-    if (k_eff > 0 && !a->scores && a->order == DC_ORDER_ANY && !a->region_hi_dev &&
+    const bool one_first = dc_one_kernel_first(a, region, k_eff);
+    if (k_eff > 0 && !a->scores && a->order == DC_ORDER_ANY && !a->region_hi_dev && (one_first || !ready) &&
         dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr)) {
         // short context: the whole layer in one kernel whose blocks are all resident (ids in no
         // particular order); reads the bf16 keys, with or without a sketch.  The state is set up
@@ -132,7 +133,7 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
             ready = 1;
         }
         rc = 0;
-        if (dc_one_kernel_first(a, region, k_eff)) {
+        if (one_first) {
             if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
             rc = dc_small_try(a, region, k_eff, w.topk, w.small_cand, w.attn, w.attn_bytes, stream, step);
         }
