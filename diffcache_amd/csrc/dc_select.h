@@ -23,6 +23,17 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v, int) {
     return v;
 }
 
+// OR over the lanes of a wave, in lane 63 (the same steps)
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, true);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, true);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, true);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, true);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 // Block-wide exclusive scan for NT threads (NT a multiple of 64, <= 1024).
 // `wtot` is LDS scratch of at least NT/64 + 1 words.  Returns the exclusive
 // prefix; *total receives the block sum.  Contains two barriers.

@@ -1012,11 +1012,16 @@ __global__ __launch_bounds__(kThreads) void pq_rescore_kernel(
 }
 
 // One block per unit: a selection among the candidates of the threshold bucket
-// fills idx_out[c_less, k).  Leaves the unit's list cursors at zero.  A chain of block barriers on few CUs: the
-// counting pass that hands out the slots itself (dc_select_counted) takes 5.9 us at 8 units and 7.0 us at
-// 64 (2048 of about 3600 candidates); a radix pass whose members reserve slots wave by wave took 7.5
-// and 8.8 us.  Lists that do not fit the LDS and threshold bins of more than kFinalThreads (ties by the
-// thousand) take the radix passes of dc_finalize_unit.
+// fills idx_out[c_less, k).  Leaves the unit's list cursors at zero.  A chain of block barriers on few CUs.  Lists of up to
+// kFinishRegs entries stay in registers, requested whole before their length is known: one counting pass over the
+// highest 11 bits in which the keys differ hands out the slots (as dc_select_counted does), with six barriers: 5.3 us at 8
+// units and 6.6 at 64 (2048 of about 3600 candidates), 5.9 and 7.3 with the list staged in LDS and eight barriers.
+// (Counting a threshold bin of more than 96 once more instead of ranking it: no faster where it applies, 0.3 us slower else.)
+// A radix pass whose members reserve slots wave by wave took 7.5 and 8.8 us.  Longer lists take dc_select_counted as long as they fit
+// the LDS; lists that do not, and threshold bins of more than kFinalThreads (ties by the
+// thousand), take the radix passes of dc_finalize_unit.
+constexpr int kFinishPer = 8, kFinishRegs = kFinishPer * kFinalThreads;
+
 __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     uint32_t *__restrict__ hist, UnitState *__restrict__ state, uint32_t *__restrict__ cand_key,
     uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride,
@@ -1025,19 +1030,18 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     __shared__ uint32_t wtot[kFinalThreads / 64 + 1];
     __shared__ uint32_t sres[4];
     __shared__ uint32_t smisc[2];
-    __shared__ uint32_t lck[kCandLds], lci[kCandLds];  // candidates are staged in LDS when they fit
+    __shared__ uint32_t s_or[kFinalThreads / 64];
+    __shared__ uint32_t lck[kCandLds], lci[kCandLds];  // longer lists are staged in LDS when they fit
     __shared__ unsigned long long tie[kFinalThreads];
     const int unit = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     UnitState *st = state + unit;
     uint32_t *ck = cand_key + (int64_t)unit * n_rows;
     uint32_t *ci = cand_idx + (int64_t)unit * n_rows;
-    // the head of the candidate list (what a list of ordinary length holds) is fetched before
-    // its length is known: one memory round trip less
-    constexpr int kHead = 4;
-    uint32_t hk[kHead], hi[kHead];
+    // the list is fetched before its length is known: one memory round trip less
+    uint32_t hk[kFinishPer], hi[kFinishPer];
 #pragma unroll
-    for (int j = 0; j < kHead; ++j) {
+    for (int j = 0; j < kFinishPer; ++j) {
         const int i = tid + j * kFinalThreads;
         hk[j] = hi[j] = 0;
         if (i < n_rows) {
@@ -1045,23 +1049,29 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
             hi[j] = ci[i];
         }
     }
+    const uint32_t k0 = ck[0];
     uint32_t n_c = st->cand_cnt;
     const uint32_t c_less = st->c_less;
+    reinterpret_cast<uint2 *>(lh)[tid] = make_uint2(0u, 0u);
     if (n_c > (uint32_t)n_rows) n_c = n_rows;
     const uint32_t kk = (uint32_t)k_eff;
     uint32_t *io = idx_out + (int64_t)unit * idx_stride;
     uint32_t *ko = sel_keys ? sel_keys + (int64_t)unit * k_eff : nullptr;
-    const bool staged = n_c <= (uint32_t)kCandLds;
-    if (staged) {
+    const bool regs = n_c <= (uint32_t)kFinishRegs, staged = !regs && n_c <= (uint32_t)kCandLds;
+    if (regs) {
+        uint32_t diff = 0u;
 #pragma unroll
-        for (int j = 0; j < kHead; ++j) {
-            const uint32_t i = (uint32_t)(tid + j * kFinalThreads);
-            if (i < n_c) {
-                lck[i] = hk[j];
-                lci[i] = hi[j];
-            }
+        for (int j = 0; j < kFinishPer; ++j)
+            if (j * kFinalThreads < (int)n_c) diff |= (uint32_t)(tid + j * kFinalThreads) < n_c ? hk[j] ^ k0 : 0u;
+        diff = wave_or(diff);
+        if (lane == 63) s_or[wave] = diff;
+    } else if (staged) {
+#pragma unroll
+        for (int j = 0; j < kFinishPer; ++j) {
+            lck[tid + j * kFinalThreads] = hk[j];
+            lci[tid + j * kFinalThreads] = hi[j];
         }
-        for (uint32_t i = tid + kHead * kFinalThreads; i < n_c; i += kFinalThreads) {
+        for (uint32_t i = tid + kFinishRegs; i < n_c; i += kFinalThreads) {
             lck[i] = ck[i];
             lci[i] = ci[i];
         }
@@ -1083,16 +1093,67 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     if (c_less >= kk) return;
     uint32_t need = kk - c_less;
     if (need > n_c) need = n_c;
-    auto put = [&](uint32_t slot, uint32_t key, uint32_t id) {
+    auto put = [&](uint32_t slot, uint32_t key, uint32_t id) __attribute__((always_inline)) {
         io[c_less + slot] = id;
         if (ko) ko[c_less + slot] = key;
     };
+    if (regs) {
+        auto each = [&](auto fn) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < kFinishPer; ++j)
+                if (j * kFinalThreads < (int)n_c && (uint32_t)(tid + j * kFinalThreads) < n_c)
+                    fn((uint32_t)(tid + j * kFinalThreads), hk[j], hi[j]);
+        };
+        if (need == n_c) {  // all of them
+            each(put);
+            return;
+        }
+        uint32_t diff = 0u;
+#pragma unroll
+        for (int w = 0; w < kFinalThreads / 64; ++w) diff |= s_or[w];
+        const int top = diff ? 32 - __clz((int)diff) : 0;
+        const int shift = top > kRadixBits ? top - kRadixBits : 0;
+        const uint32_t mask = diff ? (uint32_t)kRadixBins - 1u : 0u;  // the bits above are the same in every key
+        each([&](uint32_t, uint32_t key, uint32_t) __attribute__((always_inline)) { atomicAdd(&lh[(key >> shift) & mask], 1u); });
+        __syncthreads();
+        const uint2 h2 = reinterpret_cast<const uint2 *>(lh)[tid];
+        uint32_t total;
+        const uint32_t excl = block_excl_scan<kFinalThreads>(h2.x + h2.y, wtot, &total);
+        reinterpret_cast<uint2 *>(lh)[tid] = make_uint2(excl, excl + h2.x);
+        if (excl < need && need <= excl + h2.x + h2.y) {
+            const bool first = excl + h2.x >= need;
+            sres[0] = 2 * tid + (first ? 0 : 1);
+            sres[1] = first ? excl : excl + h2.x;
+            sres[2] = first ? h2.x : h2.y;
+        }
+        __syncthreads();
+        const uint32_t t_bin = sres[0], t_lo = sres[1], t_cnt = sres[2];
+        if (t_cnt <= (uint32_t)kFinalThreads) {
+            each([&](uint32_t, uint32_t key, uint32_t id) __attribute__((always_inline)) {
+                const uint32_t bin = (key >> shift) & mask;
+                if (bin > t_bin) return;
+                const uint32_t slot = atomicAdd(&lh[bin], 1u);
+                if (bin == t_bin) tie[slot - t_lo] = ((unsigned long long)key << 32) | id;
+                else put(slot, key, id);
+            });
+            __syncthreads();
+            if ((uint32_t)tid < t_cnt) {
+                const unsigned long long mine = tie[tid];
+                uint32_t rank = t_lo;
+                for (uint32_t j = 0; j < t_cnt; ++j) rank += tie[j] < mine ? 1u : 0u;
+                if (rank < need) put(rank, (uint32_t)(mine >> 32), (uint32_t)mine);
+            }
+            return;
+        }
+        // keys that crowd into one bin: from LDS like a longer list
+        each([&](uint32_t i, uint32_t key, uint32_t id) __attribute__((always_inline)) { lck[i] = key, lci[i] = id; });
+    }
     if (staged && dc_select_counted<false>(lck, lci, n_c, need, tie, lh, wtot, sres, smisc, put)) return;
     __syncthreads();
     // Two calls, so that the staged list is read with LDS instructions: through a pointer chosen
     // at run time every access would be a flat one, and waiting for a flat load also waits for
     // the stores issued above.
-    if (staged) dc_finalize_unit<true>(lck, lci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
+    if (regs || staged) dc_finalize_unit<true>(lck, lci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
     else dc_finalize_unit(ck, ci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
 }
 
