@@ -109,7 +109,7 @@ FusedWs carve_fused(void *base, int n_units, int n_rows, int k) {
     w.state = (UnitState *)(p + off);
     off += dc_align_up(nu * sizeof(UnitState), 256);
     w.surv = (uint2 *)(p + off);
-    off += dc_align_up(nu * nr * 8, 256);
+    off += dc_align_up(nu * (nr == 1 ? 2 : nr) * 8, 256);  // 16 bytes at least: a dense scan's words of a unit start there
     w.cand_key = (uint32_t *)(p + off);
     off += dc_align_up(nu * nr * 4, 256);
     w.cand_idx = (uint32_t *)(p + off);
