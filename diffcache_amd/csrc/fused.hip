@@ -132,7 +132,13 @@ __device__ __forceinline__ void prune_block_finish(uint32_t *lhist, const E *wst
     }
 }
 
-template <int HD>
+constexpr uint32_t kNoRow = 0xffffffffu;  // in the place of a row's key: there is no such row
+// words between the units of a dense scan's keys (16-byte rows of them)
+__host__ __device__ __forceinline__ int64_t dense_key_stride(int n_cap) { return ((int64_t)n_cap + 3) & ~3ll; }
+
+// DENSE: for scans of up to 1.75 Mi rows in all (plan_dense_keys), as in the sketch scan below: every row's 32-bit key goes to
+// the row's own place, nothing is polled, staged or listed, and blocks of equal shares all run at once.
+template <int HD, bool DENSE>
 __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, uint2 *__restrict__ surv, int n_units, int n_h, int n_cap,
@@ -141,7 +147,7 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     constexpr int LPR = HD / 8;
     constexpr int CH = LPR < 16 ? LPR : 16;
     __shared__ uint32_t lhist[DC_HIST_BINS];
-    __shared__ uint2 stage[kStage];
+    __shared__ uint2 stage[DENSE ? 1 : kStage];
     __shared__ uint32_t wtot[kThreads / 64 + 1];
     __shared__ uint32_t s_wcnt[kThreads / 64];
     __shared__ uint32_t s_base;
@@ -164,13 +170,19 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
               : (int64_t)small_chunks * kRowsPerBlockStep + (int64_t)big_id * big_steps * kRowsPerBlockStep;
     const int steps = small ? 1 : big_steps;
 
+    uint32_t *du = reinterpret_cast<uint32_t *>(surv) + (int64_t)unit * dense_key_stride(n_cap);
+    if (DENSE) {  // places behind the live end, up to the capacity that the readers go by
+        int64_t end = block_row0 + (int64_t)steps * kRowsPerBlockStep;
+        end = end < dense_key_stride(n_cap) ? end : dense_key_stride(n_cap);
+        for (int64_t r = (block_row0 > n_rows ? block_row0 : (int64_t)n_rows) + tid; r < end; r += kThreads) du[r] = kNoRow;
+    }
     if (block_row0 >= n_rows) return;  // the grid is laid out for n_cap rows
     for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
 
     const uint16_t *Ku = K + b * sb + h * sh + col * 8;
     UnitState *st = state + unit;
     const int last = n_rows - 1;
-    uint32_t tb = load_relaxed(&st->tb_run);
+    uint32_t tb = DENSE ? (uint32_t)DC_HIST_BINS : load_relaxed(&st->tb_run);
 
     float q[8];
     dc_load_query<HD>(Q, unit, q_group, col, q);
@@ -197,7 +209,7 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
                 w[j] = dc_load_stream16(Ku + r * sr);
             }
             // the threshold for the next step queues up behind this step's rows
-            if (c0 + CH >= LPR && step + 1 < steps) tb_next = load_relaxed(&st->tb_run);
+            if (!DENSE && c0 + CH >= LPR && step + 1 < steps) tb_next = load_relaxed(&st->tb_run);
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 float p = dc_group_sum<LPR>(dc_dot8(w[j], q, 0.f));
@@ -208,6 +220,13 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
         const bool valid = myrow < n_rows;
         uint32_t key = 0, bucket = 0xffffffffu;
         if (valid) dc_key_bucket(mine, mode, key, bucket);
+        if (DENSE) {
+            if (valid) {
+                du[myrow] = key < kNoRow ? key : kNoRow - 1u;
+                atomicAdd(&lhist[bucket], 1u);
+            }
+            continue;
+        }
         // Only rows that can still matter are kept and counted: the final threshold
         // bucket is never worse than tb, so it is fixed by the counts of buckets <= tb.
         const bool keep = valid && bucket <= tb;
@@ -216,6 +235,15 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
         if (keep) wstage[wcnt + __popcll(mask & lt)] = make_uint2((uint32_t)myrow, __float_as_uint(mine));
         wcnt += (uint32_t)__popcll(mask);
         tb = tb_next;
+    }
+    if (DENSE) {
+        __syncthreads();
+        uint32_t *hu = hist + (int64_t)unit * DC_HIST_BINS;
+        for (int i = tid; i < DC_HIST_BINS; i += kThreads) {
+            const uint32_t c = lhist[i];
+            if (c) atomicAdd(&hu[i], c);
+        }
+        return;
     }
     // every 4th small block and every 8th large one refresh the running threshold
     const bool refresh = small ? (chunk & 3) == 3 : ((chunk - small_chunks) & 7) == 7;
@@ -826,6 +854,80 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(
     }
 }
 
+// classify_kernel for the keys that a dense score_prune_kernel left: a block takes kKeyClassRows rows and reserves its places
+// in both lists with one returning atomic.  Bound by its chain: keys (6.4 MB at 32 units x 49933 rows) while the histogram is
+// scanned, one atomic, the members' stores.
+constexpr int kKeyClassRows = 4096;
+
+__global__ __launch_bounds__(kThreads) void key_classify_kernel(
+    const uint32_t *__restrict__ hist, UnitState *__restrict__ state, const uint2 *__restrict__ surv,
+    uint32_t *__restrict__ cand_key, uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride,
+    uint32_t *__restrict__ sel_keys, int n_units, int n_rows, int k_eff, int mode) {
+    constexpr int kVec = kKeyClassRows / kThreads / 4;
+    __shared__ uint32_t wtot[kThreads / 64 + 1];
+    __shared__ uint32_t sres[2];
+    __shared__ uint32_t sbase[2];
+    const int unit = blockIdx.x % n_units, blk = blockIdx.x / n_units;
+    const int tid = threadIdx.x;
+    const int64_t row0 = (int64_t)blk * kKeyClassRows;
+    UnitState *st = state + unit;
+    const int64_t stride = dense_key_stride(n_rows);
+    const uint32_t *du = reinterpret_cast<const uint32_t *>(surv) + (int64_t)unit * stride;
+    uint32_t keys[4 * kVec];
+#pragma unroll
+    for (int i = 0; i < kVec; ++i) {
+        const int64_t r = row0 + (i * kThreads + tid) * 4;
+        uint4 v = make_uint4(kNoRow, kNoRow, kNoRow, kNoRow);
+        if (r < stride) v = *reinterpret_cast<const uint4 *>(du + r);
+        keys[4 * i] = v.x, keys[4 * i + 1] = v.y, keys[4 * i + 2] = v.z, keys[4 * i + 3] = v.w;
+    }
+    const uint32_t kk = (uint32_t)k_eff;
+    uint32_t tb, c_less;
+    unit_threshold(hist + (int64_t)unit * DC_HIST_BINS, kk, wtot, sres, tb, c_less);
+    if (blk == 0 && tid == 0) {
+        st->c_less = c_less;
+        st->cand_cnt = tb < (uint32_t)DC_HIST_BINS ? hist[(int64_t)unit * DC_HIST_BINS + tb] : 0u;  // every row is counted
+    }
+    uint32_t sure = 0, cand = 0;  // a bit per row
+#pragma unroll
+    for (int j = 0; j < 4 * kVec; ++j) {
+        const float x = __uint_as_float((keys[j] & 0x80000000u) ? keys[j] & 0x7fffffffu : ~keys[j]);  // dc_f2ord, inverted
+        const uint32_t bucket = dc_score_bucket(mode == DC_MODE_REF_DIST ? 65536.0f - x : -x);
+        sure |= keys[j] != kNoRow && bucket < tb ? 1u << j : 0u;
+        cand |= keys[j] != kNoRow && bucket == tb ? 1u << j : 0u;
+    }
+    uint32_t tot;
+    const uint32_t ex = block_excl_scan<kThreads>(__popc(sure) | __popc(cand) << 16, wtot, &tot);
+    if (tid == 0) {
+        unsigned long long at = 0ull;
+        if (tot) at = atomicAdd(reinterpret_cast<unsigned long long *>(&st->surv_cnt), (unsigned long long)(tot & 0xffffu) << 32 | tot >> 16);
+        sbase[0] = (uint32_t)(at >> 32);
+        sbase[1] = (uint32_t)at;
+    }
+    __syncthreads();
+    uint32_t wpos = sbase[0] + (ex & 0xffffu), cpos = sbase[1] + (ex >> 16);
+    uint32_t *ck = cand_key + (int64_t)unit * n_rows, *ci = cand_idx + (int64_t)unit * n_rows;
+    uint32_t *io = idx_out + (int64_t)unit * idx_stride;
+    uint32_t *ko = sel_keys ? sel_keys + (int64_t)unit * k_eff : nullptr;
+#pragma unroll
+    for (int j = 0; j < 4 * kVec; ++j) {
+        const uint32_t row = (uint32_t)row0 + (uint32_t)(((j / 4) * kThreads + tid) * 4 + j % 4);
+        if (sure >> j & 1u) {
+            if (wpos < kk) {
+                io[wpos] = row;
+                if (ko) ko[wpos] = keys[j];
+            }
+            ++wpos;
+        } else if (cand >> j & 1u) {
+            if (cpos < (uint32_t)n_rows) {
+                ck[cpos] = keys[j];
+                ci[cpos] = row;
+            }
+            ++cpos;
+        }
+    }
+}
+
 // Second pass of the sketch path.  Several blocks per unit split the list the
 // sketch scan left ((id, approx) pairs): a row stays a candidate when
 // bucket(approx + margin) is not worse than the exact bucket of the k-th largest
@@ -1306,15 +1408,34 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
 // and the two bytes a row outweigh the list: 64 x 131004 225.8 / 237.7, 8 x 1048508 221.7 / 235.3.
 constexpr int64_t kDenseMostTiles = (4ll << 20) / kRowsPerBlockStep;
 
+// The grid of a dense scan: `most` blocks at the very most, so that none starts when the others end.  (Shares worked out from
+// all tiles together gave a few blocks more where the tiles of a unit did not divide: 24 units x 65000 rows of 256 columns 106
+// against 94 us, 56 x 30011 of 128 68.1 against 65.5.)
+void plan_shares(int64_t n_units, int64_t tiles, int64_t most, FusedPlan *p) {
+    const int64_t each = most > n_units ? most / n_units : 1, steps = (tiles + each - 1) / each;
+    p->small_chunks = 0;
+    p->big_steps = (int)steps;
+    p->blocks = n_units * ((tiles + steps - 1) / steps);
+}
+
 bool plan_dense(int64_t n_units, int n_rows, int hd, FusedPlan *p) {
     const int64_t tiles = ((int64_t)n_rows + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
     if (n_units * tiles > kDenseMostTiles) return false;
-    if (p) {
-        const int64_t most = 256 * (hd == 64 ? 4 : (hd == 128 ? 3 : 2)), steps = (n_units * tiles + most - 1) / most;
-        p->small_chunks = 0;
-        p->big_steps = (int)steps;
-        p->blocks = n_units * ((tiles + steps - 1) / steps);
-    }
+    if (p) plan_shares(n_units, tiles, 256 * (hd == 64 ? 4 : (hd == 128 ? 3 : 2)), p);
+    return true;
+}
+
+// The same for the bf16 scan, whose rows take twice the bytes and leave four of them: two blocks per CU.  Per layer, us,
+// listed / dense: 32 units x 49933 rows of 128 columns 101 / 95, 24 x 70000 100.3 / 95, 12 x 130001 95 / 89.6, 20 x 77771
+// 98.5 / 91, 8 x 81852 53.0 / 49.3, 8 x 45000 39.0 / 35.9, 2 x 131004 40.0 / 35.3, 4 x 524000 125.6 / 111.4; 24 x 65000 of 64 59.2 /
+// 55.4; 9 x 55555 of 256 71.3 / 68.8, 24 x 65000 153.3 / 154.  1024 blocks 98.6 in the first of these, 1280 94.5, 2048 96.2 (a CU
+// holds five).  Beyond it is as often slower: 16 x 131004 112.2 / 115.5, 32 x 100000 163.6 / 166.2, 32 x 131004 204.1 / 208.3.
+constexpr int64_t kDenseKeyTiles = (7ll << 18) / kRowsPerBlockStep;  // 1.75 Mi rows
+
+bool plan_dense_keys(int64_t n_units, int n_rows, FusedPlan *p) {
+    const int64_t tiles = ((int64_t)n_rows + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
+    if (n_units * tiles > kDenseKeyTiles) return false;
+    if (p) plan_shares(n_units, tiles, 512, p);
     return true;
 }
 
@@ -1375,16 +1496,23 @@ int dc_score_prune_launch(const void *k, const void *q, int n_b, int n_h, int n_
     FusedWs w;
     rc = check_ws("dc_score_prune_bf16", workspace, workspace_bytes, p.n_units, n_rows, budget, &w);
     if (rc) return rc;
+    const bool dense = plan_dense_keys(p.n_units, n_rows, &p);
     hipStream_t st = (hipStream_t)stream;
-#define DC_LAUNCH_SP(HD)                                                                           \
-    hipLaunchKernelGGL(score_prune_kernel<HD>, dim3((unsigned)p.blocks), dim3(kThreads), 0, st,    \
+#define DC_LAUNCH_SPD(HD, DN)                                                                      \
+    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dim3((unsigned)p.blocks), dim3(kThreads), 0, st, \
                        (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv,          \
                        p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, p.small_chunks,  \
                        p.big_steps, hi_dev, lo_row)
+#define DC_LAUNCH_SP(HD)                    \
+    do {                                    \
+        if (dense) DC_LAUNCH_SPD(HD, true); \
+        else DC_LAUNCH_SPD(HD, false);      \
+    } while (0)
     if (hd == 64) DC_LAUNCH_SP(64);
     else if (hd == 128) DC_LAUNCH_SP(128);
     else DC_LAUNCH_SP(256);
 #undef DC_LAUNCH_SP
+#undef DC_LAUNCH_SPD
     DC_CHECK_LAUNCH("dc_score_prune_bf16");
     return DC_OK;
 }
@@ -1418,6 +1546,13 @@ int launch_select(const char *who, const FusedWs &w, uint32_t *idx_out, int64_t 
     // the grid stays near 2048 blocks
     // one block per 4096 rows and at most 2048 blocks; below 3 Mi rows in all, one per 1024 rows
     // and at most 1024 blocks (8 x 131072 rows: 5.5 us against 7.1 us)
+    if (plan_dense_keys(n_units, n_rows, nullptr)) {
+        const int64_t blocks = (int64_t)n_units * (((int64_t)n_rows + kKeyClassRows - 1) / kKeyClassRows);
+        hipLaunchKernelGGL(key_classify_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, w.hist, w.state, w.surv, w.cand_key,
+                           w.cand_idx, idx_out, idx_unit_stride, sel_keys, n_units, n_rows, k_eff, mode);
+        DC_CHECK_LAUNCH(who);
+        return launch_finish(who, w, idx_out, idx_unit_stride, n_units, n_rows, k_eff, mode, order, reinit, st);
+    }
     const bool few = (int64_t)n_units * n_rows < (3ll << 20);
     int nblk = few ? (n_rows + 1023) / 1024 : (n_rows + 4095) / 4096;
     const int grid = few ? 1024 : 2048;
