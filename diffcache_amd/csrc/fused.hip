@@ -585,7 +585,7 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
 // dense sketch scan it leaves every key's bucket at the key's own place, and the histogram.  Nothing is polled, listed
 // or handed over before the block's end.
 //
-// Bound by instruction issue and HBM together (some 130 vector instructions per 64 keys, 32 of them the additions, 32 the
+// Bound by instruction issue and HBM together (some 118 vector instructions per 64 keys, 32 of them the additions, 32 the
 // addresses of the tables; 268 MB of codes in 46 us = 5.8 TB/s).  8 x 1048576 codes of 32 bytes: 46 us.  Listed, in blocks of
 // 4096 keys, half of a block's life went into staging the tables and closing (76 us; 70 with the wide tables, sixteen
 // waves per block).  One block of 1024 threads per CU: two 46.2, four 51; three steps of codes ahead 48.9, one 47.6;
