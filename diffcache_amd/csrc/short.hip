@@ -517,16 +517,18 @@ bool dc_short_supported(const dc_layer_args *a, int region, int k_eff) {
 // 22.8 / 19.0; 8 x 4028 19.2 / 17.3, x 16316 30.4 / 21.9, x 32533 35.1 / 30.1 / 28.4; 64 x 4028 32.2 / 28.4; 8 x 16323 of 64 33.1 / 19.2;
 // 32 x 16316 44.7 / - / 35.8; 12 x 24615 of 256 51.0 / - / 40.3; 8 x 39932 of 128 39.5 / - / 31.4 (with the longer sketch chain of
 // then).  What is left to it: groups too large for this chain's attention, as long as it takes less than the sketch
-// chain (8 x 4028 of 256 22.5 / - / 31.6, x 16316 38.7 / - / 33.0).  Two units of more than 16 Ki rows, callers
+// chain (8 x 4028 of 256 22.5 / - / 31.6, x 16316 38.7 / - / 33.0).  Without one the chain behind this one scans the bf16
+// keys and is the faster one too since its scan is dense (one kernel / bf16 chain: 8 x 39932 37.5 / 34.1, x 81900 55.8 / 47.2, 4 x
+// 163000 60.1 / 47.4, 16 x 20100 36.2 / 35.2; 16 x 39932 of 64 36.9 / 33.3; 16 x 20100 of 256 51.3 / 51.4, x 39932 79.9 / 75.6; eight
+// heads to a unit of 256, 4 x 12500 36.0 / 29.6, 32 x 16316 83.7 / 74.2).  At most two units of more than 16 Ki rows, callers
 // without a sketch up to 12 Ki rows or two units, and callers who vouch for an exclusive GPU stay with it all the same:
 // that is the route they are told of (dc_decode_layer_route) and rely on.
 bool dc_one_kernel_first(const dc_layer_args *a, int region, int k_eff) {
     const int64_t n_units = (int64_t)a->n_b * a->n_h;
-    const bool short_ok = dc_short_supported(a, region, k_eff);
     if (a->one_kernel == DC_ONE_KERNEL_EXCLUSIVE) return true;
-    if (!a->sketch_codes) return !short_ok || n_units <= 2 || region <= 12 * 1024;
+    if (!a->sketch_codes) return n_units <= 2 || region <= 12 * 1024;
     if (n_units <= 2 && region > 16 * 1024) return true;
-    return !short_ok && region <= 16 * 1024 && n_units * region * a->hd * 2 <= (32ll << 20);
+    return !dc_short_supported(a, region, k_eff) && region <= 16 * 1024 && n_units * region * a->hd * 2 <= (32ll << 20);
 }
 
 // The layer on `stream`.  sel_ws: the select part of the workspace, its histograms zero (and left so).

@@ -445,8 +445,8 @@ int dc_decode_layer_step(const dc_layer_args *args, const dc_step_args *step, vo
  * unit), dc_decode_layer can run the layer as ONE kernel whose blocks are all resident
  * (two per CU) and hand their phases over through the workspace (same results; the event pair
  * then brackets that kernel).  It does so with DC_ONE_KERNEL_EXCLUSIVE; for callers without a sketch, up to 12 Ki rows per
- * unit or two units, or where the chain of three does not apply; with a sketch, for two units of more than 16 Ki
- * rows, and for large groups of query heads up to 32 MiB of keys. No counterpart in the reference, whose layers run on the CPU pool
+ * unit or at most two units; with a sketch, for at most two units of more than 16 Ki
+ * rows each, and for large groups of query heads up to 32 MiB of keys. No counterpart in the reference, whose layers run on the CPU pool
  * (lib.rs:352-369); what it has to match is that one layer call is always right
  * (src/diffcache/base.py:150-155).
  *

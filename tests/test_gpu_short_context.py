@@ -169,7 +169,7 @@ def test_which_calls_run_as_one_kernel():
     one, chain, stream = hip.ROUTE_ONE_KERNEL, hip.ROUTE_SKETCH, hip.ROUTE_STREAM
     assert [route(8, n) for n in (4028, 16384, 32768, 40960)] == [chain] * 4
     assert [route(2, n) for n in (4028, 16384, 16385, 40960, 40961)] == [chain, chain, one, one, chain]
-    assert [route(8, n, sketch=None) for n in (4028, 12288, 12289, 32768, 40960)] == [one, one, stream, stream, one]
+    assert [route(8, n, sketch=None) for n in (4028, 12288, 12289, 32768, 40960)] == [one, one, stream, stream, stream]
     assert [route(2, n, sketch=None) for n in (4028, 40960)] == [one, one]
     assert [route(8, n, policy=hip.ONE_KERNEL_EXCLUSIVE) for n in (4028, 32768)] == [one, one]
     assert route(8, 4028, policy=hip.ONE_KERNEL_NEVER) == chain and route(8, 4028, region_hi_dev=0x1000) == chain
