@@ -1,5 +1,5 @@
 """The dense sketch scan (up to 4 Mi rows over all units: a bucket for every row at the row's own place, read back by the
-exact pass in tiles of 2048 rows): the edges of its blocks' shares and of those tiles, live ends in front of them,
+exact pass in tiles of 2048 rows): the edges of its blocks' shares and of those tiles,
 candidates that all sit in one tile.  Ids, best first, against oracle.topk_select of the GPU's dense scores
 (nsw.rs:592-630)."""
 import numpy as np
