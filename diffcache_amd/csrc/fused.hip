@@ -1408,9 +1408,9 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
 // and the two bytes a row outweigh the list: 64 x 131004 225.8 / 237.7, 8 x 1048508 221.7 / 235.3.
 constexpr int64_t kDenseMostTiles = (4ll << 20) / kRowsPerBlockStep;
 
-// The grid of a dense scan: `most` blocks at the very most, so that none starts when the others end.  (Shares worked out from
-// all tiles together gave a few blocks more where the tiles of a unit did not divide: 24 units x 65000 rows of 256 columns 106
-// against 94 us, 56 x 30011 of 128 68.1 against 65.5.)
+// The grid of a dense scan of at least one unit and one tile: `most` blocks at the very most (one per unit where there are more
+// units), so that none starts when the others end.  (Shares worked out from all tiles together gave a few blocks more where the
+// tiles of a unit did not divide: 24 units x 65000 rows of 256 columns 106 against 94 us, 56 x 30011 of 128 68.1 against 65.5.)
 void plan_shares(int64_t n_units, int64_t tiles, int64_t most, FusedPlan *p) {
     const int64_t each = most > n_units ? most / n_units : 1, steps = (tiles + each - 1) / each;
     p->small_chunks = 0;
@@ -1628,8 +1628,8 @@ int dc_sketch_scan_launch(const char *who, const void *k, const uint8_t *codes, 
     FusedPlan p;
     int rc = plan_fused(who, n_b, n_h, n_rows, budget, &p, kBigSteps, kRowsPerBlockStep, kSketchFillBlocks);
     if (rc) return rc;
-    const bool dense = plan_dense(p.n_units, n_rows, hd, &p);
     if (p.n_units == 0 || p.k_eff == 0) return DC_OK;
+    const bool dense = plan_dense(p.n_units, n_rows, hd, &p);
     DC_REQUIRE(workspace && (((uintptr_t)workspace) & 255u) == 0,
                "%s: workspace must be non-null and 256-byte aligned", who);
     const FusedWs w = carve_fused(workspace, p.n_units, n_rows, budget);

@@ -190,6 +190,29 @@ def test_invalid_arguments_of_the_pq_search_entry_point():
     assert lib.dc_pq_search_workspace_bytes(8, 1000, 64) > lib.dc_score_select_workspace_bytes(8, 1000, 64)
 
 
+@pytest.mark.parametrize("n_b,n_rows,budget", [(0, 100, 8), (1, 0, 8), (1, 100, 0), (0, 0, 0)])
+def test_empty_selections_return_before_any_launch(n_b, n_rows, budget):
+    """No units, no rows or nothing wanted is DC_OK from every entry point that selects.  In a process of its own: what
+    the grids are worked out from is zero here, and a division by it would end the process."""
+    code = f"""
+import ctypes
+from diffcache_amd import _hip
+lib = _hip.lib
+buf = (ctypes.c_char * 8192)()
+p = (ctypes.addressof(buf) + 255) // 256 * 256
+for hd in (64, 128, 256):
+    assert lib.dc_score_select_sketch_bf16(p, p, p, p, p, p, 8, {n_b}, 1, {n_rows}, hd, 0, 0, hd, 0, 0, hd, 1, {budget}, 1, 0, 0, p,
+                                           4096, None, None, None) == 0
+    assert lib.dc_score_prune_bf16(p, p, {n_b}, 1, {n_rows}, hd, 0, 0, hd, 1, {budget}, 1, p, 4096, None) == 0
+    assert lib.dc_sparse_select(p, 8, {n_b}, {n_rows}, {budget}, 1, 0, 0, p, 4096, None) == 0
+    assert lib.dc_pq_search_bf16(p, p, p, p, p, 8, {n_b}, 1, {n_rows}, hd, 32, 0, 0, hd, {budget}, {budget}, 0, p, 4096, None,
+                                 None, None) == 0
+print("all there")
+"""
+    res = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert res.returncode == 0 and "all there" in res.stdout, (res.returncode, res.stderr[-500:])
+
+
 def test_c_data_layer_handle_bookkeeping_and_errors():
     """dc_data_layer_*: the host-side mirror of lib.rs:189-404 as a C handle; everything that
     needs no GPU (creation, sizes, argument checks)."""
