@@ -23,10 +23,10 @@ struct UnitState {
     uint32_t tb_run;    // running threshold bucket (only decreases)
     uint32_t sync_cnt;  // one-kernel route (small.hip): arrivals of the unit's blocks at its barriers; zero between launches
     uint32_t pad0[30];
-    uint32_t surv_cnt;  // survivors appended so far
+    uint32_t surv_cnt;  // survivors appended so far (a scan's result, like the histogram: it may be selected from again)
+    uint32_t c_less;    // keys in buckets better than the threshold bucket
     uint32_t win_cnt;   // certain members written to idx_out (select phase)
     uint32_t cand_cnt;  // candidates of the threshold bucket (select phase)
-    uint32_t c_less;    // keys in buckets better than the threshold bucket
     uint32_t margin;    // sketch scan only: float bits of the score margin of the unit
     // the one-kernel route for short contexts (small.hip)
     uint32_t sync_err;  // a bounded wait ran out (never expected)

@@ -667,7 +667,7 @@ __global__ __launch_bounds__(kPqThreads, 4) void pq_scan_kernel(
 // members, keys in it become candidates, whose scores are worked out once more (the additions of pq_adc_score).  A block
 // takes kPqClassRows keys and reserves its places in both lists with one returning atomic.
 constexpr int kPqClassRows = 8192;
-static_assert(offsetof(UnitState, win_cnt) == offsetof(UnitState, surv_cnt) + 4 && offsetof(UnitState, surv_cnt) % 8 == 0, "one word");
+static_assert(offsetof(UnitState, cand_cnt) == offsetof(UnitState, win_cnt) + 4 && offsetof(UnitState, win_cnt) % 8 == 0, "one word");
 
 template <int M>
 __global__ __launch_bounds__(kThreads) void pq_classify_kernel(
@@ -695,10 +695,7 @@ __global__ __launch_bounds__(kThreads) void pq_classify_kernel(
     const uint32_t kk = (uint32_t)k_eff;
     uint32_t tb, c_less;
     unit_threshold(hist + (int64_t)unit * DC_HIST_BINS, kk, wtot, sres, tb, c_less);
-    if (blk == 0 && tid == 0) {
-        st->c_less = c_less;
-        st->cand_cnt = tb < (uint32_t)DC_HIST_BINS ? hist[(int64_t)unit * DC_HIST_BINS + tb] : 0u;  // every key is counted
-    }
+    if (blk == 0 && tid == 0) st->c_less = c_less;
     uint32_t sure = 0, cand = 0;  // a bit per key
     static_assert(kVec * 8 <= 32, "bits of a thread's keys");
 #pragma unroll
@@ -719,9 +716,9 @@ __global__ __launch_bounds__(kThreads) void pq_classify_kernel(
     // the other, 128 of them per unit at a million keys)
     if (tid == 0) {
         unsigned long long at = 0ull;
-        if (tot) at = atomicAdd(reinterpret_cast<unsigned long long *>(&st->surv_cnt), (unsigned long long)n_sure << 32 | n_cand);
-        sbase[0] = (uint32_t)(at >> 32);
-        sbase[1] = (uint32_t)at;
+        if (tot) at = atomicAdd(reinterpret_cast<unsigned long long *>(&st->win_cnt), (unsigned long long)n_cand << 32 | n_sure);
+        sbase[0] = (uint32_t)at;
+        sbase[1] = (uint32_t)(at >> 32);
     }
     auto list = [&](uint32_t bits, uint32_t at, uint16_t *dst) __attribute__((always_inline)) {
         while (bits) {
@@ -884,10 +881,7 @@ __global__ __launch_bounds__(kThreads) void key_classify_kernel(
     const uint32_t kk = (uint32_t)k_eff;
     uint32_t tb, c_less;
     unit_threshold(hist + (int64_t)unit * DC_HIST_BINS, kk, wtot, sres, tb, c_less);
-    if (blk == 0 && tid == 0) {
-        st->c_less = c_less;
-        st->cand_cnt = tb < (uint32_t)DC_HIST_BINS ? hist[(int64_t)unit * DC_HIST_BINS + tb] : 0u;  // every row is counted
-    }
+    if (blk == 0 && tid == 0) st->c_less = c_less;
     uint32_t sure = 0, cand = 0;  // a bit per row
 #pragma unroll
     for (int j = 0; j < 4 * kVec; ++j) {
@@ -900,9 +894,9 @@ __global__ __launch_bounds__(kThreads) void key_classify_kernel(
     const uint32_t ex = block_excl_scan<kThreads>(__popc(sure) | __popc(cand) << 16, wtot, &tot);
     if (tid == 0) {
         unsigned long long at = 0ull;
-        if (tot) at = atomicAdd(reinterpret_cast<unsigned long long *>(&st->surv_cnt), (unsigned long long)(tot & 0xffffu) << 32 | tot >> 16);
-        sbase[0] = (uint32_t)(at >> 32);
-        sbase[1] = (uint32_t)at;
+        if (tot) at = atomicAdd(reinterpret_cast<unsigned long long *>(&st->win_cnt), (unsigned long long)(tot >> 16) << 32 | (tot & 0xffffu));
+        sbase[0] = (uint32_t)at;
+        sbase[1] = (uint32_t)(at >> 32);
     }
     __syncthreads();
     uint32_t wpos = sbase[0] + (ex & 0xffffu), cpos = sbase[1] + (ex >> 16);

@@ -114,6 +114,8 @@ int dc_topk_select(const float *scores, int64_t scores_unit_stride, uint32_t *id
  *                          it also leaves the workspace as dc_select_state_init does, so
  *                          the next dc_score_prune_bf16 of the same sizes on it needs no
  *                          init call
+ *                          (with reinit == 0 the same scan may be selected from again,
+ *                          with any budget up to the scan's)
  * Replaces the same reference code as the two calls it stands for
  * (diffcache_cpu/src/nsw.rs:129-139,600-621).
  */
