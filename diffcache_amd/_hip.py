@@ -764,17 +764,21 @@ class LayerStep:
         key, again, self._again = None, self._again, True
         if again and scores is None and lse is None and scan_events is None and append is not None:
             key = (store_k.data_ptr(), store_k.shape, store_k.stride(), store_k.dtype, store_v.data_ptr(), store_v.stride(),
-                   store_v.dtype, idx_out.data_ptr(), idx_out.shape, idx_out.stride(), workspace.data_ptr(),
-                   workspace.numel(), n_sink, recent_lo, n_recent, budget, mode, order, scale, n, append[0], append[2])
+                   store_v.dtype, idx_out.data_ptr(), idx_out.shape, idx_out.stride(), idx_out.dtype, workspace.data_ptr(),
+                   workspace.numel(), n_sink, recent_lo, n_recent, budget, mode, order, scale, n, append[0], append[2],
+                   append[1] is n_recent_dev)
             if sketch is not None:
                 c = sketch.codes
                 key += (c.data_ptr(), c.shape, c.stride(), sketch.scale.data_ptr(), sketch.resid.data_ptr())
             pos_dev = append[1]
+            # (the window's counter as the append position is looked at once, and the key says so: no counter is another call)
             for t in (n_recent_dev, region_hi_dev, None if pos_dev is n_recent_dev else pos_dev, advance and advance[0]):
                 if t is not None:
                     key += (t.data_ptr(), t.numel(), t.dtype)
                 else:
                     key += (None,)
+            if advance is not None:
+                key += (advance[0].stride(),)
         s = self._step
         if key is None or key != self._key:
             self._key = None

@@ -54,3 +54,25 @@ def test_a_kept_layer_follows_its_tensors(with_sketch):
     with pytest.raises(hip.DiffCacheError):
         hip.decode_layer(q, ks, wide[..., :hd], *good[3:], **args)
     torch.cuda.synchronize()
+
+
+def test_a_kept_layer_tells_the_append_positions_apart():
+    """The token's row at pos + the window's counter, at pos + another counter, at pos alone: in any order, one LayerStep."""
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(32)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV).to(torch.bfloat16)
+    b, h, group, hd, n, sink, cap, budget = 1, 2, 2, 64, 1000, 4, 8, 96
+    hi = n - cap
+    ws = hip.alloc_workspace(hip.layer_workspace_bytes(b * h, hi - sink, budget, group, hd, budget + sink + cap + 1), DEV)
+    words = torch.tensor([2, 5], device=DEV, dtype=torch.int32)
+    window, other = words[0:1], words[1:2]
+    q, ks, vs = rnd(b, h * group, hd), rnd(b, h, n, hd), rnd(b, h, n, hd)
+    idx, out = torch.zeros((b * h, budget), device=DEV, dtype=torch.int32), torch.zeros((b, h * group, hd), device=DEV, dtype=torch.bfloat16)
+    kept = hip.LayerStep()
+    for pos_dev, row in ((window, 2), (window, 2), (None, 0), (None, 0), (window, 2), (other, 5), (None, 0), (other, 5), (window, 2)):
+        nk, nv, want_k, want_v = rnd(b, h, hd), rnd(b, h, hd), ks.clone(), vs.clone()
+        want_k[:, :, hi + row], want_v[:, :, hi + row] = nk, nv
+        hip.decode_layer(q, ks, vs, sink, hi, cap, budget, None, idx, out, ws, nk, nv, n_recent_dev=window,
+                         append=(hi, pos_dev, hi + cap), kept=kept)
+        torch.cuda.synchronize()
+        assert torch.equal(ks, want_k) and torch.equal(vs, want_v), row
