@@ -931,11 +931,9 @@ __global__ __launch_bounds__(kThreads) void key_classify_kernel(
 // holds every member of the top-k).
 constexpr int kRescoreBatch = 4;
 
-// DENSE: the scan left a bucket for every row (sketch_prune_kernel); a block takes kDensePer rows of a thread at a time, side
-// by side, and the tiles of a unit are dealt to its blocks as they come.
-constexpr int kDensePer = 8;
-
-template <int HD, bool DENSE>
+// PER > 0: the scan left a bucket for every row (sketch_prune_kernel); a block takes PER rows of a thread at a time, side
+// by side, and the tiles of a unit are dealt to its blocks as they come (dense_per_thread).  PER == 0: the list.
+template <int HD, int PER>
 __global__ __launch_bounds__(kThreads) void rescore_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, const uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, const uint2 *__restrict__ surv, uint32_t *__restrict__ cand_key,
@@ -943,7 +941,8 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
     int64_t sr, int q_group, int mode, int k_eff, int nblk, const int32_t *__restrict__ hi_dev, int lo_row) {
     constexpr int LPR = HD / 8;
     constexpr int GROUPS = kThreads / LPR;
-    constexpr int kOwn = DENSE ? kDensePer : kRescoreBatch;  // entries of a thread per batch
+    constexpr bool DENSE = PER > 0;
+    constexpr int kOwn = DENSE ? PER : kRescoreBatch;  // entries of a thread per batch
     constexpr uint32_t kPer = kOwn * kThreads;
     __shared__ uint32_t cid[kPer];
     __shared__ uint32_t ckey[kPer];
@@ -971,10 +970,18 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
     const uint16_t *du = reinterpret_cast<const uint16_t *>(surv) + (int64_t)unit * dense_stride(n_rows);
     uint32_t p[4];
     auto load_dense = [&](uint32_t t) __attribute__((always_inline)) {
-        const uint32_t i = (((uint32_t)blk + t * (uint32_t)nblk) * kThreads + (uint32_t)tid) * kDensePer;
-        uint4 v = make_uint4(~0u, ~0u, ~0u, ~0u);
-        if (i < (uint32_t)n_rows) v = *reinterpret_cast<const uint4 *>(du + i);
-        p[0] = v.x, p[1] = v.y, p[2] = v.z, p[3] = v.w;
+        const uint32_t i = (((uint32_t)blk + t * (uint32_t)nblk) * kThreads + (uint32_t)tid) * PER;
+        p[0] = p[1] = p[2] = p[3] = ~0u;
+        if (i >= (uint32_t)n_rows) return;
+        if constexpr (PER == 8) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(du + i);
+            p[0] = v.x, p[1] = v.y, p[2] = v.z, p[3] = v.w;
+        } else if constexpr (PER == 4) {
+            const uint2 v = *reinterpret_cast<const uint2 *>(du + i);
+            p[0] = v.x, p[1] = v.y;
+        } else {
+            p[0] = *reinterpret_cast<const uint32_t *>(du + i);
+        }
     };
     uint32_t n_s;
     if constexpr (DENSE) {
@@ -1005,11 +1012,11 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
 
     for (uint32_t t0 = 0; t0 < my_tiles; t0 += DENSE ? 1 : kRescoreBatch) {
         uint32_t pass = 0;
-        const uint32_t row0 = (((uint32_t)blk + t0 * (uint32_t)nblk) * kThreads + (uint32_t)tid) * kDensePer;  // DENSE
+        const uint32_t row0 = (((uint32_t)blk + t0 * (uint32_t)nblk) * kThreads + (uint32_t)tid) * PER;  // DENSE
         if constexpr (DENSE) {
             if (t0 != 0) load_dense(t0);
 #pragma unroll
-            for (int j = 0; j < kDensePer; ++j) {
+            for (int j = 0; j < PER; ++j) {
                 const uint32_t kb = j & 1 ? p[j / 2] >> 16 : p[j / 2] & 0xffffu;
                 if (row0 + j < n_s && kb <= tb) pass |= 1u << j;
             }
@@ -1419,6 +1426,19 @@ bool plan_dense(int64_t n_units, int n_rows, int hd, FusedPlan *p) {
     return true;
 }
 
+// Rows of a thread per tile of the exact pass of a dense scan: tiles of 512, 1024 or 2048 rows.  What a block scores one after
+// the other is its tiles' candidates, so short regions, and those of which much is selected, take small tiles on many
+// blocks; where every CU has work either way, a tile costs its barriers and its slot reservation.  Per selection, us, 512 / 1024 /
+// 2048: 8 units x 8000 rows of 256 columns, 2048 ids 20.2 / 24.0 / 31.8, 1 x 16000 17.1 / 19.1 / 22.5, 32 x 8000 30.6 / 32.4 /
+// 39.8, 8 x 60000 34.4 / 35.1 / 36.3, 8 x 131004 58.7 / 57.9 / 58.0, 8 x 262144 108.0 / 103.4 / 101.7; 64 x 16000 of 64, 64 ids 24.6 / 22.8 /
+// 22.3.
+// (The listed scan, which dealt its list out in pieces of 256 to one block per 1024 rows, took 26.1 in the first of these.)
+int dense_per_thread(int64_t n_units, int n_rows) {
+    const int64_t all = n_units * n_rows;
+    if (n_rows <= 32 * 1024 && all <= 384 * 1024) return 2;
+    return n_rows <= 96 * 1024 && all <= 1024 * 1024 ? 4 : 8;
+}
+
 // The same for the bf16 scan, whose rows take twice the bytes and leave four of them: two blocks per CU.  Per layer, us,
 // listed / dense: 32 units x 49933 rows of 128 columns 101 / 95, 24 x 70000 100.3 / 95, 12 x 130001 95 / 89.6, 20 x 77771
 // 98.5 / 91, 8 x 81852 53.0 / 49.3, 8 x 45000 39.0 / 35.9, 2 x 131004 40.0 / 35.3, 4 x 524000 125.6 / 111.4; 24 x 65000 of 64 59.2 /
@@ -1700,25 +1720,27 @@ int dc_sketch_select_impl(const void *k, const uint8_t *codes, const float *scal
     const int cap = p.n_units >= grid ? 1 : grid / p.n_units;
     if (nblk > cap) nblk = cap;
     if (nblk < 1) nblk = 1;
-    const bool dense = plan_dense(p.n_units, n_rows, hd, nullptr);
-    if (dense) {
-        const int tiles = (n_rows + kThreads * kDensePer - 1) / (kThreads * kDensePer);
-        if (nblk > tiles) nblk = tiles;
+    const int per = plan_dense(p.n_units, n_rows, hd, nullptr) ? dense_per_thread(p.n_units, n_rows) : 0;
+    if (per) {
+        const int tiles = (n_rows + kThreads * per - 1) / (kThreads * per);
+        nblk = tiles < cap ? tiles : cap;
     }
-#define DC_LAUNCH_RSD(HD, DN)                                                                         \
-    hipLaunchKernelGGL((rescore_kernel<HD, DN>), dim3((unsigned)p.n_units * (unsigned)nblk), dim3(kThreads), 0, \
+#define DC_LAUNCH_RSP(HD, PER)                                                                        \
+    hipLaunchKernelGGL((rescore_kernel<HD, PER>), dim3((unsigned)p.n_units * (unsigned)nblk), dim3(kThreads), 0, \
                        st, (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv, w.cand_key, \
                        w.cand_idx, p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, nblk, hi_dev, lo_row)
-#define DC_LAUNCH_RS(HD)                     \
-    do {                                     \
-        if (dense) DC_LAUNCH_RSD(HD, true);  \
-        else DC_LAUNCH_RSD(HD, false);       \
+#define DC_LAUNCH_RS(HD)                        \
+    do {                                        \
+        if (per == 2) DC_LAUNCH_RSP(HD, 2);     \
+        else if (per == 4) DC_LAUNCH_RSP(HD, 4); \
+        else if (per == 8) DC_LAUNCH_RSP(HD, 8); \
+        else DC_LAUNCH_RSP(HD, 0);              \
     } while (0)
     if (hd == 64) DC_LAUNCH_RS(64);
     else if (hd == 128) DC_LAUNCH_RS(128);
     else DC_LAUNCH_RS(256);
 #undef DC_LAUNCH_RS
-#undef DC_LAUNCH_RSD
+#undef DC_LAUNCH_RSP
     DC_CHECK_LAUNCH(who);
     return launch_finish(who, w, idx_out, idx_unit_stride, p.n_units, n_rows, p.k_eff, mode, order, 1, st);
 }

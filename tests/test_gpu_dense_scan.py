@@ -36,3 +36,31 @@ def test_dense_scan_is_exact_at_its_edges(hd, hkv, region):
                 ids = ids.cpu().numpy()
                 for u in range(hkv):
                     assert np.array_equal(ids[u], orc.topk_select(dense[u], k_eff, mode)), (law, mode, budget, ready, u)
+
+
+# tiles of 512 rows up to 32 Ki rows a unit and 384 Ki in all, of 1024 up to 96 Ki and 1 Mi, of 2048 beyond
+@pytest.mark.parametrize("hd,hkv,region", [(64, 3, 511), (128, 2, 513), (256, 2, 1025), (256, 1, 32768), (128, 1, 32769), (64, 2, 98304),
+                                           (64, 1, 98305), (64, 24, 16384), (64, 24, 16385), (64, 16, 65536), (64, 16, 65537)])
+def test_tiles_of_every_size_are_exact_at_their_edges(hd, hkv, region):
+    test_dense_scan_is_exact_at_its_edges(hd, hkv, region)
+
+
+@pytest.mark.parametrize("hkv,cap", [(3, 9001), (24, 20483)])
+def test_the_live_end_cuts_a_tile_of_any_size(hkv, cap):
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(cap)
+    hd, budget, sink = 64, 300, 4
+    k = torch.randn((1, hkv, sink + cap, hd), generator=g, device=DEV).to(torch.bfloat16)
+    q = torch.randn((1, hkv, hd), generator=g, device=DEV).to(torch.bfloat16)
+    sk = hip.Sketch(k).build(k, sink, cap)
+    ws = hip.alloc_workspace(hip.layer_workspace_bytes(hkv, cap, budget, 1, hd, budget + sink), DEV)
+    state = torch.zeros((4,), device=DEV, dtype=torch.int32)
+    for i, region in enumerate((cap, cap - 1, 8193, 8192, 4097, 1025, 513, 512, 303, 300, cap)):
+        state[1:2].fill_(sink + region)
+        idx = torch.full((hkv, budget), -1, device=DEV, dtype=torch.int32)
+        hip.decode_layer(q, k, k, sink, sink + cap, 0, budget, None, idx, torch.empty_like(q), ws, mode=0, order=hip.ORDER_BEST,
+                         one_kernel=hip.ONE_KERNEL_NEVER, select_state_ready=i > 0, sketch=sk,
+                         n_recent_dev=state[0:1], region_hi_dev=state[1:2])
+        dense = hip.score(k, q.view(hkv, hd), sink, region, 0).cpu().numpy()
+        for u in range(0, hkv, 1 + hkv // 4):
+            assert np.array_equal(idx[u].cpu().numpy(), orc.topk_select(dense[u], budget, 0)), (region, u)
