@@ -1403,11 +1403,15 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
 }
 
 // Whether the sketch scan of these sizes is a dense one, and its grid: blocks of equal shares, all running at once
-// (four per CU at 64 columns, three at 128, two at 256).  Per layer, us, listed / dense: 8 units x 131004 rows of 128 columns
-// 48.9 / 45.1, x 65468 38.5 / 35.5, 16 x 131004 75.0 / 69.5, 32 x 131004 125.4 / 121.5, 4 x 1048508 135.5 / 121.8, 128 x 32700 138.6 /
-// 135; 8 x 131004 of 64 38.4 / 32.0, 12 x 24615 of 256 44.7 / 41.4.  Beyond 4 Mi rows in all equal shares end at unequal times
-// and the two bytes a row outweigh the list: 64 x 131004 225.8 / 237.7, 8 x 1048508 221.7 / 235.3.
-constexpr int64_t kDenseMostTiles = (4ll << 20) / kRowsPerBlockStep;
+// (four per CU at 64 columns, three at 128, two at 256; 256 per unit at most, because every block adds its counts to the unit's
+// one histogram: 1 x 262107 of 64 columns 30.2 us with 1024 blocks, 20.1 with 256; listed 27.3).  Per layer, us, listed / dense: 8
+// units x 131004 rows of 128 columns 48.9 / 45.1, x 65468 38.5 / 35.5, 16 x 131004 75.0 / 69.5, 32 x 131004 125.4 / 121.5, 4 x 1048508
+// 135.5 / 121.8, 128 x 32700 138.6 / 135; 8 x 131004 of 64 38.4 / 32.0, 12 x 24615 of 256 44.7 / 41.4.  Beyond 4 Mi rows in all
+// equal shares end at unequal times and the two bytes a row outweigh the list: 64 x 131004 225.8 / 237.7, 8 x 1048508 221.7 /
+// 235.3.  From 128 columns on that shows from 2.5 Mi rows on where few rows are selected and the list is short: the selection
+// alone, 64 x 65420 of 128, 64 ids 97.9 / 105.0, 1024 ids 107.2 / 107.4, 4096 ids 128.8 / 123.3; 32 x 130878 of 256, 64 ids 174.5 /
+// 184.5, 2048 ids 197.3 / 195.8; but 24 x 109189 of 128, 64 ids 67.6 / 66.7, and 64 x 65420 of 64, 64 ids 61.7 / 62.8.
+constexpr int64_t kDenseMostTiles = (4ll << 20) / kRowsPerBlockStep, kDenseFewTiles = (5ll << 19) / kRowsPerBlockStep;
 
 // The grid of a dense scan of at least one unit and one tile: `most` blocks at the very most (one per unit where there are more
 // units), so that none starts when the others end.  (Shares worked out from all tiles together gave a few blocks more where the
@@ -1419,10 +1423,11 @@ void plan_shares(int64_t n_units, int64_t tiles, int64_t most, FusedPlan *p) {
     p->blocks = n_units * ((tiles + steps - 1) / steps);
 }
 
-bool plan_dense(int64_t n_units, int n_rows, int hd, FusedPlan *p) {
+bool plan_dense(int64_t n_units, int n_rows, int hd, int k_eff, FusedPlan *p) {
     const int64_t tiles = ((int64_t)n_rows + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
-    if (n_units * tiles > kDenseMostTiles) return false;
-    if (p) plan_shares(n_units, tiles, 256 * (hd == 64 ? 4 : (hd == 128 ? 3 : 2)), p);
+    if (n_units * tiles > (hd == 64 || k_eff >= 8 * hd ? kDenseMostTiles : kDenseFewTiles)) return false;
+    const int64_t most = 256 * (hd == 64 ? 4 : (hd == 128 ? 3 : 2));
+    if (p) plan_shares(n_units, tiles, most < 256 * n_units ? most : 256 * n_units, p);
     return true;
 }
 
@@ -1643,7 +1648,7 @@ int dc_sketch_scan_launch(const char *who, const void *k, const uint8_t *codes, 
     int rc = plan_fused(who, n_b, n_h, n_rows, budget, &p, kBigSteps, kRowsPerBlockStep, kSketchFillBlocks);
     if (rc) return rc;
     if (p.n_units == 0 || p.k_eff == 0) return DC_OK;
-    const bool dense = plan_dense(p.n_units, n_rows, hd, &p);
+    const bool dense = plan_dense(p.n_units, n_rows, hd, p.k_eff, &p);
     DC_REQUIRE(workspace && (((uintptr_t)workspace) & 255u) == 0,
                "%s: workspace must be non-null and 256-byte aligned", who);
     const FusedWs w = carve_fused(workspace, p.n_units, n_rows, budget);
@@ -1720,7 +1725,7 @@ int dc_sketch_select_impl(const void *k, const uint8_t *codes, const float *scal
     const int cap = p.n_units >= grid ? 1 : grid / p.n_units;
     if (nblk > cap) nblk = cap;
     if (nblk < 1) nblk = 1;
-    const int per = plan_dense(p.n_units, n_rows, hd, nullptr) ? dense_per_thread(p.n_units, n_rows) : 0;
+    const int per = plan_dense(p.n_units, n_rows, hd, p.k_eff, nullptr) ? dense_per_thread(p.n_units, n_rows) : 0;
     if (per) {
         const int tiles = (n_rows + kThreads * per - 1) / (kThreads * per);
         nblk = tiles < cap ? tiles : cap;

@@ -64,3 +64,20 @@ def test_the_live_end_cuts_a_tile_of_any_size(hkv, cap):
         dense = hip.score(k, q.view(hkv, hd), sink, region, 0).cpu().numpy()
         for u in range(0, hkv, 1 + hkv // 4):
             assert np.array_equal(idx[u].cpu().numpy(), orc.topk_select(dense[u], budget, 0)), (region, u)
+
+
+# from 2.5 Mi rows in all on (128 columns) the scan lists its rows unless 1024 ids or more are selected
+@pytest.mark.parametrize("region,budget", [(655360, 64), (655361, 64), (655361, 1023), (655361, 1024)])
+def test_both_sides_of_the_line_for_few_ids(region, budget):
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(region + budget)
+    hkv, hd = 4, 128
+    k = torch.randn((1, hkv, region, hd), generator=g, device=DEV, dtype=torch.bfloat16)
+    q = torch.randn((hkv, hd), generator=g, device=DEV).to(torch.bfloat16)
+    sk = hip.Sketch(k).build(k, 0, region)
+    ws = hip.alloc_workspace(hip.sketch_select_workspace_bytes(hkv, region, budget), DEV)
+    dense = hip.score(k, q, 0, region, 0).cpu().numpy()
+    for ready in (False, True):
+        ids = hip.score_select_sketch(k, sk, q, 0, region, budget, 0, hip.ORDER_BEST, workspace=ws, state_ready=ready).cpu().numpy()
+        for u in range(hkv):
+            assert np.array_equal(ids[u], orc.topk_select(dense[u], budget, 0)), (ready, u)
