@@ -196,6 +196,14 @@ __device__ __forceinline__ uint32_t dc_score_bucket(float s) {
     return (kPosBuckets - 1u) - ((m - lo) >> (23u - kSubBits));
 }
 static_assert(kPosBuckets + 512u <= DC_HIST_BINS, "bucket map exceeds the histogram");
+// The same without a branch: for a lane that maps many scores in a row.
+__device__ __forceinline__ uint32_t dc_score_bucket_flat(float s) {
+    const uint32_t b = __float_as_uint(s + 0.0f), mag = b & 0x7fffffffu;
+    constexpr uint32_t lo = (127u - 20u) << 23, hi = ((127u - 20u + kPosBinades) << 23) - 1u;
+    const uint32_t m = mag < lo ? lo : (mag > hi ? hi : mag);
+    const uint32_t pos = (kPosBuckets - 1u) - ((m - lo) >> (23u - kSubBits)), neg = kPosBuckets + (mag >> 22);
+    return (b & 0x80000000u) ? neg : pos;
+}
 
 // 32-bit ordering key (smaller = better) and its histogram bucket.  The bucket is
 // a monotone function of the key, so equal keys share a bucket.

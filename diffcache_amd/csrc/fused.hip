@@ -136,8 +136,9 @@ constexpr uint32_t kNoRow = 0xffffffffu;  // in the place of a row's key: there 
 // words between the units of a dense scan's keys (16-byte rows of them)
 __host__ __device__ __forceinline__ int64_t dense_key_stride(int n_cap) { return ((int64_t)n_cap + 3) & ~3ll; }
 
-// DENSE: for scans of up to 1.75 Mi rows in all (plan_dense_keys), as in the sketch scan below: every row's 32-bit key goes to
-// the row's own place, nothing is polled, staged or listed, and blocks of equal shares all run at once.
+// DENSE: for scans of more than 768 rows a unit and up to 1.75 Mi in all (plan_dense_keys), as in the sketch scan below:
+// every row's 32-bit key goes to the row's own place, nothing is polled, staged or listed, and blocks of equal shares all
+// run at once.
 template <int HD, bool DENSE>
 __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, uint32_t *__restrict__ hist,
@@ -886,7 +887,7 @@ __global__ __launch_bounds__(kThreads) void key_classify_kernel(
 #pragma unroll
     for (int j = 0; j < 4 * kVec; ++j) {
         const float x = __uint_as_float((keys[j] & 0x80000000u) ? keys[j] & 0x7fffffffu : ~keys[j]);  // dc_f2ord, inverted
-        const uint32_t bucket = dc_score_bucket(mode == DC_MODE_REF_DIST ? 65536.0f - x : -x);
+        const uint32_t bucket = dc_score_bucket_flat(mode == DC_MODE_REF_DIST ? 65536.0f - x : -x);
         sure |= keys[j] != kNoRow && bucket < tb ? 1u << j : 0u;
         cand |= keys[j] != kNoRow && bucket == tb ? 1u << j : 0u;
     }
@@ -1447,14 +1448,25 @@ int dense_per_thread(int64_t n_units, int n_rows) {
 // The same for the bf16 scan, whose rows take twice the bytes and leave four of them: two blocks per CU.  Per layer, us,
 // listed / dense: 32 units x 49933 rows of 128 columns 101 / 95, 24 x 70000 100.3 / 95, 12 x 130001 95 / 89.6, 20 x 77771
 // 98.5 / 91, 8 x 81852 53.0 / 49.3, 8 x 45000 39.0 / 35.9, 2 x 131004 40.0 / 35.3, 4 x 524000 125.6 / 111.4; 24 x 65000 of 64 59.2 /
-// 55.4; 9 x 55555 of 256 71.3 / 68.8, 24 x 65000 153.3 / 154.  1024 blocks 98.6 in the first of these, 1280 94.5, 2048 96.2 (a CU
-// holds five).  Beyond it is as often slower: 16 x 131004 112.2 / 115.5, 32 x 100000 163.6 / 166.2, 32 x 131004 204.1 / 208.3.
+// 55.4; 9 x 55555 of 256 71.3 / 68.8.  Beyond 1.75 Mi rows it is as often slower: 16 x 131004 112.2 / 115.5, 32 x 100000 163.6 /
+// 166.2, 32 x 131004 204.1 / 208.3.  Up to 768 rows the listed scan's few blocks are the shorter chain (96 x 304 of 64 13.0 / 13.7).
+//
+// Its grid, selections alone, us: up to 640 tiles of 256 rows a block each (24 x 5424 of 128: 264 blocks of two tiles 19.7, 528
+// of one 18.3); then 512 blocks, 1024 from 64 units on (64 x 16000 of 128 59.0 / 56.5, listed 55.1).  Above 1 Mi rows, where
+// every share is long, 1280 blocks (a CU holds five) up to 32 units and 128 columns (16 x 100003 of 64 48.7 / 45.7, listed
+// 47.5), and at 256 columns from 9 to 64 units one per CU (32 x 50000 144.5 / 139.5, listed 139.0).
 constexpr int64_t kDenseKeyTiles = (7ll << 18) / kRowsPerBlockStep;  // 1.75 Mi rows
+constexpr int kDenseKeyRows = 768;
 
-bool plan_dense_keys(int64_t n_units, int n_rows, FusedPlan *p) {
+bool plan_dense_keys(int64_t n_units, int n_rows, int hd, FusedPlan *p) {
     const int64_t tiles = ((int64_t)n_rows + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
-    if (n_units * tiles > kDenseKeyTiles) return false;
-    if (p) plan_shares(n_units, tiles, 512, p);
+    if (n_rows <= kDenseKeyRows || n_units * tiles > kDenseKeyTiles) return false;
+    if (!p) return true;
+    const int64_t all = n_units * tiles;
+    int64_t most = all <= 640 ? all : (n_units < 64 ? 512 : 1024);
+    if (all > (1ll << 20) / kRowsPerBlockStep)
+        most = hd == 256 ? (n_units > 8 && n_units <= 64 ? 256 : 512) : (n_units <= 32 ? 1280 : 512);
+    plan_shares(n_units, tiles, most, p);
     return true;
 }
 
@@ -1515,7 +1527,7 @@ int dc_score_prune_launch(const void *k, const void *q, int n_b, int n_h, int n_
     FusedWs w;
     rc = check_ws("dc_score_prune_bf16", workspace, workspace_bytes, p.n_units, n_rows, budget, &w);
     if (rc) return rc;
-    const bool dense = plan_dense_keys(p.n_units, n_rows, &p);
+    const bool dense = plan_dense_keys(p.n_units, n_rows, hd, &p);
     hipStream_t st = (hipStream_t)stream;
 #define DC_LAUNCH_SPD(HD, DN)                                                                      \
     hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dim3((unsigned)p.blocks), dim3(kThreads), 0, st, \
@@ -1565,7 +1577,7 @@ int launch_select(const char *who, const FusedWs &w, uint32_t *idx_out, int64_t 
     // the grid stays near 2048 blocks
     // one block per 4096 rows and at most 2048 blocks; below 3 Mi rows in all, one per 1024 rows
     // and at most 1024 blocks (8 x 131072 rows: 5.5 us against 7.1 us)
-    if (plan_dense_keys(n_units, n_rows, nullptr)) {
+    if (plan_dense_keys(n_units, n_rows, 0, nullptr)) {
         const int64_t blocks = (int64_t)n_units * (((int64_t)n_rows + kKeyClassRows - 1) / kKeyClassRows);
         hipLaunchKernelGGL(key_classify_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, st, w.hist, w.state, w.surv, w.cand_key,
                            w.cand_idx, idx_out, idx_unit_stride, sel_keys, n_units, n_rows, k_eff, mode);

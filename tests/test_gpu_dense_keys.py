@@ -1,4 +1,4 @@
-"""The dense bf16 scan (up to 1.75 Mi rows over all units: a 32-bit key for every row at the row's own place, classified in
+"""The dense bf16 scan (from 769 rows a unit to 1.75 Mi over all units: a 32-bit key for every row at the row's own place, classified in
 tiles of 4096 rows): the edges of its blocks' shares and of those tiles, with ties, and live ends in front of the
 capacity, for the sketch's dense scan as well.  Ids against oracle.topk_select of the GPU's dense scores (nsw.rs:592-630)."""
 import numpy as np
@@ -74,3 +74,22 @@ def test_the_live_end_comes_from_the_device(sketch):
         dense = hip.score(k, q.view(hkv, hd), sink, region, 0).cpu().numpy()
         for u in range(hkv):
             assert np.array_equal(idx[u].cpu().numpy(), orc.topk_select(dense[u], budget, 0)), (region, u)
+
+
+# up to 768 rows a unit the scan lists its survivors; up to 640 tiles of 256 rows in all every tile is a block's; other grids
+# from 64 units on and above 1 Mi rows
+@pytest.mark.parametrize("hkv,region,hd", [(3, 768, 64), (3, 769, 128), (2, 1023, 256), (24, 5424, 64), (24, 7000, 64), (64, 2561, 64),
+                                           (33, 33000, 64), (16, 70001, 64), (9, 120001, 256)])
+def test_every_grid_scans_every_row(hkv, region, hd):
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(hkv + region)
+    k = torch.randint(-1, 2, (1, hkv, region, hd), generator=g, device=DEV, dtype=torch.int8).to(torch.bfloat16)
+    q = torch.randn((hkv, hd), generator=g, device=DEV).to(torch.bfloat16)
+    budget = min(region, 700)
+    ws = hip.alloc_workspace(hip.score_select_workspace_bytes(hkv, region, budget), DEV)
+    dense = hip.score(k, q, 0, region, 0)
+    for order in (hip.ORDER_BEST, hip.ORDER_ANY):
+        ids = hip.score_select(k, q, 0, region, budget, 0, order, workspace=ws).cpu().numpy()
+        for u in range(0, hkv, 1 + hkv // 5):
+            want, got = orc.topk_select(dense[u].cpu().numpy(), budget, 0), ids[u] if order == hip.ORDER_BEST else np.sort(ids[u])
+            assert np.array_equal(got, want if order == hip.ORDER_BEST else np.sort(want)), (order, u)
