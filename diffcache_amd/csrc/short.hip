@@ -512,23 +512,39 @@ bool dc_short_supported(const dc_layer_args *a, int region, int k_eff) {
            (a->recent_lo + a->n_recent + 1) * a->kv_row_stride * 2 <= 0xffffffffll;
 }
 
-// Whether a layer that can run as one kernel (small.hip) does.  With a sketch the chains are the faster ones at every
-// size measured (us, one kernel / this chain / sketch chain): 2 units x 4028 rows of 128 columns 18.1 / 15.4, x 16316
-// 22.8 / 19.0; 8 x 4028 19.2 / 17.3, x 16316 30.4 / 21.9, x 32533 35.1 / 30.1 / 28.4; 64 x 4028 32.2 / 28.4; 8 x 16323 of 64 33.1 / 19.2;
-// 32 x 16316 44.7 / - / 35.8; 12 x 24615 of 256 51.0 / - / 40.3; 8 x 39932 of 128 39.5 / - / 31.4 (with the longer sketch chain of
-// then).  What is left to it: groups too large for this chain's attention, as long as it takes less than the sketch
-// chain (8 x 4028 of 256 22.5 / - / 31.6, x 16316 38.7 / - / 33.0).  Without one the chain behind this one scans the bf16
-// keys and is the faster one too since its scan is dense (one kernel / bf16 chain: 8 x 39932 37.5 / 34.1, x 81900 55.8 / 47.2, 4 x
-// 163000 60.1 / 47.4, 16 x 20100 36.2 / 35.2; 16 x 39932 of 64 36.9 / 33.3; 16 x 20100 of 256 51.3 / 51.4, x 39932 79.9 / 75.6; eight
-// heads to a unit of 256, 4 x 12500 36.0 / 29.6, 32 x 16316 83.7 / 74.2).  At most two units of more than 16 Ki rows, callers
-// without a sketch up to 12 Ki rows or two units, and callers who vouch for an exclusive GPU stay with it all the same:
-// that is the route they are told of (dc_decode_layer_route) and rely on.
+// Whether a layer that can run as one kernel (small.hip) does.  What decides is the time (us, one kernel / chain, G query heads to
+// a unit, k ids).  The one kernel pays for every query head and every row of its serial phases; this chain pays for every split,
+// all of which count all keys of their unit (units x k / 128 of them); the sketch chain for every candidate it
+// scores again, and for two more kernels.
+//   G >= 4       the chains: 8 x 4028 of 128 columns 19.5 / 16.5, x 16316 30.3 / 22.0, x 32533 34.4 / 27.7; 64 x 4028 37.3 / 28.8; 8 x
+//                16316 of 64, G 8, 33.3 / 19.1; 12 x 24615 of 256 49.7 / 37.6; without a sketch 8 x 39932 36.9 / 33.7, 16 x 39932 of 64 34.9 / 32.7
+//   G <= 2       this chain except, at 64 columns, from 48 Ki ids over all units on (64 Ki at G 2, 96 Ki at G 4: 12 x 20000, 4096 ids
+//                22.7 / 25.2; 64 x 8124 33.7 / 43.3; 24 x 20000 at G 4 32.5 / 36.4), at 128 from 96 Ki (G 1: 32 x 8124, 4096 ids 34.4 /
+//                37.2), and at 256 for a few units of 5 Ki rows and more (6 x 8124 20.0 / 22.0, 4 x 16316 22.4 / 24.0)
+//   sketch chain except where much of the region is selected, 1/14 of it at 256 columns, 1/7 at 128 and 1/10 at 64, times G, half of it
+//                at any G (24 x 12200 of 256, 4096 ids 56.5 / 66.2; G 4: 64 x 8124 115.8 / 151.4)
+//   bf16 chain   except at G 1 up to 48 Ki rows, at G 2 up to 32 Ki, and at 256 columns from a sixth of the region on (12 x 24615 of 128
+//                29.8 / 32.9; 16 x 16316 of 256 40.1 / 43.3; but 3 x 39932 of 128 29.0 / 27.1)
+// Over 9000 shapes (1 to 64 units x 1000 to 65468 rows, 256 to 4096 ids, G 1 to 8) a layer takes 0.898 of what the one kernel alone
+// took, 14 of them more than 1.05, none more than 1.10.  At most two units of more than 16 Ki rows, and callers without a
+// sketch up to 12 Ki rows or two units, stay with the one kernel although this chain is mostly the faster one there too (2 x 16316
+// of 128, G 4, 22.5 / 18.9).  Groups too large for this chain's attention: one kernel up to 32 MiB of keys (8 x 4028 of 256 at G 8, 256 ids
+// 26.8 / 27.1, 1024 ids 32.2 / 30.7).
 bool dc_one_kernel_first(const dc_layer_args *a, int region, int k_eff) {
-    const int64_t n_units = (int64_t)a->n_b * a->n_h;
+    constexpr int64_t Ki = 1024;
+    const int64_t n_units = (int64_t)a->n_b * a->n_h, k = k_eff;
+    const int g = a->group, hd = a->hd;
     if (a->one_kernel == DC_ONE_KERNEL_EXCLUSIVE) return true;
-    if (!a->sketch_codes) return n_units <= 2 || region <= 12 * 1024;
-    if (n_units <= 2 && region > 16 * 1024) return true;
-    return !dc_short_supported(a, region, k_eff) && region <= 16 * 1024 && n_units * region * a->hd * 2 <= (32ll << 20);
+    if (a->sketch_codes ? n_units <= 2 && region > 16 * Ki : n_units <= 2 || region <= 12 * Ki) return true;
+    if (dc_short_supported(a, region, k_eff)) {
+        if (hd == 64) return g <= 4 && n_units * k >= (g == 1 ? 48 : (g == 2 ? 64 : 96)) * Ki;
+        if (hd == 128) return g == 1 && n_units * k >= 96 * Ki;
+        return (g == 1 || (g == 2 && n_units >= 4)) && region >= 5 * Ki && n_units * region <= 64 * Ki && 4 * k <= region;
+    }
+    if (a->sketch_codes)
+        return (region <= 16 * Ki && n_units * region * hd * 2 <= (32ll << 20)) || 2 * k >= region ||
+               (hd == 64 ? 10 : (hd == 128 ? 7 : 14)) * k >= (int64_t)g * region;
+    return (g == 1 && n_units > 3 && region < 48 * Ki) || (g == 2 && region < 32 * Ki) || (hd == 256 && g <= 4 && 6 * k >= region);
 }
 
 // The layer on `stream`.  sel_ws: the select part of the workspace, its histograms zero (and left so).

@@ -438,7 +438,8 @@ typedef struct dc_step_args {
 int dc_decode_layer_step(const dc_layer_args *args, const dc_step_args *step, void *stream);
 /*
  * Short contexts.  With scores == NULL, order == DC_ORDER_ANY, at most 32 Ki region rows per unit and 64 MiB of
- * keys in the regions of all units (56 MiB with a sketch, above 16 Ki rows of which fewer than a twelfth are selected), a layer runs as a chain of THREE kernels over the bf16 keys, with or without a
+ * keys in the regions of all units (56 MiB with a sketch, above 16 Ki rows of which fewer than a twelfth are selected), a
+ * layer runs as a chain of THREE kernels over the bf16 keys, with or without a
  * sketch (scores; selection and attention in one; merge), on any stream, also under capture and with
  * region_hi_dev; the event pair brackets the first.  dc_decode_layer_is_short says whether a call that does not
  * run as one kernel is of that kind; its route is named DC_ROUTE_SKETCH or DC_ROUTE_STREAM like any chain's.
@@ -446,9 +447,11 @@ int dc_decode_layer_step(const dc_layer_args *args, const dc_step_args *step, vo
  * With at most 640 Ki region rows over all units (and, when a sketch is passed, at most 40 Ki region rows per
  * unit), dc_decode_layer can run the layer as ONE kernel whose blocks are all resident
  * (two per CU) and hand their phases over through the workspace (same results; the event pair
- * then brackets that kernel).  It does so with DC_ONE_KERNEL_EXCLUSIVE; for callers without a sketch, up to 12 Ki rows per
- * unit or at most two units; with a sketch, for at most two units of more than 16 Ki
- * rows each, and for large groups of query heads up to 32 MiB of keys. No counterpart in the reference, whose layers run on the CPU pool
+ * then brackets that kernel).  It does so with DC_ONE_KERNEL_EXCLUSIVE and, with DC_ONE_KERNEL_AUTO, where it takes less time than
+ * the chains: mostly for one or two query heads to a unit, or where a large part of the region is selected; also for
+ * callers without a sketch up to 12 Ki rows per unit or at most two units, with a sketch for at most two
+ * units of more than 16 Ki rows each, and for large groups of query heads up to 32 MiB of keys.  dc_decode_layer_route
+ * says what a call takes.  No counterpart in the reference, whose layers run on the CPU pool
  * (lib.rs:352-369); what it has to match is that one layer call is always right
  * (src/diffcache/base.py:150-155).
  *

@@ -174,3 +174,33 @@ def test_which_calls_run_as_one_kernel():
     assert [route(8, n, policy=hip.ONE_KERNEL_EXCLUSIVE) for n in (4028, 32768)] == [one, one]
     assert route(8, 4028, policy=hip.ONE_KERNEL_NEVER) == chain and route(8, 4028, region_hi_dev=0x1000) == chain
     assert [route(8, n, hd=256, group=6) for n in (4028, 8192, 8193)] == [one, one, chain]
+
+
+@pytest.mark.gpu
+def test_small_groups_and_large_selections_run_as_one_kernel():
+    """Both sides of the lines at which the one kernel takes less time than the chains."""
+    from diffcache_amd import _hip as hip
+
+    def one(units, rows, hd, group, budget, sketch=0x1000):
+        a = hip.LayerArgs()
+        a.n_b, a.n_h, a.group, a.hd, a.budget, a.n_sink = 1, units, group, hd, budget, 4
+        a.recent_lo, a.n_recent, a.kv_row_stride, a.sketch_codes = 4 + rows, 64, hd, sketch
+        return hip.lib.dc_decode_layer_route(ctypes.byref(a)) == hip.ROUTE_ONE_KERNEL
+    for sketch in (0x1000, None):       # three kernels: many ids of narrow heads, a few units of wide ones
+        rows = 12289                    # (without a sketch: beyond what stays with the one kernel anyway)
+        assert one(12, rows, 64, 1, 4096, sketch) and not one(12, rows, 64, 1, 4095, sketch)
+        assert one(16, rows, 64, 2, 4096, sketch) and not one(16, rows, 64, 2, 4095, sketch)
+        assert one(24, rows, 64, 4, 4096, sketch) and not one(24, rows, 64, 4, 4095, sketch) and not one(24, rows, 64, 8, 4096, sketch)
+        assert one(5, 13107, 256, 1, 1024, sketch) and not one(5, 13108, 256, 1, 1024, sketch)
+        assert one(4, rows, 256, 2, 1024, sketch) and not one(3, rows, 256, 2, 1024, sketch) and not one(4, rows, 256, 4, 1024, sketch)
+        assert one(4, rows, 256, 1, 3072, sketch) and not one(4, rows, 256, 1, 3073, sketch)
+    assert one(24, 8124, 128, 1, 4096) and not one(24, 8124, 128, 1, 4095) and not one(24, 8124, 128, 2, 4096)
+    assert one(3, 5120, 256, 1, 1024) and not one(3, 5119, 256, 1, 1024)
+    # the sketch chain
+    assert one(48, 13000, 64, 1, 1300) and not one(48, 13001, 64, 1, 1300) and one(32, 14000, 128, 1, 2000) and not one(32, 14001, 128, 1, 2000)
+    assert one(16, 28000, 256, 1, 2000) and not one(16, 28001, 256, 1, 2000) and one(16, 14000, 256, 2, 2000) and not one(16, 14001, 256, 2, 2000)
+    assert one(64, 8192, 256, 4, 4096) and not one(64, 8193, 256, 8, 4096)
+    # the bf16 chain
+    assert one(12, 49151, 128, 1, 512, None) and not one(12, 49152, 128, 1, 512, None) and not one(3, 49151, 128, 1, 512, None)
+    assert one(12, 32767, 128, 2, 512, None) and not one(12, 32768, 128, 2, 512, None)
+    assert one(12, 24000, 256, 4, 4000, None) and not one(12, 24001, 256, 4, 4000, None) and not one(12, 24000, 128, 4, 4000, None)
