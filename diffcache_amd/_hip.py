@@ -756,6 +756,9 @@ class LayerStep:
         self._args: Optional[LayerArgs] = None
         self._step = StepArgs()
 
+    def __reduce__(self):
+        return LayerStep, ()    # a copy keeps nothing yet: what is kept are addresses of the original's tensors
+
     def __call__(self, q, store_k, store_v, n_sink, recent_lo, n_recent, budget, scores, idx_out, out, workspace, new_k, new_v,
                  lse, mode, order, scale, select_state_ready, scan_events, sketch, n_recent_dev, one_kernel, region_hi_dev,
                  append, advance) -> None:

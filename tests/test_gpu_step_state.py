@@ -338,3 +338,30 @@ def test_prefill_cache_saved_after_decode_steps_holds_the_decoded_tokens(tmp_pat
         a = cache.decode_attention(l, q, nk, nv, order=_hip.ORDER_BEST).clone()
         c = cache2.decode_attention(l, q, nk, nv, order=_hip.ORDER_BEST).clone()
         assert torch.equal(a, c) and torch.equal(cache.idx[l], cache2.idx[l])
+
+
+def test_a_copy_of_a_cache_decodes_on_its_own():
+    """copy.deepcopy of a cache in use: the copy continues as the original does, and neither sees the other's rows."""
+    import copy
+    from diffcache_amd import DiffCache
+    g = torch.Generator(device=DEV).manual_seed(12)
+    rnd = lambda *s: torch.randn(s, generator=g, device=DEV).to(torch.bfloat16)
+    cache = DiffCache(num_layers=2, batch_size=1, max_length=1200, num_kv_heads=2, num_q_heads=4, head_dim=64, retrieval_budget=64,
+                      nsw_m=16, nsw_ef_cons=200, kvbuf_prefix_len=4, kvbuf_suffix_len=8, kvbuf_suffix_maxlen=16,
+                      attn_mass_threshold=0.9, k_check_seq=[100], r_sq=[[4.0] * 2] * 2)
+    for layer in range(2):
+        cache.prefill_update_kv_cache(rnd(1, 1000, 2, 64), rnd(1, 1000, 2, 64), layer)
+    tokens = [[(rnd(1, 4, 64), rnd(1, 2, 64), rnd(1, 2, 64)) for _ in range(2)] for _ in range(6)]
+
+    def step(c, token):
+        return [c.decode_attention(layer, *token[layer]).clone() for layer in range(2)]
+    for token in tokens[:3]:
+        step(cache, token)
+    other = copy.deepcopy(cache)
+    for token in tokens[3:]:
+        for x, y in zip(step(cache, token), step(other, token)):
+            assert torch.equal(x, y)
+    torch.cuda.synchronize()
+    for layer in range(2):
+        assert torch.equal(cache.kstore[layer], other.kstore[layer])
+        assert cache.kstore[layer].data_ptr() != other.kstore[layer].data_ptr()

@@ -115,6 +115,18 @@ def test_scan_kernels_do_not_spill():
     assert not bad, bad
 
 
+def test_kept_layer_arguments_are_copied_and_pickled_empty():
+    """A cache can be copied and pickled like any object of tensors: the copy's layers fill their arguments anew."""
+    import copy
+    import pickle
+    from diffcache_amd import _hip
+    step = _hip.LayerStep()
+    step._again, step._key, step._args = True, (1, 2), _hip.LayerArgs()
+    for other in (copy.copy(step), copy.deepcopy(step), pickle.loads(pickle.dumps(step)), copy.deepcopy([step])[0]):
+        assert isinstance(other, _hip.LayerStep) and other._args is None and other._key is None and not other._again
+        assert other._step is not step._step
+
+
 def test_wrappers_refuse_cpu_tensors():
     from diffcache_amd import _hip
     k = torch.zeros((1, 1, 16, 128), dtype=torch.bfloat16)
