@@ -105,6 +105,11 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
     hipStream_t st = (hipStream_t)stream;
     int rc;
     const uint16_t *k_region = (const uint16_t *)a->k + (int64_t)a->n_sink * a->kv_row_stride;
+    // (a policy that does not exist is refused wherever the one kernel could run, also where a chain is the faster one)
+    const bool one_form = k_eff > 0 && !a->scores && a->order == DC_ORDER_ANY && !a->region_hi_dev;
+    DC_REQUIRE((a->one_kernel >= DC_ONE_KERNEL_NEVER && a->one_kernel <= DC_ONE_KERNEL_EXCLUSIVE) || !one_form ||
+                   !dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr),
+               "dc_decode_layer: bad one_kernel policy %d", a->one_kernel);
     // The caller's word that the select state is ready counts unless a kernel of the one-kernel
     // route has reported a failure since this workspace was last initialised.
     int ready = a->select_state_ready;
@@ -118,7 +123,7 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
                                                                                              : DC_ROUTE_STREAM));
     const bool short_ok = dc_short_supported(a, region, k_eff);
     const bool one_first = dc_one_kernel_first(a, region, k_eff);
-    if (k_eff > 0 && !a->scores && a->order == DC_ORDER_ANY && !a->region_hi_dev && (one_first || !ready) &&
+    if (one_form && (one_first || !ready) &&
         dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr)) {
         // short context: the whole layer in one kernel whose blocks are all resident (ids in no
         // particular order); reads the bf16 keys, with or without a sketch.  The state is set up

@@ -204,3 +204,23 @@ def test_small_groups_and_large_selections_run_as_one_kernel():
     assert one(12, 49151, 128, 1, 512, None) and not one(12, 49152, 128, 1, 512, None) and not one(3, 49151, 128, 1, 512, None)
     assert one(12, 32767, 128, 2, 512, None) and not one(12, 32768, 128, 2, 512, None)
     assert one(12, 24000, 256, 4, 4000, None) and not one(12, 24001, 256, 4, 4000, None) and not one(12, 24000, 128, 4, 4000, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("policy", [-2, 2, 7])
+def test_a_policy_that_does_not_exist_is_refused(policy):
+    """Wherever the one kernel could run, whichever route is the faster one; before anything is launched."""
+    from diffcache_amd import _hip as hip
+    b, hkv, group, hd, budget = 1, 2, 4, 64, 64
+    for rows, order in ((500, hip.ORDER_ANY), (9000, hip.ORDER_ANY)):
+        k = torch.zeros((b, hkv, rows, hd), device=DEV, dtype=torch.bfloat16)
+        q = torch.zeros((b, hkv * group, hd), device=DEV, dtype=torch.bfloat16)
+        ws = hip.alloc_workspace(hip.layer_workspace_bytes(b * hkv, rows, budget, group, hd, budget), DEV)
+        idx, out = torch.full((b * hkv, budget), -7, device=DEV, dtype=torch.int32), torch.full_like(q, 3.0)
+        for sk in (None, hip.Sketch(k).build(k, 0, rows)):
+            for ready in (False, True):
+                with pytest.raises(hip.DiffCacheError, match="one_kernel policy"):
+                    hip.decode_layer(q, k, k, 0, rows, 0, budget, None, idx, out, ws, order=order, sketch=sk, one_kernel=policy,
+                                     select_state_ready=ready)
+        torch.cuda.synchronize()
+        assert bool((idx == -7).all()) and bool((out == 3.0).all())
