@@ -185,14 +185,18 @@ int launch_attn(int group, dim3 grid, hipStream_t st, const AttnArgs &a) {
 
 // Which split body a call runs.  The matrix-core version takes any group up to 16; the VALU
 // version (groups up to 8) stays for comparison: DIFFCACHE_ATTN_VALU=1 in the environment of the
-// process (read once) selects it wherever it applies.
-static bool attn_use_mfma(int group, int64_t max_row, int64_t ksr, int64_t vsr) {
+// process (read once) selects it wherever it applies, in place of the short chain too, which has no such version.
+bool dc_attn_valu(int group) {
     static const bool valu = [] {
         const char *e = std::getenv("DIFFCACHE_ATTN_VALU");
         return e && e[0] == '1' && e[1] == 0;
     }();
+    return valu && group <= 8;
+}
+
+static bool attn_use_mfma(int group, int64_t max_row, int64_t ksr, int64_t vsr) {
     if (group > 8) return true;
-    if (valu) return false;
+    if (dc_attn_valu(group)) return false;
     // rows are addressed with 32-bit byte offsets from the unit's first row
     const int64_t sr = ksr > vsr ? ksr : vsr;
     return (max_row + 1) * sr * 2 <= 0xffffffffll;

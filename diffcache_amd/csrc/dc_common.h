@@ -59,6 +59,7 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
                           int64_t ksh, int64_t ksr, int64_t vsb, int64_t vsh, int64_t vsr, float scale,
                           void *workspace, size_t workspace_bytes, void *stream, const int32_t *recent_lo_dev,
                           const dc_step_args *step = nullptr);
+bool dc_attn_valu(int group);  // the environment asks for the VALU version of the attention
 int dc_merge_launch(const char *who, const float *acc, const float *ml, void *out, float *lse, int n_units, int group, int hd,
                     int n_splits, const dc_step_args *step, uint32_t *clear_hist, void *stream);
 // short.hip: a decode layer in three kernels, for short contexts

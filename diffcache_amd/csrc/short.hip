@@ -502,13 +502,15 @@ constexpr int64_t kShortBytes = 64ll << 20, kShortBytesFew = 56ll << 20;
 }  // namespace
 
 // Whether a layer can take this chain: ids in any order, keys of a unit in a block's registers, row offsets of 32
-// bits, the splits' partials in the LDS that a launch gets without asking; and whether it is short enough to.
+// bits, the splits' partials in the LDS that a launch gets without asking, no wish for the VALU version of the attention; and
+// whether it is short enough to.
 bool dc_short_supported(const dc_layer_args *a, int region, int k_eff) {
     const int64_t n_units = (int64_t)a->n_b * a->n_h;
-    return a->order == DC_ORDER_ANY && !a->scores && k_eff > 0 && n_units > 0 && region >= 64 && region <= kShortMaxRows &&
+    return !dc_attn_valu(a->group) && a->order == DC_ORDER_ANY && !a->scores && k_eff > 0 && n_units > 0 && region >= 64 &&
+           region <= kShortMaxRows &&
            n_units * region * a->hd * 2 <=
-               (a->sketch_codes && region > 16 * 1024 && k_eff < region / 12 ? kShortBytesFew : kShortBytes) && a->group >= 1 && a->group * a->hd <= 1024 &&
-           (a->hd == 64 || a->hd == 128 || a->hd == 256) && a->kv_row_stride > 0 &&
+               (a->sketch_codes && region > 16 * 1024 && k_eff < region / 12 ? kShortBytesFew : kShortBytes) &&
+           a->group >= 1 && a->group * a->hd <= 1024 && (a->hd == 64 || a->hd == 128 || a->hd == 256) && a->kv_row_stride > 0 &&
            (a->recent_lo + a->n_recent + 1) * a->kv_row_stride * 2 <= 0xffffffffll;
 }
 

@@ -3,6 +3,9 @@ places of the list by itself, so what can go wrong is a split that counts differ
 oracle.  Ids against oracle.topk_select of the GPU's dense scores (nsw.rs:592-630, ties to the lower id), attention
 against the float64 softmax over the oracle's rows (base.py:134-142)."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -154,6 +157,27 @@ def test_which_calls_take_the_short_chain():
     assert short(hd=256, group=4) == 1 and short(hd=256, group=5) == 0 and short(group=8) == 1 and short(group=9) == 0
     assert short(order=hip.ORDER_BEST) == short(order=hip.ORDER_INDEX) == short(budget=0) == short(scores=0x1000) == 0
     assert short(kv_row_stride=1 << 20) == 0                                        # rows beyond 4 GiB of the unit's first
+
+
+def test_the_valu_attention_is_kept_where_it_is_asked_for():
+    """DIFFCACHE_ATTN_VALU=1 (read once per process): groups up to 8 leave this chain, whose attention is the matrix cores'."""
+    code = """
+import ctypes
+import os
+import subprocess
+import sys
+from diffcache_amd import _hip as hip
+a = hip.LayerArgs()
+a.n_b, a.n_h, a.hd, a.budget, a.n_sink, a.recent_lo, a.order, a.kv_row_stride, a.sketch_codes = 1, 8, 64, 512, 4, 4032, 0, 64, 0x1000
+a.one_kernel = hip.ONE_KERNEL_NEVER
+for g in (1, 8, 9, 16):
+    a.group = g
+    print(hip.lib.dc_decode_layer_is_short(ctypes.byref(a)), end=" ")
+"""
+    for value, want in (("1", "0 0 1 1"), ("0", "1 1 1 1")):
+        res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env={**os.environ, "DIFFCACHE_ATTN_VALU": value},
+                             cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+        assert res.stdout.split() == want.split(), (value, res.stdout, res.stderr[-300:])
 
 
 @pytest.mark.gpu
