@@ -110,6 +110,16 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
     DC_REQUIRE((a->one_kernel >= DC_ONE_KERNEL_NEVER && a->one_kernel <= DC_ONE_KERNEL_EXCLUSIVE) || !one_form ||
                    !dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr),
                "dc_decode_layer: bad one_kernel policy %d", a->one_kernel);
+    // (the short chain does not read the sketch; one that the sketch chain would refuse is refused all the same, unless the one
+    // kernel, which does not look at it either, could have taken the call)
+    const bool short_ok = dc_short_supported(a, region, k_eff);
+    if (short_ok && a->sketch_codes &&
+        !(a->sketch_scale && a->sketch_resid && dc_aligned16(a->sketch_codes + (int64_t)a->n_sink * a->sketch_row_stride) &&
+          dc_aligned16(a->sketch_scale) && dc_aligned16(a->sketch_resid) && a->sketch_batch_stride % 16 == 0 &&
+          a->sketch_head_stride % 16 == 0 && a->sketch_row_stride % 16 == 0 && a->sketch_row_stride >= a->hd))
+        DC_REQUIRE(one_form && a->one_kernel != DC_ONE_KERNEL_NEVER && dc_small_supported(n_units, region, k_eff, a->group, a->hd, true),
+                   "dc_decode_layer: the sketch needs codes, scale and resid aligned to 16 bytes, code strides in multiples of 16 "
+                   "bytes and row_stride >= hd");
     // The caller's word that the select state is ready counts unless a kernel of the one-kernel
     // route has reported a failure since this workspace was last initialised.
     int ready = a->select_state_ready;
@@ -121,7 +131,6 @@ extern "C" int dc_decode_layer_step(const dc_layer_args *a, const dc_step_args *
                               : (a->scores ? DC_ROUTE_DENSE
                                            : (a->sketch_codes && region <= DC_SKETCH_MAX_ROWS ? DC_ROUTE_SKETCH
                                                                                              : DC_ROUTE_STREAM));
-    const bool short_ok = dc_short_supported(a, region, k_eff);
     const bool one_first = dc_one_kernel_first(a, region, k_eff);
     if (one_form && (one_first || !ready) &&
         dc_small_supported(n_units, region, k_eff, a->group, a->hd, a->sketch_codes != nullptr)) {

@@ -179,6 +179,24 @@ def test_invalid_arguments_of_the_sketch_and_k_check_entry_points():
     assert rc == -22 and b"scores_unit_stride" in lib.dc_last_error()
 
 
+@pytest.mark.parametrize("region", [4000, 40000])
+def test_a_layers_sketch_is_checked_whichever_chain_runs(region):
+    """The short chain (4000 rows) does not read the sketch, but what the sketch chain (40000 rows) refuses it refuses too."""
+    from diffcache_amd import _hip
+    buf = (ctypes.c_char * 4096)()
+    p = (ctypes.addressof(buf) + 255) // 256 * 256
+    for name, bad in (("sketch_scale", None), ("sketch_resid", None), ("sketch_codes", p + 8), ("sketch_scale", p + 4), ("sketch_resid", p + 8),
+                      ("sketch_batch_stride", 8), ("sketch_head_stride", 24), ("sketch_row_stride", 136), ("sketch_row_stride", 112)):
+        a = _hip.LayerArgs()
+        a.q = a.k = a.v = a.out = a.idx_out = a.workspace = a.sketch_codes = a.sketch_scale = a.sketch_resid = p
+        a.n_b, a.n_h, a.group, a.hd, a.budget, a.idx_unit_stride, a.recent_lo = 1, 2, 4, 128, 64, 64, region
+        a.kv_row_stride = a.sketch_row_stride = 128
+        a.order, a.mode, a.one_kernel, a.workspace_bytes, a.select_state_ready = 0, 1, _hip.ONE_KERNEL_NEVER, 1 << 40, 1
+        setattr(a, name, bad)
+        assert _hip.lib.dc_decode_layer_is_short(ctypes.byref(a)) == (region == 4000)
+        assert _hip.lib.dc_decode_layer(ctypes.byref(a), None) == -22 and re.search(rb"sketch|codes|code strides", _hip.lib.dc_last_error()), name
+
+
 def test_invalid_arguments_of_the_pq_search_entry_point():
     from diffcache_amd import _hip
     lib = _hip.lib
