@@ -465,11 +465,13 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, const Attn
 #pragma unroll
     for (int w2 = 1; w2 < WAVES; ++w2) m = fmaxf(m, s_red[w2 * 16 + c]);
 
-    // P = exp(S - m): this lane's part of the A operand of P V, as the sum of two bf16 values
-    // (p = hi + lo to 2^-17 of p: with P rounded to one bf16 a slice of a few rows misses the
-    // 2e-3 bar where the terms cancel), so P V takes two instructions per 16 output columns
+    // P = exp(S - m): this lane's part of the A operand of P V, as the exact sum of three bf16 values
+    // (8 + 8 + 8 bits: the products are those of an fp32 P, as in the kernels without matrix
+    // instructions; two terms leave 2^-17 of p, per cents of an output whose terms cancel), so P V takes
+    // three instructions per 16 output columns.  (The third costs 0.4 us in 89 at four layers of 2 x 16391 tokens of 64
+    // columns, 0.7 in 137 at eight of 4096 tokens of 128; nothing that shows from 32 Ki tokens on.)
     float p[TILES * 4];
-    uint32_t pa[TILES * 2], pb[TILES * 2];
+    uint32_t pa[TILES * 2], pb[TILES * 2], pc[TILES * 2];
     float lloc = 0.f;
 #pragma unroll
     for (int t = 0; t < TILES; ++t)
@@ -481,7 +483,9 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, const Attn
 #pragma unroll
     for (int k2 = 0; k2 < TILES * 2; ++k2) {
         pa[k2] = dc_pack_bf16(p[2 * k2], p[2 * k2 + 1]);
-        pb[k2] = dc_pack_bf16(p[2 * k2] - dc_bf16_lo(pa[k2]), p[2 * k2 + 1] - dc_bf16_hi(pa[k2]));
+        const float r0 = p[2 * k2] - dc_bf16_lo(pa[k2]), r1 = p[2 * k2 + 1] - dc_bf16_hi(pa[k2]);
+        pb[k2] = dc_pack_bf16(r0, r1);
+        pc[k2] = dc_pack_bf16(r0 - dc_bf16_lo(pb[k2]), r1 - dc_bf16_hi(pb[k2]));
     }
     dc_f32x4 acc[EPL];
 #pragma unroll
@@ -494,13 +498,16 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, const Attn
         const dc_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         if constexpr (TILES == 2) {
             const dc_u32x4 ah = {pa[0], pa[1], pa[TILES * 2 - 2], pa[TILES * 2 - 1]};
-            const dc_u32x4 al = {pb[0], pb[1], pb[TILES * 2 - 2], pb[TILES * 2 - 1]};
+            const dc_u32x4 am = {pb[0], pb[1], pb[TILES * 2 - 2], pb[TILES * 2 - 1]};
+            const dc_u32x4 al = {pc[0], pc[1], pc[TILES * 2 - 2], pc[TILES * 2 - 1]};
             const dc_bf16x8 bw = __builtin_bit_cast(dc_bf16x8, dc_u32x4{bv[0], bv[1], bv[TILES * 2 - 2], bv[TILES * 2 - 1]});
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, al), bw, zero, 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, am), bw, acc[j], 0, 0, 0);
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dc_bf16x8, ah), bw, acc[j], 0, 0, 0);
         } else {
             const dc_s16x4 bw = __builtin_bit_cast(dc_s16x4, dc_u32x2{bv[0], bv[1]});
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(dc_s16x4, dc_u32x2{pb[0], pb[1]}), bw, zero, 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(dc_s16x4, dc_u32x2{pc[0], pc[1]}), bw, zero, 0, 0, 0);
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(dc_s16x4, dc_u32x2{pb[0], pb[1]}), bw, acc[j], 0, 0, 0);
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(dc_s16x4, dc_u32x2{pa[0], pa[1]}), bw, acc[j], 0, 0, 0);
         }
     }
