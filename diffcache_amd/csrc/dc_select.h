@@ -125,14 +125,28 @@ __device__ __forceinline__ void dc_for_each_pair(const uint32_t *ck, const uint3
 // `prefix`, histogram bits [top-1, top-width) and find the bin that holds the
 // rem-th smallest (1-based).  Updates prefix (bin bits filled in), rem (rank inside
 // the bin), eq (bin size) and top (= the lowest decided bit).  Uniform over the block.
+// wide (optional): kRadixCopies histograms of LDS (16-byte aligned) in which long lists are counted, a lane in copy
+// lane % kRadixCopies: additions to one word are served one after the other, and neighbours in a list are
+// neighbouring rows, whose numbers agree in the bits of a pass (select_finish_kernel over 8 units x 60001 rows that
+// tie: 74 us in one copy, 46 in eight; groups of lanes picked out by ballots and added once 102).
+constexpr int kRadixCopies = 8;
+
 template <bool IN_LDS = false, typename Get>
 __device__ __forceinline__ void block_radix_pass(Get get, uint32_t n, uint32_t &prefix, uint32_t &rem,
                                                  uint32_t &eq, int &top, uint32_t *lh, uint32_t *wtot,
-                                                 uint32_t *sres) {
+                                                 uint32_t *sres, uint32_t *wide = nullptr) {
+    static_assert(kRadixBins == 2 * kFinalThreads && kRadixCopies == 8, "a thread adds up two bins of eight copies");
     const int tid = threadIdx.x;
     const int width = top < kRadixBits ? top : kRadixBits;
     const int shift = top - width;
-    for (int i = tid; i < kRadixBins; i += kFinalThreads) lh[i] = 0;
+    const bool spread = !IN_LDS && wide && n > (uint32_t)kScanShort;
+    uint4 *const wide4 = reinterpret_cast<uint4 *>(wide);
+    if (spread) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wide4[i * kFinalThreads + tid] = make_uint4(0u, 0u, 0u, 0u);
+    } else {
+        for (int i = tid; i < kRadixBins; i += kFinalThreads) lh[i] = 0;
+    }
     __syncthreads();
     const uint32_t himask = (top >= 32) ? 0u : (0xffffffffu << top);
     constexpr bool kPlain = IN_LDS;  // a list that the caller keeps in LDS: nothing to hide
@@ -159,6 +173,10 @@ __device__ __forceinline__ void block_radix_pass(Get get, uint32_t n, uint32_t &
         for (int u = 0; u < kScanBatch; ++u) {
             const bool hit = in[u] && ((v[u] & himask) == (prefix & himask));
             const uint32_t bin = (v[u] >> shift) & ((1u << width) - 1u);
+            if (spread) {
+                if (hit) atomicAdd(&wide[bin * kRadixCopies + (tid & (kRadixCopies - 1))], 1u);
+                continue;
+            }
             const unsigned long long hits = __ballot(hit);
             if (hits == 0ull) continue;
             const int leader = (int)__builtin_ctzll(hits);
@@ -171,8 +189,20 @@ __device__ __forceinline__ void block_radix_pass(Get get, uint32_t n, uint32_t &
         }
     }
     __syncthreads();
-    // kRadixBins == 2 * kFinalThreads: each thread owns two adjacent bins
-    const uint32_t h0 = lh[2 * tid], h1 = lh[2 * tid + 1];
+    // each thread owns two adjacent bins
+    uint32_t h0 = 0u, h1 = 0u;
+    if (spread) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int c = (j + (tid >> 1)) & 3;  // (lanes start at different banks)
+            const uint4 v = wide4[4 * tid + c];
+            const uint32_t sum = v.x + v.y + v.z + v.w;
+            h0 += c < 2 ? sum : 0u;
+            h1 += c < 2 ? 0u : sum;
+        }
+    } else {
+        h0 = lh[2 * tid], h1 = lh[2 * tid + 1];
+    }
     uint32_t total;
     const uint32_t excl = block_excl_scan<kFinalThreads>(h0 + h1, wtot, &total);
     if (excl < rem && rem <= excl + h0 + h1) {
@@ -202,8 +232,8 @@ __device__ __forceinline__ void block_radix_pass(Get get, uint32_t n, uint32_t &
 template <bool IN_LDS = false, typename Get>
 __device__ __forceinline__ uint32_t block_radix_select(Get get, uint32_t n, uint32_t rem, int top, uint32_t prefix,
                                        uint32_t eq, uint32_t *lh, uint32_t *wtot, uint32_t *sres,
-                                       uint32_t *rem_out, uint32_t *n_eq) {
-    while (top > 0) block_radix_pass<IN_LDS>(get, n, prefix, rem, eq, top, lh, wtot, sres);
+                                       uint32_t *rem_out, uint32_t *n_eq, uint32_t *wide = nullptr) {
+    while (top > 0) block_radix_pass<IN_LDS>(get, n, prefix, rem, eq, top, lh, wtot, sres, wide);
     *rem_out = rem;
     *n_eq = eq;
     return prefix;
@@ -218,7 +248,7 @@ __device__ __forceinline__ uint32_t block_radix_select(Get get, uint32_t n, uint
 template <bool IN_LDS = false>
 __device__ __forceinline__ void dc_finalize_unit(const uint32_t *ck, const uint32_t *ci, uint32_t n_c, uint32_t need,
                                  uint32_t *io, int n_rows, uint32_t *lh, uint32_t *wtot,
-                                 uint32_t *sres, uint32_t *smisc, uint32_t *kout = nullptr) {
+                                 uint32_t *sres, uint32_t *smisc, uint32_t *kout = nullptr, uint32_t *wide = nullptr) {
     const int tid = threadIdx.x;
     if (need == n_c) {  // the whole candidate list is selected
 #pragma unroll 4
@@ -263,7 +293,7 @@ __device__ __forceinline__ void dc_finalize_unit(const uint32_t *ck, const uint3
         *v = ck[i];
         return true;
     };
-    if (top > 0) block_radix_pass<IN_LDS>(get_key, n_c, prefix, rem, eq, top, lh, wtot, sres);
+    if (top > 0) block_radix_pass<IN_LDS>(get_key, n_c, prefix, rem, eq, top, lh, wtot, sres, wide);
 
     if (eq <= (uint32_t)kFinalThreads) {
         // The keys whose decided bits equal the threshold bin's are few: they are
@@ -302,7 +332,7 @@ __device__ __forceinline__ void dc_finalize_unit(const uint32_t *ck, const uint3
 
     uint32_t need_eq, n_eq;
     const uint32_t t_key =
-        block_radix_select<IN_LDS>(get_key, n_c, rem, top, prefix, eq, lh, wtot, sres, &need_eq, &n_eq);
+        block_radix_select<IN_LDS>(get_key, n_c, rem, top, prefix, eq, lh, wtot, sres, &need_eq, &n_eq, wide);
 
     uint32_t t_idx = 0xffffffffu;
     if (need_eq < n_eq) {  // only the lowest ids of the tie group fit
@@ -313,7 +343,7 @@ __device__ __forceinline__ void dc_finalize_unit(const uint32_t *ck, const uint3
             return ck[i] == t_key;
         };
         uint32_t r2, e2;
-        t_idx = block_radix_select<IN_LDS>(get_idx, n_c, need_eq, hbi + 1, 0u, n_eq, lh, wtot, sres, &r2, &e2);
+        t_idx = block_radix_select<IN_LDS>(get_idx, n_c, need_eq, hbi + 1, 0u, n_eq, lh, wtot, sres, &r2, &e2, wide);
     }
 
     dc_for_each_pair_uniform<kFinalThreads, IN_LDS>(ck, ci, n_c, [&](uint32_t key, uint32_t id, bool in) {
@@ -409,6 +439,7 @@ __device__ __forceinline__ bool dc_select_counted(const uint32_t *ck, const uint
     if ((tid & 63) == 0 && diff) atomicOr(&smisc[0], diff);
     __syncthreads();
     diff = smisc[0];
+    if (diff == 0u && n > (uint32_t)kFinalThreads) return false;  // one bin, which a count would fill one addition after the other
     const int top = diff ? 32 - __clz(diff) : 0;
     const int shift = top > kRadixBits ? top - kRadixBits : 0;
     const uint32_t mask = diff ? (uint32_t)kRadixBins - 1u : 0u;  // the bits above are the same in every key

@@ -1123,7 +1123,8 @@ __global__ __launch_bounds__(kThreads) void pq_rescore_kernel(
 // (Counting a threshold bin of more than 96 once more instead of ranking it: no faster where it applies, 0.3 us slower else.)
 // A radix pass whose members reserve slots wave by wave took 7.5 and 8.8 us.  Longer lists take dc_select_counted as long as they fit
 // the LDS; lists that do not, and threshold bins of more than kFinalThreads (ties by the
-// thousand), take the radix passes of dc_finalize_unit.
+// thousand), take the radix passes of dc_finalize_unit.  Keys that are all equal are not counted first (one bin: 8 units x
+// 8000 rows that tie, a whole selection, 34 us with the count, 31 without).
 constexpr int kFinishPer = 8, kFinishRegs = kFinishPer * kFinalThreads;
 
 __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
@@ -1135,7 +1136,9 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     __shared__ uint32_t sres[4];
     __shared__ uint32_t smisc[2];
     __shared__ uint32_t s_or[kFinalThreads / 64];
-    __shared__ uint32_t lck[kCandLds], lci[kCandLds];  // longer lists are staged in LDS when they fit
+    __shared__ __align__(16) uint32_t s_list[2 * kCandLds];  // longer lists are staged in LDS when they fit
+    uint32_t *const lck = s_list, *const lci = s_list + kCandLds;
+    static_assert(kRadixCopies * kRadixBins <= 2 * kCandLds, "the counts of lists that do not fit take their place");
     __shared__ unsigned long long tie[kFinalThreads];
     const int unit = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1215,39 +1218,41 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
         uint32_t diff = 0u;
 #pragma unroll
         for (int w = 0; w < kFinalThreads / 64; ++w) diff |= s_or[w];
-        const int top = diff ? 32 - __clz((int)diff) : 0;
-        const int shift = top > kRadixBits ? top - kRadixBits : 0;
-        const uint32_t mask = diff ? (uint32_t)kRadixBins - 1u : 0u;  // the bits above are the same in every key
-        each([&](uint32_t, uint32_t key, uint32_t) __attribute__((always_inline)) { atomicAdd(&lh[(key >> shift) & mask], 1u); });
-        __syncthreads();
-        const uint2 h2 = reinterpret_cast<const uint2 *>(lh)[tid];
-        uint32_t total;
-        const uint32_t excl = block_excl_scan<kFinalThreads>(h2.x + h2.y, wtot, &total);
-        reinterpret_cast<uint2 *>(lh)[tid] = make_uint2(excl, excl + h2.x);
-        if (excl < need && need <= excl + h2.x + h2.y) {
-            const bool first = excl + h2.x >= need;
-            sres[0] = 2 * tid + (first ? 0 : 1);
-            sres[1] = first ? excl : excl + h2.x;
-            sres[2] = first ? h2.x : h2.y;
-        }
-        __syncthreads();
-        const uint32_t t_bin = sres[0], t_lo = sres[1], t_cnt = sres[2];
-        if (t_cnt <= (uint32_t)kFinalThreads) {
-            each([&](uint32_t, uint32_t key, uint32_t id) __attribute__((always_inline)) {
-                const uint32_t bin = (key >> shift) & mask;
-                if (bin > t_bin) return;
-                const uint32_t slot = atomicAdd(&lh[bin], 1u);
-                if (bin == t_bin) tie[slot - t_lo] = ((unsigned long long)key << 32) | id;
-                else put(slot, key, id);
-            });
+        if (diff != 0u || n_c <= (uint32_t)kFinalThreads) {  // (equal keys are one bin)
+            const int top = diff ? 32 - __clz((int)diff) : 0;
+            const int shift = top > kRadixBits ? top - kRadixBits : 0;
+            const uint32_t mask = diff ? (uint32_t)kRadixBins - 1u : 0u;  // the bits above are the same in every key
+            each([&](uint32_t, uint32_t key, uint32_t) __attribute__((always_inline)) { atomicAdd(&lh[(key >> shift) & mask], 1u); });
             __syncthreads();
-            if ((uint32_t)tid < t_cnt) {
-                const unsigned long long mine = tie[tid];
-                uint32_t rank = t_lo;
-                for (uint32_t j = 0; j < t_cnt; ++j) rank += tie[j] < mine ? 1u : 0u;
-                if (rank < need) put(rank, (uint32_t)(mine >> 32), (uint32_t)mine);
+            const uint2 h2 = reinterpret_cast<const uint2 *>(lh)[tid];
+            uint32_t total;
+            const uint32_t excl = block_excl_scan<kFinalThreads>(h2.x + h2.y, wtot, &total);
+            reinterpret_cast<uint2 *>(lh)[tid] = make_uint2(excl, excl + h2.x);
+            if (excl < need && need <= excl + h2.x + h2.y) {
+                const bool first = excl + h2.x >= need;
+                sres[0] = 2 * tid + (first ? 0 : 1);
+                sres[1] = first ? excl : excl + h2.x;
+                sres[2] = first ? h2.x : h2.y;
             }
-            return;
+            __syncthreads();
+            const uint32_t t_bin = sres[0], t_lo = sres[1], t_cnt = sres[2];
+            if (t_cnt <= (uint32_t)kFinalThreads) {
+                each([&](uint32_t, uint32_t key, uint32_t id) __attribute__((always_inline)) {
+                    const uint32_t bin = (key >> shift) & mask;
+                    if (bin > t_bin) return;
+                    const uint32_t slot = atomicAdd(&lh[bin], 1u);
+                    if (bin == t_bin) tie[slot - t_lo] = ((unsigned long long)key << 32) | id;
+                    else put(slot, key, id);
+                });
+                __syncthreads();
+                if ((uint32_t)tid < t_cnt) {
+                    const unsigned long long mine = tie[tid];
+                    uint32_t rank = t_lo;
+                    for (uint32_t j = 0; j < t_cnt; ++j) rank += tie[j] < mine ? 1u : 0u;
+                    if (rank < need) put(rank, (uint32_t)(mine >> 32), (uint32_t)mine);
+                }
+                return;
+            }
         }
         // keys that crowd into one bin: from LDS like a longer list
         each([&](uint32_t i, uint32_t key, uint32_t id) __attribute__((always_inline)) { lck[i] = key, lci[i] = id; });
@@ -1258,7 +1263,7 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     // at run time every access would be a flat one, and waiting for a flat load also waits for
     // the stores issued above.
     if (regs || staged) dc_finalize_unit<true>(lck, lci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
-    else dc_finalize_unit(ck, ci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr);
+    else dc_finalize_unit(ck, ci, n_c, need, io + c_less, n_rows, lh, wtot, sres, smisc, ko ? ko + c_less : nullptr, s_list);
 }
 
 // The same for ids in best-first order (k <= kSortMost): the unit's certain members (which classify_kernel
@@ -1277,7 +1282,9 @@ __global__ __launch_bounds__(kFinalThreads) void select_sorted_kernel(
     __shared__ uint32_t wtot[kFinalThreads / 64 + 1];
     __shared__ uint32_t sres[4];
     __shared__ uint32_t smisc[2];
-    __shared__ uint32_t lck[kSortedLds], lci[kSortedLds];
+    __shared__ __align__(16) uint32_t s_list[2 * kSortedLds];
+    uint32_t *const lck = s_list, *const lci = s_list + kSortedLds;
+    static_assert(kRadixCopies * kRadixBins <= 2 * kSortedLds, "the counts of lists that do not fit take their place");
     __shared__ unsigned long long buf[kSortMost + kSortBinMost];
     const int unit = blockIdx.x;
     const int tid = threadIdx.x;
@@ -1346,7 +1353,7 @@ __global__ __launch_bounds__(kFinalThreads) void select_sorted_kernel(
             dc_finalize_unit<true>(lck + c_less, lci + c_less, n_c, need - c_less, io + c_less, n_rows, lh, wtot, sres, smisc,
                                    ko + c_less);
         else
-            dc_finalize_unit(ck, ci, n_c, need - c_less, io + c_less, n_rows, lh, wtot, sres, smisc, ko + c_less);
+            dc_finalize_unit(ck, ci, n_c, need - c_less, io + c_less, n_rows, lh, wtot, sres, smisc, ko + c_less, s_list);
     }
     __syncthreads();
     int pow2 = 128;
