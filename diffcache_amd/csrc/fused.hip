@@ -666,24 +666,28 @@ __global__ __launch_bounds__(kPqThreads, 4) void pq_scan_kernel(
 
 // classify_kernel for the buckets that pq_scan_kernel left: keys in buckets better than the threshold bucket are certain
 // members, keys in it become candidates, whose scores are worked out once more (the additions of pq_adc_score).  A block
-// takes kPqClassRows keys and reserves its places in both lists with one returning atomic.
-constexpr int kPqClassRows = 8192;
+// takes ROWS keys (pq_class_rows) and reserves its places in both lists with one returning atomic.  Few candidates are scored
+// from the tables in memory, a chain of 3 us per 256 of them.  More are many of a block's keys (short units of which much is
+// selected, keys that tie), and the block stages the tables and walks its keys in order as the scan does: 3 units x 5000 keys,
+// 4096 of them selected, 6.6 us (12 from memory, in blocks of 8192); 5000 keys that tie 7.6 (65), 3 x 65000 11 (70).
 static_assert(offsetof(UnitState, cand_cnt) == offsetof(UnitState, win_cnt) + 4 && offsetof(UnitState, win_cnt) % 8 == 0, "one word");
 
-template <int M>
+template <int M, int ROWS>
 __global__ __launch_bounds__(kThreads) void pq_classify_kernel(
     const uint8_t *__restrict__ codes, const float *__restrict__ lut, const uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, const uint2 *__restrict__ surv, uint32_t *__restrict__ cand_key,
     uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride, int n_units, int n_rows, int k_eff) {
-    constexpr int kVec = kPqClassRows / kThreads / 8;  // vectors of eight buckets per thread
+    constexpr int kVec = ROWS / kThreads / 8;  // vectors of eight buckets per thread
     constexpr int NW = M / 4;
-    __shared__ uint16_t s_sure[kPqClassRows], s_cand[kPqClassRows];
+    static_assert(kVec * 8 * kThreads == ROWS && ROWS % 64 == 0 && 4 * ROWS <= 4 * kPqLutWords, "whole vectors; both lists in the tables' place");
+    __shared__ __align__(16) float s_lut[kPqLutWords];  // of blocks with many candidates; the lists before
+    uint16_t *s_sure = reinterpret_cast<uint16_t *>(s_lut), *s_cand = s_sure + ROWS;
     __shared__ uint32_t wtot[kThreads / 64 + 1];
     __shared__ uint32_t sres[2];
     __shared__ uint32_t sbase[2];
     const int unit = blockIdx.x % n_units, blk = blockIdx.x / n_units;
     const int tid = threadIdx.x;
-    const int row0 = blk * kPqClassRows;
+    const int row0 = blk * ROWS;
     UnitState *st = state + unit;
     const uint16_t *du = reinterpret_cast<const uint16_t *>(surv) + (int64_t)unit * dense_stride(n_rows);
     uint4 v[kVec];
@@ -738,15 +742,54 @@ __global__ __launch_bounds__(kThreads) void pq_classify_kernel(
     }
     const uint8_t *cu = codes + (int64_t)unit * n_rows * M;
     const float *lu = lut + (int64_t)unit * M * 256;
-    for (uint32_t i = tid; i < n_cand; i += kThreads) {
-        const uint32_t row = (uint32_t)row0 + s_cand[i], at = sbase[1] + i;
+    uint32_t *ck = cand_key + (int64_t)unit * n_rows, *ci = cand_idx + (int64_t)unit * n_rows;
+    auto load_codes = [&](uint32_t row, uint32_t (&w)[NW]) __attribute__((always_inline)) {
         const uint4 *cp = reinterpret_cast<const uint4 *>(cu + (int64_t)row * M);
-        uint32_t w[NW], rw[NW];
 #pragma unroll
         for (int x = 0; x < NW / 4; ++x) {
             const uint4 t = cp[x];
             w[4 * x] = t.x, w[4 * x + 1] = t.y, w[4 * x + 2] = t.z, w[4 * x + 3] = t.w;
         }
+    };
+    auto put = [&](uint32_t at, uint32_t row, float score) __attribute__((always_inline)) {
+        uint32_t key, bucket;
+        dc_key_bucket(score, DC_MODE_IP, key, bucket);
+        if (at < (uint32_t)n_rows) {
+            ck[at] = key;
+            ci[at] = row;
+        }
+    };
+    if (n_cand > (uint32_t)(ROWS / 8 + kThreads)) {
+        __syncthreads();  // the lists are in the tables' place
+        pq_stage_lut<M>(s_lut, lu, tid, kThreads);
+        PqLane<M> ln;
+        ln.init(tid & 63);
+        __syncthreads();
+        constexpr int kAtOnce = 4;
+#pragma unroll 1
+        for (int s0 = 0; s0 < ROWS && row0 + s0 < n_rows; s0 += kAtOnce * kThreads) {
+            uint32_t w[kAtOnce][NW], bucket[kAtOnce];
+#pragma unroll
+            for (int j = 0; j < kAtOnce; ++j) {
+                const int row = row0 + s0 + j * kThreads + tid, r = row < n_rows ? row : n_rows - 1;
+                bucket[j] = row < n_rows ? (uint32_t)du[r] : ~0u;
+                load_codes((uint32_t)r, w[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < kAtOnce; ++j) {
+                const bool in = bucket[j] == tb;
+                if (__ballot(in) == 0ull) continue;
+                const float score = pq_adc_score<M>(w[j], s_lut, ln);
+                const uint32_t at = wave_reserve(in, &sbase[1]);
+                if (in) put(at, (uint32_t)(row0 + s0 + j * kThreads + tid), score);
+            }
+        }
+        return;
+    }
+    for (uint32_t i = tid; i < n_cand; i += kThreads) {
+        const uint32_t row = (uint32_t)row0 + s_cand[i];
+        uint32_t w[NW], rw[NW];
+        load_codes(row, w);
         PqWideLane<M> ln;
         ln.init((int)(row & 63u));
         pq_rotate<M>(w, ln.rot, ln.sh, rw);
@@ -755,12 +798,7 @@ __global__ __launch_bounds__(kThreads) void pq_classify_kernel(
         for (int j = 0; j < M; ++j) e[j] = lu[((row + j) % M) * 256 + ((rw[j / 4] >> (8 * (j % 4))) & 0xffu)];
 #pragma unroll
         for (int j = 0; j < M; ++j) acc += e[j];
-        uint32_t key, bucket;
-        dc_key_bucket(acc, DC_MODE_IP, key, bucket);
-        if (at < (uint32_t)n_rows) {
-            cand_key[(int64_t)unit * n_rows + at] = key;
-            cand_idx[(int64_t)unit * n_rows + at] = row;
-        }
+        put(sbase[1] + i, row, acc);
     }
 }
 
@@ -1769,6 +1807,14 @@ int dc_sketch_select_impl(const void *k, const uint8_t *codes, const float *scal
     return launch_finish(who, w, idx_out, idx_unit_stride, p.n_units, n_rows, p.k_eff, mode, order, 1, st);
 }
 
+namespace {
+// Keys of a block of pq_classify_kernel: 8192, or 2048 where those blocks would leave CUs idle and a unit has 128 of these at
+// most, which all reserve their places with additions to one word.
+int pq_class_rows(int64_t n_units, int n_rows) {
+    return n_rows <= 128 * 2048 && n_units * ((n_rows + 8191) / 8192) < 512 ? 2048 : 8192;
+}
+}  // namespace
+
 extern "C" size_t dc_pq_search_workspace_bytes(int n_units, int n_rows, int n_cand) {
     const FusedWs w = carve_fused(nullptr, n_units, n_rows, n_cand);
     const size_t nu = n_units > 0 ? n_units : 0;
@@ -1815,7 +1861,8 @@ extern "C" int dc_pq_search_bf16(const void *k, const uint8_t *codes, const floa
     const int64_t tiles = ((int64_t)n_rows + kPqThreads - 1) / kPqThreads;
     const int64_t steps = (p.n_units * tiles + kPqBlocks - 1) / kPqBlocks;
     const int64_t blocks = p.n_units * ((tiles + steps - 1) / steps);
-    const int64_t class_blocks = p.n_units * (((int64_t)n_rows + kPqClassRows - 1) / kPqClassRows);
+    const int class_rows = pq_class_rows(p.n_units, n_rows);
+    const int64_t class_blocks = p.n_units * (((int64_t)n_rows + class_rows - 1) / class_rows);
     DC_REQUIRE(blocks < (1ll << 31) && class_blocks < (1ll << 31), "%s: grid too large", who);
     if (ev_scan_begin) (void)hipEventRecord((hipEvent_t)ev_scan_begin, st);
     if (m == 16)
@@ -1827,12 +1874,14 @@ extern "C" int dc_pq_search_bf16(const void *k, const uint8_t *codes, const floa
     DC_CHECK_LAUNCH(who);
     if (ev_scan_end) (void)hipEventRecord((hipEvent_t)ev_scan_end, st);
     // the k1 best ADC scores of every unit, in no particular order
-    if (m == 16)
-        hipLaunchKernelGGL(pq_classify_kernel<16>, dim3((unsigned)class_blocks), dim3(kThreads), 0, st, codes, lut, w.hist, w.state,
-                           w.surv, w.cand_key, w.cand_idx, cand, (int64_t)k1, p.n_units, n_rows, k1);
-    else
-        hipLaunchKernelGGL(pq_classify_kernel<32>, dim3((unsigned)class_blocks), dim3(kThreads), 0, st, codes, lut, w.hist, w.state,
-                           w.surv, w.cand_key, w.cand_idx, cand, (int64_t)k1, p.n_units, n_rows, k1);
+#define DC_LAUNCH_PC(M, ROWS)                                                                                             \
+    hipLaunchKernelGGL((pq_classify_kernel<M, ROWS>), dim3((unsigned)class_blocks), dim3(kThreads), 0, st, codes, lut, w.hist, \
+                       w.state, w.surv, w.cand_key, w.cand_idx, cand, (int64_t)k1, p.n_units, n_rows, k1)
+    if (m == 16 && class_rows == 2048) DC_LAUNCH_PC(16, 2048);
+    else if (m == 16) DC_LAUNCH_PC(16, 8192);
+    else if (class_rows == 2048) DC_LAUNCH_PC(32, 2048);
+    else DC_LAUNCH_PC(32, 8192);
+#undef DC_LAUNCH_PC
     DC_CHECK_LAUNCH(who);
     rc = launch_finish(who, w, cand, k1, p.n_units, n_rows, k1, DC_MODE_IP, DC_ORDER_ANY, 1, st);
     if (rc) return rc;
