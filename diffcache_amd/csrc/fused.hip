@@ -1857,10 +1857,9 @@ extern "C" int dc_pq_search_bf16(const void *k, const uint8_t *codes, const floa
         rc = dc_select_state_init(p.n_units, n_rows, n_cand, workspace, workspace_bytes, stream);
         if (rc) return rc;
     }
-    // equal shares for as many blocks as run at once
-    const int64_t tiles = ((int64_t)n_rows + kPqThreads - 1) / kPqThreads;
-    const int64_t steps = (p.n_units * tiles + kPqBlocks - 1) / kPqBlocks;
-    const int64_t blocks = p.n_units * ((tiles + steps - 1) / steps);
+    // equal shares, a block per CU at most
+    plan_shares(p.n_units, ((int64_t)n_rows + kPqThreads - 1) / kPqThreads, kPqBlocks, &p);
+    const int64_t blocks = p.blocks, steps = p.big_steps;
     const int class_rows = pq_class_rows(p.n_units, n_rows);
     const int64_t class_blocks = p.n_units * (((int64_t)n_rows + class_rows - 1) / class_rows);
     DC_REQUIRE(blocks < (1ll << 31) && class_blocks < (1ll << 31), "%s: grid too large", who);
