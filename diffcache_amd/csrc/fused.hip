@@ -303,7 +303,9 @@ __host__ __device__ __forceinline__ int64_t dense_stride(int n_cap) { return ((i
 // worth its poll, so nothing is polled or listed: every row's bucket of (approximation + margin) goes to the row's
 // own place, two bytes, and the exact pass reads them all.  That leaves out the block's closing round trip (the returning
 // atomic that reserves its list slots) and the refresh of the threshold behind it, and the grid can be one of equal
-// shares (sizes and times: plan_dense).
+// shares (sizes and times: plan_dense).  Nor is there a way out for rows that all tie, which a listed scan stops reading (bulk,
+// below): selections among such rows take up to 14 % longer at 256 columns (1 x 131001 rows 140 -> 160 us, 32 x 65001 322 -> 355)
+// and 6 % at 128 (32 x 65001 204 -> 215).
 template <int HD, bool SHARED_POLL, bool DENSE>
 __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kernel(
     const uint8_t *__restrict__ C, const uint16_t *__restrict__ Q, const float *__restrict__ scale,
@@ -1415,7 +1417,7 @@ extern "C" size_t dc_sketch_select_workspace_bytes(int n_units, int n_rows, int 
 
 namespace {
 
-constexpr int kSketchFillBlocks = 512;  // see plan_fused
+constexpr int kFewFillBlocks = 512;  // see plan_fused
 
 struct FusedPlan {
     int n_units, k_eff, small_chunks, big_steps;
@@ -1432,9 +1434,9 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
     // chunks per unit: up to kSmallChunks blocks of one step, then blocks of big_steps steps.
     // Short scans take fewer steps per block so that the grid still has fill_div blocks or
     // more: a block's steps run one after the other, and with few blocks the kernel
-    // lasts as long as its longest block.  (2048 for the bf16 scan; the listed sketch scan,
-    // whose blocks cost more to start and to end than their steps cost, does better with 512:
-    // 34 against 42 us at 8 units x 131072 rows, 37 against 46 us at 32 units x 32768 rows.)
+    // lasts as long as its longest block.  (2048 for the bf16 scan of many units.  With 512, for the sketch scan and the bf16
+    // scan of few units, every scan that is listed at all -- more rows than plan_dense and plan_dense_keys take --
+    // has blocks of big_steps: there a block's start and end cost more than its steps do.)
     const int64_t tiles = ((int64_t)n_rows + rows_per_step - 1) / rows_per_step;
     const int64_t fill = n_units64 * tiles / fill_div;
     if (fill < big_steps) big_steps = fill < 1 ? 1 : (int)fill;
@@ -1566,7 +1568,7 @@ int dc_score_prune_launch(const void *k, const void *q, int n_b, int n_h, int n_
     FusedPlan p;
     // (short scans of up to 32 units: eight steps per block down to 512 blocks, like the sketch scan)
     int rc = plan_fused("dc_score_prune_bf16", n_b, n_h, n_rows, budget, &p, kBigSteps, kRowsPerBlockStep,
-                        (int64_t)n_b * n_h <= 32 ? kSketchFillBlocks : 2048);
+                        (int64_t)n_b * n_h <= 32 ? kFewFillBlocks : 2048);
     if (rc) return rc;
     if (p.n_units == 0 || p.k_eff == 0) return DC_OK;
     FusedWs w;
@@ -1702,7 +1704,7 @@ int dc_sketch_scan_launch(const char *who, const void *k, const uint8_t *codes, 
     DC_REQUIRE(n_rows <= kSketchMaxRows, "%s: %d rows per unit; the sketch scan takes at most %d (use the bf16 scan)", who,
                n_rows, kSketchMaxRows);
     FusedPlan p;
-    int rc = plan_fused(who, n_b, n_h, n_rows, budget, &p, kBigSteps, kRowsPerBlockStep, kSketchFillBlocks);
+    int rc = plan_fused(who, n_b, n_h, n_rows, budget, &p, kBigSteps, kRowsPerBlockStep, kFewFillBlocks);
     if (rc) return rc;
     if (p.n_units == 0 || p.k_eff == 0) return DC_OK;
     const bool dense = plan_dense(p.n_units, n_rows, hd, p.k_eff, &p);

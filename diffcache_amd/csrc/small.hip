@@ -45,8 +45,9 @@ namespace {
 constexpr int kSmallRows = 4096;     // rows a block scores at most (their scores stay in LDS)
 constexpr int kSmallCand = 4096;     // candidates of a unit that are ranked in LDS
 constexpr int kSmallBlocks = 512;    // blocks of a launch at most: two per CU
-constexpr int64_t kSmallTotalRows = 640 * 1024;  // rows of all units that the route takes on (measured crossover)
-// ... and rows per unit when the caller brings a sketch (where it is preferred to the chains: dc_one_kernel_first).
+// Rows of all units that the route is open to, and rows per unit when the caller brings a sketch.  Where it is preferred
+// to the chains: dc_one_kernel_first.
+constexpr int64_t kSmallTotalRows = 640 * 1024;
 constexpr int kSmallSketchRows = 40 * 1024;
 constexpr int kSmallMl = 2048;       // floats of (m, l) the merge keeps in LDS: blocks per unit * G * 2
 

@@ -369,9 +369,8 @@ def test_prepared_layer_call_equals_decode_layer():
 
 
 def test_a_sketch_moves_the_crossover_to_the_chain():
-    """With a sketch the kernel chain is the faster one from about 40 Ki rows per unit on, so the
-    one-kernel route ends there; without a sketch it goes on to 640 Ki rows in all.  Both routes
-    select the same ids."""
+    """With a sketch the one-kernel route ends at 40 Ki rows per unit; without one it goes on to 640 Ki rows in
+    all.  Up to there one or two units of long regions stay with it.  Both routes select the same ids."""
     torch.manual_seed(306)
     b, hq, hkv, hd, budget = 1, 8, 2, 128, 512
     for n_ctx, want_with_sketch in ((40 * 1024 + 68, hip.ROUTE_ONE_KERNEL), (40 * 1024 + 69, hip.ROUTE_SKETCH)):

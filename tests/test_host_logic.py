@@ -84,34 +84,43 @@ def test_route_of_a_region_too_long_for_the_sketch_scan():
     assert _hip.lib.dc_decode_layer_route(ctypes.byref(a)) == _hip.ROUTE_ATTEND_ONLY
 
 
-def test_scan_kernels_do_not_spill():
-    """The scan kernels sit at the edge of their register budget (four waves per SIMD): a change
-    that makes the compiler spill costs them 10 us per launch without failing any parity test, and
-    a lambda that the compiler declines to inline keeps the arrays it is handed in scratch memory
+@pytest.mark.parametrize("source,kernels", [
+    ("fused.hip", ["score_prune_kernel", "sketch_prune_kernel", "pq_scan_kernel", "classify_kernel", "key_classify_kernel",
+                   "pq_classify_kernel", "rescore_kernel", "pq_rescore_kernel", "select_finish_kernel", "select_sorted_kernel"]),
+    ("short.hip", ["short_score_kernel", "short_attend_kernel"]),
+    ("pq.hip", ["pq_adc_kernel", "pq_encode_kernel"]),
+    ("attn.hip", ["gather_attn_mfma_kernel", "merge_kernel"]),
+])
+def test_scan_kernels_do_not_spill(source, kernels):
+    """The kernels of a decode step and of the PQ baseline, many of them at the edge of their register budget (the scans:
+    four waves per SIMD): a change that makes the compiler spill costs a scan 10 us per launch without failing any
+    parity test, and a lambda that the compiler declines to inline keeps the arrays it is handed in scratch memory
     (no "spill" in the report, only a scratch size: the head-dim-256 sketch scan ran at a quarter
-    of its speed that way).  Compiles the file that holds them once more with the compiler's
+    of its speed that way).  Compiles the files that hold them once more with the compiler's
     resource report."""
     import shutil
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc")
-    src = os.path.join(ROOT, "diffcache_amd", "csrc", "fused.hip")
+    src = os.path.join(ROOT, "diffcache_amd", "csrc", source)
     res = subprocess.run([hipcc, "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "--cuda-device-only",
                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-fno-fast-math",
                           "-Rpass-analysis=kernel-resource-usage", "-c", src, "-o", os.devnull],
                          capture_output=True, text=True, cwd=os.path.dirname(src))
     assert res.returncode == 0, res.stderr[-2000:]
-    name, seen, bad = None, 0, []
+    name, seen, bad = None, {}, []
     for line in res.stderr.splitlines():
         m = re.search(r"Function Name: (\S+)", line)
         if m:
             name = m.group(1)
         m = re.search(r"(VGPRs Spill|ScratchSize \[bytes/lane\]): (\d+)", line)
-        if m and name and ("prune_kernel" in name or "rescore_kernel" in name):
-            seen += 1
+        if m and name:
+            seen[name] = seen.get(name, 0) + 1
             if int(m.group(2)) > 0:
                 bad.append((name, m.group(1), int(m.group(2))))
-    assert seen >= 16, "the compiler's report was not understood"
+    # (mangled: a kernel's name stands behind its length)
+    missing = [k for k in kernels if not any(f"{len(k)}{k}" in n for n in seen)]
+    assert not missing and all(c == 2 for c in seen.values()), ("the compiler's report was not understood", missing)
     assert not bad, bad
 
 
