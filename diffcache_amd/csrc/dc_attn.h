@@ -294,7 +294,7 @@ __device__ __forceinline__ void dc_attn_split(const AttnArgs &a, int unit, int s
 //               The result leaves S[row 4q + i][head c], i < 4, in lane (q, c).
 //   O = P V     M = query heads, N = 16 of the HD output columns, K = the rows.  That lane's four
 //               logits per tile are, as they stand, its part of the A operand (head c, rows 4q + i)
-//               once exponentiated and split into two bf16 values (flash_attn_with_kvcache,
+//               once exponentiated and split into three bf16 values (flash_attn_with_kvcache,
 //               base.py:134-142, rounds P to one; that alone misses the 2e-3 bar on short
 //               slices).  The B operand wants, per lane, the values of ITS rows 4q + i
 //               in one output column; column n of instruction j is taken to be d = (HD/16) c + j,
