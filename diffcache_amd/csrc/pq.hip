@@ -96,10 +96,17 @@ __global__ __launch_bounds__(kThreads) void pq_adc_kernel(
 // v_min3, a compare, a select).  At the end the two lanes of a key settle its octet, each lane
 // for the key of one of the wave's two groups (v_permlane32_swap exchanges the halves), and that lane takes
 // the least of the eight in fp32, from tables whose octets are padded apart so that lanes that look at the same place of
-// different octets read different banks at fixed offsets.  200003 keys of 128 columns, 32 subspaces: 75 us, the vector ALUs issuing 95 % of
-// the kernel's time (347 instructions per wave and subspace, 192 of them the search); with tiles of 16 x 16 x 16 (half the rate of
-// the wider ones, four lanes to settle a key through LDS shuffles; 488 instructions) 96, with 32 x 32 x 8 90; torch's
-// distance matrices, written to and read from HBM four times over, took 11.8 ms.
+// different octets read different banks at fixed offsets.
+//
+// A CU holds one block, which stages the tables of its subspaces once and walks the keys; its waves take batches of 64 from a
+// counter in LDS and meet at no barrier.  200003 keys of 128 columns, 32 subspaces: 68 us (275 instructions per wave and subspace,
+// 192 of them the search, the vector ALUs issuing 94 % of the time that a CU is busy).  Blocks of 256 keys that stage for themselves took 75
+// (347 instructions); walking with equal shares per wave 74, because the older waves of a SIMD run ahead and the youngest ends
+// alone; two blocks of half the size per CU 69, one of which runs ahead; a tile's products asked for when the tile before has been searched
+// 66 to 68, 87 % of the time issuing; the last batches dealt out by subspace 69; the octets' numbers as masks in scalar registers, 20
+// instructions less, no faster.  Tiles of 16 x 16 x 16 (half the rate of the wider ones, four lanes to settle a key through LDS
+// shuffles; 488 instructions) took 96 in the blocks of 256 keys, 32 x 32 x 8 90; torch's distance matrices, written to and read from
+// HBM four times over, 11.8 ms.  16 subspaces of 8 columns 64 -> 55 us, 8 of 16 63 -> 51; 5000 keys 11.3 -> 10.6.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -111,18 +118,22 @@ __device__ __forceinline__ void split3(float x, uint32_t &a, uint32_t &b, uint32
     c = __float_as_uint(r - __uint_as_float(b));
 }
 
-constexpr int kEncGroups = 2;                              // groups of 32 keys per wave: one per half of its lanes
-constexpr int kEncKeys = kThreads / 64 * 32 * kEncGroups;  // keys per block
-constexpr int kEncSubs = 4;                                // subspaces per block: their codes leave as one word
-constexpr int kEncHalf = 12;                               // words of an octet's half norms, padded
+constexpr int kEncGroups = 2;                  // groups of 32 keys per wave: one per half of its lanes
+constexpr int kEncBatch = 32 * kEncGroups;     // keys of a wave at a time
+constexpr int kEncHalf = 12;                   // words of an octet's half norms, padded
+// subspaces whose tables a block holds, and whose codes leave together (160 KB of LDS per CU)
+__host__ __device__ constexpr int enc_subs(int ds) { return ds <= 8 ? 4 : 2; }
+// threads of a block, of which a CU takes one
+__host__ __device__ constexpr int enc_threads(int ds) { return ds <= 8 ? 1024 : 512; }
 
 // (At least two waves per SIMD asked for: with up to 256 registers the compiler leaves the results of the
 // matrix instructions in vector registers; with more it moves each through an accumulation register,
 // one instruction per value, which is what the search costs.)
 template <int DS>
-__global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
+__global__ __launch_bounds__(enc_threads(DS), enc_threads(DS) / 256) void pq_encode_kernel(
     const uint16_t *__restrict__ keys, int64_t key_stride, int64_t n, const float *__restrict__ books,
-    uint8_t *__restrict__ codes, int64_t code_stride, int m, int nc) {
+    uint8_t *__restrict__ codes, int64_t code_stride, int m, int nc, int per_column) {
+    constexpr int SUBS = enc_subs(DS), THREADS = enc_threads(DS);
     constexpr int KW = 4;                        // operand words per lane and instruction
     constexpr int NI = DS <= 4 ? 1 : 2;          // instructions per tile and eight columns (four, where there are no more)
     constexpr int KL = DS <= 4 ? 4 : 8;          // columns of a part of the centroid per lane and instruction
@@ -130,42 +141,70 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
     constexpr int XW = (DS + 1) / 2;             // words of a key's columns
     constexpr int kOctet = 8 * DS + (DS < 4 ? DS : 4);  // words of an octet's centroids, padded
     // [tile][instruction][lane][word]: a wave's operand is one stretch
-    __shared__ __align__(16) uint32_t s_a[PARTS][8 * NI * 64 * KW];
-    __shared__ __align__(16) float s_c[32 * kOctet];
-    __shared__ __align__(16) float s_half[32 * kEncHalf];
+    __shared__ __align__(16) uint32_t s_a[SUBS][PARTS][8 * NI * 64 * KW];
+    __shared__ __align__(16) float s_c[SUBS][32 * kOctet];
+    __shared__ __align__(16) float s_half[SUBS][32 * kEncHalf];
+    __shared__ uint32_t s_turn;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = lane >> 5, c = lane & 31;
     // The blocks that read the same keys (a few columns each, of lines they share) are numbered 8 apart:
     // they run on one XCD at about the same time and find the lines in its L2.
-    const int n_y = (m + kEncSubs - 1) / kEncSubs;
-    const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8;
-    const int64_t kblk = (int64_t)(turn / n_y) * 8 + xcd;
-    const int sub0 = (turn % n_y) * kEncSubs;
-    const int n_sub = m - sub0 < kEncSubs ? m - sub0 : kEncSubs;
-    const int64_t key0 = kblk * kEncKeys + wave * (32 * kEncGroups);
-    if (kblk * kEncKeys >= n) return;  // the grid is a whole number of eights
-    const uint16_t *kp[kEncGroups];
+    const int n_y = (m + SUBS - 1) / SUBS;
+    const int turn = blockIdx.x / 8;
+    const int place = turn / n_y * 8 + (int)(blockIdx.x % 8);  // among the blocks of the column
+    const int sub0 = (turn % n_y) * SUBS;
+    const int n_sub = m - sub0 < SUBS ? m - sub0 : SUBS;
+    if (place >= per_column) return;  // the grid is a whole number of eights
+    // stage the subspaces: the negated centroid in three bf16 parts, half its squared norm in three
+    for (int s = tid / 256; s < n_sub; s += THREADS / 256) {
+        const int at_c = tid & 255;  // this thread's centroid
+        // and where it sits among the tiles' rows
+        const int row = 16 * ((at_c >> 4) & 1) + 8 * ((at_c >> 2) & 1) + 4 * ((at_c >> 3) & 1) + (at_c & 3);
+        const float *cp = books + ((int64_t)(sub0 + s) * nc + (at_c < nc ? at_c : nc - 1)) * DS;
+        float cen[DS];
 #pragma unroll
-    for (int g = 0; g < kEncGroups; ++g) {
-        int64_t k = key0 + g * 32 + c;
-        k = k < n ? k : n - 1;
-        kp[g] = keys + k * key_stride;
-    }
-    float cen[DS];  // this thread's centroid of a subspace
-    auto load_centroid = [&](int sub) __attribute__((always_inline)) {
-#pragma unroll
-        for (int d = 0; d < DS; ++d) cen[d] = 0.f;
-        if (tid < nc) {
-            const float *p = books + ((int64_t)sub * nc + tid) * DS;
-#pragma unroll
-            for (int d = 0; d < DS; ++d) cen[d] = p[d];
+        for (int d = 0; d < DS; ++d) {
+            const float v = cp[d];
+            cen[d] = at_c < nc ? v : 0.f;
         }
-    };
-    uint32_t xw[kEncGroups][XW], xn[kEncGroups][XW];
-    auto load_keys = [&](int sub, uint32_t(&x)[kEncGroups][XW]) __attribute__((always_inline)) {
+        float half = 0.f;
+#pragma unroll
+        for (int d = 0; d < DS; ++d) half = fmaf(cen[d], cen[d], half);
+        half = at_c < nc ? 0.5f * half : INFINITY;  // a centroid that does not exist is never the nearest, of no key
+        s_half[s][(at_c >> 3) * kEncHalf + (at_c & 7)] = half;
+#pragma unroll
+        for (int d = 0; d < DS; ++d) s_c[s][(at_c >> 3) * kOctet + (at_c & 7) * DS + d] = cen[d];
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+            uint32_t e[4][KL];  // bf16 values in the upper halves: the three parts, the bias
+#pragma unroll
+            for (int j = 0; j < KL; ++j) {
+                e[0][j] = e[1][j] = e[2][j] = e[3][j] = 0u;
+                if (p * KL + j < DS) split3(-cen[p * KL + j < DS ? p * KL + j : 0], e[0][j], e[1][j], e[2][j]);
+            }
+            if (p == 0) split3(half, e[3][0], e[3][1], e[3][2]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)  // two instructions: r in lane 32 (r % 2) of number r / 2; one: parts 2 l and 2 l + 1 in half l
+#pragma unroll
+                for (int w = 0; w < KL / 2; ++w) {
+                    const int at = NI == 2 ? ((at_c >> 5) * 128 + r * 32 + row) * KW + w : ((at_c >> 5) * 64 + (r / 2) * 32 + row) * KW + 2 * (r % 2) + w;
+                    s_a[s][p][at] = __builtin_amdgcn_perm(e[r][2 * w + 1], e[r][2 * w], 0x07060302u);
+                }
+        }
+    }
+    const uint16_t *kp[kEncGroups];  // the batch that is loaded from
+    auto point = [&](int64_t key0) __attribute__((always_inline)) {
 #pragma unroll
         for (int g = 0; g < kEncGroups; ++g) {
-            const uint16_t *p = kp[g] + sub * DS;
+            int64_t k = key0 + g * 32 + c;
+            k = k < n ? k : n - 1;
+            kp[g] = keys + k * key_stride + sub0 * DS;
+        }
+    };
+    auto load_keys = [&](int s, uint32_t(&x)[kEncGroups][XW]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < kEncGroups; ++g) {
+            const uint16_t *p = kp[g] + s * DS;
             if constexpr (DS == 2) {
                 x[g][0] = *reinterpret_cast<const uint32_t *>(p);
             } else if constexpr (DS == 4) {
@@ -180,39 +219,19 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
             }
         }
     };
-    // where this thread's centroid sits among the tiles' rows
-    const int row = 16 * ((tid >> 4) & 1) + 8 * ((tid >> 2) & 1) + 4 * ((tid >> 3) & 1) + (tid & 3);
+    // The block's waves take its batches as they come: the older waves of a SIMD run ahead of the younger ones, and with equal
+    // shares the youngest would end alone.
+    auto take = [&](int turn) __attribute__((always_inline)) { return ((int64_t)turn * per_column + place) * kEncBatch; };
+    int64_t key0 = take(wave);
+    uint32_t xw[kEncGroups][XW], xn[kEncGroups][XW];
     uint32_t word = 0u;  // the codes of key key0 + lane
-    load_centroid(sub0);
-    load_keys(sub0, xw);
-    for (int s = 0; s < n_sub; ++s) {
-        // stage the subspace: the negated centroid in three bf16 parts, half its squared norm in three
-        float half = 0.f;
-#pragma unroll
-        for (int d = 0; d < DS; ++d) half = fmaf(cen[d], cen[d], half);
-        half = tid < nc ? 0.5f * half : INFINITY;  // a centroid that does not exist is never the nearest, of no key
-        if (s > 0) __syncthreads();               // the last subspace's tables are no longer read
-        s_half[(tid >> 3) * kEncHalf + (tid & 7)] = half;
-#pragma unroll
-        for (int d = 0; d < DS; ++d) s_c[(tid >> 3) * kOctet + (tid & 7) * DS + d] = cen[d];
-#pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
-            uint32_t e[4][KL];  // bf16 values in the upper halves: the three parts, the bias
-#pragma unroll
-            for (int j = 0; j < KL; ++j) {
-                e[0][j] = e[1][j] = e[2][j] = e[3][j] = 0u;
-                if (p * KL + j < DS) split3(-cen[p * KL + j < DS ? p * KL + j : 0], e[0][j], e[1][j], e[2][j]);
-            }
-            if (p == 0) split3(half, e[3][0], e[3][1], e[3][2]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)  // two instructions: r in lane 32 (r % 2) of number r / 2; one: parts 2 l and 2 l + 1 in half l
-#pragma unroll
-                for (int w = 0; w < KL / 2; ++w) {
-                    const int at = NI == 2 ? ((tid >> 5) * 128 + r * 32 + row) * KW + w : ((tid >> 5) * 64 + (r / 2) * 32 + row) * KW + 2 * (r % 2) + w;
-                    s_a[p][at] = __builtin_amdgcn_perm(e[r][2 * w + 1], e[r][2 * w], 0x07060302u);
-                }
-        }
-        __syncthreads();
+    int s = 0;
+    int64_t key_next = n;
+    if (tid == 0) s_turn = THREADS / 64;
+    point(key0);
+    load_keys(0, xw);
+    __syncthreads();
+    while (key0 < n) {
         // the keys' operands: the columns, and ones against the bias
         uint32_t b[kEncGroups][PARTS][NI][KW];
 #pragma unroll
@@ -227,10 +246,15 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
                     b[g][p][0][w] = x;
                     if (NI == 2 || w >= 2) b[g][p][NI - 1][w] = h == 0 ? x : one;
                 }
-        if (s + 1 < n_sub) {  // the next subspace's centroids and columns are on the way meanwhile
-            load_centroid(sub0 + s + 1);
-            load_keys(sub0 + s + 1, xn);
+        // the next columns are on the way meanwhile (past the last key they repeat it)
+        const bool last = s + 1 == n_sub;
+        if (last) {
+            uint32_t turn = 0u;
+            if (lane == 0) turn = atomicAdd(&s_turn, 1u);
+            key_next = take(__builtin_amdgcn_readfirstlane((int)turn));
+            point(key_next);
         }
+        load_keys(last ? 0 : s + 1, xn);
         float best[kEncGroups];
         uint32_t from[kEncGroups];  // 2 * tile + which of its octets
 #pragma unroll
@@ -238,33 +262,20 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
             best[g] = INFINITY;
             from[g] = 0u;
         }
-        uint32_t aw[PARTS][NI][KW], an[PARTS][NI][KW];
-        auto load_tile = [&](int t, uint32_t(&dst)[PARTS][NI][KW]) __attribute__((always_inline)) {
+        uint32_t aw[PARTS][NI][KW];
+        auto load_tile = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
             for (int p = 0; p < PARTS; ++p)
 #pragma unroll
                 for (int i = 0; i < NI; ++i) {
-                    const uint4 v = *reinterpret_cast<const uint4 *>(&s_a[p][((NI * t + i) * 64 + lane) * KW]);
-                    dst[p][i][0] = v.x, dst[p][i][1] = v.y, dst[p][i][2] = v.z, dst[p][i][3] = v.w;
+                    const uint4 v = *reinterpret_cast<const uint4 *>(&s_a[s][p][((NI * t + i) * 64 + lane) * KW]);
+                    aw[p][i][0] = v.x, aw[p][i][1] = v.y, aw[p][i][2] = v.z, aw[p][i][3] = v.w;
                 }
         };
-        load_tile(0, an);
-#pragma unroll  // (whole: the octets' numbers are constants of their instructions then, and so are the tiles' addresses)
-        for (int t = 0; t < 8; ++t) {
-#pragma unroll
-            for (int p = 0; p < PARTS; ++p)
-#pragma unroll
-                for (int i = 0; i < NI; ++i)
-#pragma unroll
-                    for (int w = 0; w < KW; ++w) aw[p][i][w] = an[p][i][w];
-            if (t < 7) load_tile(t + 1, an);  // the next tile is on the way
-            // all products first, then each step of the search for all groups: a result is some dozen
-            // cycles away from its instruction, a compare's mask two from its reader
-            f32x16 d[kEncGroups];
-#pragma unroll
-            for (int g = 0; g < kEncGroups; ++g)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) d[g][i] = 0.f;
+        // A tile's products are asked for before the tile ahead of it is searched, its operands another one earlier: a result is
+        // dozens of cycles away from its instruction.
+        f32x16 d[2][kEncGroups];
+        auto products = [&](f32x16(&dst)[kEncGroups]) __attribute__((always_inline)) {
 #pragma unroll
             for (int p = 0; p < PARTS; ++p)
 #pragma unroll
@@ -273,22 +284,34 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
                     for (int g = 0; g < kEncGroups; ++g) {
                         const uint4 av = make_uint4(aw[p][i][0], aw[p][i][1], aw[p][i][2], aw[p][i][3]);
                         const uint4 bv = make_uint4(b[g][p][i][0], b[g][p][i][1], b[g][p][i][2], b[g][p][i][3]);
-                        d[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
-                                                                       __builtin_bit_cast(bf16x8, bv), d[g], 0, 0, 0);
+                        const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                        dst[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv),
+                                                                         p == 0 && i == 0 ? zero : dst[g], 0, 0, 0);
                     }
+        };
+        load_tile(0);
+        products(d[0]);
+        load_tile(1);
+#pragma unroll  // (whole: the octets' numbers are constants of their instructions then, and so are the tiles' addresses)
+        for (int t = 0; t < 8; ++t) {
             __builtin_amdgcn_sched_barrier(0);
+            if (t < 7) products(d[(t + 1) & 1]);
+            if (t < 6) load_tile(t + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            // each step of the search for all groups: a compare's mask is two cycles from its reader
+            const f32x16(&dt)[kEncGroups] = d[t & 1];
 #pragma unroll
             for (int o = 0; o < 2; ++o) {
                 float v[kEncGroups];
                 bool less[kEncGroups];
 #pragma unroll
-                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(d[g][8 * o], d[g][8 * o + 1]), d[g][8 * o + 2]);
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(dt[g][8 * o], dt[g][8 * o + 1]), dt[g][8 * o + 2]);
 #pragma unroll
-                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][8 * o + 3]), d[g][8 * o + 4]);
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], dt[g][8 * o + 3]), dt[g][8 * o + 4]);
 #pragma unroll
-                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][8 * o + 5]), d[g][8 * o + 6]);
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], dt[g][8 * o + 5]), dt[g][8 * o + 6]);
 #pragma unroll
-                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], d[g][8 * o + 7]), best[g]);
+                for (int g = 0; g < kEncGroups; ++g) v[g] = fminf(fminf(v[g], dt[g][8 * o + 7]), best[g]);
 #pragma unroll
                 for (int g = 0; g < kEncGroups; ++g) less[g] = v[g] < best[g];
 #pragma unroll
@@ -297,7 +320,6 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
                     best[g] = v[g];
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
         }
         // The two lanes of a key hold its least value over their octets each.  The halves of the wave exchange a
         // group: half h ends with both lanes' values for group h.  (Equal values: the lower octet.)
@@ -317,10 +339,10 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
             xf[2 * w] = dc_bf16_lo(x);
             xf[2 * w + 1] = dc_bf16_hi(x);
         }
-        const float4 *hp = reinterpret_cast<const float4 *>(s_half + octet * kEncHalf);
+        const float4 *hp = reinterpret_cast<const float4 *>(s_half[s] + octet * kEncHalf);
         const float4 h0 = hp[0], h1 = hp[1];
         const float hs[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-        const float *cp = s_c + octet * kOctet;
+        const float *cp = s_c[s] + octet * kOctet;
         float dist[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -341,14 +363,22 @@ __global__ __launch_bounds__(kThreads, DS <= 4 ? 4 : 2) void pq_encode_kernel(
         for (int g = 0; g < kEncGroups; ++g)
 #pragma unroll
             for (int w = 0; w < XW; ++w) xw[g][w] = xn[g][w];
-    }
-    const int64_t k = key0 + lane;
-    if (k >= n) return;
-    uint8_t *dst = codes + k * code_stride + sub0;
-    if (n_sub == kEncSubs && (code_stride & 3) == 0) {
-        *reinterpret_cast<uint32_t *>(dst) = word;
-    } else {
-        for (int s = 0; s < n_sub; ++s) dst[s] = (uint8_t)(word >> (8 * s));
+        ++s;
+        if (!last) continue;
+        const int64_t k = key0 + lane;
+        if (k < n) {
+            uint8_t *dst = codes + k * code_stride + sub0;
+            if (SUBS == 4 && n_sub == SUBS && (code_stride & 3) == 0) {
+                *reinterpret_cast<uint32_t *>(dst) = word;
+            } else if (SUBS == 2 && n_sub == SUBS && (code_stride & 1) == 0) {
+                *reinterpret_cast<uint16_t *>(dst) = (uint16_t)word;
+            } else {
+                for (int i = 0; i < n_sub; ++i) dst[i] = (uint8_t)(word >> (8 * i));
+            }
+        }
+        key0 = key_next;
+        s = 0;
+        word = 0u;
     }
 }
 
@@ -367,13 +397,18 @@ extern "C" int dc_pq_encode_bf16(const void *keys, int64_t key_stride, int64_t n
     DC_REQUIRE(((uintptr_t)keys) % align == 0 && key_stride >= hd && (key_stride * 2) % align == 0,
                "%s: keys must be %d-byte aligned, rows included", who, align);
     DC_REQUIRE((((uintptr_t)codes) & 3u) == 0 && code_stride >= m, "%s: codes must be 4-byte aligned, rows of at least m bytes", who);
-    const int64_t blocks = ((n + kEncKeys - 1) / kEncKeys + 7) / 8 * 8 * ((m + kEncSubs - 1) / kEncSubs);
+    // blocks of a column of subspaces: four batches each, until every CU has what it holds
+    const int64_t columns = (m + enc_subs(ds) - 1) / enc_subs(ds), batches = (n + kEncBatch - 1) / kEncBatch;
+    int64_t per_column = 256 / columns;
+    if (per_column > (batches + 3) / 4) per_column = (batches + 3) / 4;
+    if (per_column < 1) per_column = 1;
+    const int64_t blocks = (per_column + 7) / 8 * 8 * columns;
     DC_REQUIRE(blocks < (1ll << 31), "%s: grid too large", who);
     const dim3 grid((unsigned)blocks);
     hipStream_t st = (hipStream_t)stream;
 #define DC_LAUNCH_ENC(DS)                                                                                            \
-    hipLaunchKernelGGL(pq_encode_kernel<DS>, grid, dim3(kThreads), 0, st, (const uint16_t *)keys, key_stride, n, books, \
-                       codes, code_stride, m, n_centroids)
+    hipLaunchKernelGGL(pq_encode_kernel<DS>, grid, dim3(enc_threads(DS)), 0, st, (const uint16_t *)keys, key_stride, n, books, \
+                       codes, code_stride, m, n_centroids, (int)per_column)
     if (ds == 2) DC_LAUNCH_ENC(2);
     else if (ds == 4) DC_LAUNCH_ENC(4);
     else if (ds == 8) DC_LAUNCH_ENC(8);

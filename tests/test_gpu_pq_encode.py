@@ -65,3 +65,18 @@ def test_encode_takes_what_it_took_before():
             want = torch.stack([torch.cdist(keys.float().view(400, m, -1)[:, j].contiguous(), books[j]).argmin(1)
                                 for j in range(m)], 1)
             assert (encode(keys, books).long() != want).float().mean() < 1e-2
+
+
+@pytest.mark.parametrize("m,ds,n", [(32, 4, 33000), (3, 2, 90001), (16, 8, 33000), (5, 16, 30001), (300, 2, 700)])
+def test_codes_do_not_depend_on_how_many_keys_there_are(m, ds, n):
+    """Many keys: a block's waves take several batches each (from 2 ** 15 keys on at 8 columns of blocks), odd numbers of
+    subspaces and columns of blocks that outnumber the CUs.  The same keys a few hundred at a time, a batch per wave, get the same codes."""
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn((n, m * ds), generator=g, device=DEV).to(torch.bfloat16)
+    books = torch.randn((m, 256, ds), generator=g, device=DEV)
+    codes = hip.pq_encode(x, books)
+    for lo in (0, n // 2 - 100, n - 401):
+        assert torch.equal(codes[lo:lo + 401], hip.pq_encode(x[lo:lo + 401].contiguous(), books))
+    far = torch.randn((0, m * ds), device=DEV).to(torch.bfloat16)
+    assert hip.pq_encode(far, books).shape == (0, m)
