@@ -97,6 +97,15 @@ __global__ __launch_bounds__(kThreads) void sketch_quantise_kernel(
     const int64_t r0 = (int64_t)blk * rows_per_block;
     int64_t r1 = r0 + rows_per_block;
     if (r1 > n_rows) r1 = n_rows;
+    // Codes of numbers are rounded by adding a constant whose unit is one (halves go to the even neighbour there too), which leaves the
+    // code in the low byte: 7.4 vector instructions an element instead of 17.  A key that is no number shows in the residual, whose
+    // maximum keeps it; the wave then works the batch out again with every comparison, as it always does where a channel's
+    // scale is so small that a zero times its reciprocal is no number.
+    constexpr float kRound = 12582912.0f + 128.0f;
+    bool odd_scale = false;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) odd_scale |= inv[i] == __builtin_inff();
+    odd_scale = __ballot(odd_scale) != 0ull;
     for (int64_t rb = r0 + grp; rb < r1; rb += GROUPS * kInFlight) {
         uint4 wv[kInFlight];
 #pragma unroll
@@ -105,28 +114,58 @@ __global__ __launch_bounds__(kThreads) void sketch_quantise_kernel(
             r = r < r1 ? r : r1 - 1;
             wv[u] = dc_load_stream16(Ku + r * sr);
         }
+        uint2 packed[kInFlight];
+        bool odd = odd_scale;
+        if (!odd) {
+#pragma unroll
+            for (int u = 0; u < kInFlight; ++u) {  // (past the end the last row once more)
+                const uint4 w = wv[u];
+                const float kv[8] = {dc_bf16_lo(w.x), dc_bf16_hi(w.x), dc_bf16_lo(w.y), dc_bf16_hi(w.y),
+                                     dc_bf16_lo(w.z), dc_bf16_hi(w.z), dc_bf16_lo(w.w), dc_bf16_hi(w.w)};
+                uint32_t y[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float f = __builtin_amdgcn_fmed3f(kv[i] * inv[i], -127.f, 127.f) + kRound;
+                    y[i] = __float_as_uint(f);
+                    res[i] = __builtin_elementwise_maximum(res[i], fabsf(fmaf(-a[i], f - kRound, kv[i])));
+                }
+                constexpr uint32_t kTwo = 0x0c0c0400u, kFour = 0x05040100u;  // the low bytes, the low halves of two words
+                packed[u].x = __builtin_amdgcn_perm(__builtin_amdgcn_perm(y[3], y[2], kTwo), __builtin_amdgcn_perm(y[1], y[0], kTwo), kFour);
+                packed[u].y = __builtin_amdgcn_perm(__builtin_amdgcn_perm(y[7], y[6], kTwo), __builtin_amdgcn_perm(y[5], y[4], kTwo), kFour);
+            }
+            bool nan = false;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) nan |= !(res[i] == res[i]);
+            odd = __ballot(nan) != 0ull;
+        }
+        if (odd) {
+            // a NaN residual must poison the bound, not vanish in the max
+#pragma unroll
+            for (int i = 0; i < 8; ++i) res[i] = res[i] == res[i] ? res[i] : __builtin_inff();
+#pragma unroll
+            for (int u = 0; u < kInFlight; ++u) {
+                const uint4 w = wv[u];
+                const float kv[8] = {dc_bf16_lo(w.x), dc_bf16_hi(w.x), dc_bf16_lo(w.y), dc_bf16_hi(w.y),
+                                     dc_bf16_lo(w.z), dc_bf16_hi(w.z), dc_bf16_lo(w.w), dc_bf16_hi(w.w)};
+                uint32_t code[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    float c = rintf(kv[i] * inv[i]);
+                    c = c > 127.f ? 127.f : (c < -127.f ? -127.f : c);
+                    if (!(c == c)) c = 0.f;  // NaN key or 0 * inf
+                    const float e = fabsf(fmaf(-a[i], c, kv[i]));
+                    if (!(e <= res[i])) res[i] = (e == e) ? e : __builtin_inff();
+                    code[i] = (uint32_t)((int)c + 128);
+                }
+                packed[u].x = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
+                packed[u].y = code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24);
+            }
+        }
 #pragma unroll
         for (int u = 0; u < kInFlight; ++u) {
             const int64_t r = rb + (int64_t)u * GROUPS;
             if (r >= r1) break;
-            const uint4 w = wv[u];
-            const float kv[8] = {dc_bf16_lo(w.x), dc_bf16_hi(w.x), dc_bf16_lo(w.y), dc_bf16_hi(w.y),
-                                 dc_bf16_lo(w.z), dc_bf16_hi(w.z), dc_bf16_lo(w.w), dc_bf16_hi(w.w)};
-            uint32_t code[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                float c = rintf(kv[i] * inv[i]);
-                c = c > 127.f ? 127.f : (c < -127.f ? -127.f : c);
-                if (!(c == c)) c = 0.f;  // NaN key or 0 * inf
-                const float e = fabsf(fmaf(-a[i], c, kv[i]));
-                // a NaN residual must poison the bound, not vanish in the max
-                if (!(e <= res[i])) res[i] = (e == e) ? e : __builtin_inff();
-                code[i] = (uint32_t)((int)c + 128);
-            }
-            uint2 packed;
-            packed.x = code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24);
-            packed.y = code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24);
-            dc_store_stream8(Cu + r * cr, packed);
+            dc_store_stream8(Cu + r * cr, packed[u]);
         }
     }
 #pragma unroll
@@ -151,10 +190,11 @@ __global__ void sketch_finalise_kernel(float *scale, int64_t n) {
 int dc_sketch_quantise_launch(const char *who, const void *k, uint8_t *codes, const float *scale, float *resid,
                               int n_units, int n_h, int n_rows, int hd, int64_t sb, int64_t sh, int64_t sr, int64_t cb,
                               int64_t ch, int64_t cr, int scale_is_amax, float *scale_out, void *stream) {
-    // rows per block: as many as leave about 2048 blocks, from 256 (a block ends with an LDS pass and
-    // HD atomics) to kRowsPerBlock
-    int64_t rpb = (int64_t)n_units * n_rows / 2048 / 256 * 256;
-    rpb = rpb < 256 ? 256 : (rpb > kRowsPerBlock ? kRowsPerBlock : rpb);
+    // Rows per block: 32 KB of keys, so that the blocks that run at a time walk the store together, as the copy that filled it did (longer
+    // blocks are each somewhere else); 256 where there are few rows in all and a block's end, an LDS pass and HD atomics to its
+    // unit's words, shows.  A prompt's layer, us, 32 KB / 64 KB / 128 KB: 16 units x 40003 rows of 128 columns 151 / 156 / 161, 8 x 131072
+    // 244 / 249 / 258, 12 x 24683 of 256 144 / 145 / 148, 16 x 40003 of 64 87 / 88 / 89; but 2 x 50000 of 128 41 / 39 / 40.
+    const int64_t rpb = (int64_t)n_units * n_rows * hd >= (1ll << 24) ? 16384 / hd : 256;
     const int64_t blocks = ((int64_t)n_rows + rpb - 1) / rpb * n_units;
     DC_REQUIRE(blocks < (1ll << 31), "%s: grid too large", who);
     const dim3 grid((unsigned)blocks);
