@@ -9,10 +9,11 @@
 // maxima for the scales, the largest |k|^2 of a head, and copies the rows that also belong to the
 // assembled buffer; the second (sketch_quantise_kernel) reads K back.  Both are bound by HBM:
 // 11 bytes per key element, 9 of which no implementation can do without.  At 16 units x 40003 rows
-// of 128 channels the two take 133 us (656 MB: 4.9 TB/s, the rate of a plain copy on this part) and
-// 49 us (246 MB: 5.0 TB/s); the torch reduction for r_sq, the two ingest calls, the three-pass sketch
-// build and the buffer copies they replace took 7.8 ms per layer, nearly all of it the reduction (one
-// batched product per token and head) and the wait for its result.
+// of 128 channels a layer takes 152 us (902 MB moved: 5.9 TB/s, where a plain copy of 2 GiB reaches 5.0); with blocks that start one after
+// the other and 17 instructions an element in the second pass 181, and the torch reduction for r_sq, the two ingest calls, the
+// three-pass sketch build and the buffer copies they replace 7.8 ms, nearly all of it the reduction (one
+// batched product per token and head) and the wait for its result.  (V stored past the caches and K through them, so that the
+// second pass finds a part of it: both past them 30 us more, both through them 16.  V first and K second in every block: no gain.)
 #include "dc_common.h"
 
 namespace {
@@ -41,9 +42,13 @@ __global__ void prefill_zero_kernel(uint32_t *amax, uint32_t *resid, int64_t n, 
     if (r_sq && i < n_h) r_sq[i] = 0u;
 }
 
-// One block copies rows_per_block rows of one unit, of V (the first half of the grid) or of K.  K goes last
-// so that as much of it as fits is still in the memory-side cache when the quantising pass
-// reads it.  A group of HD/8 lanes owns a row, 16 bytes per lane; a lane keeps its eight columns
+// Blocks of K and V together: they all run at once (a CU holds eight) and end at about the same time.  Per layer, us, with 8192 blocks
+// (fewer for short prompts), which start one after the other in the place of those that end / with 1280: 16 units x 40003 rows of
+// 128 columns 183 / 159, 8 x 32768 108 / 76, 4 x 127284 184 / 133, 64 x 10000 188 / 162, 160 x 2048 123 / 88, 16 x 40003 of 64 123 /
+// 94, 8 x 40003 of 256 179 / 159 (1024 blocks: as much, 2048: 2 to 4 more, 2560: 10 more, 512: 25 more).
+constexpr int64_t kCopyBlocks = 1280;
+
+// One block copies rows_per_block rows of one unit, of V (the first half of the grid) or of K.  A group of HD/8 lanes owns a row, 16 bytes per lane; a lane keeps its eight columns
 // for the whole block, so the column maxima stay in registers.
 template <int HD>
 __global__ __launch_bounds__(kThreads) void prefill_copy_kernel(PrefillCopy a) {
@@ -190,9 +195,11 @@ extern "C" int dc_prefill_layer_bf16(const dc_prefill_args *a, void *stream) {
                            sketch ? (uint32_t *)a->resid : nullptr, n_sc, p.r_sq, a->n_h);
         DC_CHECK_LAUNCH(who);
     }
-    // rows per block: as many as leave about 4096 blocks for K and as many for V, from 64 to 1024
-    int64_t rpb = n_units64 * a->seq / 4096 / 64 * 64;
-    rpb = rpb < 64 ? 64 : (rpb > 1024 ? 1024 : rpb);
+    // Equal shares for kCopyBlocks blocks, 64 rows at least.
+    int64_t chunks = kCopyBlocks / (2 * n_units64);
+    chunks = chunks < 1 ? 1 : chunks;
+    int64_t rpb = ((int64_t)a->seq + chunks - 1) / chunks;
+    rpb = rpb < 64 ? 64 : rpb;
     const int64_t blocks = ((int64_t)a->seq + rpb - 1) / rpb * n_units64;
     DC_REQUIRE(2 * blocks < (1ll << 31), "%s: grid too large", who);
     p.rows_per_block = (int)rpb;
