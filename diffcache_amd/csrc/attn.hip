@@ -37,15 +37,31 @@ __global__ __launch_bounds__(kThreads) void gather_attn_kernel(AttnArgs a) {
 template <int HD>
 __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, int group) {
     extern __shared__ float s_dyn[];
+    // (all arguments at once: read where they are first used, they are half a dozen round trips in a row)
+    asm volatile("" ::"s"(a.Q), "s"(a.K), "s"(a.V), "s"(a.idx), "s"(a.new_k), "s"(a.n_idx_unit), "s"(a.n_recent_dev), "s"(a.recent_lo_dev),
+                 "s"(a.n_h), "s"(a.n_idx), "s"(a.idx_stride), "s"(a.region_lo), "s"(a.n_sink), "s"(a.recent_lo), "s"(a.n_recent),
+                 "s"(a.n_total), "s"(a.n_splits), "s"(a.ksb), "s"(a.ksh), "s"(a.ksr), "s"(a.vsb), "s"(a.vsh), "s"(a.vsr), "s"(group));
     // Split-major: a grid a little larger than what the device holds at once (config 3: 1088
     // blocks on 1024 places) then ends on every unit's last, partial split instead of on the last
     // units' full ones.
-    const int n_units = (int)(gridDim.x / (unsigned)a.n_splits);
-    const int unit = blockIdx.x % n_units, split = blockIdx.x / n_units;
+    const int unit = blockIdx.x, split = blockIdx.y;
+    // the ids of all tiles first: one round trip, which the lengths and the query share (a tile's ids asked for when those of the
+    // tile before were there, behind the lengths and the query: 5.8 us instead of 5.2 at 8 units x 1093 rows of 128 columns)
+    constexpr int TILES = mfma_tiles(HD);
+    uint32_t id[TILES];
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const uint32_t *ids = a.idx + (int64_t)unit * a.idx_stride;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const int p = split * (kAttnWaves * 16 * TILES) + (wave * TILES + t) * 16 + (lane & 15);
+            id[t] = 0u;
+            if (a.n_idx > 0) id[t] = ids[p < a.n_idx ? p : a.n_idx - 1];
+        }
+    }
     AttnFrame<HD> f;
     f.load(a, group, unit);
-    const uint32_t *ids = a.idx + (int64_t)unit * a.idx_stride;
-    dc_attn_split_mfma<HD, kAttnWaves, mfma_tiles(HD)>(a, f, group, unit, split, s_dyn, [ids](int p) { return ids[p]; });
+    dc_attn_split_mfma<HD, kAttnWaves, TILES>(a, f, group, unit, split, s_dyn, [&id](int t, int) { return id[t]; });
 }
 
 // The splits of one query head, combined: out[u, g, :] = sum_s w_s acc_s / sum_s w_s l_s with
@@ -69,6 +85,7 @@ __global__ __launch_bounds__(256) void merge_kernel(const float *__restrict__ ws
                                                     int32_t *__restrict__ adv_state, int adv_limit,
                                                     uint32_t *__restrict__ clear_hist) {
     constexpr int kLanes = HD / 4, kParts = 256 / kLanes;
+    asm volatile("" ::"s"(ws_acc), "s"(ws_ml), "s"(out), "s"(lse), "s"(group), "s"(n_splits), "s"(adv_state), "s"(adv_limit), "s"(clear_hist));
     __shared__ float4 s_acc[256];
     const int ug = blockIdx.x;  // unit * group + g
     const int unit = ug / group, g = ug % group;
@@ -76,40 +93,42 @@ __global__ __launch_bounds__(256) void merge_kernel(const float *__restrict__ ws
     const int64_t slot0 = (int64_t)unit * n_splits * group + g;  // split s at slot0 + s * group
     const float2 *ml = reinterpret_cast<const float2 *>(ws_ml) + slot0;
     const float4 *pa = reinterpret_cast<const float4 *>(ws_acc) + slot0 * kLanes + col;
-    auto load_ml = [&](int sp) __attribute__((always_inline)) {
-        float2 p = make_float2(-INFINITY, 0.f);
-        if (sp < n_splits) p = ml[(int64_t)sp * group];
-        if (!(p.y > 0.f)) p.x = -INFINITY;
-        return p;
+    auto load_ml = [&](int sp) __attribute__((always_inline)) { return ml[(sp < n_splits ? sp : n_splits - 1) * group]; };
+    auto known = [&](float2 p, int sp) __attribute__((always_inline)) {  // a split that counts, or none
+        const bool in = sp < n_splits && p.y > 0.f;
+        return make_float2(in ? p.x : -INFINITY, sp < n_splits ? p.y : 0.f);
     };
     float4 v[kMergeBatch];
     float2 p[kMergeBatch];
+    // (without a branch to a thread: the last split again in the place of one that does not exist, told apart when all are there)
     auto load_rows = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kMergeBatch; ++j) {
-            const int sp = s0 + part + j * kParts;
             v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
             p[j] = make_float2(-INFINITY, 0.f);
-            if (sp < n_splits) {
-                p[j] = ml[(int64_t)sp * group];
-                v[j] = pa[(int64_t)sp * group * kLanes];
+            if (s0 + j * kParts < n_splits) {  // (uniform: what no thread has a split for is not asked for)
+                const int sp = s0 + part + j * kParts, at = (sp < n_splits ? sp : n_splits - 1) * group;
+                p[j] = ml[at];
+                v[j] = pa[(int64_t)at * kLanes];
             }
         }
     };
-    const float2 own = load_ml(lane);
+    float2 own = load_ml(lane);
     load_rows(0);
+    __builtin_amdgcn_sched_barrier(0);
+    own = known(own, lane);
     // the step is counted here because no block of this kernel reads the state
     if (adv_state && blockIdx.x == 0 && tid == 255) dc_state_advance(adv_state, 1, adv_limit);
     if (clear_hist && g == 0)
         reinterpret_cast<uint4 *>(clear_hist + (int64_t)unit * DC_HIST_BINS)[tid] = make_uint4(0u, 0u, 0u, 0u);
     float M = own.x;
-    for (int sp = lane + 64; sp < n_splits; sp += 64) M = fmaxf(M, load_ml(sp).x);
+    for (int sp = lane + 64; sp < n_splits; sp += 64) M = fmaxf(M, known(load_ml(sp), sp).x);
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
     auto weight = [&](float m) __attribute__((always_inline)) { return m > -INFINITY ? __expf(m - M) : 0.f; };
     float L = weight(own.x) * own.y;
     for (int sp = lane + 64; sp < n_splits; sp += 64) {
-        const float2 o = load_ml(sp);
+        const float2 o = known(load_ml(sp), sp);
         L = fmaf(weight(o.x), o.y, L);
     }
 #pragma unroll
@@ -118,11 +137,12 @@ __global__ __launch_bounds__(256) void merge_kernel(const float *__restrict__ ws
     for (int s0 = 0;;) {
 #pragma unroll
         for (int j = 0; j < kMergeBatch; ++j) {
-            const float w = p[j].y > 0.f ? weight(p[j].x) : 0.f;
-            acc.x = fmaf(w, v[j].x, acc.x);
-            acc.y = fmaf(w, v[j].y, acc.y);
-            acc.z = fmaf(w, v[j].z, acc.z);
-            acc.w = fmaf(w, v[j].w, acc.w);
+            const bool in = s0 + part + j * kParts < n_splits;
+            const float w = in && p[j].y > 0.f ? weight(p[j].x) : 0.f;
+            acc.x = fmaf(w, in ? v[j].x : 0.f, acc.x);
+            acc.y = fmaf(w, in ? v[j].y : 0.f, acc.y);
+            acc.z = fmaf(w, in ? v[j].z : 0.f, acc.z);
+            acc.w = fmaf(w, in ? v[j].w : 0.f, acc.w);
         }
         s0 += kParts * kMergeBatch;
         if (s0 >= n_splits) break;
@@ -285,6 +305,7 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
     int rc = 0;
     if (mfma) {
         const size_t lds = mfma_shared_bytes(hd, group);
+        const dim3 grid((unsigned)n_units, (unsigned)plan.n_splits);
         if (hd == 64) hipLaunchKernelGGL(gather_attn_mfma_kernel<64>, grid, dim3(kThreads), lds, st, aa, group);
         else if (hd == 128) hipLaunchKernelGGL(gather_attn_mfma_kernel<128>, grid, dim3(kThreads), lds, st, aa, group);
         else hipLaunchKernelGGL(gather_attn_mfma_kernel<256>, grid, dim3(kThreads), lds, st, aa, group);

@@ -339,6 +339,12 @@ struct AttnFrame {
     dc_u32x4 bq[CH];
     __device__ __forceinline__ void load(const AttnArgs &a, int G, int unit) {
         const int lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+        // (the query first: the lengths are waited for on the spot)
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) {
+            bq[ch] = dc_u32x4{0u, 0u, 0u, 0u};
+            if (c < G) bq[ch] = *reinterpret_cast<const dc_u32x4 *>(a.Q + ((int64_t)unit * G + c) * HD + ch * 32 + q * 8);
+        }
         n_recent = a.n_recent, n_total = a.n_total;
         recent_lo = a.recent_lo_dev ? (int64_t)*a.recent_lo_dev : a.recent_lo;
         if (a.n_recent_dev) {  // the window's length may live on the device (cache_seqlens, base.py:134-142)
@@ -352,15 +358,11 @@ struct AttnFrame {
             const uint32_t ne = a.n_idx_unit[unit];
             n_eff = ne < (uint32_t)a.n_idx ? (int)ne : a.n_idx;
         }
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            bq[ch] = dc_u32x4{0u, 0u, 0u, 0u};
-            if (c < G) bq[ch] = *reinterpret_cast<const dc_u32x4 *>(a.Q + ((int64_t)unit * G + c) * HD + ch * 32 + q * 8);
-        }
     }
 };
 
-// id_of(p): the selected id at position p < n_idx of the unit's list (relative to the region).
+// id_of(t, p): the selected id at position p of the unit's list (relative to the region), which is this lane's of tile t; any value
+// for positions from n_idx on.
 template <int HD, int WAVES, int TILES, typename Ids>
 __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, const AttnFrame<HD> &f, int G, int unit, int split,
                                                    float *s_mem, Ids id_of) {
@@ -385,15 +387,11 @@ __device__ __forceinline__ void dc_attn_split_mfma(const AttnArgs &a, const Attn
     uint32_t rowk[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        const int vj = p0 + t * 16 + c;
-        uint32_t r = 0;
-        if (live(vj)) {
-            if (vj < n_idx) r = (uint32_t)(a.region_lo + id_of(vj));
-            else if (vj < n_idx + n_sink) r = (uint32_t)(vj - n_idx);
-            else if (vj < n_idx + n_sink + n_recent) r = (uint32_t)(f.recent_lo + (vj - n_idx - n_sink));
-            else r = kNewToken;
-        }
-        rowk[t] = r;
+        const int vj = p0 + t * 16 + c, at = vj - n_idx;
+        uint32_t r = at < n_sink + n_recent ? (uint32_t)(f.recent_lo + (at - n_sink)) : kNewToken;
+        r = at < n_sink ? (uint32_t)at : r;
+        r = at < 0 ? (uint32_t)(a.region_lo + id_of(t, vj)) : r;
+        rowk[t] = live(vj) ? r : 0u;
     }
     const __amdgpu_buffer_rsrc_t rk = dc_rows_rsrc(a.K + b * a.ksb + h * a.ksh);
     const __amdgpu_buffer_rsrc_t rv = dc_rows_rsrc(a.V + b * a.vsb + h * a.vsh);

@@ -286,47 +286,48 @@ __device__ __forceinline__ float dc_dot8(const uint4 &w, const float (&q)[8], fl
 // This lane's 8 query values (columns col*8 .. col*8+7) of one unit.  A GQA
 // group (q_group > 1) is averaged in fp32 in ascending head order, divided once
 // and rounded to bf16, as torch's bf16 mean does (diffcache.py:193).  The loads
-// of up to 8 heads are issued together; a serial loop covers larger groups.
-template <int HD>
-__device__ __forceinline__ void dc_load_query(const uint16_t *__restrict__ Q, int64_t unit,
-                                              int q_group, int col, float (&q)[8]) {
-    const uint16_t *qp = Q + unit * q_group * HD + col * 8;
-    uint4 raw[8];
+// of up to 8 heads are issued together, without a branch to a head (the last head again in the place of one that
+// does not exist); a serial loop covers larger groups.  A group of a power of two is multiplied by the exact reciprocal.
+__device__ __forceinline__ void dc_add_head(const uint4 &w, bool in, float (&acc)[8]) {
+    const uint32_t x[4] = {in ? w.x : 0u, in ? w.y : 0u, in ? w.z : 0u, in ? w.w : 0u};
 #pragma unroll
-    for (int g = 0; g < 8; ++g) {
-        raw[g] = make_uint4(0u, 0u, 0u, 0u);
-        if (g < q_group) raw[g] = *reinterpret_cast<const uint4 *>(qp + (int64_t)g * HD);
+    for (int i = 0; i < 4; ++i) {
+        acc[2 * i] += dc_bf16_lo(x[i]);
+        acc[2 * i + 1] += dc_bf16_hi(x[i]);
     }
+}
+template <int HD>
+__device__ __forceinline__ void dc_load_query(const uint16_t *__restrict__ Q, int64_t unit, int q_group, int col, float (&q)[8]) {
+    const uint16_t *qp = Q + unit * q_group * HD + col * 8;
+    auto head = [&](int g) __attribute__((always_inline)) {
+        return *reinterpret_cast<const uint4 *>(qp + (g < q_group ? g : q_group - 1) * HD);
+    };
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+    if (q_group == 1) {
+        dc_add_head(head(0), true, acc);
+    } else if (q_group <= 4) {
+        uint4 raw[4];
 #pragma unroll
-    for (int g = 0; g < 8; ++g) {
-        if (g < q_group) {
-            acc[0] += dc_bf16_lo(raw[g].x);
-            acc[1] += dc_bf16_hi(raw[g].x);
-            acc[2] += dc_bf16_lo(raw[g].y);
-            acc[3] += dc_bf16_hi(raw[g].y);
-            acc[4] += dc_bf16_lo(raw[g].z);
-            acc[5] += dc_bf16_hi(raw[g].z);
-            acc[6] += dc_bf16_lo(raw[g].w);
-            acc[7] += dc_bf16_hi(raw[g].w);
-        }
-    }
-    for (int g = 8; g < q_group; ++g) {
-        const uint4 r = *reinterpret_cast<const uint4 *>(qp + (int64_t)g * HD);
-        acc[0] += dc_bf16_lo(r.x);
-        acc[1] += dc_bf16_hi(r.x);
-        acc[2] += dc_bf16_lo(r.y);
-        acc[3] += dc_bf16_hi(r.y);
-        acc[4] += dc_bf16_lo(r.z);
-        acc[5] += dc_bf16_hi(r.z);
-        acc[6] += dc_bf16_lo(r.w);
-        acc[7] += dc_bf16_hi(r.w);
+        for (int g = 0; g < 4; ++g) raw[g] = head(g);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) dc_add_head(raw[g], g < q_group, acc);
+    } else {
+        uint4 raw[8];
+#pragma unroll
+        for (int g = 0; g < 8; ++g) raw[g] = head(g);
+#pragma unroll
+        for (int g = 0; g < 8; ++g) dc_add_head(raw[g], g < q_group, acc);
+        for (int g = 8; g < q_group; ++g) dc_add_head(*reinterpret_cast<const uint4 *>(qp + (int64_t)g * HD), true, acc);
     }
     if (q_group == 1) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) q[i] = acc[i];
+    } else if ((q_group & (q_group - 1)) == 0) {
+        const float r = 1.0f / (float)q_group;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q[i] = dc_bf16_to_f32(dc_f32_to_bf16(acc[i] * r));
     } else {
         const float n = (float)q_group;
 #pragma unroll

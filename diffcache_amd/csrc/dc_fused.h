@@ -43,9 +43,15 @@ __device__ __forceinline__ uint32_t load_relaxed(const uint32_t *p) {
 
 // Exact threshold bucket of a unit from its complete histogram: the bucket that
 // holds the k-th best key, and how many keys sit in better buckets.  Called by
-// all kThreads threads; the result is uniform.  `wtot`, `sres`: LDS scratch.
-__device__ __forceinline__ void unit_threshold(const uint32_t *__restrict__ hu, uint32_t kk,
-                                               uint32_t *wtot, uint32_t *sres, uint32_t &tb,
+// all kThreads threads; the result is uniform.  `wtot`, `sres`: LDS scratch.  UnitBins asks for the histogram, ahead of other work.
+struct UnitBins {
+    uint4 t[kBinsPerThread / 4];
+    __device__ __forceinline__ void request(const uint32_t *__restrict__ hu) {
+#pragma unroll
+        for (int i = 0; i < kBinsPerThread / 4; ++i) t[i] = reinterpret_cast<const uint4 *>(hu)[threadIdx.x * (kBinsPerThread / 4) + i];
+    }
+};
+__device__ __forceinline__ void unit_threshold(const UnitBins &hist, uint32_t kk, uint32_t *wtot, uint32_t *sres, uint32_t &tb,
                                                uint32_t &c_less) {
     const int tid = threadIdx.x;
     if (tid == 0) {
@@ -56,7 +62,7 @@ __device__ __forceinline__ void unit_threshold(const uint32_t *__restrict__ hu, 
     uint32_t sum = 0;
 #pragma unroll
     for (int i = 0; i < kBinsPerThread / 4; ++i) {
-        const uint4 t = reinterpret_cast<const uint4 *>(hu)[tid * (kBinsPerThread / 4) + i];
+        const uint4 t = hist.t[i];
         bins[4 * i + 0] = t.x;
         bins[4 * i + 1] = t.y;
         bins[4 * i + 2] = t.z;
@@ -81,6 +87,12 @@ __device__ __forceinline__ void unit_threshold(const uint32_t *__restrict__ hu, 
     __syncthreads();
     tb = sres[0];
     c_less = sres[1];
+}
+__device__ __forceinline__ void unit_threshold(const uint32_t *__restrict__ hu, uint32_t kk, uint32_t *wtot, uint32_t *sres,
+                                               uint32_t &tb, uint32_t &c_less) {
+    UnitBins bins;
+    bins.request(hu);
+    unit_threshold(bins, kk, wtot, sres, tb, c_less);
 }
 
 struct FusedWs {

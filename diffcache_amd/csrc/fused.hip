@@ -283,7 +283,12 @@ __device__ __forceinline__ float group_max(float v) {
 // 16 rows x 64 bytes takes half lines, which streaming loads fetch twice (205 us instead of 180 us at 64 units x
 // 131004 rows of 128).  A step of 64 rows of 128 takes 284 vector instructions in all, 532 with fp32 arithmetic on the
 // codes; the kernel is bound by memory latency at few units and by HBM at many.  The first rows, the
-// query, scales and residuals are all requested at the block's start, one round trip instead of three.
+// query, scales and residuals are all requested at the block's start, one round trip instead of three, and little stands in
+// front of them: the arguments are read at once, the unit and the chunk are the grid's dimensions, the heads of a group are asked for without
+// a branch each.  (Clock stamps, 8 x 32533 rows of 128: the first rows are there after 2.8 to 4.5 us, 3.5 to 5.8 before that; the kernel
+// ends after 8.1, 8.9 before.  Two steps of rows ahead instead of one, or the query in front of the rows: no earlier, the memory
+// system is busy by then.)  Layers, us, before / after that and the like of it in the exact pass and the attention: 8 x 32533 29.6 / 28.7, 8 x
+// 131004 46.8 / 46.2, 64 x 65420 126.3 / 123.5, 12 x 24615 of 256 38.9 / 38.0, 8 x 16316 (short chain) 24.5 / 23.6.
 // Measured before / after (kernel trace): 8 x 131004 rows of 128 29.8 / 27.3 us, 4 x 127028 19.6 / 17.7, 64 x 131004
 // 185.1 / 180.8, 8 x 1048508 183.1 / 179.1, 8 x 16323 of 64 11.1 / 9.5.
 constexpr uint32_t kBulkKeep = 96;      // of the 128 rows of a wave's first two steps
@@ -319,6 +324,9 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     constexpr int TILES = 4 * S;          // tiles of a wave's 64 rows
     constexpr int kLoads = TILES * KS;    // 16-byte loads of a lane per step
     constexpr int LPQ = HD / 8;           // lanes that hold a copy of the weights, eight each
+    // (all arguments at once: read where they are first used, they are half a dozen round trips in a row)
+    asm volatile("" ::"s"(C), "s"(Q), "s"(scale), "s"(resid), "s"(hist), "s"(state), "s"(surv), "s"(n_units), "s"(n_h), "s"(n_cap), "s"(cb),
+                 "s"(ch), "s"(cr), "s"(q_group), "s"(mode), "s"(k_eff), "s"(small_chunks), "s"(big_steps), "s"(hi_dev), "s"(lo_row));
     const int n_rows = dc_live_rows(n_cap, hi_dev, lo_row);
     __shared__ uint32_t lhist[DC_HIST_BINS];
     __shared__ __align__(16) uint8_t s_w[4][HD];  // the weights' digits, lowest first
@@ -328,8 +336,7 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     __shared__ uint32_t s_wcnt[kThreads / 64];
     __shared__ uint32_t s_base;
 
-    const int unit = blockIdx.x % n_units;
-    const int chunk = blockIdx.x / n_units;
+    const int unit = blockIdx.x, chunk = blockIdx.y;
     const int b = unit / n_h, h = unit % n_h;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -337,16 +344,15 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     const int grp = lane >> 4, side = S == 1 ? 0 : lane & 1, par = S == 1 ? 0 : (grp ^ lane) & 1;
     const int own_row = S == 1 ? lane : (4 * side + 2 * par + (grp >> 1)) * 8 + ((lane & 15) >> 1);
 
-    const bool small = chunk < small_chunks;
-    const int big_chunks = (int)(gridDim.x / n_units) - small_chunks;
-    const int big_id = small ? 0 : (int)(((int64_t)(chunk - small_chunks) + (int64_t)unit * 7) % big_chunks);
+    const bool small = !DENSE && chunk < small_chunks;
+    const int big_chunks = (int)gridDim.y - small_chunks;
+    const int big_id = DENSE ? chunk : (small ? 0 : (int)(((uint32_t)(chunk - small_chunks) + (uint32_t)unit * 7u) % (uint32_t)big_chunks));
     const int64_t block_row0 =
         small ? (int64_t)chunk * kRowsPerBlockStep
               : (int64_t)small_chunks * kRowsPerBlockStep + (int64_t)big_id * big_steps * kRowsPerBlockStep;
     const int steps = small ? 1 : big_steps;
 
     if (block_row0 >= n_rows) return;  // the grid is laid out for n_cap rows
-    for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
 
     const uint8_t *Cu = C + b * cb + h * ch + (grp * S + side) * 16;
     UnitState *st = state + unit;
@@ -375,6 +381,7 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
     // the first rows are under way while the weights are worked out
     uint4 ca[kLoads], cb2[kLoads];
     load_step(0, ca);
+    for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
 
     // The weights q_d * a_d as whole multiples of 2^w_exp, |multiple| < 2^30, in four signed digits
     // of base 256, and the margin.  Every wave works them out for itself and leaves one digit
@@ -983,6 +990,9 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
     constexpr int LPR = HD / 8;
     constexpr int GROUPS = kThreads / LPR;
     constexpr bool DENSE = PER > 0;
+    if constexpr (DENSE)  // all arguments at once (in the scan, too); the pass over a list is 2 us slower with it
+        asm volatile("" ::"s"(K), "s"(Q), "s"(hist), "s"(state), "s"(surv), "s"(cand_key), "s"(cand_idx), "s"(n_units), "s"(n_h), "s"(n_rows),
+                     "s"(sb), "s"(sh), "s"(sr), "s"(q_group), "s"(mode), "s"(k_eff), "s"(nblk), "s"(hi_dev), "s"(lo_row));
     constexpr int kOwn = DENSE ? PER : kRescoreBatch;  // entries of a thread per batch
     constexpr uint32_t kPer = kOwn * kThreads;
     __shared__ uint32_t cid[kPer];
@@ -990,8 +1000,7 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
     __shared__ uint32_t wtot[kThreads / 64 + 1];
     __shared__ uint32_t sres[2];
     __shared__ uint32_t s_base;
-    const int unit = blockIdx.x % n_units;
-    const int blk = blockIdx.x / n_units;
+    const int unit = blockIdx.x, blk = blockIdx.y;
     const int b = unit / n_h, h = unit % n_h;
     const int tid = threadIdx.x;
     const int grp = tid / LPR, col = tid % LPR;
@@ -1025,9 +1034,9 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
         }
     };
     uint32_t n_s;
+    UnitBins bins;
     if constexpr (DENSE) {
         load_dense(0u);
-        n_s = (uint32_t)dc_live_rows(n_rows, hi_dev, lo_row);
     } else {
 #pragma unroll
         for (int j = 0; j < kRescoreBatch; ++j) {
@@ -1037,10 +1046,13 @@ __global__ __launch_bounds__(kThreads) void rescore_kernel(
         }
         n_s = st->surv_cnt;
     }
+    bins.request(hist + (int64_t)unit * DC_HIST_BINS);
+    __builtin_amdgcn_sched_barrier(0);  // (the query's sums are not worked out ahead of that)
     float q[8];
     dc_load_query<HD>(Q, unit, q_group, col, q);
+    if constexpr (DENSE) n_s = (uint32_t)dc_live_rows(n_rows, hi_dev, lo_row);
     uint32_t tb, c_less;
-    unit_threshold(hist + (int64_t)unit * DC_HIST_BINS, (uint32_t)k_eff, wtot, sres, tb, c_less);
+    unit_threshold(bins, (uint32_t)k_eff, wtot, sres, tb, c_less);
     if (n_s > (uint32_t)n_rows) n_s = n_rows;
     constexpr uint32_t kTile = DENSE ? kPer : (uint32_t)kThreads;
     const uint32_t n_tiles = (n_s + kTile - 1) / kTile;
@@ -1171,6 +1183,8 @@ __global__ __launch_bounds__(kFinalThreads) void select_finish_kernel(
     uint32_t *__restrict__ hist, UnitState *__restrict__ state, uint32_t *__restrict__ cand_key,
     uint32_t *__restrict__ cand_idx, uint32_t *__restrict__ idx_out, int64_t idx_stride,
     uint32_t *__restrict__ sel_keys, int n_rows, int k_eff, int reinit) {
+    asm volatile("" ::"s"(hist), "s"(state), "s"(cand_key), "s"(cand_idx), "s"(idx_out), "s"(idx_stride), "s"(sel_keys), "s"(n_rows), "s"(k_eff),
+                 "s"(reinit));  // all arguments at once
     __shared__ uint32_t lh[kRadixBins];
     __shared__ uint32_t wtot[kFinalThreads / 64 + 1];
     __shared__ uint32_t sres[4];
@@ -1722,7 +1736,7 @@ int dc_sketch_scan_launch(const char *who, const void *k, const uint8_t *codes, 
     }
     if (ev_scan_begin) (void)hipEventRecord((hipEvent_t)ev_scan_begin, st);
 #define DC_LAUNCH_SK(HD, SP, DN)                                                                    \
-    hipLaunchKernelGGL((sketch_prune_kernel<HD, SP, DN>), dim3((unsigned)p.blocks), dim3(kThreads), 0, st,  \
+    hipLaunchKernelGGL((sketch_prune_kernel<HD, SP, DN>), dim3((unsigned)p.n_units, (unsigned)(p.blocks / p.n_units)), dim3(kThreads), 0, st,  \
                        codes, (const uint16_t *)q, scale, resid, w.hist, w.state, w.surv, p.n_units,    \
                        n_h, n_rows, cb, ch, cr, q_group, mode, p.k_eff, p.small_chunks, p.big_steps, hi_dev, lo_row)
     const bool shared_poll = p.n_units <= kSharedPollUnits;
@@ -1790,7 +1804,7 @@ int dc_sketch_select_impl(const void *k, const uint8_t *codes, const float *scal
         nblk = tiles < cap ? tiles : cap;
     }
 #define DC_LAUNCH_RSP(HD, PER)                                                                        \
-    hipLaunchKernelGGL((rescore_kernel<HD, PER>), dim3((unsigned)p.n_units * (unsigned)nblk), dim3(kThreads), 0, \
+    hipLaunchKernelGGL((rescore_kernel<HD, PER>), dim3((unsigned)p.n_units, (unsigned)nblk), dim3(kThreads), 0, \
                        st, (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv, w.cand_key, \
                        w.cand_idx, p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, nblk, hi_dev, lo_row)
 #define DC_LAUNCH_RS(HD)                        \

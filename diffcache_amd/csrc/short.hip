@@ -77,8 +77,10 @@ __global__ __launch_bounds__(kThreads) void short_score_kernel(
     constexpr int PART = 64 / LPR * NL;       // rows of a part
     constexpr int WAVES = kThreads / 64;
     __shared__ uint32_t lhist[DC_HIST_BINS];
+    asm volatile("" ::"s"(K), "s"(Q), "s"(hist), "s"(keys), "s"(key_stride), "s"(n_units), "s"(n_h), "s"(n_cap), "s"(sb), "s"(sh), "s"(sr),
+                 "s"(q_group), "s"(mode), "s"(parts), "s"(hi_dev), "s"(lo_row));  // all arguments at once
     const int n_rows = dc_live_rows(n_cap, hi_dev, lo_row);
-    const int unit = blockIdx.x % n_units, blk = blockIdx.x / n_units;
+    const int unit = blockIdx.x, blk = blockIdx.y;
     const int b = unit / n_h, h = unit % n_h;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int grp = lane / LPR, col = lane % LPR;
@@ -483,7 +485,7 @@ __global__ __launch_bounds__(kSplitThreads) void short_attend_kernel(AttnArgs a,
     }
     const uint32_t *own = sh.own;
     dc_attn_split_mfma<HD, kSplitWaves, 1>(a, f, group, unit, split, s_dyn,
-                                           [own, slot0](int p) { return own[(uint32_t)p - slot0]; });
+                                           [own, slot0](int, int p) { return own[((uint32_t)p - slot0) % kSplitRows]; });
 }
 
 // Blocks of the score kernel, where rows allow: two per CU.  Between 256 and 1024 a layer of up to 8 units x 8 Ki rows
@@ -586,7 +588,7 @@ int dc_short_layer(const dc_layer_args *a, int region, int k_eff, void *sel_ws, 
     const bool fine = region <= 2 * 4 * kSplitThreads;  // NV <= 2 of short_attend_kernel
     if (a->ev_scan_begin) (void)hipEventRecord((hipEvent_t)a->ev_scan_begin, st);
 #define DC_LAUNCH_SSF(HD, FN)                                                                                         \
-    hipLaunchKernelGGL((short_score_kernel<HD, FN>), dim3((unsigned)(n_units * bpu)), dim3(kThreads), 0, st, k_region,       \
+    hipLaunchKernelGGL((short_score_kernel<HD, FN>), dim3((unsigned)n_units, (unsigned)bpu), dim3(kThreads), 0, st, k_region,       \
                        (const uint16_t *)a->q, w.hist, keys, key_stride, n_units, a->n_h, region, a->kv_batch_stride,  \
                        a->kv_head_stride, a->kv_row_stride, a->group, a->mode, (int)parts, a->region_hi_dev, a->n_sink)
 #define DC_LAUNCH_SS(HD)                    \
