@@ -138,13 +138,18 @@ __host__ __device__ __forceinline__ int64_t dense_key_stride(int n_cap) { return
 
 // DENSE: for scans of more than 768 rows a unit and up to 1.75 Mi in all (plan_dense_keys), as in the sketch scan below:
 // every row's 32-bit key goes to the row's own place, nothing is polled, staged or listed, and blocks of equal shares all
-// run at once.
+// run at once.  Its loads come in halves of a step (quarters at 256 columns), two of them in flight, the first two ahead of the query; a
+// step's sixteen at a time, behind the query and behind the step before them: per layer, us, 32 units x 49933 rows of 128 95.2 / 93.4, 4 x
+// 127028 44.8 / 43.1, 16 x 65404 of 64 44.5 / 43.6, 64 x 16432 71.8 / 71.1, 8 x 131004 67.5 / 67.9.
 template <int HD, bool DENSE>
 __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, uint2 *__restrict__ surv, int n_units, int n_h, int n_cap,
     int64_t sb, int64_t sh, int64_t sr, int q_group, int mode, int k_eff, int small_chunks,
     int big_steps, const int32_t *__restrict__ hi_dev, int lo_row) {
+    if constexpr (DENSE)  // all arguments at once: read where they are first used, they are half a dozen round trips in a row
+        asm volatile("" ::"s"(K), "s"(Q), "s"(hist), "s"(surv), "s"(n_units), "s"(n_h), "s"(n_cap), "s"(sb), "s"(sh), "s"(sr), "s"(q_group),
+                     "s"(mode), "s"(big_steps), "s"(hi_dev), "s"(lo_row));
     constexpr int LPR = HD / 8;
     constexpr int CH = LPR < 16 ? LPR : 16;
     __shared__ uint32_t lhist[DC_HIST_BINS];
@@ -154,18 +159,17 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     __shared__ uint32_t s_base;
     const int n_rows = dc_live_rows(n_cap, hi_dev, lo_row);
 
-    const int unit = blockIdx.x % n_units;
-    const int chunk = blockIdx.x / n_units;
+    const int unit = blockIdx.x, chunk = blockIdx.y;
     const int b = unit / n_h, h = unit % n_h;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int grp = lane / LPR, col = lane % LPR;
 
-    const bool small = chunk < small_chunks;
+    const bool small = !DENSE && chunk < small_chunks;
     // Units sit a power of two apart in memory; rotating each unit's order of large
     // chunks keeps blocks that run together from walking the same address offsets.
-    const int big_chunks = (int)(gridDim.x / n_units) - small_chunks;
-    const int big_id = small ? 0 : (int)(((int64_t)(chunk - small_chunks) + (int64_t)unit * 7) % big_chunks);
+    const int big_chunks = (int)gridDim.y - small_chunks;
+    const int big_id = DENSE ? chunk : (small ? 0 : (int)(((uint32_t)(chunk - small_chunks) + (uint32_t)unit * 7u) % (uint32_t)big_chunks));
     const int64_t block_row0 =
         small ? (int64_t)chunk * kRowsPerBlockStep
               : (int64_t)small_chunks * kRowsPerBlockStep + (int64_t)big_id * big_steps * kRowsPerBlockStep;
@@ -178,12 +182,73 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
         for (int64_t r = (block_row0 > n_rows ? block_row0 : (int64_t)n_rows) + tid; r < end; r += kThreads) du[r] = kNoRow;
     }
     if (block_row0 >= n_rows) return;  // the grid is laid out for n_cap rows
-    for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
 
     const uint16_t *Ku = K + b * sb + h * sh + col * 8;
     UnitState *st = state + unit;
     const int last = n_rows - 1;
-    uint32_t tb = DENSE ? (uint32_t)DC_HIST_BINS : load_relaxed(&st->tb_run);
+    if constexpr (DENSE) {
+        // A step's rows in parts of eight loads, two of them on the way at any time, the first two before the query is there; past the
+        // end of the block its last row again, so that the number of loads in flight is known.
+        constexpr int NL = 8, PARTS = LPR / NL;
+        const int64_t blk_end = block_row0 + (int64_t)steps * kRowsPerBlockStep - 1;
+        const int64_t blk_last = blk_end < (int64_t)last ? blk_end : (int64_t)last;
+        auto load_part = [&](int i, uint4 (&w)[NL]) __attribute__((always_inline)) {
+            const int64_t row = block_row0 + (int64_t)(i / PARTS) * kRowsPerBlockStep + wave * 64 + grp * LPR + i % PARTS * NL;
+#pragma unroll
+            for (int j = 0; j < NL; ++j) {
+                const int64_t at = row + j > blk_last ? blk_last : row + j;
+                w[j] = dc_load_stream16(Ku + at * sr);
+            }
+        };
+        uint4 wa[NL], wb[NL];
+        load_part(0, wa);
+        load_part(1, wb);
+        for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
+        float q[8];
+        dc_load_query<HD>(Q, unit, q_group, col, q);
+        __syncthreads();
+        const int64_t first = block_row0 + wave * 64;
+        int my_steps = 0;  // of this wave, those that hold rows
+        if (first < n_rows) {
+            const int64_t left = ((int64_t)n_rows - first + kRowsPerBlockStep - 1) / kRowsPerBlockStep;
+            my_steps = left < steps ? (int)left : steps;
+        }
+        float mine = 0.f;
+        auto work_part = [&](int i, const uint4 (&w)[NL]) __attribute__((always_inline)) {
+            const int c0 = i % PARTS * NL;
+#pragma unroll
+            for (int j = 0; j < NL; ++j) {
+                const float p = dc_group_sum<LPR>(dc_dot8(w[j], q, 0.f));
+                mine = col == c0 + j ? p : mine;
+            }
+            if (i % PARTS != PARTS - 1) return;
+            const int64_t row = first + (int64_t)(i / PARTS) * kRowsPerBlockStep + lane;
+            if (row < n_rows) {
+                uint32_t key, bucket;
+                dc_key_bucket(mine, mode, key, bucket);
+                du[row] = key < kNoRow ? key : kNoRow - 1u;
+                atomicAdd(&lhist[bucket], 1u);
+            }
+        };
+        const int parts = my_steps * PARTS;
+        int i = 0;
+        for (; i + 1 < parts; i += 2) {
+            work_part(i, wa);
+            load_part(i + 2, wa);
+            work_part(i + 1, wb);
+            load_part(i + 3, wb);
+        }
+        if (i < parts) work_part(i, wa);
+        __syncthreads();
+        uint32_t *hu = hist + (int64_t)unit * DC_HIST_BINS;
+        for (int i = tid; i < DC_HIST_BINS; i += kThreads) {
+            const uint32_t c = lhist[i];
+            if (c) atomicAdd(&hu[i], c);
+        }
+        return;
+    }
+    for (int i = tid; i < DC_HIST_BINS; i += kThreads) lhist[i] = 0;
+    uint32_t tb = load_relaxed(&st->tb_run);
 
     float q[8];
     dc_load_query<HD>(Q, unit, q_group, col, q);
@@ -210,7 +275,7 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
                 w[j] = dc_load_stream16(Ku + r * sr);
             }
             // the threshold for the next step queues up behind this step's rows
-            if (!DENSE && c0 + CH >= LPR && step + 1 < steps) tb_next = load_relaxed(&st->tb_run);
+            if (c0 + CH >= LPR && step + 1 < steps) tb_next = load_relaxed(&st->tb_run);
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 float p = dc_group_sum<LPR>(dc_dot8(w[j], q, 0.f));
@@ -221,13 +286,6 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
         const bool valid = myrow < n_rows;
         uint32_t key = 0, bucket = 0xffffffffu;
         if (valid) dc_key_bucket(mine, mode, key, bucket);
-        if (DENSE) {
-            if (valid) {
-                du[myrow] = key < kNoRow ? key : kNoRow - 1u;
-                atomicAdd(&lhist[bucket], 1u);
-            }
-            continue;
-        }
         // Only rows that can still matter are kept and counted: the final threshold
         // bucket is never worse than tb, so it is fixed by the counts of buckets <= tb.
         const bool keep = valid && bucket <= tb;
@@ -236,15 +294,6 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
         if (keep) wstage[wcnt + __popcll(mask & lt)] = make_uint2((uint32_t)myrow, __float_as_uint(mine));
         wcnt += (uint32_t)__popcll(mask);
         tb = tb_next;
-    }
-    if (DENSE) {
-        __syncthreads();
-        uint32_t *hu = hist + (int64_t)unit * DC_HIST_BINS;
-        for (int i = tid; i < DC_HIST_BINS; i += kThreads) {
-            const uint32_t c = lhist[i];
-            if (c) atomicAdd(&hu[i], c);
-        }
-        return;
     }
     // every 4th small block and every 8th large one refresh the running threshold
     const bool refresh = small ? (chunk & 3) == 3 : ((chunk - small_chunks) & 7) == 7;
@@ -1514,7 +1563,7 @@ int dense_per_thread(int64_t n_units, int n_rows) {
 //
 // Its grid, selections alone, us: up to 640 tiles of 256 rows a block each (24 x 5424 of 128: 264 blocks of two tiles 19.7, 528
 // of one 18.3); then 512 blocks, 1024 from 64 units on (64 x 16000 of 128 59.0 / 56.5, listed 55.1).  Above 1 Mi rows, where
-// every share is long, 1280 blocks (a CU holds five) up to 32 units and 128 columns (16 x 100003 of 64 48.7 / 45.7, listed
+// every share is long, 1280 blocks (a CU holds four; 1024: 95.5 us instead of 93.2 a layer of 32 x 49933 rows of 128) up to 32 units and 128 columns (16 x 100003 of 64 48.7 / 45.7, listed
 // 47.5), and at 256 columns from 9 to 64 units one per CU (32 x 50000 144.5 / 139.5, listed 139.0).
 constexpr int64_t kDenseKeyTiles = (7ll << 18) / kRowsPerBlockStep;  // 1.75 Mi rows
 constexpr int kDenseKeyRows = 768;
@@ -1591,7 +1640,7 @@ int dc_score_prune_launch(const void *k, const void *q, int n_b, int n_h, int n_
     const bool dense = plan_dense_keys(p.n_units, n_rows, hd, &p);
     hipStream_t st = (hipStream_t)stream;
 #define DC_LAUNCH_SPD(HD, DN)                                                                      \
-    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dim3((unsigned)p.blocks), dim3(kThreads), 0, st, \
+    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dim3((unsigned)p.n_units, (unsigned)(p.blocks / p.n_units)), dim3(kThreads), 0, st, \
                        (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv,          \
                        p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, p.small_chunks,  \
                        p.big_steps, hi_dev, lo_row)
