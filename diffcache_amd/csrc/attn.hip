@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kThreads) void gather_attn_kernel(AttnArgs a) {
 
 // The same split on the matrix cores (dc_attn_split_mfma); the group is a run-time value here
 // because the products are padded to 16 heads anyway.
-template <int HD>
+template <int HD, int TILES>
 __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, int group) {
     extern __shared__ float s_dyn[];
     // (all arguments at once: read where they are first used, they are half a dozen round trips in a row)
@@ -47,7 +47,6 @@ __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, 
     const int unit = blockIdx.x, split = blockIdx.y;
     // the ids of all tiles first: one round trip, which the lengths and the query share (a tile's ids asked for when those of the
     // tile before were there, behind the lengths and the query: 5.8 us instead of 5.2 at 8 units x 1093 rows of 128 columns)
-    constexpr int TILES = mfma_tiles(HD);
     uint32_t id[TILES];
     {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -222,12 +221,22 @@ static bool attn_use_mfma(int group, int64_t max_row, int64_t ksr, int64_t vsr) 
     return (max_row + 1) * sr * 2 <= 0xffffffffll;
 }
 
-extern "C" size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_rows_attended) {
+// what a call cannot do without
+static size_t attn_least_bytes(int n_units, int group, int hd, int n_rows_attended) {
     if (n_units <= 0 || group <= 0 || hd < 8) return 256;
     // room for either split body (the slices of the VALU version are shorter for large groups)
     const size_t a = carve_attn(nullptr, n_units, group, hd, plan_attn(hd, group, n_rows_attended, false).n_splits).bytes;
     const size_t b = carve_attn(nullptr, n_units, group, hd, plan_attn(hd, group, n_rows_attended, true).n_splits).bytes;
     return a > b ? a : b;
+}
+
+extern "C" size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_rows_attended) {
+    const size_t least = attn_least_bytes(n_units, group, hd, n_rows_attended);
+    if (n_units <= 0 || group <= 0 || hd < 8) return least;
+    // and for slices of 64 rows, which this list or a shorter one takes where there is room
+    const int most = attn_fine_rows(n_units), n = n_rows_attended < most ? n_rows_attended : most;
+    const size_t fine = carve_attn(nullptr, n_units, group, hd, plan_attn(hd, group, n, true, true).n_splits).bytes;
+    return least > fine ? least : fine;
 }
 
 // Argument checks and the two launches shared by dc_gather_attn_bf16 (caller's workspace),
@@ -269,8 +278,14 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
                "%s: workspace must be non-null and 256-byte aligned", who);
     const bool mfma = attn_use_mfma(group, recent_lo + n_recent, ksr, vsr);
     DC_REQUIRE(mfma || group <= 8, "%s: group %d needs rows within 4 GiB of the unit's first row", who, group);
-    const AttnPlan plan = plan_attn(hd, group, n_total, mfma);
-    const AttnWs w = carve_attn(workspace, n_units, group, hd, plan.n_splits);
+    bool fine = mfma && hd <= 128 && n_total <= attn_fine_rows(n_units);
+    AttnPlan plan = plan_attn(hd, group, n_total, mfma, fine);
+    AttnWs w = carve_attn(workspace, n_units, group, hd, plan.n_splits);
+    if (fine && workspace_bytes < w.bytes) {  // (a workspace of fewer slices, the static scratch among them)
+        fine = false;
+        plan = plan_attn(hd, group, n_total, mfma);
+        w = carve_attn(workspace, n_units, group, hd, plan.n_splits);
+    }
     if (workspace_bytes < w.bytes) {
         dc_set_error("%s: workspace %zu bytes < %zu needed", who, workspace_bytes, w.bytes);
         return DC_ENOMEM;
@@ -306,9 +321,14 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
     if (mfma) {
         const size_t lds = mfma_shared_bytes(hd, group);
         const dim3 grid((unsigned)n_units, (unsigned)plan.n_splits);
-        if (hd == 64) hipLaunchKernelGGL(gather_attn_mfma_kernel<64>, grid, dim3(kThreads), lds, st, aa, group);
-        else if (hd == 128) hipLaunchKernelGGL(gather_attn_mfma_kernel<128>, grid, dim3(kThreads), lds, st, aa, group);
-        else hipLaunchKernelGGL(gather_attn_mfma_kernel<256>, grid, dim3(kThreads), lds, st, aa, group);
+#define DC_LAUNCH_GA(HD, TILES) \
+    hipLaunchKernelGGL((gather_attn_mfma_kernel<HD, TILES>), grid, dim3(kThreads), lds, st, aa, group)
+        if (hd == 64 && fine) DC_LAUNCH_GA(64, 1);
+        else if (hd == 64) DC_LAUNCH_GA(64, 2);
+        else if (hd == 128 && fine) DC_LAUNCH_GA(128, 1);
+        else if (hd == 128) DC_LAUNCH_GA(128, 2);
+        else DC_LAUNCH_GA(256, 1);
+#undef DC_LAUNCH_GA
     } else if (hd == 64) rc = launch_attn<64>(group, grid, st, aa);
     else if (hd == 128) rc = launch_attn<128>(group, grid, st, aa);
     else rc = launch_attn<256>(group, grid, st, aa);
@@ -376,7 +396,7 @@ extern "C" int dc_gather_attn_static_bf16(const void *q, const void *k, const vo
     DC_REQUIRE(n_units < (1 << 20), "%s: too many units", who);
     const int64_t n_total = (int64_t)n_idx + n_sink + n_recent + (new_k ? 1 : 0);
     DC_REQUIRE(n_total < (1ll << 31), "%s: too many rows", who);
-    const size_t need = dc_attn_workspace_bytes((int)n_units, group, hd, (int)n_total);
+    const size_t need = attn_least_bytes((int)n_units, group, hd, (int)n_total);
     if (need > kStaticScratchBytes) {
         dc_set_error("%s: %lld units x %lld attended rows (group %d, head_dim %d) need %zu bytes of scratch; "
                      "the static scratch holds %zu (use dc_gather_attn_bf16 with a workspace)",

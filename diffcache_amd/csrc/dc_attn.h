@@ -26,10 +26,18 @@ struct AttnPlan {
     int n_splits;
 };
 
-// mfma: the split runs on the matrix cores (dc_attn_split_mfma), whose slice does not depend on the group
-inline AttnPlan plan_attn(int hd, int group, int n_total, bool mfma) {
+// Slices of 64 rows instead of 128 (up to 128 columns) where that leaves no more of them than CUs: a CU takes some 45 KB of rows in a
+// microsecond.  Rows of a unit's list up to which that holds.  Per layer, us, 128 / 64 rows: 8 units x 1093 rows of 128
+// columns 28.5 / 27.9 (144 blocks), 8 x 581 43.6 / 43.0, 2 x 1093 29.3 / 28.7, 8 x 1093 of 64 30.2 / 29.7; but 16 x 1093 44.7 / 45.2 (288), 32 x 581
+// 67.7 / 68.3, 8 x 2117 46.6 / 46.9 (272).
+constexpr int kFineBlocks = 256;
+inline int attn_fine_rows(int n_units) { return kFineBlocks / (n_units > 0 ? n_units : 1) * 64; }
+
+// mfma: the split runs on the matrix cores (dc_attn_split_mfma), whose slice does not depend on the group; fine: of 64 rows at any
+// head_dim
+inline AttnPlan plan_attn(int hd, int group, int n_total, bool mfma, bool fine = false) {
     AttnPlan p;
-    p.rows_per_split = mfma ? kAttnWaves * 16 * (hd <= 128 ? 2 : 1) : (kAttnThreads / (hd / 8)) * rows_per_group(group);
+    p.rows_per_split = mfma ? kAttnWaves * 16 * (hd <= 128 && !fine ? 2 : 1) : (kAttnThreads / (hd / 8)) * rows_per_group(group);
     p.n_splits = n_total > 0 ? (n_total + p.rows_per_split - 1) / p.rows_per_split : 1;
     return p;
 }
@@ -312,7 +320,6 @@ typedef uint32_t dc_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t dc_u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kMfmaMaxGroup = 16;
-__host__ __device__ constexpr int mfma_tiles(int hd) { return hd <= 128 ? 2 : 1; }
 // bytes of LDS: per-wave maxima and sums of 16 heads, per-wave partial outputs of G heads
 inline size_t mfma_shared_bytes(int hd, int group, int waves = kAttnWaves) {
     return (size_t)(2 * waves * 16 + waves * group * hd) * sizeof(float);
