@@ -353,9 +353,9 @@ struct AttnFrame {
             if (c < G) bq[ch] = *reinterpret_cast<const dc_u32x4 *>(a.Q + ((int64_t)unit * G + c) * HD + ch * 32 + q * 8);
         }
         n_recent = a.n_recent, n_total = a.n_total;
-        recent_lo = a.recent_lo_dev ? (int64_t)*a.recent_lo_dev : a.recent_lo;
+        recent_lo = a.recent_lo_dev ? (int64_t)dc_step_word(a.recent_lo_dev) : a.recent_lo;
         if (a.n_recent_dev) {  // the window's length may live on the device (cache_seqlens, base.py:134-142)
-            int cur = *a.n_recent_dev;
+            int cur = dc_step_word(a.n_recent_dev);
             cur = cur < 0 ? 0 : (cur < n_recent ? cur : n_recent);
             n_total -= n_recent - cur;
             n_recent = cur;

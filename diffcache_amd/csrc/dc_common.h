@@ -261,12 +261,18 @@ __device__ __forceinline__ float dc_group_sum(float v) {
     return v;
 }
 
+// A device word of the step (dc_step_state) that no block of the reading kernel changes: a scalar load, also where the compiler can no
+// longer tell that nothing does.
+__device__ __forceinline__ int32_t dc_step_word(const int32_t *p) {
+    return *(const __attribute__((address_space(4))) int32_t *)p;
+}
+
 // Rows of a retrieval region that are live.  The kernels' grids and lists are laid out for
 // n_cap rows; with hi_dev the region ends at the row that device word names (it moves up when the
 // recent window is rolled over, between replays of a captured step), lo_row being its first row.
 __device__ __forceinline__ int dc_live_rows(int n_cap, const int32_t *hi_dev, int lo_row) {
     if (!hi_dev) return n_cap;
-    const int v = *hi_dev - lo_row;
+    const int v = dc_step_word(hi_dev) - lo_row;
     return v < 0 ? 0 : (v < n_cap ? v : n_cap);
 }
 
