@@ -98,9 +98,9 @@ __global__ __launch_bounds__(kThreads) void sketch_quantise_kernel(
     int64_t r1 = r0 + rows_per_block;
     if (r1 > n_rows) r1 = n_rows;
     // Codes of numbers are rounded by adding a constant whose unit is one (halves go to the even neighbour there too), which leaves the
-    // code in the low byte: 7.4 vector instructions an element instead of 17.  A key that is no number shows in the residual, whose
-    // maximum keeps it; the wave then works the batch out again with every comparison, as it always does where a channel's
-    // scale is so small that a zero times its reciprocal is no number.
+    // code in the low byte: 7.4 vector instructions an element instead of 17.  A key that is not finite leaves a residual that is infinite
+    // or no number, whose maximum keeps it; the wave then works the batch out again with every comparison, and the rest of its block, as
+    // it always does where a channel's scale is so small that a zero times its reciprocal is no number.
     constexpr float kRound = 12582912.0f + 128.0f;
     bool odd_scale = false;
 #pragma unroll
@@ -133,10 +133,10 @@ __global__ __launch_bounds__(kThreads) void sketch_quantise_kernel(
                 packed[u].x = __builtin_amdgcn_perm(__builtin_amdgcn_perm(y[3], y[2], kTwo), __builtin_amdgcn_perm(y[1], y[0], kTwo), kFour);
                 packed[u].y = __builtin_amdgcn_perm(__builtin_amdgcn_perm(y[7], y[6], kTwo), __builtin_amdgcn_perm(y[5], y[4], kTwo), kFour);
             }
-            bool nan = false;
+            bool wide = false;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) nan |= !(res[i] == res[i]);
-            odd = __ballot(nan) != 0ull;
+            for (int i = 0; i < 8; ++i) wide |= !(res[i] < __builtin_inff());
+            odd = __ballot(wide) != 0ull;
         }
         if (odd) {
             // a NaN residual must poison the bound, not vanish in the max

@@ -55,3 +55,26 @@ def test_codes_scales_and_bounds(kind, hd, rows):
             assert np.array_equal(codes[u], c)
             assert np.array_equal(scale[u], s)
             assert np.array_equal(resid[u], np.maximum(r, before[u]) if keep else r)
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_infinite_keys_in_a_channel_that_was_zeros_at_the_fit(hd):
+    """A kept scale of zero: the product of the key and the reciprocal is no number there, the residual is infinite and the code that of
+    zero, in every row and whatever else is in its batch."""
+    from diffcache_amd import _hip as hip
+    g = torch.Generator().manual_seed(hd)
+    k = torch.randn((1, 2, 700, hd), generator=g)
+    k[:, :, :, 3] = 0.0
+    k = k.to(torch.bfloat16)
+    sk = hip.Sketch(k.to(DEV)).build(k.to(DEV), 0, 700)
+    scale, before = (t.cpu().reshape(2, hd).numpy().copy() for t in (sk.scale, sk.resid))
+    k[0, 0, 350, 3] = float("inf")
+    k[0, 1, 1, 3] = float("nan")
+    k[0, 1, 699, 3] = float("-inf")
+    sk.build(k.to(DEV), 0, 700, keep_scale=True)
+    codes = sk.codes.cpu().reshape(2, -1, hd)[:, :700].numpy()
+    for u in range(2):
+        c, _, r = _want(k.float()[0, u].numpy(), scale[u])
+        assert np.array_equal(codes[u], c)
+        assert np.array_equal(sk.resid.cpu().reshape(2, hd).numpy()[u], np.maximum(r, before[u]))
+        assert np.array_equal(sk.scale.cpu().reshape(2, hd).numpy()[u], scale[u])
