@@ -47,6 +47,11 @@ __global__ void prefill_zero_kernel(uint32_t *amax, uint32_t *resid, int64_t n, 
 // 128 columns 183 / 159, 8 x 32768 108 / 76, 4 x 127284 184 / 133, 64 x 10000 188 / 162, 160 x 2048 123 / 88, 16 x 40003 of 64 123 /
 // 94, 8 x 40003 of 256 179 / 159 (1024 blocks: as much, 2048: 2 to 4 more, 2560: 10 more, 512: 25 more).
 constexpr int64_t kCopyBlocks = 1280;
+// Beyond 64 units and 80 Mi key elements more and shorter blocks, which start one after the other: there a block of 1280 is a whole prompt of
+// its unit or a large part of it.  Per layer, us, 8192 / 1280 / these: 256 units x 4000 rows of 128 columns 297 / 329 / 293, 160 x 8000 372 /
+// 404 / 354, 320 x 4000 386 / 423 / 369, 400 x 4096 433 / 459 / 428, 400 x 4000 of 64 233 / 256 / 227, 328 x 2048 196 / 183 / 172; 320 x 4000
+// of 64, just below, 205 / 185 / 193.  (Pieces of 64 rows: 200 x 4000 215 -> 209, 256 x 2000 of 256 columns 250 -> 242; 16 x 40003, below, 154 -> 157.)
+constexpr int64_t kCopyBlocksMany = 6144, kManyUnits = 64, kManyElements = 80ll << 20;
 
 // One block copies rows_per_block rows of one unit, of V (the first half of the grid) or of K.  A group of HD/8 lanes owns a row, 16 bytes per lane; a lane keeps its eight columns
 // for the whole block, so the column maxima stay in registers.
@@ -195,10 +200,12 @@ extern "C" int dc_prefill_layer_bf16(const dc_prefill_args *a, void *stream) {
                            sketch ? (uint32_t *)a->resid : nullptr, n_sc, p.r_sq, a->n_h);
         DC_CHECK_LAUNCH(who);
     }
-    // Equal shares for kCopyBlocks blocks, 64 rows at least.
-    int64_t chunks = kCopyBlocks / (2 * n_units64);
+    // Equal shares for kCopyBlocks blocks, 64 rows at least; in long copies of many units more and shorter ones, whole pieces of 64 rows.
+    const bool many = n_units64 > kManyUnits && n_units64 * a->seq * a->hd > kManyElements;
+    int64_t chunks = (many ? kCopyBlocksMany : kCopyBlocks) / (2 * n_units64);
     chunks = chunks < 1 ? 1 : chunks;
     int64_t rpb = ((int64_t)a->seq + chunks - 1) / chunks;
+    if (many) rpb = (rpb + 63) / 64 * 64;
     rpb = rpb < 64 ? 64 : rpb;
     const int64_t blocks = ((int64_t)a->seq + rpb - 1) / rpb * n_units64;
     DC_REQUIRE(2 * blocks < (1ll << 31), "%s: grid too large", who);

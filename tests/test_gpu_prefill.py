@@ -112,3 +112,12 @@ def test_a_prefill_under_capture_is_refused():
     with torch.cuda.graph(torch.cuda.CUDAGraph()):
         with pytest.raises(Exception, match="captured"):
             cache.prefill_update_kv_cache(k, k, 0)
+
+
+@pytest.mark.parametrize("hd,b,h,seq,prefix,suffix", [
+    (64, 41, 8, 300, 4, 64),         # one block to a unit's whole prompt
+    (128, 11, 8, 7450, 4, 64),       # just beyond 80 Mi key elements of 88 units: shorter blocks, in pieces of 64 rows
+    (256, 65, 1, 5043, 128, 128),    # the same of 256 columns, one unit beyond the line
+])
+def test_prefills_of_many_units_match_copies_and_sketch_build(hd, b, h, seq, prefix, suffix):
+    test_prefill_layer_matches_copies_and_sketch_build(hd, b, h, seq, prefix, suffix)
