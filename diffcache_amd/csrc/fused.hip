@@ -166,10 +166,14 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     const int grp = lane / LPR, col = lane % LPR;
 
     const bool small = !DENSE && chunk < small_chunks;
-    // Units sit a power of two apart in memory; rotating each unit's order of large
-    // chunks keeps blocks that run together from walking the same address offsets.
-    const int big_chunks = (int)gridDim.y - small_chunks;
-    const int big_id = DENSE ? chunk : (small ? 0 : (int)(((uint32_t)(chunk - small_chunks) + (uint32_t)unit * 7u) % (uint32_t)big_chunks));
+    // Units may sit a power of two apart in memory; rotating each unit's order of chunks keeps blocks that run together from walking
+    // the same address offsets: large chunks of the listed scan by seven a unit; those of the dense scan, of which a grid holds few, so
+    // that the units start evenly apart.  (Dense, per layer, us, without / by seven / evenly: 8 units of 131072 rows of 128 columns 74.1 / 65.2 /
+    // 64.6, 4 of 262144 71.0 / 69.3 / 65.6, 8 of 65536 of 256 71.1 / 67.1 / 67.0, 4 of 131072 of 256 70.9 / 69.4 / 66.1; 8 of 140128 of 128 69.3 /
+    // - / 70.6.  Not at 64 columns: 8 of 131072 40.7 / 41.9 / 42.0, 32 of 50129 57.9 / - / 60.1; in the dense sketch scan it changes nothing.)
+    const uint32_t chunks = gridDim.y - (DENSE ? 0u : (uint32_t)small_chunks), at = (uint32_t)(chunk - (DENSE ? 0 : small_chunks));
+    const uint32_t apart = !DENSE ? 7u : (HD == 64 ? 0u : (chunks > gridDim.x ? chunks / gridDim.x : 1u));
+    const int big_id = DENSE && HD == 64 ? chunk : (small ? 0 : (int)((at + (uint32_t)unit * apart) % chunks));
     const int64_t block_row0 =
         small ? (int64_t)chunk * kRowsPerBlockStep
               : (int64_t)small_chunks * kRowsPerBlockStep + (int64_t)big_id * big_steps * kRowsPerBlockStep;
