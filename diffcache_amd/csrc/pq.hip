@@ -126,13 +126,45 @@ __host__ __device__ constexpr int enc_subs(int ds) { return ds <= 8 ? 4 : 2; }
 // threads of a block, of which a CU takes one
 __host__ __device__ constexpr int enc_threads(int ds) { return ds <= 8 ? 1024 : 512; }
 
+// Blocks of a column of subspaces, of the last one, which may have fewer of them, of all.
+struct EncGrid {
+    int per_column, last, blocks;
+};
+
+// A block per CU, in shares as equal as they come: the last column gets blocks by its number of subspaces.  Where the columns do not divide
+// the CUs, or outnumber them, more and shorter blocks may fill them better in two or more turns, each of which costs a block about four
+// batches to stage and start.  (256 / columns blocks of each, in a grid rounded up to eights, gave XCDs unequal numbers of them, some more than
+// they have CUs.  200003 keys, us, blocks of 256 keys / that / this: 12 subspaces of 8 columns 50 / 67 / 43, 6 of 16 58 / 64 / 41, 24 of
+// 4 58 / 94 / 53, 96 of 2 207 / 347 / 194, 5 of 8 29 / 25 / 20; 30001 keys, 272 of 2 95 / 276 / 93, 1040 of 2 384 / 2213 / 390.)
+static bool plan_encode(int m, int subs, int64_t n, EncGrid *g) {
+    const int64_t columns = (m + subs - 1) / subs, batches = (n + kEncBatch - 1) / kEncBatch;
+    const int64_t whole = columns > 1 ? subs : m, last = m - (columns - 1) * subs;  // subspaces of a column, of the last
+    auto last_of = [&](int64_t per) { return (per * last + whole - 1) / whole; };
+    auto all_of = [&](int64_t per) { return (columns - 1) * per + last_of(per); };
+    const int64_t most = (batches + 3) / 4;  // four batches each at least
+    int64_t best = INT64_MAX, at = 1;
+    for (int64_t turns = 1; turns <= 8; ++turns) {
+        int64_t per = 256 * turns * whole / m + 1;
+        while (per > 1 && all_of(per) > 256 * turns) --per;
+        if (per > most) per = most;
+        const int64_t cost = (all_of(per) + 255) / 256 * ((batches + per - 1) / per + 4);
+        if (cost < best) best = cost, at = per;
+        if (per == most || all_of(per) == 256 * turns) break;
+    }
+    if (all_of(at) >= (1ll << 31)) return false;
+    g->per_column = (int)at;
+    g->last = (int)last_of(at);
+    g->blocks = (int)all_of(at);
+    return true;
+}
+
 // (At least two waves per SIMD asked for: with up to 256 registers the compiler leaves the results of the
 // matrix instructions in vector registers; with more it moves each through an accumulation register,
 // one instruction per value, which is what the search costs.)
 template <int DS>
 __global__ __launch_bounds__(enc_threads(DS), enc_threads(DS) / 256) void pq_encode_kernel(
     const uint16_t *__restrict__ keys, int64_t key_stride, int64_t n, const float *__restrict__ books,
-    uint8_t *__restrict__ codes, int64_t code_stride, int m, int nc, int per_column) {
+    uint8_t *__restrict__ codes, int64_t code_stride, int m, int nc, EncGrid grid) {
     constexpr int SUBS = enc_subs(DS), THREADS = enc_threads(DS);
     constexpr int KW = 4;                        // operand words per lane and instruction
     constexpr int NI = DS <= 4 ? 1 : 2;          // instructions per tile and eight columns (four, where there are no more)
@@ -147,14 +179,23 @@ __global__ __launch_bounds__(enc_threads(DS), enc_threads(DS) / 256) void pq_enc
     __shared__ uint32_t s_turn;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = lane >> 5, c = lane & 31;
-    // The blocks that read the same keys (a few columns each, of lines they share) are numbered 8 apart:
-    // they run on one XCD at about the same time and find the lines in its L2.
+    // The blocks that read the same keys (a few columns each, of lines they share) are next to each other in an order of which every XCD
+    // takes an eighth in one piece: they run on one XCD at about the same time and find the lines in its L2.
     const int n_y = (m + SUBS - 1) / SUBS;
-    const int turn = blockIdx.x / 8;
-    const int place = turn / n_y * 8 + (int)(blockIdx.x % 8);  // among the blocks of the column
-    const int sub0 = (turn % n_y) * SUBS;
+    const int xcd = blockIdx.x % 8, more = grid.blocks % 8;
+    int at = xcd * (grid.blocks / 8) + (xcd < more ? xcd : more) + (int)blockIdx.x / 8;
+    int place, col;  // among the blocks of the column; the column
+    if (at < grid.last * n_y) {
+        place = at / n_y;
+        col = at % n_y;
+    } else {  // the last column has no more
+        at -= grid.last * n_y;
+        place = grid.last + at / (n_y - 1);
+        col = at % (n_y - 1);
+    }
+    const int per_column = col == n_y - 1 ? grid.last : grid.per_column;
+    const int sub0 = col * SUBS;
     const int n_sub = m - sub0 < SUBS ? m - sub0 : SUBS;
-    if (place >= per_column) return;  // the grid is a whole number of eights
     // stage the subspaces: the negated centroid in three bf16 parts, half its squared norm in three
     for (int s = tid / 256; s < n_sub; s += THREADS / 256) {
         const int at_c = tid & 255;  // this thread's centroid
@@ -397,18 +438,13 @@ extern "C" int dc_pq_encode_bf16(const void *keys, int64_t key_stride, int64_t n
     DC_REQUIRE(((uintptr_t)keys) % align == 0 && key_stride >= hd && (key_stride * 2) % align == 0,
                "%s: keys must be %d-byte aligned, rows included", who, align);
     DC_REQUIRE((((uintptr_t)codes) & 3u) == 0 && code_stride >= m, "%s: codes must be 4-byte aligned, rows of at least m bytes", who);
-    // blocks of a column of subspaces: four batches each, until every CU has what it holds
-    const int64_t columns = (m + enc_subs(ds) - 1) / enc_subs(ds), batches = (n + kEncBatch - 1) / kEncBatch;
-    int64_t per_column = 256 / columns;
-    if (per_column > (batches + 3) / 4) per_column = (batches + 3) / 4;
-    if (per_column < 1) per_column = 1;
-    const int64_t blocks = (per_column + 7) / 8 * 8 * columns;
-    DC_REQUIRE(blocks < (1ll << 31), "%s: grid too large", who);
-    const dim3 grid((unsigned)blocks);
+    EncGrid g;
+    DC_REQUIRE(plan_encode(m, enc_subs(ds), n, &g), "%s: grid too large", who);
+    const dim3 grid((unsigned)g.blocks);
     hipStream_t st = (hipStream_t)stream;
 #define DC_LAUNCH_ENC(DS)                                                                                            \
     hipLaunchKernelGGL(pq_encode_kernel<DS>, grid, dim3(enc_threads(DS)), 0, st, (const uint16_t *)keys, key_stride, n, books, \
-                       codes, code_stride, m, n_centroids, (int)per_column)
+                       codes, code_stride, m, n_centroids, g)
     if (ds == 2) DC_LAUNCH_ENC(2);
     else if (ds == 4) DC_LAUNCH_ENC(4);
     else if (ds == 8) DC_LAUNCH_ENC(8);

@@ -80,3 +80,32 @@ def test_codes_do_not_depend_on_how_many_keys_there_are(m, ds, n):
         assert torch.equal(codes[lo:lo + 401], hip.pq_encode(x[lo:lo + 401].contiguous(), books))
     far = torch.randn((0, m * ds), device=DEV).to(torch.bfloat16)
     assert hip.pq_encode(far, books).shape == (0, m)
+
+
+@pytest.mark.parametrize("m,ds,n", [(5, 8, 33000), (6, 16, 20001), (12, 8, 33000), (7, 2, 90001), (33, 4, 20001), (96, 2, 9001), (136, 2, 5003),
+                                    (1, 8, 33000), (27, 16, 3001), (1040, 2, 700)])
+def test_codes_of_columns_that_do_not_divide_the_grid(m, ds, n):
+    """Columns of subspaces that do not divide an XCD's CUs, a last column of fewer subspaces, more columns than CUs."""
+    test_codes_do_not_depend_on_how_many_keys_there_are(m, ds, n)
+
+
+@pytest.mark.parametrize("m,ds,like,n", [(12, 8, 16, 200003), (24, 4, 32, 200003), (96, 2, 64, 100003), (272, 2, 128, 60001)])
+def test_a_subspace_takes_no_longer_where_their_number_is_no_power_of_two(m, ds, like, n):
+    """Blocks that the CUs or the XCDs hold unequal numbers of are twice as long; `like` subspaces fill both evenly."""
+    from diffcache_amd import _hip as hip
+    took = []
+    for mm in (m, like):
+        x = torch.randn((n, mm * ds), device=DEV).to(torch.bfloat16)
+        books = torch.randn((mm, 256, ds), device=DEV)
+        times = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            hip.pq_encode(x, books)
+            a.record()
+            for _ in range(5):
+                hip.pq_encode(x, books)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        took.append(min(times) / mm)
+    assert took[0] < 1.3 * took[1]
