@@ -233,9 +233,11 @@ static size_t attn_least_bytes(int n_units, int group, int hd, int n_rows_attend
 extern "C" size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_rows_attended) {
     const size_t least = attn_least_bytes(n_units, group, hd, n_rows_attended);
     if (n_units <= 0 || group <= 0 || hd < 8) return least;
-    // and for slices of 64 rows, which this list or a shorter one takes where there is room
-    const int most = attn_fine_rows(n_units), n = n_rows_attended < most ? n_rows_attended : most;
-    const size_t fine = carve_attn(nullptr, n_units, group, hd, plan_attn(hd, group, n, true, true).n_splits).bytes;
+    // And for slices of 64 rows, which a list of up to so many rows takes where there is room: those of this call or, so that a workspace
+    // for more units or rows is enough for fewer, of any smaller one.
+    if (hd > 128) return least;
+    const int64_t slices = n_units * (n_rows_attended > 0 ? ((int64_t)n_rows_attended + 63) / 64 : 1);
+    const size_t fine = carve_attn(nullptr, 1, group, hd, slices < kFineBlocks ? (int)slices : kFineBlocks).bytes;
     return least > fine ? least : fine;
 }
 

@@ -380,3 +380,18 @@ def test_layer_workspace_of_a_long_region_covers_every_shorter_one(n_units):
     regions = sorted({r + d for r in (256, 1024, 4096, 16384, 32768, 40960, 65536, 81920, 131072) for d in (-68, 0, 1, 60)})
     need = [lib.dc_layer_workspace_bytes(n_units, r, 1024, 4, 128, 1024 + 4 + 128 + 1) for r in regions]
     assert all(a <= b for a, b in zip(need, need[1:]))
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_attention_workspace_of_more_units_or_rows_covers_fewer(hd):
+    """A workspace laid out once for the largest batch and list serves every smaller one: also where only the smaller
+    one takes slices of 64 rows."""
+    from diffcache_amd import _hip
+    rows = [1, 63, 64, 65, 127, 128, 129, 192, 256, 300, 1000, 1024, 1093, 2048, 4097, 16384, 16385, 40000]
+    for group in (1, 4, 12, 16):
+        before = [0] * len(rows)
+        for units in range(1, 300):
+            need = [_hip.lib.dc_attn_workspace_bytes(units, group, hd, n) for n in rows]
+            assert all(a <= b for a, b in zip(need, need[1:])), (units, group)
+            assert all(a <= b for a, b in zip(before, need)), (units, group)
+            before = need
