@@ -44,7 +44,8 @@ __global__ __launch_bounds__(kThreads) void gather_attn_mfma_kernel(AttnArgs a, 
     // Split-major: a grid a little larger than what the device holds at once (config 3: 1088
     // blocks on 1024 places) then ends on every unit's last, partial split instead of on the last
     // units' full ones.
-    const int unit = blockIdx.x, split = blockIdx.y;
+    const int unit = blockIdx.x, split = dc_chunk();
+    if (split >= a.n_splits) return;
     // the ids of all tiles first: one round trip, which the lengths and the query share (a tile's ids asked for when those of the
     // tile before were there, behind the lengths and the query: 5.8 us instead of 5.2 at 8 units x 1093 rows of 128 columns)
     uint32_t id[TILES];
@@ -322,7 +323,7 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
     int rc = 0;
     if (mfma) {
         const size_t lds = mfma_shared_bytes(hd, group);
-        const dim3 grid((unsigned)n_units, (unsigned)plan.n_splits);
+        const dim3 grid = dc_unit_grid(n_units, plan.n_splits);
 #define DC_LAUNCH_GA(HD, TILES) \
     hipLaunchKernelGGL((gather_attn_mfma_kernel<HD, TILES>), grid, dim3(kThreads), lds, st, aa, group)
         if (hd == 64 && fine) DC_LAUNCH_GA(64, 1);

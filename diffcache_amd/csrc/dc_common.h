@@ -261,6 +261,15 @@ __device__ __forceinline__ float dc_group_sum(float v) {
     return v;
 }
 
+// Blocks of a grid whose first dimension is the units and whose others are the chunks of a unit, which need not fit the second (it and the
+// third hold 65535): the kernel numbers them with dc_chunk() and leaves those beyond the last alone.
+constexpr int kMostChunksY = 32768;
+inline dim3 dc_unit_grid(int n_units, int64_t chunks) {
+    return dim3((unsigned)n_units, (unsigned)(chunks < kMostChunksY ? chunks : kMostChunksY),
+                (unsigned)((chunks + kMostChunksY - 1) / kMostChunksY));
+}
+__device__ __forceinline__ int dc_chunk() { return (int)(blockIdx.z * (unsigned)kMostChunksY + blockIdx.y); }
+
 // A device word of the step (dc_step_state) that no block of the reading kernel changes: a scalar load, also where the compiler can no
 // longer tell that nothing does.
 __device__ __forceinline__ int32_t dc_step_word(const int32_t *p) {

@@ -146,10 +146,10 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, uint2 *__restrict__ surv, int n_units, int n_h, int n_cap,
     int64_t sb, int64_t sh, int64_t sr, int q_group, int mode, int k_eff, int small_chunks,
-    int big_steps, const int32_t *__restrict__ hi_dev, int lo_row) {
+    int big_steps, int n_chunks, const int32_t *__restrict__ hi_dev, int lo_row) {
     if constexpr (DENSE)  // all arguments at once: read where they are first used, they are half a dozen round trips in a row
         asm volatile("" ::"s"(K), "s"(Q), "s"(hist), "s"(surv), "s"(n_units), "s"(n_h), "s"(n_cap), "s"(sb), "s"(sh), "s"(sr), "s"(q_group),
-                     "s"(mode), "s"(big_steps), "s"(hi_dev), "s"(lo_row));
+                     "s"(mode), "s"(big_steps), "s"(n_chunks), "s"(hi_dev), "s"(lo_row));
     constexpr int LPR = HD / 8;
     constexpr int CH = LPR < 16 ? LPR : 16;
     __shared__ uint32_t lhist[DC_HIST_BINS];
@@ -159,7 +159,8 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     __shared__ uint32_t s_base;
     const int n_rows = dc_live_rows(n_cap, hi_dev, lo_row);
 
-    const int unit = blockIdx.x, chunk = blockIdx.y;
+    const int unit = blockIdx.x, chunk = DENSE ? (int)blockIdx.y : dc_chunk();
+    if (!DENSE && chunk >= n_chunks) return;
     const int b = unit / n_h, h = unit % n_h;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     // that the units start evenly apart.  (Dense, per layer, us, without / by seven / evenly: 8 units of 131072 rows of 128 columns 74.1 / 65.2 /
     // 64.6, 4 of 262144 71.0 / 69.3 / 65.6, 8 of 65536 of 256 71.1 / 67.1 / 67.0, 4 of 131072 of 256 70.9 / 69.4 / 66.1; 8 of 140128 of 128 69.3 /
     // - / 70.6.  Not at 64 columns: 8 of 131072 40.7 / 41.9 / 42.0, 32 of 50129 57.9 / - / 60.1; in the dense sketch scan it changes nothing.)
-    const uint32_t chunks = gridDim.y - (DENSE ? 0u : (uint32_t)small_chunks), at = (uint32_t)(chunk - (DENSE ? 0 : small_chunks));
+    const uint32_t chunks = (uint32_t)(n_chunks - (DENSE ? 0 : small_chunks)), at = (uint32_t)(chunk - (DENSE ? 0 : small_chunks));
     const uint32_t apart = !DENSE ? 7u : (HD == 64 ? 0u : (chunks > gridDim.x ? chunks / gridDim.x : 1u));
     const int big_id = DENSE && HD == 64 ? chunk : (small ? 0 : (int)((at + (uint32_t)unit * apart) % chunks));
     const int64_t block_row0 =
@@ -352,6 +353,7 @@ constexpr uint32_t kBulkKeep = 96;      // of the 128 rows of a wave's first two
 // such regions down the bf16 route.
 constexpr int kSketchRowBits = 22;
 constexpr int kSketchMaxRows = 1 << kSketchRowBits;
+static_assert(kSketchMaxRows / kRowsPerBlockStep <= 65535, "the chunks of a unit are the second dimension of the scan's grid");
 static_assert(kSketchMaxRows == DC_SKETCH_MAX_ROWS && DC_HIST_BINS <= (1 << (32 - kSketchRowBits)), "row and bucket share a word");
 __device__ __forceinline__ uint32_t sketch_entry(uint32_t bucket, uint32_t row) { return (bucket << kSketchRowBits) | row; }
 // words of two bytes between the units of a dense scan's buckets (16-byte rows of them)
@@ -1644,10 +1646,10 @@ int dc_score_prune_launch(const void *k, const void *q, int n_b, int n_h, int n_
     const bool dense = plan_dense_keys(p.n_units, n_rows, hd, &p);
     hipStream_t st = (hipStream_t)stream;
 #define DC_LAUNCH_SPD(HD, DN)                                                                      \
-    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dim3((unsigned)p.n_units, (unsigned)(p.blocks / p.n_units)), dim3(kThreads), 0, st, \
+    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dc_unit_grid(p.n_units, p.blocks / p.n_units), dim3(kThreads), 0, st, \
                        (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv,          \
                        p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, p.small_chunks,  \
-                       p.big_steps, hi_dev, lo_row)
+                       p.big_steps, (int)(p.blocks / p.n_units), hi_dev, lo_row)
 #define DC_LAUNCH_SP(HD)                    \
     do {                                    \
         if (dense) DC_LAUNCH_SPD(HD, true); \
