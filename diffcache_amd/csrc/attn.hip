@@ -222,18 +222,12 @@ static bool attn_use_mfma(int group, int64_t max_row, int64_t ksr, int64_t vsr) 
     return (max_row + 1) * sr * 2 <= 0xffffffffll;
 }
 
-// what a call cannot do without
-static size_t attn_least_bytes(int n_units, int group, int hd, int n_rows_attended) {
+extern "C" size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_rows_attended) {
     if (n_units <= 0 || group <= 0 || hd < 8) return 256;
     // room for either split body (the slices of the VALU version are shorter for large groups)
     const size_t a = carve_attn(nullptr, n_units, group, hd, plan_attn(hd, group, n_rows_attended, false).n_splits).bytes;
     const size_t b = carve_attn(nullptr, n_units, group, hd, plan_attn(hd, group, n_rows_attended, true).n_splits).bytes;
-    return a > b ? a : b;
-}
-
-extern "C" size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_rows_attended) {
-    const size_t least = attn_least_bytes(n_units, group, hd, n_rows_attended);
-    if (n_units <= 0 || group <= 0 || hd < 8) return least;
+    const size_t least = a > b ? a : b;
     // And for slices of 64 rows, which a list of up to so many rows takes where there is room: those of this call or, so that a workspace
     // for more units or rows is enough for fewer, of any smaller one.
     if (hd > 128) return least;
@@ -284,7 +278,7 @@ int dc_gather_attn_common(const char *who, const void *q, const void *k, const v
     bool fine = mfma && hd <= 128 && n_total <= attn_fine_rows(n_units);
     AttnPlan plan = plan_attn(hd, group, n_total, mfma, fine);
     AttnWs w = carve_attn(workspace, n_units, group, hd, plan.n_splits);
-    if (fine && workspace_bytes < w.bytes) {  // (a workspace of fewer slices, the static scratch among them)
+    if (fine && workspace_bytes < w.bytes) {  // (the static scratch has room for 256 slices of any group)
         fine = false;
         plan = plan_attn(hd, group, n_total, mfma);
         w = carve_attn(workspace, n_units, group, hd, plan.n_splits);
@@ -367,6 +361,7 @@ std::mutex g_scratch_mutex;
 
 }  // namespace
 
+static_assert((size_t)kFineBlocks * kMfmaMaxGroup * (128 + 2) * 4 + 512 <= kStaticScratchBytes, "slices of 64 rows fit whenever those of 128 do");
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 extern "C" int dc_gather_attn_bf16(const void *q, const void *k, const void *v, const uint32_t *idx,
@@ -399,7 +394,7 @@ extern "C" int dc_gather_attn_static_bf16(const void *q, const void *k, const vo
     DC_REQUIRE(n_units < (1 << 20), "%s: too many units", who);
     const int64_t n_total = (int64_t)n_idx + n_sink + n_recent + (new_k ? 1 : 0);
     DC_REQUIRE(n_total < (1ll << 31), "%s: too many rows", who);
-    const size_t need = attn_least_bytes((int)n_units, group, hd, (int)n_total);
+    const size_t need = dc_attn_workspace_bytes((int)n_units, group, hd, (int)n_total);
     if (need > kStaticScratchBytes) {
         dc_set_error("%s: %lld units x %lld attended rows (group %d, head_dim %d) need %zu bytes of scratch; "
                      "the static scratch holds %zu (use dc_gather_attn_bf16 with a workspace)",

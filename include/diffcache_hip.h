@@ -192,7 +192,13 @@ int dc_gather_rows_bf16(const void *k, const void *v, const uint32_t *idx, void 
                         int64_t src_row_stride, int64_t dst_batch_stride, int64_t dst_head_stride,
                         int64_t dst_row_stride, void *stream);
 
-/* Bytes of workspace dc_gather_attn_bf16 needs. */
+/*
+ * Bytes of workspace for dc_gather_attn_bf16; those for some sizes are enough for fewer units
+ * or rows.  Short lists of few units are worked on in slices of 64 rows, which take the larger
+ * part of it; with a smaller workspace that has room for slices of 128 the call takes those,
+ * whose sums are rounded in another order (the last bits of out and lse may differ), and with
+ * less still it returns DC_ENOMEM.
+ */
 size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_rows_attended);
 
 /*
@@ -230,7 +236,7 @@ int dc_gather_attn_bf16(const void *q, const void *k, const void *v, const uint3
  * dc_gather_attn_bf16 for callers that cannot allocate device memory or bring a workspace
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc):
  * the same kernels, the same arguments without `workspace`, the same results bit for
- * bit.  The per-split softmax partials live in a static device array of
+ * bit as with a workspace of dc_attn_workspace_bytes.  The per-split softmax partials live in a static device array of
  * DC_ATTN_STATIC_SCRATCH_BYTES inside the library (one copy per GPU, held until the
  * process ends); a call that needs more -- dc_attn_workspace_bytes(n_b*n_h, group, hd,
  * n_idx + n_sink + n_recent + 1) -- returns DC_ENOMEM and launches nothing.  The call
