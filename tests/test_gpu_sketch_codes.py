@@ -78,3 +78,25 @@ def test_infinite_keys_in_a_channel_that_was_zeros_at_the_fit(hd):
         assert np.array_equal(codes[u], c)
         assert np.array_equal(sk.resid.cpu().reshape(2, hd).numpy()[u], np.maximum(r, before[u]))
         assert np.array_equal(sk.scale.cpu().reshape(2, hd).numpy()[u], scale[u])
+
+
+@pytest.mark.parametrize("hd,rows", [(64, 65549), (128, 32801), (256, 16421)])
+def test_codes_of_long_stores(hd, rows):
+    """Beyond 2 ** 24 key elements blocks take 32 KB of keys (256, 128, 64 rows): ragged last blocks, a key that is no number in a
+    late one and in the last, element by element against numpy."""
+    from diffcache_amd import _hip as hip
+    units = 4
+    assert units * rows * hd >= 1 << 24
+    g = torch.Generator().manual_seed(rows)
+    k = torch.randn((2, 2, rows, hd), generator=g)
+    k[0, 1, rows - 130, 9] = float("nan")
+    k[1, 0, rows - 1, 2] = float("-inf")
+    k = k.to(torch.bfloat16)
+    sk = hip.Sketch(k.to(DEV)).build(k.to(DEV), 0, rows)
+    codes = sk.codes.cpu().reshape(units, -1, hd)[:, :rows].numpy()
+    scale, resid = (t.cpu().reshape(units, hd).numpy() for t in (sk.scale, sk.resid))
+    for u in range(units):
+        c, s, r = _want(k.float().reshape(units, rows, hd)[u].numpy())
+        assert np.array_equal(codes[u], c)
+        assert np.array_equal(scale[u], s)
+        assert np.array_equal(resid[u], r)
