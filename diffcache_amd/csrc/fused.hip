@@ -137,8 +137,8 @@ constexpr uint32_t kNoRow = 0xffffffffu;  // in the place of a row's key: there 
 __host__ __device__ __forceinline__ int64_t dense_key_stride(int n_cap) { return ((int64_t)n_cap + 3) & ~3ll; }
 
 // DENSE: for scans of more than 768 rows a unit and up to 1.75 Mi in all (plan_dense_keys), as in the sketch scan below:
-// every row's 32-bit key goes to the row's own place, nothing is polled, staged or listed, and blocks of equal shares all
-// run at once.  Its loads come in halves of a step (quarters at 256 columns), two of them in flight, the first two ahead of the query; a
+// every row's 32-bit key goes to the row's own place, nothing is polled, staged or listed, and blocks take equal shares; a CU
+// runs four at a time, above 1 Mi rows some start late (plan_dense_keys).  Its loads come in halves of a step (quarters at 256 columns), two of them in flight, the first two ahead of the query; a
 // step's sixteen at a time, behind the query and behind the step before them: per layer, us, 32 units x 49933 rows of 128 95.2 / 93.4, 4 x
 // 127028 44.8 / 43.1, 16 x 65404 of 64 44.5 / 43.6, 64 x 16432 71.8 / 71.1, 8 x 131004 67.5 / 67.9.
 template <int HD, bool DENSE>
@@ -1531,7 +1531,7 @@ int plan_fused(const char *who, int n_b, int n_h, int n_rows, int budget, FusedP
 constexpr int64_t kDenseMostTiles = (4ll << 20) / kRowsPerBlockStep, kDenseFewTiles = (5ll << 19) / kRowsPerBlockStep;
 
 // The grid of a dense scan of at least one unit and one tile: `most` blocks at the very most (one per unit where there are more
-// units), so that none starts when the others end.  (Shares worked out from all tiles together gave a few blocks more where the
+// units), which is as many as run at a time, so that none starts when the others end, but for the largest bf16 scans.  (Shares worked out from all tiles together gave a few blocks more where the
 // tiles of a unit did not divide: 24 units x 65000 rows of 256 columns 106 against 94 us, 56 x 30011 of 128 68.1 against 65.5.)
 void plan_shares(int64_t n_units, int64_t tiles, int64_t most, FusedPlan *p) {
     const int64_t each = most > n_units ? most / n_units : 1, steps = (tiles + each - 1) / each;
@@ -1568,9 +1568,12 @@ int dense_per_thread(int64_t n_units, int n_rows) {
 // 166.2, 32 x 131004 204.1 / 208.3.  Up to 768 rows the listed scan's few blocks are the shorter chain (96 x 304 of 64 13.0 / 13.7).
 //
 // Its grid, selections alone, us: up to 640 tiles of 256 rows a block each (24 x 5424 of 128: 264 blocks of two tiles 19.7, 528
-// of one 18.3); then 512 blocks, 1024 from 64 units on (64 x 16000 of 128 59.0 / 56.5, listed 55.1).  Above 1 Mi rows, where
-// every share is long, 1280 blocks (a CU holds four; 1024: 95.5 us instead of 93.2 a layer of 32 x 49933 rows of 128) up to 32 units and 128 columns (16 x 100003 of 64 48.7 / 45.7, listed
-// 47.5), and at 256 columns from 9 to 64 units one per CU (32 x 50000 144.5 / 139.5, listed 139.0).
+// of one 18.3); then 512 blocks, 1024 from 64 units on (64 x 16000 of 128 59.0 / 56.5, listed 55.1).  (768 instead of 512, per layer: 8 x 131004 of
+// 128 67.1 -> 63.8, but 16 x 39932 48.5 -> 50.3, 4 x 199932 53.3 -> 55.2, 8 x 44932 35.6 -> 36.9, 8 x 99932 of 64 36.7 -> 38.3: no line between
+// them is known.)  Above 1 Mi rows, where every share is long, 1280 blocks up to 32 units and 128 columns: a CU holds four, but the shorter
+// shares outweigh the late start of some (per layer, 1024 / 1280: 32 x 49933 of 128 93.9 / 91.9, 16 x 99932 89.7 / 87.9; 16 x 100003 of 64
+// 56.3 / 55.2, 32 x 49933 59.3 / 58.0, 8 x 199932 54.7 / 53.7); at 256 columns from 9 to 64 units one per CU (32 x 50000 144.5 / 139.5,
+// listed 139.0).
 constexpr int64_t kDenseKeyTiles = (7ll << 18) / kRowsPerBlockStep;  // 1.75 Mi rows
 constexpr int kDenseKeyRows = 768;
 

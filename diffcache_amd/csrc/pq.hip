@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kThreads) void pq_adc_kernel(
 //
 // A CU holds one block, which stages the tables of its subspaces once and walks the keys; its waves take batches of 64 from a
 // counter in LDS and meet at no barrier.  200003 keys of 128 columns, 32 subspaces: 68 us (275 instructions per wave and subspace,
-// 192 of them the search, the vector ALUs issuing 94 % of the time that a CU is busy).  Blocks of 256 keys that stage for themselves took 75
+// 192 of them the search, the vector ALUs issuing 95 % of the time that a CU is busy).  Blocks of 256 keys that stage for themselves took 75
 // (347 instructions); walking with equal shares per wave 74, because the older waves of a SIMD run ahead and the youngest ends
 // alone; two blocks of half the size per CU 69, one of which runs ahead; a tile's products asked for when the tile before has been searched
 // 66 to 68, 87 % of the time issuing; the last batches dealt out by subspace 69; the octets' numbers as masks in scalar registers, 20
@@ -158,8 +158,8 @@ static bool plan_encode(int m, int subs, int64_t n, EncGrid *g) {
     return true;
 }
 
-// (At least two waves per SIMD asked for: with up to 256 registers the compiler leaves the results of the
-// matrix instructions in vector registers; with more it moves each through an accumulation register,
+// (A CU's one block is four waves to a SIMD, of up to 128 registers, two of up to 256 at 16 columns: within 256 the compiler leaves the
+// results of the matrix instructions in vector registers; with more it moves each through an accumulation register,
 // one instruction per value, which is what the search costs.)
 template <int DS>
 __global__ __launch_bounds__(enc_threads(DS), enc_threads(DS) / 256) void pq_encode_kernel(
