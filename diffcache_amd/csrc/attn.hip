@@ -231,7 +231,7 @@ extern "C" size_t dc_attn_workspace_bytes(int n_units, int group, int hd, int n_
     // And for slices of 64 rows, which a list of up to so many rows takes where there is room: those of this call or, so that a workspace
     // for more units or rows is enough for fewer, of any smaller one.
     if (hd > 128) return least;
-    const int64_t slices = n_units * (n_rows_attended > 0 ? ((int64_t)n_rows_attended + 63) / 64 : 1);
+    const int64_t each = n_rows_attended > 0 ? ((int64_t)n_rows_attended + 63) / 64 : 1, slices = n_units * (each < kFineSlices ? each : kFineSlices);
     const size_t fine = carve_attn(nullptr, 1, group, hd, slices < kFineBlocks ? (int)slices : kFineBlocks).bytes;
     return least > fine ? least : fine;
 }

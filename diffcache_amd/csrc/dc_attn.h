@@ -29,9 +29,13 @@ struct AttnPlan {
 // Slices of 64 rows instead of 128 (up to 128 columns) where that leaves no more of them than CUs: a CU takes some 45 KB of rows in a
 // microsecond.  Rows of a unit's list up to which that holds.  Per layer, us, 128 / 64 rows: 8 units x 1093 rows of 128
 // columns 28.5 / 27.9 (144 blocks), 8 x 581 43.6 / 43.0, 2 x 1093 29.3 / 28.7, 8 x 1093 of 64 30.2 / 29.7; but 16 x 1093 44.7 / 45.2 (288), 32 x 581
-// 67.7 / 68.3, 8 x 2117 46.6 / 46.9 (272).
-constexpr int kFineBlocks = 256;
-inline int attn_fine_rows(int n_units) { return kFineBlocks / (n_units > 0 ? n_units : 1) * 64; }
+// 67.7 / 68.3, 8 x 2117 46.6 / 46.9 (272).  And no more than 64 of a unit, which are what the merge takes at once: the attention alone of
+// 1 x 4000 rows of 128 8.3 / 8.1, 4 x 4000 8.6 / 8.2, but 3 x 5000 8.7 / 9.5, 1 x 8000 8.6 / 9.6, 1 x 16000 10.3 / 12.7 (of 64 8.4 / 9.9).
+constexpr int kFineBlocks = 256, kFineSlices = 64;
+inline int attn_fine_rows(int n_units) {
+    const int each = kFineBlocks / (n_units > 0 ? n_units : 1);
+    return (each < kFineSlices ? each : kFineSlices) * 64;
+}
 
 // mfma: the split runs on the matrix cores (dc_attn_split_mfma), whose slice does not depend on the group; fine: of 64 rows at any
 // head_dim
