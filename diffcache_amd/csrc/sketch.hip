@@ -193,8 +193,12 @@ int dc_sketch_quantise_launch(const char *who, const void *k, uint8_t *codes, co
     // Rows per block: 32 KB of keys, so that the blocks that run at a time walk the store together, as the copy that filled it did (longer
     // blocks are each somewhere else); 256 where there are few rows in all and a block's end, an LDS pass and HD atomics to its
     // unit's words, shows.  A prompt's layer, us, 32 KB / 64 KB / 128 KB: 16 units x 40003 rows of 128 columns 151 / 156 / 161, 8 x 131072
-    // 244 / 249 / 258, 12 x 24683 of 256 144 / 145 / 148, 16 x 40003 of 64 87 / 88 / 89; but 2 x 50000 of 128 41 / 39 / 40.
-    const int64_t rpb = (int64_t)n_units * n_rows * hd >= (1ll << 24) ? 16384 / hd : 256;
+    // 244 / 249 / 258, 12 x 24683 of 256 144 / 145 / 148, 16 x 40003 of 64 87 / 88 / 89.  Below four units the atomics to a unit's words, one
+    // behind the other, take longer than the keys: 64 KB for two units, 128 for one.  This pass alone, us: 2 x 131072 28.4 / 23.3 / 22.0, 2 x
+    // 500000 88 / 68 / 73, 2 x 65536 17.0 / 13.9 / 15.8, 1 x 262144 45.9 / 32.3 / 26.5, 1 x 1000000 156 / 92 / 76, 1 x 500000 of 256 156 / 92 /
+    // 76; 4 x 131072 40.7 / 42.7 / 40.0, 3 x 100000 24.4 / 23.6 / 26.1.
+    const int64_t kb32 = 16384 / hd, each = n_units == 1 ? 4 : (n_units == 2 ? 2 : 1);
+    const int64_t rpb = (int64_t)n_units * n_rows * hd >= (1ll << 24) ? kb32 * each : 256;
     const int64_t blocks = ((int64_t)n_rows + rpb - 1) / rpb * n_units;
     DC_REQUIRE(blocks < (1ll << 31), "%s: grid too large", who);
     const dim3 grid((unsigned)blocks);

@@ -100,3 +100,21 @@ def test_codes_of_long_stores(hd, rows):
         assert np.array_equal(codes[u], c)
         assert np.array_equal(scale[u], s)
         assert np.array_equal(resid[u], r)
+
+
+@pytest.mark.parametrize("units,hd,rows", [(1, 64, 262401), (1, 256, 65551), (2, 128, 65665), (3, 128, 43700)])
+def test_codes_of_long_stores_of_few_units(units, hd, rows):
+    """The same with one unit, two (blocks of 128 and 64 KB of keys) and three."""
+    from diffcache_amd import _hip as hip
+    assert units * rows * hd >= 1 << 24
+    g = torch.Generator().manual_seed(rows)
+    k = torch.randn((1, units, rows, hd), generator=g)
+    k[0, units - 1, rows - 500, 9] = float("nan")
+    k = k.to(torch.bfloat16)
+    sk = hip.Sketch(k.to(DEV)).build(k.to(DEV), 0, rows)
+    codes = sk.codes.cpu().reshape(units, -1, hd)[:, :rows].numpy()
+    for u in range(units):
+        c, s, r = _want(k.float()[0, u].numpy())
+        assert np.array_equal(codes[u], c)
+        assert np.array_equal(sk.scale.cpu().reshape(units, hd).numpy()[u], s)
+        assert np.array_equal(sk.resid.cpu().reshape(units, hd).numpy()[u], r)
