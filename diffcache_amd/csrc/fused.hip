@@ -146,10 +146,10 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     const uint16_t *__restrict__ K, const uint16_t *__restrict__ Q, uint32_t *__restrict__ hist,
     UnitState *__restrict__ state, uint2 *__restrict__ surv, int n_units, int n_h, int n_cap,
     int64_t sb, int64_t sh, int64_t sr, int q_group, int mode, int k_eff, int small_chunks,
-    int big_steps, int n_chunks, const int32_t *__restrict__ hi_dev, int lo_row) {
+    int big_steps, int n_chunks, uint32_t apart, const int32_t *__restrict__ hi_dev, int lo_row) {
     if constexpr (DENSE)  // all arguments at once: read where they are first used, they are half a dozen round trips in a row
         asm volatile("" ::"s"(K), "s"(Q), "s"(hist), "s"(surv), "s"(n_units), "s"(n_h), "s"(n_cap), "s"(sb), "s"(sh), "s"(sr), "s"(q_group),
-                     "s"(mode), "s"(big_steps), "s"(n_chunks), "s"(hi_dev), "s"(lo_row));
+                     "s"(mode), "s"(big_steps), "s"(n_chunks), "s"(apart), "s"(hi_dev), "s"(lo_row));
     constexpr int LPR = HD / 8;
     constexpr int CH = LPR < 16 ? LPR : 16;
     __shared__ uint32_t lhist[DC_HIST_BINS];
@@ -171,10 +171,14 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
     // the same address offsets: large chunks of the listed scan by seven a unit; those of the dense scan, of which a grid holds few, so
     // that the units start evenly apart.  (Dense, per layer, us, without / by seven / evenly: 8 units of 131072 rows of 128 columns 74.1 / 65.2 /
     // 64.6, 4 of 262144 71.0 / 69.3 / 65.6, 8 of 65536 of 256 71.1 / 67.1 / 67.0, 4 of 131072 of 256 70.9 / 69.4 / 66.1; 8 of 140128 of 128 69.3 /
-    // - / 70.6.  Not at 64 columns: 8 of 131072 40.7 / 41.9 / 42.0, 32 of 50129 57.9 / - / 60.1; in the dense sketch scan it changes nothing.)
-    const uint32_t chunks = (uint32_t)(n_chunks - (DENSE ? 0 : small_chunks)), at = (uint32_t)(chunk - (DENSE ? 0 : small_chunks));
-    const uint32_t apart = !DENSE ? 7u : (HD == 64 ? 0u : (chunks > gridDim.x ? chunks / gridDim.x : 1u));
-    const int big_id = DENSE && HD == 64 ? chunk : (small ? 0 : (int)((at + (uint32_t)unit * apart) % chunks));
+    // - / 70.1.  Not at 64 columns: 8 of 131072 40.7 / 41.9 / 42.0, 32 of 50129 57.9 / - / 60.1; in the dense sketch scan it changes nothing.)
+    int big_id = chunk;
+    if constexpr (!DENSE) {
+        big_id = small ? 0 : (int)(((uint32_t)(chunk - small_chunks) + (uint32_t)unit * 7u) % (uint32_t)(n_chunks - small_chunks));
+    } else if constexpr (HD > 64) {  // apart: n_chunks / n_units in 1/65536 (without a division here, in front of the first loads)
+        big_id += (int)((uint32_t)unit * apart >> 16);
+        big_id -= big_id < n_chunks ? 0 : n_chunks;
+    }
     const int64_t block_row0 =
         small ? (int64_t)chunk * kRowsPerBlockStep
               : (int64_t)small_chunks * kRowsPerBlockStep + (int64_t)big_id * big_steps * kRowsPerBlockStep;
@@ -237,13 +241,19 @@ __global__ __launch_bounds__(kThreads) void score_prune_kernel(
         };
         const int parts = my_steps * PARTS;
         int i = 0;
-        for (; i + 1 < parts; i += 2) {
+        // From 128 columns on the number of parts is even and the last two are worked on without further loads, which a short block would
+        // wait for at its end (selections of 8 x 17940 rows of 128 19.2 -> 18.5 us; at 64 columns 32 x 49933 take 1 us longer with that).
+        constexpr int kAhead = PARTS > 1 ? 3 : 1;
+        for (; i + kAhead < parts; i += 2) {
             work_part(i, wa);
             load_part(i + 2, wa);
             work_part(i + 1, wb);
             load_part(i + 3, wb);
         }
-        if (i < parts) work_part(i, wa);
+        if (i < parts) {
+            work_part(i, wa);
+            if (PARTS > 1) work_part(i + 1, wb);
+        }
         __syncthreads();
         uint32_t *hu = hist + (int64_t)unit * DC_HIST_BINS;
         for (int i = tid; i < DC_HIST_BINS; i += kThreads) {
@@ -1647,12 +1657,15 @@ int dc_score_prune_launch(const void *k, const void *q, int n_b, int n_h, int n_
     rc = check_ws("dc_score_prune_bf16", workspace, workspace_bytes, p.n_units, n_rows, budget, &w);
     if (rc) return rc;
     const bool dense = plan_dense_keys(p.n_units, n_rows, hd, &p);
+    const int n_chunks = (int)(p.blocks / p.n_units);
+    // (dense: 1280 chunks at most, so that no unit's share of them leaves 32 bits)
+    const uint32_t apart = dense ? ((uint32_t)n_chunks << 16) / (uint32_t)p.n_units : 0u;
     hipStream_t st = (hipStream_t)stream;
 #define DC_LAUNCH_SPD(HD, DN)                                                                      \
-    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dc_unit_grid(p.n_units, p.blocks / p.n_units), dim3(kThreads), 0, st, \
+    hipLaunchKernelGGL((score_prune_kernel<HD, DN>), dc_unit_grid(p.n_units, n_chunks), dim3(kThreads), 0, st, \
                        (const uint16_t *)k, (const uint16_t *)q, w.hist, w.state, w.surv,          \
                        p.n_units, n_h, n_rows, sb, sh, sr, q_group, mode, p.k_eff, p.small_chunks,  \
-                       p.big_steps, (int)(p.blocks / p.n_units), hi_dev, lo_row)
+                       p.big_steps, n_chunks, apart, hi_dev, lo_row)
 #define DC_LAUNCH_SP(HD)                    \
     do {                                    \
         if (dense) DC_LAUNCH_SPD(HD, true); \

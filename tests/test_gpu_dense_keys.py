@@ -93,3 +93,10 @@ def test_every_grid_scans_every_row(hkv, region, hd):
         for u in range(0, hkv, 1 + hkv // 5):
             want, got = orc.topk_select(dense[u].cpu().numpy(), budget, 0), ids[u] if order == hip.ORDER_BEST else np.sort(ids[u])
             assert np.array_equal(got, want if order == hip.ORDER_BEST else np.sort(want)), (order, u)
+
+
+@pytest.mark.parametrize("hkv,region,hd", [(64, 2561, 128), (700, 800, 128), (520, 1500, 256), (100, 5000, 256), (7, 20000, 128), (24, 7000, 128),
+                                           (5, 300001, 128), (63, 9000, 128)])
+def test_rotated_chunks_scan_every_row(hkv, region, hd):
+    """More units than chunks, fewer, numbers that do not divide; blocks of one, two, three and more steps."""
+    test_every_grid_scans_every_row(hkv, region, hd)
