@@ -52,6 +52,11 @@ constexpr int64_t kCopyBlocks = 1280;
 // 404 / 354, 320 x 4000 386 / 423 / 369, 400 x 4096 433 / 459 / 428, 400 x 4000 of 64 233 / 256 / 227, 328 x 2048 196 / 183 / 172; 320 x 4000
 // of 64, just below, 205 / 185 / 193.  (Pieces of 64 rows: 200 x 4000 215 -> 209, 256 x 2000 of 256 columns 250 -> 242; 16 x 40003, below, 154 -> 157.)
 constexpr int64_t kCopyBlocksMany = 6144, kManyUnits = 64, kManyElements = 80ll << 20;
+// Without a sketch, whose pass over the keys is the other half of the time, and beyond 96 Mi key elements of any number of units, more and
+// shorter ones still.  Per layer, us, 8192 / 1280 / 6144 / these: 32 units x 32000 rows of 128 columns 214 / 230 / 221 / 214, 1 x 2000000
+// 402 / 422 / 412 / 395, 8 x 131072 223 / 225 / 223 / 212, 128 x 8000 216 / 229 / 223 / 216, 400 x 2000 of 256 315 / 347 / 322 / 316, 64 x
+// 40000 of 64 281 / 289 / 283 / 280; below the line 64 x 10000 144 / 139 / 135 / 144, 16 x 40003 142 / 135 / 135 / 141.
+constexpr int64_t kCopyBlocksLong = 12288, kLongElements = 96ll << 20;
 
 // One block copies rows_per_block rows of one unit, of V (the first half of the grid) or of K.  A group of HD/8 lanes owns a row, 16 bytes per lane; a lane keeps its eight columns
 // for the whole block, so the column maxima stay in registers.
@@ -200,12 +205,15 @@ extern "C" int dc_prefill_layer_bf16(const dc_prefill_args *a, void *stream) {
                            sketch ? (uint32_t *)a->resid : nullptr, n_sc, p.r_sq, a->n_h);
         DC_CHECK_LAUNCH(who);
     }
-    // Equal shares for kCopyBlocks blocks, 64 rows at least; in long copies of many units more and shorter ones, whole pieces of 64 rows.
-    const bool many = n_units64 > kManyUnits && n_units64 * a->seq * a->hd > kManyElements;
-    int64_t chunks = (many ? kCopyBlocksMany : kCopyBlocks) / (2 * n_units64);
+    // Equal shares for kCopyBlocks blocks, 64 rows at least; in long copies for more of them, whole pieces of 64 rows.
+    const int64_t elements = n_units64 * a->seq * a->hd;
+    int64_t most = kCopyBlocks;
+    if (!sketch && elements > kLongElements) most = kCopyBlocksLong;
+    else if (n_units64 > kManyUnits && elements > kManyElements) most = kCopyBlocksMany;
+    int64_t chunks = most / (2 * n_units64);
     chunks = chunks < 1 ? 1 : chunks;
     int64_t rpb = ((int64_t)a->seq + chunks - 1) / chunks;
-    if (many) rpb = (rpb + 63) / 64 * 64;
+    if (most != kCopyBlocks) rpb = (rpb + 63) / 64 * 64;
     rpb = rpb < 64 ? 64 : rpb;
     const int64_t blocks = ((int64_t)a->seq + rpb - 1) / rpb * n_units64;
     DC_REQUIRE(2 * blocks < (1ll << 31), "%s: grid too large", who);

@@ -121,3 +121,22 @@ def test_a_prefill_under_capture_is_refused():
 ])
 def test_prefills_of_many_units_match_copies_and_sketch_build(hd, b, h, seq, prefix, suffix):
     test_prefill_layer_matches_copies_and_sketch_build(hd, b, h, seq, prefix, suffix)
+
+
+@pytest.mark.parametrize("hd,b,h,seq", [(128, 3, 1, 262145), (64, 37, 8, 5333), (256, 2, 3, 65537)])
+def test_long_prefills_without_a_sketch_match_copies(hd, b, h, seq):
+    """Just beyond 96 Mi key elements: other blocks than with a sketch."""
+    from diffcache_amd import _hip as hip
+    assert 96 << 20 < b * h * seq * hd < 97 << 20
+    g = torch.Generator(device=DEV).manual_seed(seq)
+    k, v = (torch.empty((b, seq, h, hd), device=DEV, dtype=torch.bfloat16).normal_(generator=g) for _ in range(2))
+    ks, vs = (torch.full((b, h, seq + 3, hd), 7.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    kb, vb = (torch.full((b, h, 20, hd), 9.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    r_sq = torch.full((h,), 1e30, device=DEV)
+    hip.prefill_layer(ks, vs, k, v, 4, 9, kb, vb, r_sq=r_sq)
+    for store, src, buf in ((ks, k, kb), (vs, v, vb)):
+        src = src.permute(0, 2, 1, 3)
+        assert torch.equal(store[:, :, :seq], src) and bool((store[:, :, seq:] == 7.0).all())
+        assert torch.equal(buf[:, :, :13], torch.cat([src[:, :, :4], src[:, :, seq - 9:]], dim=2)) and bool((buf[:, :, 13:] == 9.0).all())
+    want = k.double().pow(2).sum(-1).amax(dim=(0, 1))
+    assert bool(((r_sq.double() - want).abs() <= hd * 2.0 ** -24 * want).all())
