@@ -478,8 +478,12 @@ __global__ __launch_bounds__(kThreads, HD <= 128 ? 4 : 1) void sketch_prune_kern
         e = dc_group_sum<LPQ>(e);
         wmax = group_max<LPQ>(wmax);
         margin = dc_sketch_margin(e, wabs, mode);
-        // weights that are not finite leave every approximation undefined: such rows are kept
-        poison = wabs < __builtin_inff() ? 0.f : __uint_as_float(0x7fc00000u);
+        // Weights or a margin that are not finite (an infinite residual; no number where the query is zero there) bound no row: all are kept,
+        // their approximation being no number of positive sign, whose bucket is the best, whatever the margin's sign or an
+        // approximation that overflows would make of their sum.
+        const bool bound = wabs < __builtin_inff() && margin < __builtin_inff();
+        poison = bound ? 0.f : __uint_as_float(0x7fc00000u);
+        margin = bound ? margin : 0.f;
         w_exp = __builtin_amdgcn_frexp_expf(wmax) - 30;
         uint32_t dig[8];
 #pragma unroll

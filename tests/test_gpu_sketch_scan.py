@@ -35,3 +35,26 @@ def test_scan_keeps_the_top_rows(hd, n, k, law):
     for mode in (hip.MODE_IP, hip.MODE_REF_DIST):
         want = hip.topk_select(hip.score(store, q, 1, n, mode), k, mode, hip.ORDER_BEST)
         assert torch.equal(hip.score_select_sketch(store, sk, q, 1, n, k, mode, hip.ORDER_BEST), want)
+
+
+@pytest.mark.parametrize("hd,qg", [(64, 1), (128, 4), (256, 3)])
+@pytest.mark.parametrize("rows", [237, 5003])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_rows_without_a_number_are_selected_as_by_the_bf16_scan(mode, rows, hd, qg):
+    """Infinite and undefined keys leave no bound: every row goes to the exact pass, also one whose approximation overflows, and a
+    selection of all rows names all of them."""
+    from diffcache_amd import _hip as hip
+    g = torch.Generator(device="cuda").manual_seed(rows + hd)
+    h = 6
+    k = torch.randn((1, h, rows, hd), generator=g, device="cuda")
+    for u, bad in enumerate((float("inf"), -float("inf"), float("nan"), 3e38, 1e-39)):
+        k[0, u, torch.randint(0, rows, (20,), generator=g, device="cuda"), torch.randint(0, hd, (20,), generator=g, device="cuda")] = bad
+    k = k.to(torch.bfloat16)
+    q = (2 * torch.randn((h * qg, hd), generator=g, device="cuda")).to(torch.bfloat16)
+    k[0, 5, rows // 2, 7] = float("inf")
+    q[5 * qg:, 7] = 0.0                     # an infinite residual times zero
+    sk = hip.Sketch(k).build(k, 0, rows)
+    for budget in (rows, rows - 3, 200):
+        want = hip.score_select(k, q, 0, rows, budget, mode=mode, order=hip.ORDER_BEST, q_group=qg)
+        got = hip.score_select_sketch(k, sk, q, 0, rows, budget, mode=mode, order=hip.ORDER_BEST, q_group=qg)
+        assert torch.equal(got, want), budget
